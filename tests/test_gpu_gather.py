@@ -1,0 +1,127 @@
+"""GPU: convolutions over channels-last copies (vh_gather.hip) at the edges of
+their tiles, stages and stride phases, against the oracle under the parity gate."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.parity import k_conv_dgrad, k_conv_fwd, k_conv_wgrad
+from tests.test_gpu_parity import DEV, DTYPES, check, host, prep, rng
+from volta_amd import nn as vnn
+
+pytestmark = pytest.mark.gpu
+
+# (B, C, O, H, W, K, S, P): shapes outside the specialised kernels (odd widths, strides)
+CASES = [
+    (1, 3, 5, 3, 1, 3, 1, 1),        # one column, channels below one 16-byte unit
+    (2, 33, 31, 7, 7, 3, 1, 1),      # 31 and 33 rows: one 32-row tile / one row of a second
+    (1, 64, 65, 9, 15, 3, 1, 1),     # 65 rows, 135 positions: one past the tile both ways
+    (3, 130, 129, 9, 9, 3, 2, 1),    # 129 and 130 channels, phases of 4, 2, 2 and 1 taps
+    (2, 8, 200, 5, 5, 1, 2, 0),      # K = 8: less than one stage; phases without taps
+    (2, 20, 12, 6, 7, 5, 3, 2),      # nine phases
+    (2, 7, 9, 10, 3, 2, 4, 0),       # stride 4 past the width, taps missing in most phases
+    (2, 12, 20, 11, 13, 3, 1, 3),    # padding wider than the kernel reaches
+    (64, 9, 80, 33, 31, 3, 1, 1),    # 128-row tiles, channels 9 -> 16 padded
+    (80, 24, 64, 33, 31, 3, 1, 1),   # 64 x 256 tiles
+    (16, 16, 16, 45, 45, 3, 1, 1),   # weight gradient split many ways
+    (2, 72, 136, 5, 7, 3, 1, 1),     # weight gradient split a few ways, channels past 64
+]
+
+
+def _ids(c):
+    return "B{}C{}O{}H{}W{}K{}S{}P{}".format(*c)
+
+
+@pytest.mark.parametrize("case", CASES, ids=_ids)
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_gather_conv_all_passes(case, dt):
+    B, C, O, H, W, K, S, P = case
+    g = rng(sum(case) + 11)
+    x, xt = prep(g.standard_normal((B, C, H, W)), dt)
+    w, wt = prep(g.standard_normal((O, C, K, K)) * np.sqrt(2.0 / (C * K * K)), dt)
+    b, bt = prep(g.uniform(-1, 1, (O,)), dt)
+    conv = vnn.Conv2d(C, O, K, S, P, device=DEV, dtype=DTYPES[dt])
+    conv.weight, conv.bias = wt, bt
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    kw = dict(stride=(S, S), pad=(P, P))
+    y = conv.forward(xt)
+    bb = b[None, :, None, None]
+    check(y, oracle.direct_conv, (x, w), dt, "y", kw, extra_ref=bb, extra_scale=np.abs(bb), k=k_conv_fwd(C, K, K))
+    assert np.array_equal(host(conv.forward(xt, relu=True)), np.maximum(host(y), 0))
+    dy, dyt = prep(g.standard_normal(tuple(y.shape)), dt)
+    kwg = k_conv_wgrad(B, y.shape[2], y.shape[3])
+    dx, dw, db = conv.backward(dyt, xt)  # one call: the copy of dy is shared
+    check(dx, oracle.direct_conv_backward_input, (dy, w, x.shape), dt, "dx", kw, k=k_conv_dgrad(O, K, K))
+    check(dw, oracle.direct_conv_backward_weight, (dy, x, w.shape), dt, "dw", kw, k=kwg)
+    check(db, oracle.conv_bias_grad, (dy,), dt, "db", k=kwg)
+    # each gradient alone, and the input gradient under a ReLU mask
+    assert np.array_equal(host(conv.backward(dyt, xt, weight_grad=False)[0]), host(dx))
+    _, dw1, db1 = conv.backward(dyt, xt, input_grad=False)
+    assert np.array_equal(host(dw1), host(dw)) and np.array_equal(host(db1), host(db))
+    masked = host(conv.backward(dyt, xt, weight_grad=False, relu_input=True)[0])
+    assert np.array_equal(masked, np.where(x > 0, host(dx), 0))
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_gather_padding_does_not_leak(dt):
+    """An infinity reaches the outputs whose window or channel holds it and no
+    other: the channel, position and stage padding is never multiplied with it."""
+    B, C, O, H, W = 2, 5, 7, 9, 11
+    conv = vnn.Conv2d(C, O, 3, 1, 1, device=DEV, dtype=DTYPES[dt])
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    x = torch.ones((B, C, H, W), device=DEV, dtype=DTYPES[dt])
+    dy = torch.ones((B, O, H, W), device=DEV, dtype=DTYPES[dt])
+    x[1, 4, 8, 10] = float("inf")
+    y = np.isfinite(host(conv.forward(x)))
+    assert y[0].all() and y[1, :, :7].all() and y[1, :, :, :9].all() and not y[1, :, 7:, 9:].any()
+    dw = np.isfinite(host(conv.backward(dy, x)[1]))
+    # the corner (8, 10) is under tap rows and columns 1 and 2 only
+    assert dw[:, :4].all() and dw[:, 4, 0].all() and dw[:, 4, :, 0].all() and not dw[:, 4, 1:, 1:].any()
+    x[1, 4, 8, 10] = 1
+    dy[1, 6, 8, 10] = float("inf")
+    dx, dw, db = (np.isfinite(host(t)) for t in conv.backward(dy, x))
+    assert dx[0].all() and dx[1, :, :7].all() and not dx[1, :, 7:, 9:].any()
+    assert dw[:6].all() and db[:6].all() and not db[6]
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_gather_conv_transpose(dt):
+    B, CI, CO, H, W, K, S, P = 3, 24, 20, 7, 5, 4, 2, 1
+    g = rng(5)
+    x, xt = prep(g.standard_normal((B, CI, H, W)), dt)
+    w, wt = prep(g.normal(0, 0.1, (CI, CO, K, K)), dt)
+    b, bt = prep(g.uniform(-1, 1, (CO,)), dt)
+    ct = vnn.ConvTranspose2d(CI, CO, K, S, P, device=DEV, dtype=DTYPES[dt])
+    ct.weight, ct.bias = wt, bt
+    y = ct.forward(xt)
+    kw = dict(stride=(S, S), pad=(P, P))
+    check(y, oracle.conv_transpose_forward, (x, w, b), dt, "y", kw, k=CI * K * K + 1)
+    dy, dyt = prep(g.standard_normal(tuple(y.shape)), dt)
+    got = ct.backward(dyt, xt)
+    ks = (CO * K * K, B * H * W, B * y.shape[2] * y.shape[3])
+    for i, (what, t) in enumerate(zip(("dx", "dw", "db"), got)):
+        check(t, lambda *a, i=i, **k: oracle.conv_transpose_backward(*a, **k)[i], (dy, x, w), dt, what, kw, k=ks[i])
+    assert np.array_equal(host(ct.backward(dyt, xt, weight_grad=False)[0]), host(got[0]))
+
+
+def test_gather_falls_back_without_workspace():
+    """A capture on a stream whose workspace holds what the generic path needs
+    but not the copies is still accepted, and right."""
+    conv = vnn.Conv2d(16, 16, 3, 1, 1, use_bias=False, device=DEV)
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    small, big = torch.randn(1, 16, 31, 31, device=DEV), torch.randn(64, 16, 31, 31, device=DEV)
+    want = conv.forward(big)
+    out = torch.empty_like(want)
+    cap = torch.cuda.Stream()
+    cap.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(cap):
+        conv.forward(small)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=cap):
+        conv.forward(big, out=out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((out - want).abs().max()) <= 2 * 144 * 2.0 ** -24 * float(want.abs().max()) * 16

@@ -164,6 +164,11 @@ static int ws_get(hipStream_t st, size_t bytes, void** out) {
   return VH_OK;
 }
 
+// A request of a path that has another to fall back on: no workspace where the
+// fixed scratch is too small, the stream is being captured and its workspace
+// would have to grow, or the device is out of memory.
+static bool ws_try(hipStream_t st, size_t bytes, void** out) { return bytes > 0 && ws_get(st, bytes, out) == VH_OK; }
+
 // Carves aligned sub-buffers out of one workspace request.
 struct Carve {
   size_t off = 0;
@@ -277,6 +282,14 @@ static ConvGeom geom_of(const ConvDims& d) {
 #define VH_DISPATCH(dtype, FN, ...) \
   ((dtype) == VH_BF16 ? FN<bf16>(__VA_ARGS__) : FN<float>(__VA_ARGS__))
 
+// The channels-last path, where its workspace can be had: true with its status in *r.
+static bool gather_try(int dt, const GatherCall& c, hipStream_t st, int* r) {
+  void* ws;
+  if (!ws_try(st, gather_ws(dt, c), &ws)) return false;
+  *r = gather_run(dt, c, ws, st);
+  return true;
+}
+
 // ------------------------------------------------------------------ conv passes
 // 1x1 kernel, no padding, equal strides >= 2 (the ResNet projection shortcut).
 static bool is_strided_pointwise(const ConvDims& d) {
@@ -299,8 +312,10 @@ static bool is_3x3_s1_p1(const ConvDims& d) {
 }
 
 // act: 1 = ReLU on the output (fused into the epilogue where the kernel has it).
+// defer: a pass that takes the channels-last path is only put down in it (the
+// caller runs it, together with the other passes it put down; the same below).
 static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, void* y, const ConvDims& d,
-                     hipStream_t st, int act = 0) {
+                     hipStream_t st, int act = 0, GatherCall* defer = nullptr) {
   if (dt == VH_BF16 && is_strided_pointwise(d) && g_fast_paths) {
     int r = pw_conv_bf16_fwd(x, w, bias, y, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, (int)d.SH, st);
     if (r != VH_ERR_UNSUPPORTED) return r == VH_OK && act ? relu_after(dt, y, d.B * d.O * d.HO * d.WO, st) : r;
@@ -350,6 +365,20 @@ static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, voi
     int r = halo_conv_bf16(x, w, 0, wt, bias, y, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, (int)d.KH,
                            (int)d.KW, (int)d.PH, (int)d.PW, st, act);
     if (r != VH_ERR_UNSUPPORTED) return r;
+  }
+  if (g_fast_paths) {
+    GatherCall gc{};
+    GatherCall& c = defer ? *defer : gc;
+    c.g = g;
+    c.x = x;
+    c.w = w;
+    c.bias = bias;
+    c.y = y;
+    c.act = act;
+    int r = VH_OK;
+    if (defer || gather_try(dt, gc, st, &r)) return r;
+    VH_TRY(ws_get(st, cv.off, &ws));
+    wt = at(ws, o_w);
   }
   VH_TRY(VH_DISPATCH(dt, run_relayout, w, wt, (int)d.O, (int)d.C, (int)RS, 0, st));
   const int vec = dt == VH_BF16 ? 8 : 4;
@@ -479,7 +508,7 @@ static int dgrad_phases(int dt, const void* dy, const void* w, const void* bias,
 // mask: the layer input, when it came from a ReLU: dx is zeroed where it is not
 // positive (the ReLU backward of the layer below, fused where the kernel has it).
 static int igemm_dgrad(int dt, const void* dy, const void* w, void* dx, const ConvDims& d, hipStream_t st,
-                       const void* mask = nullptr, size_t* need = nullptr) {
+                       const void* mask = nullptr, size_t* need = nullptr, GatherCall* defer = nullptr) {
   ConvGeom g = geom_of(d);
   const long RS = d.KH * d.KW;
   const size_t wbytes = std::max((size_t)d.O * d.C * RS * elem_size(dt),
@@ -534,10 +563,23 @@ static int igemm_dgrad(int dt, const void* dy, const void* w, void* dx, const Co
     int r = pw_conv_bf16_dgrad(dy, w, dx, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, (int)d.SH, st);
     if (r != VH_ERR_UNSUPPORTED) return r == VH_OK && mask ? mask_after(dt, mask, dx, d.B * d.C * d.H * d.W, st) : r;
   }
+  if (g_fast_paths) {
+    GatherCall gc{};
+    GatherCall& c = defer ? *defer : gc;
+    c.g = g;
+    c.dy = dy;
+    c.w = w;
+    c.mask = mask;
+    c.dx = dx;
+    int r = VH_OK;
+    if (defer || gather_try(dt, gc, st, &r)) return r;
+  }
   if ((d.SH > 1 || d.SW > 1) && g_fast_paths) {
     int r = dgrad_phases(dt, dy, w, nullptr, dx, d, st, mask);  // unsupported only beyond 16 phases
     if (r != VH_ERR_UNSUPPORTED) return r;
   }
+  VH_TRY(ws_get(st, cv.off, &ws));
+  wd = at(ws, o_w);
   VH_TRY(VH_DISPATCH(dt, run_relayout, w, wd, (int)d.O, (int)d.C, (int)RS, 1, st, 0));
   const int vec = dt == VH_BF16 ? 8 : 4;
   p.args.a = Operand{wd, (int)(RS * d.O), (int)d.C, ((RS * d.O) % vec) == 0};
@@ -553,7 +595,7 @@ static int igemm_dgrad(int dt, const void* dy, const void* w, void* dx, const Co
 // split-K over output positions: rows = O (A = dY), columns = (kh, kw, c)
 // (B = gather of x), stored OIHW.
 static int igemm_wgrad(int dt, const void* dy, const void* x, void* dw, void* db, bool* db_done,
-                       const ConvDims& d, hipStream_t st, size_t* need = nullptr) {
+                       const ConvDims& d, hipStream_t st, size_t* need = nullptr, GatherCall* defer = nullptr) {
   if (db_done) *db_done = false;
   size_t most = 0;  // sizing mode: the largest request of the paths that run
   if (dt == VH_BF16 && d.SH == 1 && d.SW == 1 && g_fast_paths) {
@@ -607,6 +649,20 @@ static int igemm_wgrad(int dt, const void* dy, const void* x, void* dw, void* db
     }
   }
   ConvGeom g = geom_of(d);
+  if (g_fast_paths && !need) {
+    GatherCall gc{};
+    GatherCall& c = defer ? *defer : gc;
+    c.g = g;
+    c.dy = dy;
+    c.x = x;
+    c.dw = dw;
+    c.db = db;
+    int r = VH_OK;
+    if (defer || gather_try(dt, gc, st, &r)) {
+      if (r == VH_OK && db_done) *db_done = db != nullptr;
+      return r;
+    }
+  }
   const long RS = d.KH * d.KW;
   IgemmPlan p{};
   p.dtype = dt;
@@ -1301,12 +1357,21 @@ static int conv2d_backward_impl(int dtype, int algo, const void* out_grad, const
     if (grad_input || grad_weight) VH_TRY(im2col_bwd(dtype, out_grad, input, weight, grad_input, grad_weight, d, st));
     if (mask) VH_TRY(mask_after(dtype, mask, grad_input, d.B * d.C * d.H * d.W, st));
   } else if (algo == VH_ALGO_IGEMM) {
-    if (grad_input) VH_TRY(igemm_dgrad(dtype, out_grad, weight, grad_input, d, st, mask));
-    if (grad_weight) {
-      bool db_done = false;
-      VH_TRY(igemm_wgrad(dtype, out_grad, input, grad_weight, grad_bias, &db_done, d, st));
-      if (db_done) grad_bias = nullptr;
+    // both gradients on the channels-last path: one call, sharing the copy of out_grad
+    GatherCall gc{};
+    GatherCall* defer = grad_input && grad_weight ? &gc : nullptr;
+    bool db_done = false;
+    if (grad_input) VH_TRY(igemm_dgrad(dtype, out_grad, weight, grad_input, d, st, mask, nullptr, defer));
+    if (grad_weight)
+      VH_TRY(igemm_wgrad(dtype, out_grad, input, grad_weight, grad_bias, &db_done, d, st, nullptr, defer));
+    int r;
+    if (gc.dx && gc.dw && gather_try(dtype, gc, st, &r)) {
+      VH_TRY(r);
+    } else {
+      if (gc.dx) VH_TRY(igemm_dgrad(dtype, out_grad, weight, grad_input, d, st, mask));
+      if (gc.dw) VH_TRY(igemm_wgrad(dtype, out_grad, input, grad_weight, grad_bias, &db_done, d, st));
     }
+    if (db_done) grad_bias = nullptr;
   } else {
     ConvGeom g = geom_of(d);
     if (grad_input) VH_TRY(VH_DISPATCH(dtype, run_direct_dgrad, out_grad, weight, grad_input, g, st));
@@ -1401,6 +1466,16 @@ int vh_conv_transpose2d_forward(int dtype, const void* input, const void* weight
   const ConvGeom gs = geom_of(d);
   if (g_fast_paths && dgrad_smallc_ok(gs))  // at most 4 output channels
     return VH_DISPATCH(dtype, run_dgrad_smallc, input, weight, bias, nullptr, output, gs, st);
+  if (g_fast_paths) {
+    GatherCall gc{};
+    gc.g = gs;
+    gc.dy = input;
+    gc.w = weight;
+    gc.bias = bias;
+    gc.dx = output;
+    int r;
+    if (gather_try(dtype, gc, st, &r)) return r;
+  }
   if ((d.SH > 1 || d.SW > 1) && g_fast_paths) {
     int r = dgrad_phases(dtype, input, weight, bias, output, d, st);
     if (r != VH_ERR_UNSUPPORTED) return r;
@@ -1460,7 +1535,11 @@ int vh_conv_transpose2d_backward(int dtype, const void* out_grad, const void* in
     if (grad_bias) VH_TRY(bias_grad_nchw(dtype, out_grad, grad_bias, d.B, d.C, d.H * d.W, st));
     return VH_OK;
   }
-  if (grad_input) VH_TRY(igemm_fwd(dtype, out_grad, weight, nullptr, grad_input, d, st));
+  // both gradients on the channels-last path: one call, sharing the copy of out_grad
+  GatherCall gc{};
+  GatherCall* defer = grad_input && grad_weight ? &gc : nullptr;
+  if (grad_input) VH_TRY(igemm_fwd(dtype, out_grad, weight, nullptr, grad_input, d, st, 0, defer));
+  bool dw_done = false;
   if (grad_weight && dtype == VH_F32 && g_fast_paths) {
     // up-sampling layer to a few channels: dW (and dB) in one MFMA pass over the positions
     const ConvGeom g = geom_of(d);
@@ -1469,11 +1548,20 @@ int vh_conv_transpose2d_backward(int dtype, const void* out_grad, const void* in
       void* ws;
       VH_TRY(ws_get(st, nb, &ws));
       const int r = convt_cell_wgrad_f32(input, out_grad, grad_weight, grad_bias, g, (float*)ws, nb, st);
-      if (r == VH_OK) return VH_OK;
-      if (r != VH_ERR_UNSUPPORTED) return r;
+      if (r != VH_OK && r != VH_ERR_UNSUPPORTED) return r;
+      dw_done = r == VH_OK;
+      if (dw_done) grad_bias = nullptr;
     }
   }
-  if (grad_weight) VH_TRY(igemm_wgrad(dtype, input, out_grad, grad_weight, nullptr, nullptr, d, st));
+  if (grad_weight && !dw_done)
+    VH_TRY(igemm_wgrad(dtype, input, out_grad, grad_weight, nullptr, nullptr, d, st, nullptr, defer));
+  int r;
+  if (gc.y && gc.dw && gather_try(dtype, gc, st, &r)) {
+    VH_TRY(r);
+  } else {
+    if (gc.y) VH_TRY(igemm_fwd(dtype, out_grad, weight, nullptr, grad_input, d, st));
+    if (gc.dw) VH_TRY(igemm_wgrad(dtype, input, out_grad, grad_weight, nullptr, nullptr, d, st));
+  }
   if (grad_bias) VH_TRY(bias_grad_nchw(dtype, out_grad, grad_bias, d.B, d.C, d.H * d.W, st));
   return VH_OK;
 }

@@ -1,0 +1,1081 @@
+// vh_gather.hip -- convolutions of any geometry as implicit GEMMs over
+// channels-last copies (bf16 and fp32), for gfx950 MFMA.
+//
+// A convolution pass whose shape fits none of the specialised kernels (odd
+// widths, strides, fp32) spends its time on the gather: in NCHW the values an
+// MFMA operand needs -- consecutive channels of one position -- lie a plane
+// apart, so every 16-byte LDS unit takes 4 or 8 scalar loads with their own
+// bounds checks, and the matrix cores wait (measured: 70-90 TFLOP/s bf16, 60-70
+// of 157 fp32).  Here one pass over the tensor (gather_prep_kernel) first writes
+// it as [N][Hp][Wp][Cp]: channels last, padded to whole 16-byte units, with the
+// convolution's zero border in place.  After it
+//  * every operand unit is 16 contiguous, aligned bytes: it goes from global
+//    memory straight into LDS (buffer_load_dwordx4 ... lds), no registers;
+//  * a unit's address is base(position) + offset(tap, channel unit): no bounds
+//    checks, whatever the stride and padding.
+// The copy costs one read and one write of the tensor, 2 of the R*S + 1 times
+// that the product reads it.
+//
+// gather_conv_kernel: D[o][position], forward and (one stride phase at a time,
+// every phase a stride-1 convolution over its own taps) input gradient; weights
+// re-laid out to [m][tap][Cp] by the same prep launch.
+// gather_wgrad_kernel: D[o][(tap, c)] summed over positions: both operands are
+// rows of positions, so the k index is the slow one of both tiles; bf16
+// fragments come from transposing LDS reads (ds_read_b64_tr_b16), fp32 ones from
+// 4-byte reads.  Split over positions, fp32 partials added in a fixed order by
+// gather_wgrad_reduce_kernel.
+#include <type_traits>
+
+#include "vh_kernels.hpp"
+
+namespace vh {
+
+namespace {
+
+typedef unsigned int u32x4g __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2g __attribute__((ext_vector_type(2)));
+
+constexpr int kOORg = (int)0x80000000u;  // buffer offset past every range: loads 0, stores dropped
+constexpr int kMaxPhases = 16;
+constexpr long kMaxBytesG = (1L << 31) - 4096;  // every tensor is addressed with 32-bit byte offsets
+
+template <typename T>
+struct GT {
+  static constexpr int ES = sizeof(typename Elem<T>::storage);
+  static constexpr int UE = 16 / ES;   // elements per 16-byte unit
+  static constexpr int BK = 128 / ES;  // k per stage: 8 units per K-major row
+  using frag = std::conditional_t<ES == 2, bf16x8, float2>;
+  static constexpr int STEPS = ES == 2 ? 4 : 8;  // fragment reads per stage (16 k, or one unit of 4 k)
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_g(const void* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, bytes, 0x00020000);
+}
+
+// s_waitcnt vmcnt(0) lgkmcnt(0), then the block barrier
+__device__ __forceinline__ void gather_sync() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// all MFMAs of one fragment step: independent accumulators back to back
+template <int FM, int FN>
+__device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const bf16x8 (&a)[FM], const bf16x8 (&b)[FN]) {
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], c[i][j], 0, 0, 0);
+}
+// the two k pairs of a 4-k unit: k lanes take k 2t + (lane / 32) in step t
+template <int FM, int FN>
+__device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const float2 (&a)[FM], const float2 (&b)[FN]) {
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].x, b[j].x, c[i][j], 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].y, b[j].y, c[i][j], 0, 0, 0);
+}
+
+// ---------------------------------------------------------------- preparation
+// One tensor copied from [N][C][H][W] to [N][Hp][Wp][Cp] with (padT, padL) zero
+// rows and columns before it (rows and columns past Hp / Wp are dropped).
+struct PackSeg {
+  const void* src;
+  void* dst;
+  int C, H, W, Cp, Hp, Wp, padT, padL;
+  int src_bytes, npos, ncg;  // npos = N*Hp*Wp; channel groups of GROUP channels
+  FastDiv fHpWp, fWp, fcg;
+};
+
+// The weights [O][C][KH][KW] as [phase][m][tap][Kc] (rows padded to whole
+// stages with zeros): transposed = 0: m = o, Kc = channels; 1 (input gradient):
+// m = c, Kc = output channels, taps of the phase in reverse order.
+struct WeightSeg {
+  const void* src;
+  void* dst;
+  int O, C, KH, KW, transposed, CU;
+  int sh, sw, ph, pw;            // input gradient: strides and padding (phase of a tap)
+  int nph;
+  int units, total;              // copied units of all phases; with the row tails
+  FastDiv fRS, fM, fKW;
+  // per phase (a * sw + b): dst offset in units, units per row, taps, tap columns; rows < 0: no such phase
+  int off[kMaxPhases], row_units[kMaxPhases], taps[kMaxPhases], cols[kMaxPhases];
+};
+
+struct PrepArgs {
+  PackSeg p[2];
+  WeightSeg w;
+  int b0, b1, b2;  // blocks of p[0], p[0..1], p[0..1] and w
+};
+
+// A wave copies 64 positions x 64 bytes of channels: a lane loads its position's
+// channels one by one (64 neighbouring positions per load), then the wave's 16-byte
+// units change lanes through LDS so that a store covers 64 contiguous bytes of 16
+// positions (stored by their own lanes they would be 64 scattered 16-byte pieces).
+// Slot of unit u of position l: u ^ ((l >> 2) & 3), conflict-free both ways.
+template <typename T>
+__device__ __forceinline__ void pack_block(const PackSeg& s, int blk, uint4* lds) {
+  using ST = typename Elem<T>::storage;
+  constexpr int ES = GT<T>::ES, UE = GT<T>::UE, GROUP = 64 / ES;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t pt, cg;
+  s.fcg.divmod((uint32_t)(blk * 4 + wave), pt, cg);
+  const int pos = (int)pt * 64 + lane, c0 = (int)cg * GROUP;
+  if ((int)pt * 64 >= s.npos) return;
+  uint32_t n, hw, h, w;
+  s.fHpWp.divmod((uint32_t)min(pos, s.npos - 1), n, hw);
+  s.fWp.divmod(hw, h, w);
+  const int hi = (int)h - s.padT, wi = (int)w - s.padL, HW = s.H * s.W;
+  const bool in = pos < s.npos && (unsigned)hi < (unsigned)s.H && (unsigned)wi < (unsigned)s.W;
+  const int voff = in ? ((int)n * s.C * HW + hi * s.W + wi) * ES : kOORg;
+  const __amdgpu_buffer_rsrc_t r = rsrc_g(s.src, s.src_bytes);
+  ST v[GROUP];
+#pragma unroll
+  for (int j = 0; j < GROUP; ++j) {
+    const int c = c0 + j;
+    if constexpr (ES == 2)
+      v[j] = c < s.C ? __builtin_amdgcn_raw_buffer_load_b16(r, voff, c * HW * ES, 0) : (ST)0;
+    else
+      v[j] = c < s.C ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, c * HW * ES, 0)) : 0.f;
+  }
+  uint4* t = lds + wave * 256;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    uint4 q;
+    __builtin_memcpy(&q, v + u * UE, 16);
+    t[lane * 4 + (u ^ ((lane >> 2) & 3))] = q;
+  }
+  __builtin_amdgcn_wave_barrier();  // a wave's own LDS operations complete in order
+  ST* d = reinterpret_cast<ST*>(s.dst) + c0 + (lane & 3) * UE;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int l = 16 * i + (lane >> 2), q = (int)pt * 64 + l;
+    const uint4 o = t[l * 4 + ((lane & 3) ^ ((l >> 2) & 3))];
+    if (q < s.npos && c0 + (lane & 3) * UE < s.Cp) *reinterpret_cast<uint4*>(d + (size_t)q * s.Cp) = o;
+  }
+}
+
+// One 16-byte unit per thread: (channel unit, m, tap) with the tap fastest, so
+// that a wave's loads run along the stored (channel, tap) index.
+template <typename T>
+__device__ __forceinline__ void weight_block(const WeightSeg& s, int blk) {
+  using ST = typename Elem<T>::storage;
+  constexpr int UE = GT<T>::UE;
+  const int id = blk * 256 + threadIdx.x;
+  if (id >= s.total) return;
+  uint4* dst = reinterpret_cast<uint4*>(s.dst);
+  const int RS = s.KH * s.KW, M = s.transposed ? s.C : s.O, KC = s.transposed ? s.O : s.C;
+  if (id >= s.units) {  // the zero tail of row m of a phase
+    int t = id - s.units;
+    for (int f = 0; f < s.nph; ++f) {
+      const int tail = s.row_units[f] - s.taps[f] * s.CU, cnt = tail * M;
+      if (s.off[f] < 0) continue;
+      if (t < cnt) {
+        const int m = t / tail, u = t - m * tail;
+        dst[(size_t)s.off[f] + (size_t)m * s.row_units[f] + s.taps[f] * s.CU + u] = make_uint4(0, 0, 0, 0);
+        return;
+      }
+      t -= cnt;
+    }
+    return;
+  }
+  uint32_t q, tap, cu, m;
+  s.fRS.divmod((uint32_t)id, q, tap);
+  s.fM.divmod(q, cu, m);
+  const ST* src = reinterpret_cast<const ST*>(s.src);
+  ST v[UE];
+#pragma unroll
+  for (int j = 0; j < UE; ++j) {
+    const int kc = (int)cu * UE + j;
+    const size_t idx = s.transposed ? ((size_t)kc * s.C + m) * RS + tap : ((size_t)m * s.C + kc) * RS + tap;
+    v[j] = kc < KC ? src[idx] : (ST)0;
+  }
+  int f = 0, t = (int)tap;
+  if (s.transposed) {
+    uint32_t kh, kw;
+    s.fKW.divmod(tap, kh, kw);
+    // the phase whose input rows this tap reaches: a = (kh - ph) mod sh
+    const int i = (int)kh / s.sh, j = (int)kw / s.sw;
+    int a = ((int)kh - s.ph) % s.sh, b = ((int)kw - s.pw) % s.sw;
+    a += a < 0 ? s.sh : 0;
+    b += b < 0 ? s.sw : 0;
+    f = a * s.sw + b;
+    if (s.off[f] < 0) return;  // fewer input rows or columns than the stride: no such phase
+    t = s.taps[f] - 1 - (i * s.cols[f] + j);
+  }
+  uint4 o;
+  __builtin_memcpy(&o, v, 16);
+  dst[(size_t)s.off[f] + (size_t)m * s.row_units[f] + t * s.CU + cu] = o;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void gather_prep_kernel(PrepArgs a) {
+  __shared__ uint4 lds[4 * 256];
+  const int b = blockIdx.x;
+  if (b < a.b0)
+    pack_block<T>(a.p[0], b, lds);
+  else if (b < a.b1)
+    pack_block<T>(a.p[1], b - a.b0, lds);
+  else
+    weight_block<T>(a.w, b - a.b1);
+}
+
+// ---------------------------------------------------------------- forward, input gradient
+// One stride phase (the forward pass is a single one): positions (n, i, j) of an
+// Hc x Wc grid, reading x at rows i*sh + r (+ the phase's offset, in off0).
+struct ConvPhase {
+  int w_off, w_bytes;   // weights of the phase: byte offset, size
+  int nst, units;       // stages, channel units of all taps
+  int off0;             // byte offset of tap 0 of position (0, 0)
+  int N, tiles, tile0;  // positions; tiles; first tile of the phase in the grid
+  int sub_a, sub_b;     // output position (osh*i + sub_a, osw*j + sub_b)
+  FastDiv fHW, fW, fS;
+};
+
+struct ConvArgs {
+  const char* w;
+  const void* x;
+  void* y;
+  const void* bias;
+  const void* mask;
+  int M, tiles_m, CU, x_bytes, y_bytes;
+  int img, rowb, colb;   // bytes between images, input rows and columns of x
+  int sh, sw, act;       // act: 0 none, 1 ReLU, 2 zero where mask <= 0
+  int OH, OW, osh, osw;  // output extents and strides
+  int nph, tiles;
+  FastDiv fCU;
+  ConvPhase ph[kMaxPhases];
+};
+
+// Tile BM x BN, four waves of WM x WN, two LDS stages of 128 bytes per row: row r
+// of 8 units, slot t holds k unit t ^ ((r >> 1) & 7), so that a fragment read (16
+// lanes = 16 rows of one unit) is spread over all banks.  Copy instruction c
+// brings rows 8c .. 8c+7; wave w issues c = w, w + 4, ..: their parity is the
+// wave's, which makes a lane's k unit the same in all of them.
+template <typename T, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
+  using ST = typename Elem<T>::storage;
+  using G = GT<T>;
+  using Frag = typename G::frag;
+  constexpr int ES = G::ES, FM = WM / 32, FN = WN / 32, NWN = BN / WN, AC = BM / 32, BC = BN / 32;
+  static_assert((BM / WM) * (BN / WN) == 4, "four waves");
+  __shared__ __attribute__((aligned(16))) u32x4g S0[(BM + BN) * 8];
+  __shared__ __attribute__((aligned(16))) u32x4g S1[(BM + BN) * 8];
+
+  // consecutive tiles on one XCD (the grid is a multiple of 8), m fastest: the
+  // m-tiles of one position tile share its gathered rows in that L2
+  const int lb = xcd_map(blockIdx.x, gridDim.x);
+  if (lb >= g.tiles) return;
+  int f = 0;
+  while (f + 1 < g.nph && lb >= g.ph[f + 1].tile0) ++f;
+  const ConvPhase& p = g.ph[f];
+  const int tl = lb - p.tile0, tn = tl / g.tiles_m;
+  const int m0 = (tl - tn * g.tiles_m) * BM, n0 = tn * BN;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave / NWN) * WM, wn = (wave % NWN) * WN;
+  const int l8 = lane >> 3, ku0 = (lane & 7) ^ ((wave & 1) * 4 + (l8 >> 1));
+
+  int aoff[AC], boff[BC];
+#pragma unroll
+  for (int i = 0; i < AC; ++i) aoff[i] = ((m0 + 8 * (wave + 4 * i) + l8) * p.nst * 8 + ku0) * 16;
+#pragma unroll
+  for (int i = 0; i < BC; ++i) {
+    const int pos = n0 + 8 * (wave + 4 * i) + l8;
+    uint32_t n, hw, h, w;
+    p.fHW.divmod((uint32_t)min(pos, p.N - 1), n, hw);
+    p.fW.divmod(hw, h, w);
+    boff[i] = pos < p.N ? (int)n * g.img + (int)h * g.sh * g.rowb + (int)w * g.sw * g.colb + p.off0 : kOORg;
+  }
+  const __amdgpu_buffer_rsrc_t ar = rsrc_g(g.w + p.w_off, p.w_bytes), br = rsrc_g(g.x, g.x_bytes);
+  auto issue = [&](u32x4g* st, int s) {
+    const uint32_t la = lds_byte_addr(st);
+    const int ask = s * 128;
+#pragma unroll
+    for (int i = 0; i < AC; ++i) lds_copy16(ar, aoff[i], ask, la + (wave + 4 * i) * 1024);
+    // this lane's unit of the stage: its tap and channel unit
+    const int ku = s * 8 + ku0;
+    uint32_t tap, cu, r, c;
+    g.fCU.divmod((uint32_t)ku, tap, cu);
+    p.fS.divmod(tap, r, c);
+    const int off = ku < p.units ? (int)r * g.rowb + (int)c * g.colb + (int)cu * 16 : kOORg;
+#pragma unroll
+    for (int i = 0; i < BC; ++i) lds_copy16(br, boff[i] + off, 0, la + BM * 128 + (wave + 4 * i) * 1024);
+  };
+
+  const int row_l = lane & 31, half_l = lane >> 5;
+  auto read1 = [&](const char* tile, int row0, int kk) {  // fragment of rows row0 .. +31, step kk
+    const int u = ES == 2 ? 2 * kk + half_l : kk;
+    const char* q = tile + (row0 + row_l) * 128 + (u ^ ((row_l >> 1) & 7)) * 16;
+    const u32x4g v = *reinterpret_cast<const u32x4g*>(q);
+    if constexpr (ES == 2) {
+      return __builtin_bit_cast(bf16x8, v);
+    } else {
+      const uint32_t a = half_l ? v[1] : v[0], b = half_l ? v[3] : v[2];
+      return make_float2(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+    }
+  };
+  struct Frags {
+    Frag a[FM], b[FN];
+  };
+  auto read = [&](const u32x4g* st, int kk, Frags& q) {
+    const char* at = reinterpret_cast<const char*>(st);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) q.a[i] = read1(at, wm + 32 * i, kk);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) q.b[j] = read1(at + BM * 128, wn + 32 * j, kk);
+  };
+  f32x16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+  auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
+
+  // stage s sits in buffer s % 2; fa holds its first step on entry.  The copies
+  // of stage s+1 go into the other buffer, whose stage s-1 every wave finished
+  // reading before the last barrier; the reads of step k+1 are issued ahead of
+  // the MFMAs of step k.
+  Frags fa, fb;
+  const int nst = p.nst;
+  issue(S0, 0);
+  gather_sync();
+  read(S0, 0, fa);
+  auto body = [&](auto BUF, int s) {
+    constexpr int B = decltype(BUF)::value;
+    u32x4g* cur = B == 0 ? S0 : S1;
+    u32x4g* nxt = B == 0 ? S1 : S0;
+    if (s + 1 < nst) issue(nxt, s + 1);
+#pragma unroll
+    for (int kk = 1; kk < G::STEPS; kk += 2) {
+      read(cur, kk, fb);
+      mma(fa);
+      if (kk + 1 < G::STEPS) {
+        read(cur, kk + 1, fa);
+      } else if (s + 1 < nst) {
+        gather_sync();
+        read(nxt, 0, fa);
+      }
+      mma(fb);
+    }
+  };
+  int s = 0;
+  for (; s + 1 < nst; s += 2) {
+    body(std::integral_constant<int, 0>{}, s);
+    body(std::integral_constant<int, 1>{}, s + 1);
+  }
+  if (s < nst) body(std::integral_constant<int, 0>{}, s);
+
+  // epilogue: (+ bias), ReLU or mask, one rounding; lanes walk positions
+  const __amdgpu_buffer_rsrc_t yr = rsrc_g(g.y, g.y_bytes);
+  const int plane = g.OH * g.OW * ES;
+  int voff[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int pos = n0 + wn + 32 * j + row_l;
+    uint32_t n, hw, h, w;
+    p.fHW.divmod((uint32_t)min(pos, p.N - 1), n, hw);
+    p.fW.divmod(hw, h, w);
+    voff[j] = pos < p.N ? (int)n * g.M * plane + (((int)h * g.osh + p.sub_a) * g.OW + (int)w * g.osw + p.sub_b) * ES +
+                              half_l * 4 * plane
+                        : kOORg;
+  }
+  auto row_of = [&](int i, int v) { return m0 + wm + 32 * i + (v >> 2) * 8 + (v & 3); };  // + 4 * half_l
+  uint32_t keep[FM][FN];  // bit v: mask > 0; read before the first store
+  if (g.act == 2) {
+    const __amdgpu_buffer_rsrc_t mr = rsrc_g(g.mask, g.y_bytes);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        keep[i][j] = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int row = row_of(i, v), o = row + 4 * half_l < g.M ? voff[j] : kOORg;
+          float m;
+          if constexpr (ES == 2)
+            m = bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(mr, o, row * plane, 0));
+          else
+            m = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mr, o, row * plane, 0));
+          keep[i][j] |= (m > 0.f ? 1u : 0u) << v;
+        }
+      }
+  }
+  const ST* bias = reinterpret_cast<const ST*>(g.bias);
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int row = row_of(i, v);
+      const bool ok = row + 4 * half_l < g.M;
+      const float bv = bias && ok ? Elem<T>::to_f32(bias[row + 4 * half_l]) : 0.f;
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        float r = acc[i][j][v] + bv;
+        if (g.act == 1) r = fmaxf(r, 0.f);
+        if (g.act == 2 && !((keep[i][j] >> v) & 1)) r = 0.f;
+        const int o = ok ? voff[j] : kOORg;
+        if constexpr (ES == 2)
+          __builtin_amdgcn_raw_buffer_store_b16(Elem<T>::from_f32(r), yr, o, row * plane, 0);
+        else
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), yr, o, row * plane, 0);
+      }
+    }
+}
+
+// ---------------------------------------------------------------- weight gradient
+struct WgradArgs {
+  const void* dy;  // [N][..][..][Op] (base already at position (0, 0, 0))
+  const void* x;   // [N][Hp][Wp][Cp]
+  float* part;     // [split][O][RS * Cp]
+  float* dbpart;   // [split][O] or nullptr
+  int O, NC, K;    // rows, columns (RS * Cp), positions
+  int tiles_m, tiles_n, per;  // stages per split
+  int dy_bytes, x_bytes;
+  int dimg, drow, dcol;       // bytes between images, rows and columns of dy
+  int ximg, xrow, xcol;       // the same of x, per output row / column (strides applied)
+  int trow, tcol;             // bytes between tap rows and columns
+  int cs_shift;               // bias gradient: 4 << cs_shift columns of o per block
+  FastDiv fPQ, fQ, fCU, fS;
+};
+
+// Operand tile of BK k rows (positions) x R columns: UR units per k row, copy
+// instruction c brings k rows (64 / UR) c ..; slot t of k row kr holds unit
+// t ^ swz(kr), which spreads a fragment's reads over the banks.
+template <typename T, int R>
+struct MnTile {
+  static constexpr int ES = GT<T>::ES, UR = R * ES / 16, RPI = 64 / UR, INSTR = GT<T>::BK / RPI, CPW = INSTR / 4;
+  __device__ static int swz(int kr) {
+    if (ES == 4) return 8 * (kr & 1);
+    return UR == 8 ? 4 * ((kr >> 1) & 1) : 4 * (kr & 3);
+  }
+};
+
+template <typename T, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
+  using G = GT<T>;
+  using Frag = typename G::frag;
+  using TA = MnTile<T, BM>;
+  using TB = MnTile<T, BN>;
+  constexpr int ES = G::ES, UE = G::UE, BK = G::BK, FM = WM / 32, FN = WN / 32, NWN = BN / WN;
+  constexpr int A_UNITS = BK * TA::UR, B_UNITS = BK * TB::UR;
+  static_assert((BM / WM) * (BN / WN) == 4 && TA::CPW >= 1 && TB::CPW >= 1, "tile");
+  __shared__ __attribute__((aligned(16))) u32x4g S0[A_UNITS + B_UNITS];
+  __shared__ __attribute__((aligned(16))) u32x4g S1[A_UNITS + B_UNITS];
+
+  // the tiles of one split share its positions: consecutive on one XCD
+  const int nt = g.tiles_m * g.tiles_n;
+  const int lb = xcd_map(blockIdx.x, gridDim.x);
+  const int z = lb / nt, tl = lb - z * nt;
+  const int kb = z * g.per * BK, ke = min(g.K, kb + g.per * BK);
+  if (kb >= ke) return;
+  const int tm = tl % g.tiles_m, m0 = tm * BM, tn = tl / g.tiles_m, n0 = tn * BN;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave / NWN) * WM, wn = (wave % NWN) * WN;
+
+  // this lane's k row of copy instruction wave + 4 i, and its column unit
+  const int akr = TA::RPI * wave + lane / TA::UR, bkr = TB::RPI * wave + lane / TB::UR;
+  const int au = m0 / UE + ((lane % TA::UR) ^ TA::swz(akr)), bu = n0 / UE + ((lane % TB::UR) ^ TB::swz(bkr));
+  const int acol = au * 16 < g.dcol ? au * 16 : kOORg;  // dcol = bytes of a dy position
+  uint32_t tap, cu, r, c;
+  g.fCU.divmod((uint32_t)bu, tap, cu);
+  g.fS.divmod(tap, r, c);
+  const int bcol = bu * UE < g.NC ? (int)r * g.trow + (int)c * g.tcol + (int)cu * 16 : kOORg;
+  const __amdgpu_buffer_rsrc_t ar = rsrc_g(g.dy, g.dy_bytes), br = rsrc_g(g.x, g.x_bytes);
+  auto issue = [&](u32x4g* st, int k0) {
+    const uint32_t la = lds_byte_addr(st);
+    auto place = [&](int k, int img, int row, int col) {
+      uint32_t n, pq, p, q;
+      g.fPQ.divmod((uint32_t)min(k, g.K - 1), n, pq);
+      g.fQ.divmod(pq, p, q);
+      return k < ke ? (int)n * img + (int)p * row + (int)q * col : kOORg;
+    };
+#pragma unroll
+    for (int i = 0; i < TA::CPW; ++i)
+      lds_copy16(ar, place(k0 + akr + 4 * TA::RPI * i, g.dimg, g.drow, g.dcol) + acol, 0, la + (wave + 4 * i) * 1024);
+#pragma unroll
+    for (int i = 0; i < TB::CPW; ++i)
+      lds_copy16(br, place(k0 + bkr + 4 * TB::RPI * i, g.ximg, g.xrow, g.xcol) + bcol, 0,
+                 la + A_UNITS * 16 + (wave + 4 * i) * 1024);
+  };
+
+  const int row_l = lane & 31, half_l = lane >> 5;
+  typedef short v4i16 __attribute__((ext_vector_type(4)));
+  typedef short v8i16 __attribute__((ext_vector_type(8)));
+  auto read1 = [&](auto TILE, const char* tile, int col0, int kk) {  // fragment of columns col0 .. +31
+    using Tl = decltype(TILE);
+    if constexpr (ES == 2) {
+      // transposing reads: k rows 16 kk + 8 half_l + (lane & 15) / 4 and + 4
+      const int kr = 8 * half_l + ((lane & 15) >> 2);
+      const int in = (2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * 16 + 8 * (lane & 1);
+      const __attribute__((address_space(3))) char* q =
+          (const __attribute__((address_space(3))) char*)tile + (16 * kk + kr) * Tl::UR * 16 + in +
+          ((col0 >> 3) ^ Tl::swz(kr)) * 16;
+      const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)q);
+      const v4i16 hi =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(q + 4 * Tl::UR * 16));
+      const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      return __builtin_bit_cast(bf16x8, v);
+    } else {
+      const int col = col0 + row_l, u = (col >> 2) ^ (8 * half_l);  // k rows 4 kk + half_l and + 2
+      const char* q = tile + ((4 * kk + half_l) * Tl::UR + u) * 16 + (col & 3) * 4;
+      return make_float2(*reinterpret_cast<const float*>(q), *reinterpret_cast<const float*>(q + 2 * Tl::UR * 16));
+    }
+  };
+  struct Frags {
+    Frag a[FM], b[FN];
+  };
+  auto read = [&](const u32x4g* st, int kk, Frags& q) {
+    const char* at = reinterpret_cast<const char*>(st);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) q.a[i] = read1(TA{}, at, wm + 32 * i, kk);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) q.b[j] = read1(TB{}, at + A_UNITS * 16, wn + 32 * j, kk);
+  };
+  f32x16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+  auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
+
+  // bias gradient: the blocks of one m-tile share its BM columns of o; each sums
+  // 4 << cs_shift of them from the staged tiles, a thread 4 columns of every
+  // (256 / ng)-th k row
+  const int cs_w = 4 << g.cs_shift, cs_c0 = tn * cs_w, ng = cs_w >> 2;
+  const bool cs_blk = g.dbpart != nullptr && cs_c0 < BM;
+  const int cs_c = cs_c0 + 4 * (tid & (ng - 1)), cs_k0 = tid >> g.cs_shift;
+  float csum[4] = {0.f, 0.f, 0.f, 0.f};
+  auto colsum = [&](const u32x4g* st) {
+    const char* at = reinterpret_cast<const char*>(st);
+    for (int kr = cs_k0; kr < BK; kr += 256 >> g.cs_shift) {
+      const char* q = at + (kr * TA::UR + ((cs_c / UE) ^ TA::swz(kr))) * 16 + (cs_c % UE) * ES;
+      if constexpr (ES == 2) {
+        const u32x2g v = *reinterpret_cast<const u32x2g*>(q);
+        csum[0] += __builtin_bit_cast(float, v[0] << 16);
+        csum[1] += __builtin_bit_cast(float, v[0] & 0xffff0000u);
+        csum[2] += __builtin_bit_cast(float, v[1] << 16);
+        csum[3] += __builtin_bit_cast(float, v[1] & 0xffff0000u);
+      } else {
+        const float4 v = *reinterpret_cast<const float4*>(q);
+        csum[0] += v.x;
+        csum[1] += v.y;
+        csum[2] += v.z;
+        csum[3] += v.w;
+      }
+    }
+  };
+
+  Frags fa, fb;
+  const int nst = (ke - kb + BK - 1) / BK;
+  issue(S0, kb);
+  gather_sync();
+  read(S0, 0, fa);
+  auto body = [&](auto BUF, int s) {
+    constexpr int B = decltype(BUF)::value;
+    u32x4g* cur = B == 0 ? S0 : S1;
+    u32x4g* nxt = B == 0 ? S1 : S0;
+    if (s + 1 < nst) issue(nxt, kb + (s + 1) * BK);
+    if (cs_blk) colsum(cur);
+#pragma unroll
+    for (int kk = 1; kk < G::STEPS; kk += 2) {
+      read(cur, kk, fb);
+      mma(fa);
+      if (kk + 1 < G::STEPS) {
+        read(cur, kk + 1, fa);
+      } else if (s + 1 < nst) {
+        gather_sync();
+        read(nxt, 0, fa);
+      }
+      mma(fb);
+    }
+  };
+  int s = 0;
+  for (; s + 1 < nst; s += 2) {
+    body(std::integral_constant<int, 0>{}, s);
+    body(std::integral_constant<int, 1>{}, s + 1);
+  }
+  if (s < nst) body(std::integral_constant<int, 0>{}, s);
+
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int row = m0 + wm + 32 * i + (v >> 2) * 8 + half_l * 4 + (v & 3);
+      if (row < g.O) {
+        float* d = g.part + ((size_t)z * g.O + row) * g.NC;
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          const int col = n0 + wn + 32 * j + row_l;
+          if (col < g.NC) d[col] = acc[i][j][v];
+        }
+      }
+    }
+  if (cs_blk) {  // the k-row group sums, added in group order
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(S0);  // [256 / ng][cs_w]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[cs_k0 * cs_w + cs_c - cs_c0 + e] = csum[e];
+    __syncthreads();
+    const int o = m0 + cs_c0 + tid;
+    if (tid < cs_w && cs_c0 + tid < BM && o < g.O) {
+      float t = 0.f;
+      for (int j = 0; j < 256 >> g.cs_shift; ++j) t += red[j * cs_w + tid];
+      g.dbpart[(size_t)z * g.O + o] = t;
+    }
+  }
+}
+
+// dW[o][c][tap] and db[o] from the splits' partials [split][o][tap][Cp], added in
+// a fixed order.  Few splits: block (o, 64 channels), in split order, through LDS
+// so that the store is contiguous.
+template <typename T>
+__global__ __launch_bounds__(256) void gather_wgrad_reduce_kernel(const float* __restrict__ part,
+                                                                  const float* __restrict__ dbpart, void* dw, void* db,
+                                                                  int O, int C, int Cp, int RS, int splits) {
+  using ST = typename Elem<T>::storage;
+  extern __shared__ float tile[];  // [RS][65]
+  const int o = blockIdx.x, c0 = blockIdx.y * 64, nc = min(64, C - c0);
+  const size_t NC = (size_t)RS * Cp, slab = NC * O;
+  for (int i = threadIdx.x; i < RS * 64; i += 256) {
+    const int rs = i >> 6, cl = i & 63;
+    float t = 0.f;
+    if (cl < nc) {
+      const float* q = part + (size_t)o * NC + (size_t)rs * Cp + c0 + cl;
+#pragma unroll 8
+      for (int z = 0; z < splits; ++z) t += q[z * slab];
+    }
+    tile[rs * 65 + cl] = t;
+  }
+  __syncthreads();
+  ST* d = reinterpret_cast<ST*>(dw) + ((size_t)o * C + c0) * RS;
+  for (int i = threadIdx.x; i < nc * RS; i += 256) {
+    const int cl = i / RS, rs = i - cl * RS;
+    d[i] = Elem<T>::from_f32(tile[rs * 65 + cl]);
+  }
+  if (db && blockIdx.y == 0 && threadIdx.x == 0) {
+    float t = 0.f;
+    for (int z = 0; z < splits; ++z) t += dbpart[(size_t)z * O + o];
+    reinterpret_cast<ST*>(db)[o] = Elem<T>::from_f32(t);
+  }
+}
+
+// Many splits of few weights: float4 quads of one (o, tap), the splits dealt to
+// 2^lg_g groups of threads (blocks nb .. take the bias gradient).
+template <typename T>
+__global__ __launch_bounds__(256) void gather_wgrad_reduce_vec4_kernel(const float* __restrict__ part,
+                                                                       const float* __restrict__ dbpart, void* dw,
+                                                                       void* db, int O, int C, FastDiv fCp, FastDiv fRS,
+                                                                       int splits, int lg_g, int nb) {
+  using ST = typename Elem<T>::storage;
+  if ((int)blockIdx.x >= nb) {
+    reduce_splits_block(dbpart, splits, O, [&](long i, float v) { reinterpret_cast<ST*>(db)[i] = Elem<T>::from_f32(v); },
+                        (int)blockIdx.x - nb, (int)gridDim.x - nb);
+    return;
+  }
+  const int RS = (int)fRS.d;
+  reduce_splits_vec4_block(
+      part, splits, (long)O * RS * fCp.d, lg_g,
+      [&](long i, float v) {
+        uint32_t ot, c, o, tap;
+        fCp.divmod((uint32_t)i, ot, c);
+        fRS.divmod(ot, o, tap);
+        if ((int)c < C) reinterpret_cast<ST*>(dw)[((size_t)o * C + c) * RS + tap] = Elem<T>::from_f32(v);
+      },
+      (int)blockIdx.x, nb);
+}
+
+// ---------------------------------------------------------------- host side
+int round_up(long v, int m) { return (int)((v + m - 1) / m * m); }
+size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
+
+template <typename T>
+long pack_bytes(int N, int Hp, int Wp, int Cp) {
+  return (long)N * Hp * Wp * Cp * GT<T>::ES;
+}
+
+template <typename T>
+PackSeg pack_seg(const void* src, void* dst, int N, int C, int H, int W, int Cp, int Hp, int Wp, int padT, int padL) {
+  constexpr int GROUP = 64 / GT<T>::ES;
+  PackSeg s{};
+  s.src = src;
+  s.dst = dst;
+  s.C = C;
+  s.H = H;
+  s.W = W;
+  s.Cp = Cp;
+  s.Hp = Hp;
+  s.Wp = Wp;
+  s.padT = padT;
+  s.padL = padL;
+  s.src_bytes = (int)((long)N * C * H * W * GT<T>::ES);
+  s.npos = N * Hp * Wp;
+  s.ncg = (Cp + GROUP - 1) / GROUP;
+  s.fHpWp = FastDiv((uint32_t)(Hp * Wp));
+  s.fWp = FastDiv((uint32_t)Wp);
+  s.fcg = FastDiv((uint32_t)s.ncg);
+  return s;
+}
+
+int pack_blocks(const PackSeg& s) { return (int)(((long)(s.npos + 63) / 64 * s.ncg + 3) / 4); }
+
+template <typename T>
+int launch_prep(PrepArgs& a, int npack, bool weights, hipStream_t st) {
+  a.b0 = npack > 0 ? pack_blocks(a.p[0]) : 0;
+  a.b1 = a.b0 + (npack > 1 ? pack_blocks(a.p[1]) : 0);
+  a.b2 = a.b1 + (weights ? (a.w.total + 255) / 256 : 0);
+  gather_prep_kernel<T><<<dim3((unsigned)a.b2), 256, 0, st>>>(a);
+  VH_LAUNCH_CHECK();
+  return VH_OK;
+}
+
+template <typename T, int BM, int BN, int WM, int WN>
+int launch_conv_tile(ConvArgs& a, hipStream_t st) {
+  a.tiles_m = (a.M + BM - 1) / BM;
+  a.tiles = 0;
+  for (int f = 0; f < a.nph; ++f) {
+    a.ph[f].tile0 = a.tiles;
+    a.ph[f].tiles = a.tiles_m * ((a.ph[f].N + BN - 1) / BN);
+    a.tiles += a.ph[f].tiles;
+  }
+  gather_conv_kernel<T, BM, BN, WM, WN><<<dim3((unsigned)((a.tiles + 7) / 8 * 8)), 256, 0, st>>>(a);
+  VH_LAUNCH_CHECK();
+  return VH_OK;
+}
+
+template <typename T>
+int launch_conv(ConvArgs& a, hipStream_t st) {
+  long n = 0;
+  for (int f = 0; f < a.nph; ++f) n += a.ph[f].N;
+  auto grid = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((n + bn - 1) / bn); };
+  // rows computed with 128- and 64-row tiles: the wider tile reads the gathered
+  // rows half as often, so it may waste a little
+  const long w128 = round_up(a.M, 128), w64 = round_up(a.M, 64);
+  if (a.M > 64 && w128 * 7 <= w64 * 8 && grid(128, 128) >= 256) return launch_conv_tile<T, 128, 128, 64, 64>(a, st);
+  if (a.M <= 32) return launch_conv_tile<T, 32, 128, 32, 32>(a, st);
+  if (grid(64, 256) >= 256) return launch_conv_tile<T, 64, 256, 64, 64>(a, st);
+  return launch_conv_tile<T, 64, 128, 32, 64>(a, st);
+}
+
+struct Geo {
+  int Cp, Op, Hp, Wp;              // x copy: channels, padded extents
+  int Pp, Qp, dT, dL;              // dy copy: padded extents, zero rows and columns before it
+};
+
+template <typename T>
+bool make_geo(const ConvGeom& g, Geo& o) {
+  constexpr int UE = GT<T>::UE;
+  o.Cp = round_up(g.C, UE);
+  o.Op = round_up(g.O, UE);
+  o.Hp = (g.P - 1) * g.sh + g.R;
+  o.Wp = (g.Q - 1) * g.sw + g.S;
+  // dy rows that the input-gradient phases reach: i + (a + ph) / sh - t
+  int lo_h = 0, hi_h = g.P - 1, lo_w = 0, hi_w = g.Q - 1;
+  auto reach = [](int in, int s, int p, int k, int& lo, int& hi) {
+    for (int a = 0; a < s && a < in; ++a) {
+      const int k0 = (a + p) % s, taps = k0 < k ? (k - k0 + s - 1) / s : 0;
+      if (!taps) continue;
+      const int off = (a + p - k0) / s, n = (in - a + s - 1) / s;
+      lo = std::min(lo, off - (taps - 1));
+      hi = std::max(hi, off + n - 1);
+    }
+  };
+  reach(g.H, g.sh, g.ph, g.R, lo_h, hi_h);
+  reach(g.W, g.sw, g.pw, g.S, lo_w, hi_w);
+  o.dT = -lo_h;
+  o.dL = -lo_w;
+  o.Pp = hi_h - lo_h + 1;
+  o.Qp = hi_w - lo_w + 1;
+  const long ES = GT<T>::ES;
+  for (long b : {(long)g.N * g.C * g.H * g.W * ES, (long)g.N * g.O * g.P * g.Q * ES, (long)g.N * o.Hp * o.Wp * o.Cp * ES,
+                 (long)g.N * o.Pp * o.Qp * o.Op * ES, (long)(g.O + 128) * (g.R * g.S + 1) * (o.Cp + 64) * ES,
+                 (long)(g.C + 128) * (g.R * g.S + 1) * (o.Op + 64) * ES})
+    if (b > kMaxBytesG) return false;
+  return true;
+}
+
+// Phases of the input gradient with taps, in (a, b) order.
+struct DPhase {
+  int a, b, Hc, Wc, Rc, Sc, offa, offb;
+};
+int dgrad_phase_list(const ConvGeom& g, DPhase* ph) {
+  int n = 0;
+  for (int a = 0; a < g.sh; ++a)
+    for (int b = 0; b < g.sw; ++b) {
+      DPhase& f = ph[n++];
+      f.a = a;
+      f.b = b;
+      f.Hc = a < g.H ? (g.H - a + g.sh - 1) / g.sh : 0;
+      f.Wc = b < g.W ? (g.W - b + g.sw - 1) / g.sw : 0;
+      const int kh0 = (a + g.ph) % g.sh, kw0 = (b + g.pw) % g.sw;
+      f.Rc = kh0 < g.R ? (g.R - kh0 + g.sh - 1) / g.sh : 0;
+      f.Sc = kw0 < g.S ? (g.S - kw0 + g.sw - 1) / g.sw : 0;
+      f.offa = (a + g.ph - kh0) / g.sh;
+      f.offb = (b + g.pw - kw0) / g.sw;
+    }
+  return n;
+}
+
+struct WgradPlan {
+  int BM, BN, splits, per;
+};
+
+template <typename T>
+WgradPlan wgrad_plan(const ConvGeom& g, const Geo& o) {
+  constexpr int BK = GT<T>::BK;
+  WgradPlan p;
+  const int NC = g.R * g.S * o.Cp;
+  const long K = (long)g.N * g.P * g.Q;
+  const bool wide = g.O > 64 && round_up(g.O, 128) * 7 <= round_up(g.O, 64) * 8;
+  p.BM = wide ? 128 : 64;
+  p.BN = 128;
+  const long tiles = (long)((g.O + p.BM - 1) / p.BM) * ((NC + p.BN - 1) / p.BN);
+  const long stages = (K + BK - 1) / BK;
+  // two blocks per CU; at least 4 stages each, since a split costs a write and
+  // a read of its partial tile
+  long want = std::max<long>(1, 512 / tiles);
+  want = std::min(want, std::max<long>(1, stages / 4));
+  p.per = (int)((stages + want - 1) / want);
+  p.splits = (int)((stages + p.per - 1) / p.per);
+  return p;
+}
+
+// Workspace of a call: the copies of x and dy, the weights, the partials.
+struct Layout {
+  size_t x = 0, dy = 0, w = 0, part = 0, bytes = 0;
+};
+
+template <typename T>
+bool make_layout(const GatherCall& c, const Geo& o, Layout& l) {
+  const ConvGeom& g = c.g;
+  constexpr int UE = GT<T>::UE;
+  auto take = [&](size_t b) {
+    const size_t at = l.bytes;
+    l.bytes += align256(b);
+    return at;
+  };
+  if (c.y || c.dw) l.x = take((size_t)pack_bytes<T>(g.N, o.Hp, o.Wp, o.Cp));
+  if (c.dx) l.dy = take((size_t)pack_bytes<T>(g.N, o.Pp, o.Qp, o.Op));
+  else if (c.dw) l.dy = take((size_t)pack_bytes<T>(g.N, g.P, g.Q, o.Op));
+  if (c.y) l.w = take((size_t)g.O * ((g.R * g.S * o.Cp / UE + 7) / 8) * 128);
+  if (c.dx) {
+    if (c.y || g.sh * g.sw > kMaxPhases) return false;
+    DPhase ph[kMaxPhases];
+    const int n = dgrad_phase_list(g, ph);
+    size_t wu = 1;
+    for (int f = 0; f < n; ++f) wu += (size_t)g.C * ((ph[f].Rc * ph[f].Sc * (o.Op / UE) + 7) / 8) * 8;
+    l.w = take(wu * 16);
+  }
+  if (c.dw) l.part = take((size_t)wgrad_plan<T>(g, o).splits * g.O * (g.R * g.S * o.Cp + 1) * sizeof(float));
+  return true;
+}
+
+template <typename T>
+void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, char* ws, const Layout& l) {
+  constexpr int ES = GT<T>::ES, UE = GT<T>::UE;
+  const ConvGeom& g = c.g;
+  const int RS = g.R * g.S;
+  s.src = c.w;
+  s.dst = ws + l.w;
+  s.O = g.O;
+  s.C = g.C;
+  s.KH = g.R;
+  s.KW = g.S;
+  s.fRS = FastDiv((uint32_t)RS);
+  s.fKW = FastDiv((uint32_t)g.S);
+  a.w = ws + l.w;
+  a.bias = c.bias;
+  if (c.y) {
+    const int CU = o.Cp / UE, units = RS * CU, nst = (units + 7) / 8;
+    s.CU = CU;
+    s.sh = s.sw = s.nph = 1;
+    s.units = g.O * units;
+    s.total = g.O * nst * 8;
+    s.row_units[0] = nst * 8;
+    s.taps[0] = RS;
+    s.cols[0] = g.S;
+    s.fM = FastDiv((uint32_t)g.O);
+    a.x = ws + l.x;
+    a.y = c.y;
+    a.M = g.O;
+    a.CU = CU;
+    a.x_bytes = (int)pack_bytes<T>(g.N, o.Hp, o.Wp, o.Cp);
+    a.y_bytes = (int)((long)g.N * g.O * g.P * g.Q * ES);
+    a.colb = o.Cp * ES;
+    a.rowb = o.Wp * a.colb;
+    a.img = o.Hp * a.rowb;
+    a.sh = g.sh;
+    a.sw = g.sw;
+    a.act = c.act;
+    a.OH = g.P;
+    a.OW = g.Q;
+    a.osh = a.osw = 1;
+    a.nph = 1;
+    a.fCU = FastDiv((uint32_t)CU);
+    ConvPhase& p = a.ph[0];
+    p.w_bytes = g.O * nst * 128;
+    p.nst = nst;
+    p.units = units;
+    p.N = g.N * g.P * g.Q;
+    p.fHW = FastDiv((uint32_t)(g.P * g.Q));
+    p.fW = FastDiv((uint32_t)g.Q);
+    p.fS = FastDiv((uint32_t)g.S);
+    return;
+  }
+  const int CU = o.Op / UE;
+  DPhase ph[kMaxPhases];
+  const int n = dgrad_phase_list(g, ph);
+  s.transposed = 1;
+  s.CU = CU;
+  s.sh = g.sh;
+  s.sw = g.sw;
+  s.ph = g.ph;
+  s.pw = g.pw;
+  s.nph = n;
+  s.units = g.C * RS * CU;
+  s.fM = FastDiv((uint32_t)g.C);
+  a.x = ws + l.dy;
+  a.y = c.dx;
+  a.mask = c.mask;
+  a.act = c.mask ? 2 : 0;
+  a.M = g.C;
+  a.CU = CU;
+  a.x_bytes = (int)pack_bytes<T>(g.N, o.Pp, o.Qp, o.Op);
+  a.y_bytes = (int)((long)g.N * g.C * g.H * g.W * ES);
+  a.colb = o.Op * ES;
+  a.rowb = o.Qp * a.colb;
+  a.img = o.Pp * a.rowb;
+  a.sh = a.sw = 1;
+  a.OH = g.H;
+  a.OW = g.W;
+  a.osh = g.sh;
+  a.osw = g.sw;
+  a.fCU = FastDiv((uint32_t)CU);
+  int off = 0, tails = 0;
+  for (int f = 0; f < n; ++f) {
+    const DPhase& q = ph[f];
+    const int taps = q.Rc * q.Sc, units = taps * CU, nst = (units + 7) / 8;
+    const bool live = q.Hc > 0 && q.Wc > 0;
+    s.off[f] = live ? off : -1;
+    s.row_units[f] = nst * 8;
+    s.taps[f] = taps;
+    s.cols[f] = std::max(1, q.Sc);
+    if (!live) continue;
+    tails += g.C * (nst * 8 - units);
+    ConvPhase& p = a.ph[a.nph++];
+    p.w_off = off * 16;
+    p.w_bytes = g.C * nst * 128;
+    p.nst = nst;
+    p.units = units;
+    p.off0 = (q.offa - (q.Rc - 1) + o.dT) * a.rowb + (q.offb - (q.Sc - 1) + o.dL) * a.colb;
+    p.N = g.N * q.Hc * q.Wc;
+    p.sub_a = q.a;
+    p.sub_b = q.b;
+    p.fHW = FastDiv((uint32_t)(q.Hc * q.Wc));
+    p.fW = FastDiv((uint32_t)q.Wc);
+    p.fS = FastDiv((uint32_t)std::max(1, q.Sc));
+    off += g.C * nst * 8;
+  }
+  s.total = s.units + tails;
+  // the phases with most taps first: the short ones fill the last wave
+  std::stable_sort(a.ph, a.ph + a.nph, [](const ConvPhase& p, const ConvPhase& q) { return p.nst > q.nst; });
+}
+
+template <typename T>
+int run_wgrad(const GatherCall& c, const Geo& o, char* ws, const Layout& l, hipStream_t st) {
+  constexpr int ES = GT<T>::ES, UE = GT<T>::UE;
+  const ConvGeom& g = c.g;
+  const WgradPlan p = wgrad_plan<T>(g, o);
+  // the copy of dy has the input gradient's border when both are computed
+  const int Pd = c.dx ? o.Pp : g.P, Qd = c.dx ? o.Qp : g.Q, dT = c.dx ? o.dT : 0, dL = c.dx ? o.dL : 0;
+  WgradArgs a{};
+  a.dcol = o.Op * ES;
+  a.drow = Qd * a.dcol;
+  a.dimg = Pd * a.drow;
+  const long skip = (long)dT * a.drow + (long)dL * a.dcol;
+  a.dy = ws + l.dy + skip;
+  a.dy_bytes = (int)(pack_bytes<T>(g.N, Pd, Qd, o.Op) - skip);
+  a.x = ws + l.x;
+  a.x_bytes = (int)pack_bytes<T>(g.N, o.Hp, o.Wp, o.Cp);
+  a.O = g.O;
+  a.NC = g.R * g.S * o.Cp;
+  a.K = g.N * g.P * g.Q;
+  a.part = reinterpret_cast<float*>(ws + l.part);
+  a.dbpart = c.db ? a.part + (size_t)p.splits * g.O * a.NC : nullptr;
+  a.tiles_m = (g.O + p.BM - 1) / p.BM;
+  a.tiles_n = (a.NC + p.BN - 1) / p.BN;
+  a.per = p.per;
+  a.tcol = o.Cp * ES;
+  a.trow = o.Wp * a.tcol;
+  a.xcol = g.sw * a.tcol;
+  a.xrow = g.sh * a.trow;
+  a.ximg = o.Hp * a.trow;
+  a.cs_shift = colsum_shift(a.tiles_n, p.BM);
+  a.fPQ = FastDiv((uint32_t)(g.P * g.Q));
+  a.fQ = FastDiv((uint32_t)g.Q);
+  a.fCU = FastDiv((uint32_t)(o.Cp / UE));
+  a.fS = FastDiv((uint32_t)g.S);
+  const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * p.splits));
+  if (p.BM == 128)
+    gather_wgrad_kernel<T, 128, 128, 64, 64><<<grid, 256, 0, st>>>(a);
+  else
+    gather_wgrad_kernel<T, 64, 128, 32, 64><<<grid, 256, 0, st>>>(a);
+  VH_LAUNCH_CHECK();
+  const int RS = g.R * g.S;
+  if (p.splits > 8) {
+    const int lg = reduce_vec4_lg_groups(p.splits), nb = reduce_vec4_grid((long)g.O * a.NC, lg);
+    const int ndb = c.db ? reduce_splits_grid(g.O) : 0;
+    gather_wgrad_reduce_vec4_kernel<T><<<dim3((unsigned)(nb + ndb)), 256, 0, st>>>(
+        a.part, a.dbpart, c.dw, c.db, g.O, g.C, FastDiv((uint32_t)o.Cp), FastDiv((uint32_t)RS), p.splits, lg, nb);
+  } else {
+    gather_wgrad_reduce_kernel<T><<<dim3((unsigned)g.O, (unsigned)((g.C + 63) / 64)), 256, (size_t)RS * 65 * sizeof(float),
+                                    st>>>(a.part, a.dbpart, c.dw, c.db, g.O, g.C, o.Cp, RS, p.splits);
+  }
+  VH_LAUNCH_CHECK();
+  return VH_OK;
+}
+
+template <typename T>
+size_t call_ws(const GatherCall& c) {
+  Geo o;
+  Layout l;
+  // more than 64 taps: beyond the reduction's LDS tile
+  if (c.g.N <= 0 || c.g.R * c.g.S > 64 || !make_geo<T>(c.g, o) || !make_layout<T>(c, o, l)) return 0;
+  return l.bytes;
+}
+
+template <typename T>
+int run_call(const GatherCall& c, char* ws, hipStream_t st) {
+  Geo o;
+  Layout l;
+  if (!make_geo<T>(c.g, o) || !make_layout<T>(c, o, l)) return VH_ERR_UNSUPPORTED;
+  const ConvGeom& g = c.g;
+  PrepArgs pa{};
+  ConvArgs a{};
+  int np = 0;
+  if (c.y || c.dw) pa.p[np++] = pack_seg<T>(c.x, ws + l.x, g.N, g.C, g.H, g.W, o.Cp, o.Hp, o.Wp, g.ph, g.pw);
+  if (c.dx)
+    pa.p[np++] = pack_seg<T>(c.dy, ws + l.dy, g.N, g.O, g.P, g.Q, o.Op, o.Pp, o.Qp, o.dT, o.dL);
+  else if (c.dw)
+    pa.p[np++] = pack_seg<T>(c.dy, ws + l.dy, g.N, g.O, g.P, g.Q, o.Op, g.P, g.Q, 0, 0);
+  if (c.y || c.dx) conv_args<T>(a, pa.w, c, o, ws, l);
+  int r = launch_prep<T>(pa, np, c.y || c.dx, st);
+  if (r == VH_OK && (c.y || c.dx)) r = launch_conv<T>(a, st);
+  if (r == VH_OK && c.dw) r = run_wgrad<T>(c, o, ws, l, st);
+  return r;
+}
+
+}  // namespace
+
+size_t gather_ws(int dt, const GatherCall& c) { return dt == VH_BF16 ? call_ws<bf16>(c) : call_ws<float>(c); }
+
+int gather_run(int dt, const GatherCall& c, void* ws, hipStream_t st) {
+  return dt == VH_BF16 ? run_call<bf16>(c, static_cast<char*>(ws), st) : run_call<float>(c, static_cast<char*>(ws), st);
+}
+
+}  // namespace vh

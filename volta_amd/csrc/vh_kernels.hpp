@@ -166,6 +166,22 @@ size_t halo_wgrad3x3_f32_ws(const void* dy, const void* x, int N, int C, int H, 
 int halo_wgrad3x3_f32(const void* dy, const void* x, void* dw, void* db, int N, int C, int H, int W, int O,
                       float* ws, size_t ws_bytes, hipStream_t st);
 
+// ---- convolutions of any geometry over channels-last copies (vh_gather.hip) ----
+// One call computes any of: y (forward; act 0 none, 1 ReLU) or dx (input
+// gradient, 0 where mask, laid out like dx, is not positive) -- with an optional
+// bias per output channel -- and dw with an optional db.  Null outputs are
+// skipped; y and dx do not go together.
+struct GatherCall {
+  ConvGeom g;
+  const void *x, *dy, *w, *bias, *mask;
+  void *y, *dx, *dw, *db;
+  int act;
+};
+// Workspace bytes; 0: unsupported (a tensor beyond 32-bit byte offsets, more than
+// 64 taps, more than 16 stride phases).
+size_t gather_ws(int dt, const GatherCall& c);
+int gather_run(int dt, const GatherCall& c, void* ws, hipStream_t st);
+
 // ---- dense bf16 products (vh_dense.hip) ----
 // C[M][N] = A . B (+ bias[N] per column), bf16 in and out.  A is stored
 // [M][lda] (K contiguous) or, with at, [K][lda] (M contiguous); B is stored
