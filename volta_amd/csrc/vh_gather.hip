@@ -44,8 +44,8 @@ struct GT {
   static constexpr int ES = sizeof(typename Elem<T>::storage);
   static constexpr int UE = 16 / ES;   // elements per 16-byte unit
   static constexpr int BK = 128 / ES;  // k per stage: 8 units per K-major row
-  using frag = std::conditional_t<ES == 2, bf16x8, float2>;
-  static constexpr int STEPS = ES == 2 ? 4 : 8;  // fragment reads per stage (16 k, or one unit of 4 k)
+  // K-major fragment of one step (2 units): 8 bf16, or 4 fp32 = 4 MFMAs of 2 k
+  using frag = std::conditional_t<ES == 2, bf16x8, f32x4>;
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_g(const void* p, int bytes) {
@@ -65,17 +65,14 @@ __device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const bf16x8 (&a)[F
 #pragma unroll
     for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], c[i][j], 0, 0, 0);
 }
-// the two k pairs of a 4-k unit: k lanes take k 2t + (lane / 32) in step t
 template <int FM, int FN>
-__device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const float2 (&a)[FM], const float2 (&b)[FN]) {
+__device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const f32x4 (&a)[FM], const f32x4 (&b)[FN]) {
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].x, b[j].x, c[i][j], 0, 0, 0);
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].y, b[j].y, c[i][j], 0, 0, 0);
+      for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][t], b[j][t], c[i][j], 0, 0, 0);
 }
 
 // ---------------------------------------------------------------- preparation
@@ -89,9 +86,14 @@ struct PackSeg {
   FastDiv fHpWp, fWp, fcg;
 };
 
-// The weights [O][C][KH][KW] as [phase][m][tap][Kc] (rows padded to whole
-// stages with zeros): transposed = 0: m = o, Kc = channels; 1 (input gradient):
-// m = c, Kc = output channels, taps of the phase in reverse order.
+// The weights [O][C][KH][KW] as rows [phase][m] of 16-byte channel units, padded
+// to whole stages with zeros: transposed = 0: m = o, units of channels; 1 (input
+// gradient): m = c, units of output channels, taps of the phase in reverse order.
+// Order of the product's k index (units): chunks of 8 channel units, in each the
+// taps, so that a stage is one tap of one chunk and the R*S stages that read the
+// same values of the other operand follow each other (its lines stay in L1 / L2;
+// tap-major, 9 passes over all channels, ran at L2-miss rate: 3x3 384->128 @32
+// bf16 72 us); the last chunk holds the CU % 8 units left.
 struct WeightSeg {
   const void* src;
   void* dst;
@@ -207,7 +209,9 @@ __device__ __forceinline__ void weight_block(const WeightSeg& s, int blk) {
   }
   uint4 o;
   __builtin_memcpy(&o, v, 16);
-  dst[(size_t)s.off[f] + (size_t)m * s.row_units[f] + t * s.CU + cu] = o;
+  const int full = s.CU & ~7, c = (int)cu;
+  const int ku = c < full ? (c & ~7) * s.taps[f] + t * 8 + (c & 7) : full * s.taps[f] + t * (s.CU - full) + c - full;
+  dst[(size_t)s.off[f] + (size_t)m * s.row_units[f] + ku] = o;
 }
 
 template <typename T>
@@ -227,11 +231,11 @@ __global__ __launch_bounds__(256) void gather_prep_kernel(PrepArgs a) {
 // Hc x Wc grid, reading x at rows i*sh + r (+ the phase's offset, in off0).
 struct ConvPhase {
   int w_off, w_bytes;   // weights of the phase: byte offset, size
-  int nst, units;       // stages, channel units of all taps
+  int nst, units, full; // stages, channel units of all taps, those of whole chunks
   int off0;             // byte offset of tap 0 of position (0, 0)
-  int N, tiles, tile0;  // positions; tiles; first tile of the phase in the grid
+  int N;                // positions
   int sub_a, sub_b;     // output position (osh*i + sub_a, osw*j + sub_b)
-  FastDiv fHW, fW, fS;
+  FastDiv fHW, fW, fT, fS;  // by positions per image and row, taps, tap columns
 };
 
 struct ConvArgs {
@@ -240,89 +244,105 @@ struct ConvArgs {
   void* y;
   const void* bias;
   const void* mask;
-  int M, tiles_m, CU, x_bytes, y_bytes;
+  int M, tiles_m, full, x_bytes, y_bytes;  // full: channel units in whole chunks of 8
   int img, rowb, colb;   // bytes between images, input rows and columns of x
   int sh, sw, act;       // act: 0 none, 1 ReLU, 2 zero where mask <= 0
   int OH, OW, osh, osw;  // output extents and strides
   int nph, tiles;
-  FastDiv fCU;
+  FastDiv ftail;         // by the channel units of the last chunk
   ConvPhase ph[kMaxPhases];
 };
 
 // Tile BM x BN, four waves of WM x WN, two LDS stages of 128 bytes per row: row r
 // of 8 units, slot t holds k unit t ^ ((r >> 1) & 7), so that a fragment read (16
 // lanes = 16 rows of one unit) is spread over all banks.  Copy instruction c
-// brings rows 8c .. 8c+7; wave w issues c = w, w + 4, ..: their parity is the
-// wave's, which makes a lane's k unit the same in all of them.
+// brings rows 8c .. 8c+7, a lane's k unit depends on c's parity.
+// A tile of fewer than four waves' WM x WN is computed by KS groups of waves that
+// take every KS-th stage each (their sums added in group order at the end): for
+// grids of few positions, which larger tiles would leave on a part of the CUs.
 template <typename T, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
   using ST = typename Elem<T>::storage;
   using G = GT<T>;
   using Frag = typename G::frag;
-  constexpr int ES = G::ES, FM = WM / 32, FN = WN / 32, NWN = BN / WN, AC = BM / 32, BC = BN / 32;
-  static_assert((BM / WM) * (BN / WN) == 4, "four waves");
-  __shared__ __attribute__((aligned(16))) u32x4g S0[(BM + BN) * 8];
-  __shared__ __attribute__((aligned(16))) u32x4g S1[(BM + BN) * 8];
+  constexpr int ES = G::ES, FM = WM / 32, FN = WN / 32, NWN = BN / WN;
+  constexpr int WPG = (BM / WM) * (BN / WN), KS = 4 / WPG;  // waves per group, groups
+  constexpr int AC = BM / 8 / WPG, BC = BN / 8 / WPG;       // copy instructions per wave and stage
+  static_assert(WPG * KS == 4, "four waves");
+  __shared__ __attribute__((aligned(16))) u32x4g S0[KS * (BM + BN) * 8];
+  __shared__ __attribute__((aligned(16))) u32x4g S1[KS * (BM + BN) * 8];
 
-  // consecutive tiles on one XCD (the grid is a multiple of 8), m fastest: the
-  // m-tiles of one position tile share its gathered rows in that L2
+  // consecutive tiles on one XCD (the grid is a multiple of 8): the m-tiles of one
+  // position tile share its gathered rows in that L2, and so do its stride phases,
+  // whose interleaved stores meet there again
   const int lb = xcd_map(blockIdx.x, gridDim.x);
   if (lb >= g.tiles) return;
-  int f = 0;
-  while (f + 1 < g.nph && lb >= g.ph[f + 1].tile0) ++f;
-  const ConvPhase& p = g.ph[f];
-  const int tl = lb - p.tile0, tn = tl / g.tiles_m;
-  const int m0 = (tl - tn * g.tiles_m) * BM, n0 = tn * BN;
+  const int tn = lb / (g.tiles_m * g.nph), in = lb - tn * g.tiles_m * g.nph;
+  const int f = in / g.tiles_m;
+  const ConvPhase p = g.ph[f];
+  const int m0 = (in - f * g.tiles_m) * BM, n0 = tn * BN;
+  if (n0 >= p.N) return;
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), grp = wv / WPG, wave = wv % WPG;
   const int wm = (wave / NWN) * WM, wn = (wave % NWN) * WN;
-  const int l8 = lane >> 3, ku0 = (lane & 7) ^ ((wave & 1) * 4 + (l8 >> 1));
+  const int l8 = lane >> 3;
+  // k unit in copy instruction wave + WPG i: the parity is the wave's, or i's if WPG = 1
+  auto unit0 = [&](int i) { return (lane & 7) ^ (((WPG == 1 ? i : wave) & 1) * 4 + (l8 >> 1)); };
 
   int aoff[AC], boff[BC];
 #pragma unroll
-  for (int i = 0; i < AC; ++i) aoff[i] = ((m0 + 8 * (wave + 4 * i) + l8) * p.nst * 8 + ku0) * 16;
+  for (int i = 0; i < AC; ++i) aoff[i] = ((m0 + 8 * (wave + WPG * i) + l8) * p.nst * 8 + unit0(i)) * 16;
 #pragma unroll
   for (int i = 0; i < BC; ++i) {
-    const int pos = n0 + 8 * (wave + 4 * i) + l8;
+    const int pos = n0 + 8 * (wave + WPG * i) + l8;
     uint32_t n, hw, h, w;
     p.fHW.divmod((uint32_t)min(pos, p.N - 1), n, hw);
     p.fW.divmod(hw, h, w);
     boff[i] = pos < p.N ? (int)n * g.img + (int)h * g.sh * g.rowb + (int)w * g.sw * g.colb + p.off0 : kOORg;
   }
   const __amdgpu_buffer_rsrc_t ar = rsrc_g(g.w + p.w_off, p.w_bytes), br = rsrc_g(g.x, g.x_bytes);
-  auto issue = [&](u32x4g* st, int s) {
-    const uint32_t la = lds_byte_addr(st);
+  auto issue = [&](u32x4g* st, int sk) {
+    const int s = sk * KS + grp;  // this group's stage
+    const uint32_t la = lds_byte_addr(st) + grp * (BM + BN) * 128;
     const int ask = s * 128;
 #pragma unroll
-    for (int i = 0; i < AC; ++i) lds_copy16(ar, aoff[i], ask, la + (wave + 4 * i) * 1024);
+    for (int i = 0; i < AC; ++i)
+      lds_copy16(ar, KS == 1 || s < p.nst ? aoff[i] : kOORg, ask, la + (wave + WPG * i) * 1024);
     // this lane's unit of the stage: its tap and channel unit
-    const int ku = s * 8 + ku0;
-    uint32_t tap, cu, r, c;
-    g.fCU.divmod((uint32_t)ku, tap, cu);
-    p.fS.divmod(tap, r, c);
-    const int off = ku < p.units ? (int)r * g.rowb + (int)c * g.colb + (int)cu * 16 : kOORg;
+    auto tap_off = [&](int ku0) {
+      const int ku = s * 8 + ku0;
+      uint32_t tap, cu, r, c;
+      if (s * 8 < p.full) {  // a whole chunk: the stage is one tap of it
+        uint32_t chunk;
+        p.fT.divmod((uint32_t)s, chunk, tap);
+        cu = chunk * 8 + ku0;
+      } else {
+        g.ftail.divmod((uint32_t)(ku - p.full), tap, cu);
+        cu += g.full;
+      }
+      p.fS.divmod(tap, r, c);
+      // past the last unit: out of every range (sign bit)
+      return ((int)r * g.rowb + (int)c * g.colb + (int)cu * 16) | ((p.units - 1 - ku) & kOORg);
+    };
+    const int off0 = tap_off(unit0(0)), off1 = WPG == 1 ? tap_off(unit0(1)) : off0;
 #pragma unroll
-    for (int i = 0; i < BC; ++i) lds_copy16(br, boff[i] + off, 0, la + BM * 128 + (wave + 4 * i) * 1024);
+    for (int i = 0; i < BC; ++i)
+      lds_copy16(br, boff[i] + (i & 1 ? off1 : off0), 0, la + BM * 128 + (wave + WPG * i) * 1024);
   };
 
   const int row_l = lane & 31, half_l = lane >> 5;
-  auto read1 = [&](const char* tile, int row0, int kk) {  // fragment of rows row0 .. +31, step kk
-    const int u = ES == 2 ? 2 * kk + half_l : kk;
-    const char* q = tile + (row0 + row_l) * 128 + (u ^ ((row_l >> 1) & 7)) * 16;
-    const u32x4g v = *reinterpret_cast<const u32x4g*>(q);
-    if constexpr (ES == 2) {
-      return __builtin_bit_cast(bf16x8, v);
-    } else {
-      const uint32_t a = half_l ? v[1] : v[0], b = half_l ? v[3] : v[2];
-      return make_float2(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
-    }
+  // fragment of rows row0 .. +31, step kk: the lanes of half h take unit 2 kk + h
+  // (fp32: MFMA t of the step multiplies element t of both units)
+  auto read1 = [&](const char* tile, int row0, int kk) {
+    return __builtin_bit_cast(Frag, *reinterpret_cast<const u32x4g*>(
+                                        tile + (row0 + row_l) * 128 + ((2 * kk + half_l) ^ ((row_l >> 1) & 7)) * 16));
   };
   struct Frags {
     Frag a[FM], b[FN];
   };
   auto read = [&](const u32x4g* st, int kk, Frags& q) {
-    const char* at = reinterpret_cast<const char*>(st);
+    const char* at = reinterpret_cast<const char*>(st) + grp * (BM + BN) * 128;
 #pragma unroll
     for (int i = 0; i < FM; ++i) q.a[i] = read1(at, wm + 32 * i, kk);
 #pragma unroll
@@ -337,10 +357,11 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
 
   // stage s sits in buffer s % 2; fa holds its first step on entry.  The copies
   // of stage s+1 go into the other buffer, whose stage s-1 every wave finished
-  // reading before the last barrier; the reads of step k+1 are issued ahead of
-  // the MFMAs of step k.
+  // reading before the last barrier.  The reads of step k+1 are kept ahead of the
+  // MFMAs of step k (left alone the compiler sinks them to their use, and every
+  // step waits for LDS).
   Frags fa, fb;
-  const int nst = p.nst;
+  const int nst = (p.nst + KS - 1) / KS;
   issue(S0, 0);
   gather_sync();
   read(S0, 0, fa);
@@ -350,16 +371,20 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
     u32x4g* nxt = B == 0 ? S1 : S0;
     if (s + 1 < nst) issue(nxt, s + 1);
 #pragma unroll
-    for (int kk = 1; kk < G::STEPS; kk += 2) {
+    for (int kk = 1; kk < 4; kk += 2) {
       read(cur, kk, fb);
+      __builtin_amdgcn_sched_barrier(0);
       mma(fa);
-      if (kk + 1 < G::STEPS) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (kk + 1 < 4) {
         read(cur, kk + 1, fa);
       } else if (s + 1 < nst) {
         gather_sync();
         read(nxt, 0, fa);
       }
+      __builtin_amdgcn_sched_barrier(0);
       mma(fb);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   int s = 0;
@@ -368,6 +393,33 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
     body(std::integral_constant<int, 1>{}, s + 1);
   }
   if (s < nst) body(std::integral_constant<int, 0>{}, s);
+
+  if constexpr (KS > 1) {  // the groups' sums, added in group order
+    float* red = reinterpret_cast<float*>(S0);
+    constexpr int TILE = FM * FN * 1024;
+    static_assert((KS - 1) * WPG * TILE * 4 <= (int)sizeof(S0), "group sums exceed a stage");
+    __syncthreads();
+    if (grp > 0) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            red[((grp - 1) * WPG + wave) * TILE + ((i * FN + j) * 16 + v) * 64 + lane] = acc[i][j][v];
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int q = 0; q < KS - 1; ++q)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            acc[i][j][v] += red[(q * WPG + wave) * TILE + ((i * FN + j) * 16 + v) * 64 + lane];
+  }
 
   // epilogue: (+ bias), ReLU or mask, one rounding; lanes walk positions
   const __amdgpu_buffer_rsrc_t yr = rsrc_g(g.y, g.y_bytes);
@@ -457,7 +509,6 @@ struct MnTile {
 template <typename T, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   using G = GT<T>;
-  using Frag = typename G::frag;
   using TA = MnTile<T, BM>;
   using TB = MnTile<T, BN>;
   constexpr int ES = G::ES, UE = G::UE, BK = G::BK, FM = WM / 32, FN = WN / 32, NWN = BN / WN;
@@ -507,42 +558,79 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   const int row_l = lane & 31, half_l = lane >> 5;
   typedef short v4i16 __attribute__((ext_vector_type(4)));
   typedef short v8i16 __attribute__((ext_vector_type(8)));
-  auto read1 = [&](auto TILE, const char* tile, int col0, int kk) {  // fragment of columns col0 .. +31
+  // bf16, step of 16 k: fragment f of a wave's columns col0 .. is columns
+  // 32 f + lane % 32, by transposing reads (k rows 8 half + (lane & 15) / 4 and + 4)
+  auto read_tr = [&](auto TILE, const char* tile, int col, int kk) {
     using Tl = decltype(TILE);
-    if constexpr (ES == 2) {
-      // transposing reads: k rows 16 kk + 8 half_l + (lane & 15) / 4 and + 4
-      const int kr = 8 * half_l + ((lane & 15) >> 2);
-      const int in = (2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * 16 + 8 * (lane & 1);
-      const __attribute__((address_space(3))) char* q =
-          (const __attribute__((address_space(3))) char*)tile + (16 * kk + kr) * Tl::UR * 16 + in +
-          ((col0 >> 3) ^ Tl::swz(kr)) * 16;
-      const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)q);
-      const v4i16 hi =
-          __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(q + 4 * Tl::UR * 16));
-      const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      return __builtin_bit_cast(bf16x8, v);
-    } else {
-      const int col = col0 + row_l, u = (col >> 2) ^ (8 * half_l);  // k rows 4 kk + half_l and + 2
-      const char* q = tile + ((4 * kk + half_l) * Tl::UR + u) * 16 + (col & 3) * 4;
-      return make_float2(*reinterpret_cast<const float*>(q), *reinterpret_cast<const float*>(q + 2 * Tl::UR * 16));
+    const int kr = 8 * half_l + ((lane & 15) >> 2);
+    const int in = (2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * 16 + 8 * (lane & 1);
+    const __attribute__((address_space(3))) char* q = (const __attribute__((address_space(3))) char*)tile +
+                                                      (16 * kk + kr) * Tl::UR * 16 + in + ((col >> 3) ^ Tl::swz(kr)) * 16;
+    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)q);
+    const v4i16 hi =
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(q + 4 * Tl::UR * 16));
+    const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(bf16x8, v);
+  };
+  // fp32, step of 8 k (MFMA t: k rows 2 t and 2 t + 1 of it, one per half): with
+  // two fragments per wave they are the even and the odd columns, one 8-byte read
+  auto read_pair = [&](auto TILE, auto F, const char* tile, int col0, int kk, float (&v)[decltype(F)::value][4]) {
+    using Tl = decltype(TILE);
+    constexpr int N = decltype(F)::value;
+    const int col = col0 + N * row_l, u = (col >> 2) ^ (8 * half_l);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const char* q = tile + ((8 * kk + 2 * t + half_l) * Tl::UR + u) * 16 + (col & 3) * 4;
+      if constexpr (N == 2) {
+        const float2 p = *reinterpret_cast<const float2*>(q);
+        v[0][t] = p.x;
+        v[1][t] = p.y;
+      } else {
+        v[0][t] = *reinterpret_cast<const float*>(q);
+      }
     }
   };
-  struct Frags {
-    Frag a[FM], b[FN];
+  static_assert(FM <= 2 && FN <= 2, "fragments per wave");
+  struct FragsB {
+    bf16x8 a[FM], b[FN];
   };
+  struct FragsF {
+    float a[FM][4], b[FN][4];
+  };
+  using Frags = std::conditional_t<ES == 2, FragsB, FragsF>;
   auto read = [&](const u32x4g* st, int kk, Frags& q) {
     const char* at = reinterpret_cast<const char*>(st);
+    const char* bt = at + A_UNITS * 16;
+    if constexpr (ES == 2) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i) q.a[i] = read1(TA{}, at, wm + 32 * i, kk);
+      for (int i = 0; i < FM; ++i) q.a[i] = read_tr(TA{}, at, wm + 32 * i, kk);
 #pragma unroll
-    for (int j = 0; j < FN; ++j) q.b[j] = read1(TB{}, at + A_UNITS * 16, wn + 32 * j, kk);
+      for (int j = 0; j < FN; ++j) q.b[j] = read_tr(TB{}, bt, wn + 32 * j, kk);
+    } else {
+      read_pair(TA{}, std::integral_constant<int, FM>{}, at, wm, kk, q.a);
+      read_pair(TB{}, std::integral_constant<int, FN>{}, bt, wn, kk, q.b);
+    }
   };
+  // row / column of the wave's tile that element e of fragment f stands for
+  auto spread = [&](int F, int f, int e) { return ES == 4 && F == 2 ? 2 * e + f : 32 * f + e; };
   f32x16 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
-  auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
+  auto mma = [&](const Frags& q) {
+    if constexpr (ES == 2) {
+      mma_all<FM, FN>(acc, q.a, q.b);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(q.a[i][t], q.b[j][t], acc[i][j], 0, 0, 0);
+    }
+  };
 
   // bias gradient: the blocks of one m-tile share its BM columns of o; each sums
   // 4 << cs_shift of them from the staged tiles, a thread 4 columns of every
@@ -583,16 +671,20 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
     if (s + 1 < nst) issue(nxt, kb + (s + 1) * BK);
     if (cs_blk) colsum(cur);
 #pragma unroll
-    for (int kk = 1; kk < G::STEPS; kk += 2) {
+    for (int kk = 1; kk < 4; kk += 2) {
       read(cur, kk, fb);
+      __builtin_amdgcn_sched_barrier(0);
       mma(fa);
-      if (kk + 1 < G::STEPS) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (kk + 1 < 4) {
         read(cur, kk + 1, fa);
       } else if (s + 1 < nst) {
         gather_sync();
         read(nxt, 0, fa);
       }
+      __builtin_amdgcn_sched_barrier(0);
       mma(fb);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   int s = 0;
@@ -606,12 +698,12 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const int row = m0 + wm + 32 * i + (v >> 2) * 8 + half_l * 4 + (v & 3);
+      const int row = m0 + wm + spread(FM, i, (v >> 2) * 8 + half_l * 4 + (v & 3));
       if (row < g.O) {
         float* d = g.part + ((size_t)z * g.O + row) * g.NC;
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          const int col = n0 + wn + 32 * j + row_l;
+          const int col = n0 + wn + spread(FN, j, row_l);
           if (col < g.NC) d[col] = acc[i][j][v];
         }
       }
@@ -738,28 +830,46 @@ template <typename T, int BM, int BN, int WM, int WN>
 int launch_conv_tile(ConvArgs& a, hipStream_t st) {
   a.tiles_m = (a.M + BM - 1) / BM;
   a.tiles = 0;
-  for (int f = 0; f < a.nph; ++f) {
-    a.ph[f].tile0 = a.tiles;
-    a.ph[f].tiles = a.tiles_m * ((a.ph[f].N + BN - 1) / BN);
-    a.tiles += a.ph[f].tiles;
-  }
+  for (int f = 0; f < a.nph; ++f) a.tiles = std::max(a.tiles, (a.ph[f].N + BN - 1) / BN);
+  a.tiles *= a.tiles_m * a.nph;
   gather_conv_kernel<T, BM, BN, WM, WN><<<dim3((unsigned)((a.tiles + 7) / 8 * 8)), 256, 0, st>>>(a);
   VH_LAUNCH_CHECK();
   return VH_OK;
 }
 
+// Measured over 26 shapes of each type (3x3, 32 .. 512 channels, 1.5k .. 1M
+// positions): what counts is the number of 64 x 64 tiles, g64.
+//  * below one block per CU the waves split K instead (8 x 11 x 11 positions, 217
+//    -> 224 channels: 47 us with 64 x 64 tiles, 32 with 32 x 64 in two groups, 23
+//    with 32 x 32 in four; the two cross at about 80 tiles);
+//  * fp32 keeps 64 x 64 above that: five blocks a CU cover each other's copies and
+//    stores, and larger tiles gain nothing (64 x 128: 0 .. 3 % slower);
+//  * bf16 products are ten times shorter, so a CU's copies count: 64 x 128 tiles
+//    from four blocks a CU (64 -> 192 @28x29 N=64: 33.2 -> 29.8 us), 128 x 128
+//    where one round of two blocks a CU covers the grid (3x3 s2 64 -> 128 @56: 29.7
+//    -> 28.2), K in two groups of waves for deep products of one to two blocks a CU
+//    (256 @14x15 N=32: 30.6 -> 26.3; shallow ones lose to the extra sum).
 template <typename T>
 int launch_conv(ConvArgs& a, hipStream_t st) {
   long n = 0;
-  for (int f = 0; f < a.nph; ++f) n += a.ph[f].N;
+  int nst = 0;
+  for (int f = 0; f < a.nph; ++f) {
+    n += a.ph[f].N;
+    nst = std::max(nst, a.ph[f].nst);
+  }
   auto grid = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((n + bn - 1) / bn); };
-  // rows computed with 128- and 64-row tiles: the wider tile reads the gathered
-  // rows half as often, so it may waste a little
-  const long w128 = round_up(a.M, 128), w64 = round_up(a.M, 64);
-  if (a.M > 64 && w128 * 7 <= w64 * 8 && grid(128, 128) >= 256) return launch_conv_tile<T, 128, 128, 64, 64>(a, st);
-  if (a.M <= 32) return launch_conv_tile<T, 32, 128, 32, 32>(a, st);
-  if (grid(64, 256) >= 256) return launch_conv_tile<T, 64, 256, 64, 64>(a, st);
-  return launch_conv_tile<T, 64, 128, 32, 64>(a, st);
+  const long g64 = grid(64, 64);
+  if (a.M <= 32 && grid(32, 128) >= 256) return launch_conv_tile<T, 32, 128, 32, 32>(a, st);
+  if (g64 < 80) return launch_conv_tile<T, 32, 32, 32, 32>(a, st);
+  if (g64 < 256) return launch_conv_tile<T, 32, 64, 32, 32>(a, st);
+  if constexpr (GT<T>::ES == 2) {
+    const bool fits128 = a.M > 64 && round_up(a.M, 128) * 7 <= round_up(a.M, 64) * 8;
+    if (fits128 && grid(128, 128) >= 256 && grid(128, 128) <= 512)
+      return launch_conv_tile<T, 128, 128, 64, 64>(a, st);
+    if (g64 >= 1024) return launch_conv_tile<T, 64, 128, 32, 64>(a, st);
+    if (g64 < 512 && nst >= 16) return launch_conv_tile<T, 64, 64, 64, 32>(a, st);
+  }
+  return launch_conv_tile<T, 64, 64, 32, 32>(a, st);
 }
 
 struct Geo {
@@ -822,24 +932,23 @@ int dgrad_phase_list(const ConvGeom& g, DPhase* ph) {
 }
 
 struct WgradPlan {
-  int BM, BN, splits, per;
+  int splits, per;
 };
 
+// 64 x 64 tiles, positions split for about four blocks a CU (measured on 13 shapes
+// of each type against 64 x 128, 128 x 64 and 128 x 128 tiles at one to four blocks
+// a CU: best or within 3 % on all; on few weights the larger tiles' zero padding
+// and partials cost up to 2x).  A split costs a write and a read of its partial
+// tile: at least 4 stages each, 8 once every CU has a block (217 -> 224 channels at
+// 8 x 11 x 11 positions, fp32: 32.2 -> 25 us).
 template <typename T>
 WgradPlan wgrad_plan(const ConvGeom& g, const Geo& o) {
   constexpr int BK = GT<T>::BK;
   WgradPlan p;
-  const int NC = g.R * g.S * o.Cp;
-  const long K = (long)g.N * g.P * g.Q;
-  const bool wide = g.O > 64 && round_up(g.O, 128) * 7 <= round_up(g.O, 64) * 8;
-  p.BM = wide ? 128 : 64;
-  p.BN = 128;
-  const long tiles = (long)((g.O + p.BM - 1) / p.BM) * ((NC + p.BN - 1) / p.BN);
-  const long stages = (K + BK - 1) / BK;
-  // two blocks per CU; at least 4 stages each, since a split costs a write and
-  // a read of its partial tile
-  long want = std::max<long>(1, 512 / tiles);
-  want = std::min(want, std::max<long>(1, stages / 4));
+  const long tiles = (long)((g.O + 63) / 64) * ((g.R * g.S * o.Cp + 63) / 64);
+  const long stages = ((long)g.N * g.P * g.Q + BK - 1) / BK;
+  long want = std::min(std::max<long>(1, 1024 / tiles), std::max<long>(1, stages / 4));
+  if (tiles * want > 256) want = std::max<long>((256 + tiles - 1) / tiles, std::min(want, stages / 8));
   p.per = (int)((stages + want - 1) / want);
   p.splits = (int)((stages + p.per - 1) / p.per);
   return p;
@@ -903,7 +1012,7 @@ void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, cha
     a.x = ws + l.x;
     a.y = c.y;
     a.M = g.O;
-    a.CU = CU;
+    a.full = CU & ~7;
     a.x_bytes = (int)pack_bytes<T>(g.N, o.Hp, o.Wp, o.Cp);
     a.y_bytes = (int)((long)g.N * g.O * g.P * g.Q * ES);
     a.colb = o.Cp * ES;
@@ -916,11 +1025,13 @@ void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, cha
     a.OW = g.Q;
     a.osh = a.osw = 1;
     a.nph = 1;
-    a.fCU = FastDiv((uint32_t)CU);
+    a.ftail = FastDiv((uint32_t)std::max(1, CU & 7));
     ConvPhase& p = a.ph[0];
     p.w_bytes = g.O * nst * 128;
     p.nst = nst;
     p.units = units;
+    p.full = RS * a.full;
+    p.fT = FastDiv((uint32_t)RS);
     p.N = g.N * g.P * g.Q;
     p.fHW = FastDiv((uint32_t)(g.P * g.Q));
     p.fW = FastDiv((uint32_t)g.Q);
@@ -944,7 +1055,7 @@ void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, cha
   a.mask = c.mask;
   a.act = c.mask ? 2 : 0;
   a.M = g.C;
-  a.CU = CU;
+  a.full = CU & ~7;
   a.x_bytes = (int)pack_bytes<T>(g.N, o.Pp, o.Qp, o.Op);
   a.y_bytes = (int)((long)g.N * g.C * g.H * g.W * ES);
   a.colb = o.Op * ES;
@@ -955,7 +1066,7 @@ void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, cha
   a.OW = g.W;
   a.osh = g.sh;
   a.osw = g.sw;
-  a.fCU = FastDiv((uint32_t)CU);
+  a.ftail = FastDiv((uint32_t)std::max(1, CU & 7));
   int off = 0, tails = 0;
   for (int f = 0; f < n; ++f) {
     const DPhase& q = ph[f];
@@ -972,6 +1083,8 @@ void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, cha
     p.w_bytes = g.C * nst * 128;
     p.nst = nst;
     p.units = units;
+    p.full = taps * a.full;
+    p.fT = FastDiv((uint32_t)std::max(1, taps));
     p.off0 = (q.offa - (q.Rc - 1) + o.dT) * a.rowb + (q.offb - (q.Sc - 1) + o.dL) * a.colb;
     p.N = g.N * q.Hc * q.Wc;
     p.sub_a = q.a;
@@ -982,8 +1095,6 @@ void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, cha
     off += g.C * nst * 8;
   }
   s.total = s.units + tails;
-  // the phases with most taps first: the short ones fill the last wave
-  std::stable_sort(a.ph, a.ph + a.nph, [](const ConvPhase& p, const ConvPhase& q) { return p.nst > q.nst; });
 }
 
 template <typename T>
@@ -1007,24 +1118,21 @@ int run_wgrad(const GatherCall& c, const Geo& o, char* ws, const Layout& l, hipS
   a.K = g.N * g.P * g.Q;
   a.part = reinterpret_cast<float*>(ws + l.part);
   a.dbpart = c.db ? a.part + (size_t)p.splits * g.O * a.NC : nullptr;
-  a.tiles_m = (g.O + p.BM - 1) / p.BM;
-  a.tiles_n = (a.NC + p.BN - 1) / p.BN;
+  a.tiles_m = (g.O + 63) / 64;
+  a.tiles_n = (a.NC + 63) / 64;
   a.per = p.per;
   a.tcol = o.Cp * ES;
   a.trow = o.Wp * a.tcol;
   a.xcol = g.sw * a.tcol;
   a.xrow = g.sh * a.trow;
   a.ximg = o.Hp * a.trow;
-  a.cs_shift = colsum_shift(a.tiles_n, p.BM);
+  a.cs_shift = colsum_shift(a.tiles_n, 64);
   a.fPQ = FastDiv((uint32_t)(g.P * g.Q));
   a.fQ = FastDiv((uint32_t)g.Q);
   a.fCU = FastDiv((uint32_t)(o.Cp / UE));
   a.fS = FastDiv((uint32_t)g.S);
   const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * p.splits));
-  if (p.BM == 128)
-    gather_wgrad_kernel<T, 128, 128, 64, 64><<<grid, 256, 0, st>>>(a);
-  else
-    gather_wgrad_kernel<T, 64, 128, 32, 64><<<grid, 256, 0, st>>>(a);
+  gather_wgrad_kernel<T, 64, 64, 32, 32><<<grid, 256, 0, st>>>(a);
   VH_LAUNCH_CHECK();
   const int RS = g.R * g.S;
   if (p.splits > 8) {
