@@ -1,0 +1,89 @@
+"""GPU: products of any size (vh_mm.hip) at the edges of their tiles, stages, K
+splits and padded rows, against the oracle under the parity gate."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.test_gpu_parity import DEV, DTYPES, check, host, prep, rng
+from volta_amd import nn as vnn
+from volta_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+# (m, k, n)
+CASES = [
+    (1, 1, 1), (31, 9, 33),      # below one tile, one unit of k and a bit
+    (33, 64, 65), (65, 65, 31),  # one past a tile, one past a stage
+    (40, 3000, 24),              # few tiles: K split over blocks
+    (129, 4097, 70),             # the same with padded rows, a split's last stage partial
+    (300, 96, 1000), (257, 130, 255),
+    (520, 250, 520),             # 64 x 64 tiles (bf16: 32 x 64)
+    (1030, 72, 1100),            # 64 x 64 / 64 x 128 tiles with remainders
+    (2060, 40, 2072),            # 128 x 128 tiles (bf16) with remainders, aligned rows
+    (2050, 33, 2310),            # the same, padded rows
+    (4100, 16, 2056),            # 128 x 256 producer / consumer tiles (bf16 forward)
+]
+
+
+@pytest.mark.parametrize("mkn", CASES)
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_mm_family(mkn, dt):
+    m, k, n = mkn
+    g = rng(m * 3 + k * 5 + n)
+    a, at = prep(g.standard_normal((m, k)), dt)
+    b, bt = prep(g.standard_normal((k, n)), dt)
+    gr, grt = prep(g.standard_normal((m, n)), dt)
+    check(ops.gpu_matmul(at, bt, m, k, n), oracle.matmul, (a, b), dt, "matmul", k=k)
+    check(ops.gpu_matmul_backward_a(grt, bt, m, k, n), oracle.matmul_backward_a, (gr, b), dt, "dA", k=n)
+    check(ops.gpu_matmul_backward_b(at, grt, m, k, n), oracle.matmul_backward_b, (a, gr), dt, "dB", k=m)
+
+
+@pytest.mark.parametrize("shape", [(3, 5, 7), (34, 3846, 80), (256, 784, 512), (1000, 60, 44), (70, 1030, 900)])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_mm_linear(shape, dt):
+    m, i, o = shape
+    g = rng(m + i + o)
+    x, xt = prep(g.standard_normal((m, i)), dt)
+    w, wt = prep(g.uniform(-0.5, 0.5, (i, o)), dt)
+    b, bt = prep(g.uniform(-1, 1, (o,)), dt)
+    dy, dyt = prep(g.standard_normal((m, o)), dt)
+    lin = vnn.Linear(i, o, device=DEV, dtype=DTYPES[dt])
+    lin.weight, lin.bias = wt, bt
+    check(lin.forward(xt), oracle.linear_forward, (x, w, b), dt, "y", k=i + 1)
+    got = lin.backward(dyt, xt)  # dX and dW in one launch
+    for q, (what, k) in enumerate((("dx", o), ("dw", m), ("db", m))):
+        check(got[q], lambda *a, q=q: oracle.linear_backward(*a)[q], (dy, x, w), dt, what, k=k)
+    one = lin.backward(dyt, xt, input_grad=False)
+    for q, what in ((1, "dw"), (2, "db")):
+        check(one[q], lambda *a, q=q: oracle.linear_backward(*a)[q], (dy, x, w), dt, what + " alone", k=m)
+    assert lin.backward(dyt, xt, weight_grad=False)[0].shape == xt.shape
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_mm_unaligned_operands(dt):
+    """Views that start off a 16-byte boundary take the padded copies."""
+    m, k, n = 70, 64, 48
+    g = rng(9)
+    a, _ = prep(g.standard_normal((m, k)), dt)
+    b, _ = prep(g.standard_normal((k, n)), dt)
+
+    def view(x):
+        t = torch.empty(x.size + 1, device=DEV, dtype=DTYPES[dt])[1:].view(x.shape)
+        t.copy_(torch.from_numpy(x))
+        return t
+
+    check(ops.gpu_matmul(view(a), view(b), m, k, n), oracle.matmul, (a, b), dt, "matmul", k=k)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("mkn", [(5, 7, 9), (40, 3001, 24)])
+def test_mm_padding_does_not_leak(mkn, dt):
+    """An infinity stays in its row and column: stage, row and unit padding is zero."""
+    m, k, n = mkn
+    a, b = torch.ones((m, k), device=DEV, dtype=DTYPES[dt]), torch.ones((k, n), device=DEV, dtype=DTYPES[dt])
+    a[m - 1, k - 1] = float("inf")
+    c = np.isfinite(host(ops.gpu_matmul(a, b, m, k, n)))
+    assert c[: m - 1].all() and not c[m - 1].any()
+    db = np.isfinite(host(ops.gpu_matmul_backward_b(a, torch.ones((m, n), device=DEV, dtype=DTYPES[dt]), m, k, n)))
+    assert db[: k - 1].all() and not db[k - 1].any()

@@ -853,60 +853,44 @@ static int direct_wgrad(int dt, const void* dy, const void* x, void* dw, const C
 
 
 // ------------------------------------------------------------------ GEMM entry helper
-// bf16 products on the dense kernel: either operand may be stored with its
-// contraction index contiguous (KD_DENSE_K) or its row index contiguous
-// (KD_DENSE_MN: stored [K][rows], read by transposing LDS reads).  Returns
-// VH_ERR_UNSUPPORTED when the shapes or alignments do not fit.
-static int dense_bf16(int ak, int bk, const void* a, int lda, const void* b, int ldb, void* c, int ldc, long M,
-                      long N, long K, const void* bias, hipStream_t st, void* colsum = nullptr) {
-  const bool at = ak == KD_DENSE_MN, bt = bk == KD_DENSE_MN;
-  if (!dense_bf16_ok(M, N, K, at, lda, bt, ldb, ldc, a, b, c)) return VH_ERR_UNSUPPORTED;
-  // a grid of few tiles over a long K: the split-K implicit GEMM fills the chip instead
-  if (((M + 127) / 128) * ((N + 127) / 128) < 64 && K > 2048) return VH_ERR_UNSUPPORTED;
-  return dense_bf16_gemm(a, lda, at, b, ldb, bt, c, ldc, (int)M, (int)N, (int)K, bias, st, colsum);
-}
-
-// Linear's dX and dW (K-major x K-major, MN-major x MN-major) as one launch of
-// the dense kernel when both take its 128 x 128 tiles: each grid alone would
-// hold one block per CU.  VH_ERR_UNSUPPORTED: run them separately.
-static int dense_bf16_pair(const DenseProblem& p0, const DenseProblem& p1, hipStream_t st) {
-  for (const DenseProblem* p : {&p0, &p1}) {
-    if (std::max({(long)p->M * p->K, (long)p->K * p->N, (long)p->M * p->N}) > kMaxElems) return VH_ERR_UNSUPPORTED;
-    if (!dense_bf16_ok(p->M, p->N, p->K, p->at, p->lda, p->bt, p->ldb, p->ldc, p->a, p->b, p->c))
+// A product (or a Linear layer's dX and dW as a pair) on the large whole-tile
+// kernels (vh_dense.hip, vh_dense_f32.hip); VH_ERR_UNSUPPORTED: not one of theirs.
+static int dense_large(int dt, const DenseProblem* p, int np, const void* bias, hipStream_t st) {
+  const bool b16 = dt == VH_BF16;
+  for (int i = 0; i < np; ++i)
+    if (!(b16 ? dense_bf16_ok : dense_f32_ok)(p[i].M, p[i].N, p[i].K, p[i].at, p[i].lda, p[i].bt, p[i].ldb, p[i].ldc,
+                                              p[i].a, p[i].b, p[i].c))
       return VH_ERR_UNSUPPORTED;
-    if (((p->M + 127L) / 128) * ((p->N + 127L) / 128) < 64 && p->K > 2048) return VH_ERR_UNSUPPORTED;
-  }
-  return dense_bf16_gemm_pair(p0, p1, st);
+  if (np == 2) return b16 ? dense_bf16_gemm_pair(p[0], p[1], st) : dense_f32_gemm_pair(p[0], p[1], st);
+  const DenseProblem& q = *p;
+  if (b16) return dense_bf16_gemm(q.a, q.lda, q.at, q.b, q.ldb, q.bt, q.c, q.ldc, q.M, q.N, q.K, bias, st);
+  return bias ? VH_ERR_UNSUPPORTED : dense_f32_gemm(q.a, q.lda, q.at, q.b, q.ldb, q.bt, q.c, q.ldc, q.M, q.N, q.K, st);
 }
 
-static int dense_f32_pair(const DenseProblem& p0, const DenseProblem& p1, hipStream_t st) {
-  for (const DenseProblem* p : {&p0, &p1}) {
-    if (std::max({(long)p->M * p->K, (long)p->K * p->N, (long)p->M * p->N}) > kMaxElems) return VH_ERR_UNSUPPORTED;
-    if (!dense_f32_ok(p->M, p->N, p->K, p->at, p->lda, p->bt, p->ldb, p->ldc, p->a, p->b, p->c))
-      return VH_ERR_UNSUPPORTED;
+// The large kernels, or those for any size (vh_mm.hip) where their workspace can be
+// had: true with the status in *r.
+static bool product_try(int dt, const DenseProblem* p, int np, const void* bias, hipStream_t st, int* r) {
+  bool plain = true;  // column sums of a single product: vh_mm.hip
+  for (int i = 0; i < np; ++i) {
+    if (std::max({(long)p[i].M * p[i].K, (long)p[i].K * p[i].N, (long)p[i].M * p[i].N}) > kMaxElems) return false;
+    plain = plain && (np == 2 || !p[i].colsum);
   }
-  return dense_f32_gemm_pair(p0, p1, st);
-}
-
-static int dense_f32(int ak, int bk, const void* a, int lda, const void* b, int ldb, void* c, int ldc, long M,
-                     long N, long K, const void* bias, hipStream_t st) {
-  const bool at = ak == KD_DENSE_MN, bt = bk == KD_DENSE_MN;
-  if (!dense_f32_ok(M, N, K, at, lda, bt, ldb, ldc, a, b, c)) return VH_ERR_UNSUPPORTED;
-  // a grid of few tiles over a long K: the split-K implicit GEMM fills the chip instead
-  if (((M + 63) / 64) * ((N + 127) / 128) < 128 && K > 1024) return VH_ERR_UNSUPPORTED;
-  return dense_f32_gemm(a, lda, at, b, ldb, bt, c, ldc, (int)M, (int)N, (int)K, bias, st);
+  if (plain && (*r = dense_large(dt, p, np, bias, st)) != VH_ERR_UNSUPPORTED) return true;
+  bool ok;
+  const size_t bytes = mm_ws(dt, p, np, &ok);
+  void* ws = nullptr;
+  if (!ok || (bytes && !ws_try(st, bytes, &ws))) return false;
+  *r = mm_run(dt, p, np, bias, ws, st);
+  return true;
 }
 
 static int gemm(int dt, int ak, int bk, const void* a, int lda, const void* b, int ldb, void* c, int ldc,
                 long M, long N, long K, const void* bias, int bias_mode, hipStream_t st) {
   VH_TRY(check_sizes({M * K, K * N, M * N}));
-  if (dt == VH_BF16 && g_fast_paths && (bias == nullptr || bias_mode == 2)) {
-    int r = dense_bf16(ak, bk, a, lda, b, ldb, c, ldc, M, N, K, bias, st);
-    if (r != VH_ERR_UNSUPPORTED) return r;
-  }
-  if (dt == VH_F32 && g_fast_paths && (bias == nullptr || bias_mode == 2)) {
-    int r = dense_f32(ak, bk, a, lda, b, ldb, c, ldc, M, N, K, bias, st);
-    if (r != VH_ERR_UNSUPPORTED) return r;
+  if (g_fast_paths && (bias == nullptr || bias_mode == 2) && std::max({M, N, K}) < (1L << 31)) {
+    const DenseProblem p{a, lda, ak == KD_DENSE_MN, b, ldb, bk == KD_DENSE_MN, c, ldc, (int)M, (int)N, (int)K, nullptr};
+    int r;
+    if (product_try(dt, &p, 1, bias, st, &r)) return r;
   }
   IgemmPlan p{};
   p.dtype = dt;
@@ -1577,6 +1561,18 @@ int vh_linear_forward(int dtype, const void* x, const void* weight, const void* 
               m, out_features, in_features, bias, 2, S(stream));
 }
 
+// Whether a Linear layer's dX and dW go in one launch: on the whole-tile pair
+// kernels, or where the two grids of 64 x 64 tiles leave room in four blocks a CU.
+static bool linear_pair(int dt, const DenseProblem* p) {
+  long g64 = 0;
+  bool whole = true;
+  for (int i = 0; i < 2; ++i) {
+    g64 += ((p[i].M + 63L) / 64) * ((p[i].N + 63L) / 64);
+    whole = whole && p[i].M % 128 == 0 && p[i].N % 256 == 0 && p[i].K % 128 == 0;
+  }
+  return dt == VH_F32 || whole || g64 <= 1024;
+}
+
 int vh_linear_backward(int dtype, const void* out_grad, const void* x, const void* weight, void* grad_x,
                        void* grad_weight, void* grad_bias, int64_t m, int64_t in_features, int64_t out_features,
                        void* stream) {
@@ -1585,38 +1581,26 @@ int vh_linear_backward(int dtype, const void* out_grad, const void* x, const voi
   if (m < 0 || in_features < 0 || out_features < 0) return set_error(VH_ERR_BAD_SHAPE, "negative dimension");
   if (!out_grad || (grad_x && !weight) || (grad_weight && !x)) return set_error(VH_ERR_BAD_ARG, "null pointer");
   hipStream_t st = S(stream);
-  if (dtype == VH_BF16 && g_fast_paths && grad_x && grad_weight && m * in_features * out_features &&
+  if (g_fast_paths && grad_weight && m && in_features && out_features &&
       std::max({m, in_features, out_features}) < (1L << 31)) {
-    // db as the column sums of dY inside the dW tiles
-    const DenseProblem dx{out_grad, (int)out_features, false, weight, (int)out_features, false,
-                          grad_x, (int)in_features, (int)m, (int)in_features, (int)out_features, nullptr};
-    const DenseProblem dw{x, (int)in_features, true, out_grad, (int)out_features, true,
-                          grad_weight, (int)out_features, (int)in_features, (int)out_features, (int)m, grad_bias};
-    const int r = dense_bf16_pair(dx, dw, st);
-    if (r != VH_OK && r != VH_ERR_UNSUPPORTED) return r;
-    if (r == VH_OK) grad_x = grad_weight = grad_bias = nullptr;  // all done
-  }
-  if (dtype == VH_F32 && g_fast_paths && grad_x && grad_weight && m * in_features * out_features &&
-      std::max({m, in_features, out_features}) < (1L << 31)) {
-    // the same pair in fp32 (whole 128 x 256 tiles only), db as column sums of dY
-    const DenseProblem dx{out_grad, (int)out_features, false, weight, (int)out_features, false,
-                          grad_x, (int)in_features, (int)m, (int)in_features, (int)out_features, nullptr};
-    const DenseProblem dw{x, (int)in_features, true, out_grad, (int)out_features, true,
-                          grad_weight, (int)out_features, (int)in_features, (int)out_features, (int)m, grad_bias};
-    const int r = dense_f32_pair(dx, dw, st);
-    if (r != VH_OK && r != VH_ERR_UNSUPPORTED) return r;
-    if (r == VH_OK) grad_x = grad_weight = grad_bias = nullptr;  // all done
+    // db as the column sums of dY inside the dW tiles; dX and dW in one launch
+    // unless either alone fills the chip (a bf16 product then takes larger tiles)
+    const DenseProblem p[2] = {{out_grad, (int)out_features, false, weight, (int)out_features, false, grad_x,
+                                (int)in_features, (int)m, (int)in_features, (int)out_features, nullptr},
+                               {x, (int)in_features, true, out_grad, (int)out_features, true, grad_weight,
+                                (int)out_features, (int)in_features, (int)out_features, (int)m, grad_bias}};
+    int r;
+    if (grad_x && linear_pair(dtype, p) && product_try(dtype, p, 2, nullptr, st, &r)) {
+      VH_TRY(r);
+      grad_x = grad_weight = grad_bias = nullptr;  // all done
+    } else if (product_try(dtype, p + 1, 1, nullptr, st, &r)) {
+      VH_TRY(r);
+      grad_weight = grad_bias = nullptr;
+    }
   }
   if (grad_x && m * in_features)
     VH_TRY(gemm(dtype, KD_DENSE_K, KD_DENSE_K, out_grad, (int)out_features, weight, (int)out_features, grad_x,
                 (int)in_features, m, in_features, out_features, nullptr, 0, st));
-  if (grad_weight && grad_bias && dtype == VH_BF16 && g_fast_paths && m * in_features * out_features &&
-      std::max({m * in_features, m * out_features, in_features * out_features}) <= kMaxElems) {
-    const int r = dense_bf16(KD_DENSE_MN, KD_DENSE_MN, x, (int)in_features, out_grad, (int)out_features,
-                             grad_weight, (int)out_features, in_features, out_features, m, nullptr, st, grad_bias);
-    if (r != VH_OK && r != VH_ERR_UNSUPPORTED) return r;
-    if (r == VH_OK) grad_weight = grad_bias = nullptr;  // dW and db done
-  }
   if (grad_weight && in_features * out_features)
     VH_TRY(gemm(dtype, KD_DENSE_MN, KD_DENSE_MN, x, (int)in_features, out_grad, (int)out_features, grad_weight,
                 (int)out_features, in_features, out_features, m, nullptr, 0, st));

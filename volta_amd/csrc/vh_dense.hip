@@ -1,23 +1,22 @@
 // vh_dense.hip -- dense bf16 matrix products (matmul, its gradients, Linear) on
 // gfx950 MFMA (v_mfma_f32_32x32x16_bf16), fp32 accumulation.
 //
-// One kernel for C[M][N] = A . B with either operand stored either way:
-// "K-major" (row-major [rows][K], the contraction index contiguous: A[M][K],
-// B[N][K]) or "MN-major" ([K][rows], the row index contiguous: A stored
-// [K][M], B stored [K][N] -- matmul's B, the weight gradient's A and G).  Every
-// operand tile is a plain copy of 16-byte units into LDS in its stored order.
-// An MFMA fragment (8 consecutive k of one row) of a K-major tile is one
-// ds_read_b128; of an MN-major tile ([k][row] in LDS) it is two
-// ds_read_b64_tr_b16, gfx950's transposing LDS read: within each group of 16
-// lanes, lane i names 4 consecutive elements of row i/4 (elements
+// C[M][N] = A . B with either operand stored either way: "K-major" (row-major
+// [rows][K], the contraction index contiguous: A[M][K], B[N][K]) or "MN-major"
+// ([K][rows], the row index contiguous: A stored [K][M], B stored [K][N] --
+// matmul's B, the weight gradient's A and G).  Every operand tile is a plain copy
+// of 16-byte units into LDS in its stored order.  An MFMA fragment (8 consecutive k
+// of one row) of a K-major tile is one ds_read_b128; of an MN-major tile ([k][row]
+// in LDS) it is two ds_read_b64_tr_b16, gfx950's transposing LDS read: within each
+// group of 16 lanes, lane i names 4 consecutive elements of row i/4 (elements
 // 4*(i%4) .. +3), and lane j receives element j of each of the 4 rows, i.e. 4
 // consecutive k of column j.  No operand is transposed in memory.
 //
-// Block: 256 threads (2 x 2 waves), tile BM x BN, K in stages of 64; two LDS
-// stages and two register sets: the loads of stage k+2 are issued before the
-// MFMAs of stage k (kept there by sched_barrier), the stores of stage k+1 into
-// LDS follow them.  XCD-aware block order: the blocks resident on one XCD
-// cover groups of 8 m-tiles x a few n-tiles, sharing A and B slices in L2.
+// Two kernels: whole 256 x 256 (a Linear pair: 128 x 256) tiles copied straight into
+// LDS, and 128 x 256 producer / consumer tiles for large K-major x MN-major products
+// that are not whole (4104 x 4096 x 4104: 162 us, 180 on the tiles of vh_mm.hip,
+// which take every other product).  XCD-aware block order: the blocks resident on
+// one XCD cover groups of 8 m-tiles x a few n-tiles, sharing A and B slices in L2.
 #include <type_traits>
 
 #include "vh_kernels.hpp"
@@ -40,7 +39,7 @@ struct DenseArgs {
   const uint16_t* b;     // [N][ldb] (K-major) or [K][ldb] (MN-major)
   uint16_t* c;           // [M][ldc]
   const uint16_t* bias;  // [N] or nullptr (added to every row)
-  uint16_t* colsum;      // [N] or nullptr: column sums of an MN-major B over K (128 x 128 tiles only)
+  uint16_t* colsum;      // [N] or nullptr: column sums of an MN-major B over K (the pair)
   int cs_shift;          // columns per block of the column sums: 4 << cs_shift (set at launch)
   int vec_epi;           // C 16-byte aligned, ldc and N multiples of 8: 16-byte stores through LDS
   int M, N, K, lda, ldb, ldc;
@@ -48,8 +47,8 @@ struct DenseArgs {
   int tiles_m, tiles_n;
 };
 
-template <int BM, int BN, bool AT = false, bool BT = false>
 struct DenseCfg {
+  static constexpr int BM = 128, BN = 256;
   static constexpr int BK = 64;            // contraction elements per stage
   static constexpr int KU = BK / 8;        // 16-byte units per row per stage
   static constexpr int PU = KU + 1;        // K-major tile: LDS row pitch in units (odd: conflict-free)
@@ -57,35 +56,28 @@ struct DenseCfg {
   static constexpr int AIT = BM * KU / 256, BIT = BN * KU / 256;  // load units per thread
   // MN-major tile: BK rows of R elements, pitch R + 32 elements (row starts 64
   // bytes apart mod 256: the four rows of a transposing read hit disjoint banks)
-  static constexpr int mn_pitch(int R) { return R / 8 + 4; }
-  static constexpr int A_UNITS = AT ? BK * mn_pitch(BM) : BM * PU;
-  static constexpr int B_UNITS = BT ? BK * mn_pitch(BN) : BN * PU;
+  static constexpr int BPU = BN / 8 + 4;
+  static constexpr int A_UNITS = BM * PU, B_UNITS = BK * BPU;
   static constexpr int STAGE = A_UNITS + B_UNITS;  // units per LDS stage
-  // producer / consumer tiles with an MN-major B: room after the two stages
-  // for the producers' column-sum exchange (256 / (BN / 8) k-row groups x at
-  // most BN columns, fp32)
-  static constexpr int CS_BYTES = BT ? 256 / (BN / 8) * BN * 4 : 0;
-  static constexpr size_t lds_bytes(bool pc) { return (size_t)2 * STAGE * 16 + (pc ? CS_BYTES : 0); }
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, bytes, 0x00020000);
 }
 
-// PC: 512 threads; waves 0-3 only multiply (consumers, the accumulators),
-// waves 4-7 only load the next stages into registers and store them into the
-// other LDS buffer (producers, threads 256-511 serving the load map of threads
-// 0-255).  Neither role holds the other's registers, so two waves run per SIMD
-// and the loads leave the multiplying waves' instruction stream.
-// One block's tile: logical block lb of the grid order below.
-template <int BM, int BN, bool BIAS, bool PC, bool AT, bool BT>
-__device__ __forceinline__ void gemm_bf16_tile(const DenseArgs& g, const int lb) {
-  using Cfg = DenseCfg<BM, BN, AT, BT>;
-  constexpr int FM = Cfg::FM, FN = Cfg::FN, PU = Cfg::PU, STAGE = Cfg::STAGE;
-  constexpr int APU = Cfg::mn_pitch(BM), BPU = Cfg::mn_pitch(BN);  // MN-major LDS pitches (units)
+// 128 x 256 tiles of a K-major A and an MN-major B, any M and N.  512 threads;
+// waves 0-3 only multiply (consumers, the accumulators), waves 4-7 only load the
+// next stages into registers and store them into the other LDS buffer (producers,
+// threads 256-511).  Neither role holds the other's registers, so two waves run per
+// SIMD and the loads leave the multiplying waves' instruction stream.
+template <bool BIAS>
+__global__ __launch_bounds__(512) void gemm_bf16_kernel(DenseArgs g) {
+  using Cfg = DenseCfg;
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, FM = Cfg::FM, FN = Cfg::FN, PU = Cfg::PU, BPU = Cfg::BPU, STAGE = Cfg::STAGE;
   extern __shared__ __attribute__((aligned(16))) u32x4d lds[];
-  const bool producer = PC && threadIdx.x >= 256;
-  const int tid = PC ? (int)(threadIdx.x & 255u) : (int)threadIdx.x, lane = tid & 63;
+  const int lb = xcd_block(g.tiles_m * g.tiles_n);
+  const bool producer = threadIdx.x >= 256;
+  const int tid = (int)(threadIdx.x & 255u), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
   // logical block -> tile in groups of up to 8 m-tiles: consecutive logical
@@ -97,89 +89,40 @@ __device__ __forceinline__ void gemm_bf16_tile(const DenseArgs& g, const int lb)
   const int in_grp = lb - grp * kGroupM * g.tiles_n;
   const int m0 = (first_m + in_grp % gm) * BM, n0 = (in_grp / gm) * BN;
 
-  // Load items.  K-major operand: unit u = tid + 256*it -> row u / KU, k unit
-  // u % KU (= tid % KU); global offset of k0 = 0 (the stage's k0 is a scalar
-  // offset).  MN-major operand: unit u -> k row u / (R/8), row unit u % (R/8);
-  // the k row's bound is checked per unit (a scalar offset is not range-checked,
-  // so an unused unit carries an out-of-range per-lane offset).
+  // Load items.  A: unit u = tid + 256*it -> row u / KU, k unit u % KU (= tid %
+  // KU); global offset of k0 = 0 (the stage's k0 is a scalar offset).  B: unit u ->
+  // k row u / (BN/8), row unit u % (BN/8); the k row's bound is checked per unit (a
+  // scalar offset is not range-checked, so an unused unit carries an out-of-range
+  // per-lane offset).
   const int cu = tid % Cfg::KU;
-  int a_off[Cfg::AIT], b_off[Cfg::BIT], a_kr[Cfg::AIT], b_kr[Cfg::BIT], a_l[Cfg::AIT], b_l[Cfg::BIT];
+  int a_off[Cfg::AIT], b_off[Cfg::BIT], b_kr[Cfg::BIT], a_l[Cfg::AIT], b_l[Cfg::BIT];
 #pragma unroll
   for (int it = 0; it < Cfg::AIT; ++it) {
-    const int u = tid + it * 256;
-    if constexpr (AT) {
-      const int kr = u / (BM / 8), ru = u % (BM / 8);
-      a_kr[it] = kr;
-      a_off[it] = m0 + ru * 8 < g.M ? (kr * g.lda + m0 + ru * 8) * 2 : kOOR;
-      a_l[it] = kr * APU + ru;
-    } else {
-      const int r = u / Cfg::KU;
-      a_kr[it] = cu * 8;
-      a_off[it] = m0 + r < g.M ? ((m0 + r) * g.lda + cu * 8) * 2 : kOOR;
-      a_l[it] = r * PU + cu;
-    }
+    const int r = (tid + it * 256) / Cfg::KU;
+    a_off[it] = m0 + r < g.M ? ((m0 + r) * g.lda + cu * 8) * 2 : kOOR;
+    a_l[it] = r * PU + cu;
   }
 #pragma unroll
   for (int it = 0; it < Cfg::BIT; ++it) {
-    const int u = tid + it * 256;
-    if constexpr (BT) {
-      const int kr = u / (BN / 8), ru = u % (BN / 8);
-      b_kr[it] = kr;
-      b_off[it] = n0 + ru * 8 < g.N ? (kr * g.ldb + n0 + ru * 8) * 2 : kOOR;
-      b_l[it] = Cfg::A_UNITS + kr * BPU + ru;
-    } else {
-      const int r = u / Cfg::KU;
-      b_kr[it] = cu * 8;
-      b_off[it] = n0 + r < g.N ? ((n0 + r) * g.ldb + cu * 8) * 2 : kOOR;
-      b_l[it] = Cfg::A_UNITS + r * PU + cu;
-    }
+    const int u = tid + it * 256, kr = u / (BN / 8), ru = u % (BN / 8);
+    b_kr[it] = kr;
+    b_off[it] = n0 + ru * 8 < g.N ? (kr * g.ldb + n0 + ru * 8) * 2 : kOOR;
+    b_l[it] = Cfg::A_UNITS + kr * BPU + ru;
   }
   const __amdgpu_buffer_rsrc_t ar = rsrc(g.a, g.a_bytes), br = rsrc(g.b, g.b_bytes);
 
   u32x4d areg[2][Cfg::AIT], breg[2][Cfg::BIT];
   auto gload = [&](auto SET, int k0) {
     constexpr int s = decltype(SET)::value;
-    // k0 as a scalar offset: k0 elements along a K-major row, k0 rows of an MN-major operand
-    const int ask = AT ? k0 * g.lda * 2 : k0 * 2, bsk = BT ? k0 * g.ldb * 2 : k0 * 2;
+    const int ask = k0 * 2, bsk = k0 * g.ldb * 2;
 #pragma unroll
     for (int it = 0; it < Cfg::AIT; ++it)  // K % 8 == 0: a K-major unit is all in or all out
       areg[s][it] = __builtin_bit_cast(
-          u32x4d, __builtin_amdgcn_raw_buffer_load_b128(ar, k0 + a_kr[it] < g.K ? a_off[it] : kOOR, ask, 0));
+          u32x4d, __builtin_amdgcn_raw_buffer_load_b128(ar, k0 + cu * 8 < g.K ? a_off[it] : kOOR, ask, 0));
 #pragma unroll
     for (int it = 0; it < Cfg::BIT; ++it)
       breg[s][it] = __builtin_bit_cast(
           u32x4d, __builtin_amdgcn_raw_buffer_load_b128(br, k0 + b_kr[it] < g.K ? b_off[it] : kOOR, bsk, 0));
-  };
-  // Column sums of B over K (a Linear weight gradient's bias gradient, B = dY
-  // stored [K][N]).  The tiling's tiles_m blocks of a column tile each own
-  // 4 << cs_shift of its columns (block of m-tile mt: columns mt * width ..
-  // + width - 1), so every column is summed by exactly one block, over all K.
-  //  * 4-wave blocks: from the staged LDS tile -- a thread adds 4 consecutive
-  //    owned columns of the k rows tid >> cs_shift (+ 256 >> cs_shift ...) of
-  //    each stage, in stage order; the thread sums are added in k-row order.
-  //  * producer / consumer blocks: the producers add the owned B units they
-  //    hold in registers before storing them (a thread's units all cover the
-  //    same 8 columns: unit tid + 256 it has row unit tid % (BN / 8)), stage by
-  //    stage; the 256 / (BN / 8) k-row group sums are added in group order.
-  constexpr bool CS = BT;
-  constexpr int RU = BN / 8;  // row units per k row of the B tile
-  static_assert(256 % RU == 0, "a thread's B units must share their columns");
-  const int cs_w = 4 << g.cs_shift, cs_c0 = (m0 / BM) * cs_w;
-  const bool cs_on = CS && g.colsum != nullptr;  // block-uniform
-  const bool cs_blk = cs_on && cs_c0 < BN;
-  const int cs_g = tid & ((1 << g.cs_shift) - 1), cs_k0 = tid >> g.cs_shift;
-  const int cs_ru = tid % RU;
-  const bool cs_own = cs_blk && cs_ru * 8 >= cs_c0 && cs_ru * 8 < cs_c0 + cs_w;
-  float csum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  auto colsum_stage = [&](int st) {
-    const char* bt = reinterpret_cast<const char*>(lds + st * STAGE + Cfg::A_UNITS);
-    for (int k = cs_k0; k < Cfg::BK; k += 256 >> g.cs_shift) {
-      const u32x2d v = *reinterpret_cast<const u32x2d*>(bt + k * BPU * 16 + (cs_c0 + cs_g * 4) * 2);
-      csum[0] += __builtin_bit_cast(float, v[0] << 16);
-      csum[1] += __builtin_bit_cast(float, v[0] & 0xffff0000u);
-      csum[2] += __builtin_bit_cast(float, v[1] << 16);
-      csum[3] += __builtin_bit_cast(float, v[1] & 0xffff0000u);
-    }
   };
   auto sstore = [&](auto SET, int st) {
     constexpr int s = decltype(SET)::value;
@@ -188,173 +131,71 @@ __device__ __forceinline__ void gemm_bf16_tile(const DenseArgs& g, const int lb)
     for (int it = 0; it < Cfg::AIT; ++it) base[a_l[it]] = areg[s][it];
 #pragma unroll
     for (int it = 0; it < Cfg::BIT; ++it) base[b_l[it]] = breg[s][it];
-    if constexpr (CS && PC) {
-      if (cs_own) {
-#pragma unroll
-        for (int it = 0; it < Cfg::BIT; ++it)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const unsigned w = breg[s][it][e];
-            csum[2 * e] += __builtin_bit_cast(float, w << 16);
-            csum[2 * e + 1] += __builtin_bit_cast(float, w & 0xffff0000u);
-          }
-      }
-    }
   };
 
-  f32x16 acc[FM][FN];
-  auto zero_acc = [&]() {
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
-  };
-  if (!PC) zero_acc();
   const int row_l = lane & 31, half_l = lane >> 5;
-  // transposing reads of an MN-major tile: lane l reads k row 8*(l/32) + (l%16)/4
+  // transposing reads of the MN-major tile: lane l reads k row 8*(l/32) + (l%16)/4
   // (+4 for the second half of the fragment), elements 16*((l/16)%2) + 4*(l%4) .. +3
   const int tr_row = 8 * half_l + ((lane & 15) >> 2), tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  auto frag_mn = [&](const u32x4d* tile, int pitch_units, int ks, int col0) {
+  auto frag_mn = [&](const u32x4d* tile, int ks, int col0) {
     typedef short v4i16 __attribute__((ext_vector_type(4)));
     const __attribute__((address_space(3))) char* p =
-        (const __attribute__((address_space(3))) char*)(tile) +
-        (((ks * 8 + tr_row) * pitch_units) * 16 + (col0 + tr_col) * 2);
+        (const __attribute__((address_space(3))) char*)(tile) + (((ks * 8 + tr_row) * BPU) * 16 + (col0 + tr_col) * 2);
     const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)p);
     const v4i16 hi =
-        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(p + 4 * pitch_units * 16));
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(p + 4 * BPU * 16));
     typedef short v8i16 __attribute__((ext_vector_type(8)));
     const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     return __builtin_bit_cast(bf16x8, v);
   };
-  auto compute = [&](int st) {
-    const u32x4d* ap = lds + st * STAGE + (wm + row_l) * PU + half_l;
-    const u32x4d* bp = lds + st * STAGE + Cfg::A_UNITS + (wn + row_l) * PU + half_l;
-    const u32x4d* at = lds + st * STAGE;
-    const u32x4d* bt = lds + st * STAGE + Cfg::A_UNITS;
+
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  const int nk = (g.K + Cfg::BK - 1) / Cfg::BK;
+  // one barrier per stage on both sides; stage k is multiplied from buffer
+  // k & 1 while the producers store stage k+1 into the other buffer (read
+  // by the consumers before the previous barrier) and load stage k+3
+  if (producer) {
+    gload(I0{}, 0);
+    if (nk > 1) gload(I1{}, Cfg::BK);
+    __builtin_amdgcn_sched_barrier(0);
+    sstore(I0{}, 0);
+    if (nk > 2) gload(I0{}, 2 * Cfg::BK);
+    __syncthreads();
+    for (int kt = 0; kt < nk; kt += 2) {
+      if (kt + 1 < nk) sstore(I1{}, 1);
+      if (kt + 3 < nk) gload(I1{}, (kt + 3) * Cfg::BK);
+      __syncthreads();
+      if (kt + 1 >= nk) break;
+      if (kt + 2 < nk) sstore(I0{}, 0);
+      if (kt + 4 < nk) gload(I0{}, (kt + 4) * Cfg::BK);
+      __syncthreads();
+    }
+    return;
+  }
+  f32x16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+  __syncthreads();
+  for (int kt = 0; kt < nk; ++kt) {
+    const u32x4d* ap = lds + (kt & 1) * STAGE + (wm + row_l) * PU + half_l;
+    const u32x4d* bt = lds + (kt & 1) * STAGE + Cfg::A_UNITS;
 #pragma unroll
     for (int ks = 0; ks < Cfg::KU; ks += 2) {
       bf16x8 af[FM], bf[FN];
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-        af[i] = AT ? frag_mn(at, APU, ks, wm + i * 32) : __builtin_bit_cast(bf16x8, ap[i * 32 * PU + ks]);
+      for (int i = 0; i < FM; ++i) af[i] = __builtin_bit_cast(bf16x8, ap[i * 32 * PU + ks]);
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
-        bf[j] = BT ? frag_mn(bt, BPU, ks, wn + j * 32) : __builtin_bit_cast(bf16x8, bp[j * 32 * PU + ks]);
+      for (int j = 0; j < FN; ++j) bf[j] = frag_mn(bt, ks, wn + j * 32);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
     }
-    if constexpr (CS && !PC) {  // after the stage's MFMAs are issued: the adds overlap their execution
-      if (cs_blk) colsum_stage(st);
-    }
-  };
-
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
-  const int nk = (g.K + Cfg::BK - 1) / Cfg::BK;
-  if constexpr (PC) {
-    // one barrier per stage on both sides; stage k is multiplied from buffer
-    // k & 1 while the producers store stage k+1 into the other buffer (read
-    // by the consumers before the previous barrier) and load stage k+3
-    if (producer) {
-      gload(I0{}, 0);
-      if (nk > 1) gload(I1{}, Cfg::BK);
-      __builtin_amdgcn_sched_barrier(0);
-      sstore(I0{}, 0);
-      if (nk > 2) gload(I0{}, 2 * Cfg::BK);
-      __syncthreads();
-      for (int kt = 0; kt < nk; kt += 2) {
-        if (kt + 1 < nk) sstore(I1{}, 1);
-        if (kt + 3 < nk) gload(I1{}, (kt + 3) * Cfg::BK);
-        __syncthreads();
-        if (kt + 1 >= nk) break;
-        if (kt + 2 < nk) sstore(I0{}, 0);
-        if (kt + 4 < nk) gload(I0{}, (kt + 4) * Cfg::BK);
-        __syncthreads();
-      }
-      if constexpr (CS) {
-        if (cs_on) {
-          float* red = reinterpret_cast<float*>(lds + 2 * STAGE);  // [256 / RU][cs_w]
-          if (cs_own) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) red[(tid / RU) * cs_w + cs_ru * 8 - cs_c0 + e] = csum[e];
-          }
-          __syncthreads();  // matched by the consumers after their last stage
-          const int n = n0 + cs_c0 + tid;
-          if (cs_blk && tid < cs_w && n < g.N) {
-            float t = 0.f;
-            for (int j = 0; j < 256 / RU; ++j) t += red[j * cs_w + tid];
-            g.colsum[n] = f32_to_bf16(t);
-          }
-        }
-      }
-      return;
-    }
-    zero_acc();
     __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-      compute(kt & 1);
-      __syncthreads();
-    }
-    if constexpr (CS) {
-      if (cs_on) __syncthreads();  // the producers' column-sum exchange
-    }
-  } else {
-  // invariant at an even stage k: LDS buffer 0 holds stage k, register set 1
-  // holds stage k+1 (in flight), set 0 is free
-  gload(I0{}, 0);
-  if (nk > 1) gload(I1{}, Cfg::BK);
-  __builtin_amdgcn_sched_barrier(0);
-  sstore(I0{}, 0);
-  __syncthreads();
-  int kt = 0;
-  for (; kt + 3 < nk; kt += 2) {
-    gload(I0{}, (kt + 2) * Cfg::BK);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(0);
-    __builtin_amdgcn_sched_barrier(0);
-    sstore(I1{}, 1);
-    __syncthreads();
-    gload(I1{}, (kt + 3) * Cfg::BK);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(1);
-    __builtin_amdgcn_sched_barrier(0);
-    sstore(I0{}, 0);
-    __syncthreads();
-  }
-  const int rem = nk - kt;  // 1, 2 or 3 stages left
-  if (rem == 3) gload(I0{}, (kt + 2) * Cfg::BK);
-  __builtin_amdgcn_sched_barrier(0);
-  compute(0);
-  if (rem >= 2) {
-    sstore(I1{}, 1);
-    __syncthreads();
-    compute(1);
-    if (rem == 3) {
-      sstore(I0{}, 0);
-      __syncthreads();
-      compute(0);
-    }
-  }
-  }
-
-  if constexpr (CS && !PC) {
-    if (cs_blk) {  // per owned column: the 256 >> cs_shift k-row sums, added in k-row order
-      static_assert(256 * 4 * 4 <= 2 * STAGE * 16, "column-sum exchange exceeds the LDS stages");
-      __syncthreads();  // every wave is done reading the last stage
-      float* red = reinterpret_cast<float*>(lds);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) red[cs_k0 * cs_w + cs_g * 4 + e] = csum[e];
-      __syncthreads();
-      const int n = n0 + cs_c0 + tid;
-      if (tid < cs_w && n < g.N) {
-        float t = 0.f;
-        for (int j = 0; j < 256 >> g.cs_shift; ++j) t += red[j * cs_w + tid];
-        g.colsum[n] = f32_to_bf16(t);
-      }
-    }
   }
 
   const __amdgpu_buffer_rsrc_t cr = rsrc(g.c, g.c_bytes);
@@ -364,7 +205,6 @@ __device__ __forceinline__ void gemm_bf16_tile(const DenseArgs& g, const int lb)
     // (8) stores per lane instead of 128 (64) two-byte ones
     constexpr int WMR = FM * 32, WN = FN * 32, EP = WN + 8, CPR = WN / 8, RPI = 64 / CPR;
     static_assert(4 * WMR * EP * 2 <= 2 * STAGE * 16, "epilogue tiles exceed the LDS stages");
-    if constexpr (!PC) __syncthreads();  // PC: the consumers' last stage barrier already passed
     uint16_t* eb = reinterpret_cast<uint16_t*>(lds) + wave * WMR * EP;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
@@ -405,27 +245,6 @@ __device__ __forceinline__ void gemm_bf16_tile(const DenseArgs& g, const int lb)
                                                 voff, row * g.ldc * 2, 0);
       }
   }
-}
-
-template <int BM, int BN, bool BIAS, bool PC = false, bool AT = false, bool BT = false>
-__global__ __launch_bounds__(PC ? 512 : 256)
-void gemm_bf16_kernel(DenseArgs g) {
-  gemm_bf16_tile<BM, BN, BIAS, PC, AT, BT>(g, xcd_block(g.tiles_m * g.tiles_n));
-}
-
-// Two independent products in one launch: blocks 0 .. T0-1 take the first
-// product's tiles, the rest the second's.  Meant for pairs whose grids would
-// each leave half the chip idle (a Linear layer's dX and dW): together they
-// fill it -- 128 x 256 producer / consumer tiles, one block per CU, when the
-// two grids reach a block per CU, else 128 x 128 tiles at two blocks per CU.
-template <int BN, bool PC, bool AT0, bool BT0, bool AT1, bool BT1>
-__global__ __launch_bounds__(PC ? 512 : 256)
-void gemm_bf16_pair_kernel(DenseArgs g0, DenseArgs g1) {
-  const int t0 = g0.tiles_m * g0.tiles_n, h = blockIdx.x;
-  if (h < t0)
-    gemm_bf16_tile<128, BN, false, PC, AT0, BT0>(g0, xcd_map(h, t0));
-  else
-    gemm_bf16_tile<128, BN, false, PC, AT1, BT1>(g1, xcd_map(h - t0, g1.tiles_m * g1.tiles_n));
 }
 
 // ---------------------------------------------------------------- BM x 256 tiles, direct-to-LDS loads
@@ -728,30 +547,16 @@ void gemm_bf16_d2l_pair_kernel(DenseArgs g0, DenseArgs g1) {
 
 bool fits(long bytes) { return bytes >= 0 && bytes < (1L << 31) - 64; }
 
-template <int BM, int BN, bool BIAS, bool PC, bool AT, bool BT>
+template <bool BIAS>
 int launch_gemm(const DenseArgs& a0, hipStream_t st) {
-  using Cfg = DenseCfg<BM, BN, AT, BT>;
-  auto kern = gemm_bf16_kernel<BM, BN, BIAS, PC, AT, BT>;
-  const size_t lds = Cfg::lds_bytes(PC);
+  auto kern = gemm_bf16_kernel<BIAS>;
   VH_LDS_LIMIT_ONCE(kern);
   DenseArgs a = a0;
-  a.tiles_m = (a.M + BM - 1) / BM;
-  a.tiles_n = (a.N + BN - 1) / BN;
-  a.cs_shift = colsum_shift(a.tiles_m, BN);
-  kern<<<dim3((unsigned)(a.tiles_m * a.tiles_n)), PC ? 512 : 256, lds, st>>>(a);
+  a.tiles_m = (a.M + DenseCfg::BM - 1) / DenseCfg::BM;
+  a.tiles_n = (a.N + DenseCfg::BN - 1) / DenseCfg::BN;
+  kern<<<dim3((unsigned)(a.tiles_m * a.tiles_n)), 512, (size_t)2 * DenseCfg::STAGE * 16, st>>>(a);
   VH_LAUNCH_CHECK();
   return VH_OK;
-}
-
-// 128 x 256 tiles (one block per CU, producer / consumer form, 64 x 128 per
-// consumer wave) when the grid still fills the chip, else 128 x 128 (two
-// blocks per CU of four waves that both load and multiply: already two waves
-// per SIMD, and measured as fast as or faster than a split form)
-template <bool AT, bool BT>
-int launch_layout(const DenseArgs& g, bool big, hipStream_t st) {
-  if (big)
-    return g.bias ? launch_gemm<128, 256, true, true, AT, BT>(g, st) : launch_gemm<128, 256, false, true, AT, BT>(g, st);
-  return g.bias ? launch_gemm<128, 128, true, false, AT, BT>(g, st) : launch_gemm<128, 128, false, false, AT, BT>(g, st);
 }
 
 }  // namespace
@@ -792,8 +597,8 @@ bool dense_big(int M, int N) { return (long)((M + 127) / 128) * ((N + 255) / 256
 // The 256 x 256 direct-to-LDS kernel: whole tiles only (no bounds checks in
 // its loads or stores), K in whole stages, 16-byte aligned rows of every
 // operand, and a grid of at least one block per CU.
-bool dense_d2l(const DenseArgs& g, bool colsum) {
-  return !colsum && g.M % 256 == 0 && g.N % 256 == 0 && g.K % (2 * kD2lBK) == 0 && g.vec_epi &&
+bool dense_d2l(const DenseArgs& g) {
+  return g.M % 256 == 0 && g.N % 256 == 0 && g.K % (2 * kD2lBK) == 0 && g.vec_epi &&
          (long)(g.M / 256) * (g.N / 256) >= 256;
 }
 
@@ -810,16 +615,16 @@ int launch_d2l(const DenseArgs& a0, hipStream_t st) {
 }  // namespace
 
 int dense_bf16_gemm(const void* a, int lda, bool at, const void* b, int ldb, bool bt, void* c, int ldc, int M,
-                    int N, int K, const void* bias, hipStream_t st, void* colsum) {
-  const bool big = dense_big(M, N);
-  if (colsum && (!bt || bias)) return VH_ERR_UNSUPPORTED;
-  const DenseArgs g = dense_args(a, lda, at, b, ldb, bt, c, ldc, M, N, K, bias, colsum);
-  if (dense_d2l(g, colsum != nullptr)) {
-    if (at) return bt ? launch_d2l<true, true>(g, st) : launch_d2l<true, false>(g, st);
+                    int N, int K, const void* bias, hipStream_t st) {
+  if (at && !bt) return VH_ERR_UNSUPPORTED;
+  const DenseArgs g = dense_args(a, lda, at, b, ldb, bt, c, ldc, M, N, K, bias, nullptr);
+  if (dense_d2l(g)) {
+    if (at) return launch_d2l<true, true>(g, st);
     return bt ? launch_d2l<false, true>(g, st) : launch_d2l<false, false>(g, st);
   }
-  if (at) return bt ? launch_layout<true, true>(g, big, st) : launch_layout<true, false>(g, big, st);
-  return bt ? launch_layout<false, true>(g, big, st) : launch_layout<false, false>(g, big, st);
+  // not whole tiles, at least one block per CU
+  if (at || !bt || !dense_big(M, N)) return VH_ERR_UNSUPPORTED;
+  return bias ? launch_gemm<true>(g, st) : launch_gemm<false>(g, st);
 }
 
 namespace {
@@ -835,20 +640,6 @@ int launch_d2l_pair(DenseArgs a0, DenseArgs a1, hipStream_t st) {
   return VH_OK;
 }
 
-template <int BN, bool PC>
-int launch_pair(DenseArgs a0, DenseArgs a1, hipStream_t st) {
-  for (DenseArgs* a : {&a0, &a1}) {
-    a->tiles_m = (a->M + 127) / 128;
-    a->tiles_n = (a->N + BN - 1) / BN;
-    a->cs_shift = colsum_shift(a->tiles_m, BN);
-  }
-  auto kern = gemm_bf16_pair_kernel<BN, PC, false, false, true, true>;
-  const size_t lds = std::max(DenseCfg<128, BN, false, false>::lds_bytes(PC), DenseCfg<128, BN, true, true>::lds_bytes(PC));
-  VH_LDS_LIMIT_ONCE(kern);
-  kern<<<dim3((unsigned)(a0.tiles_m * a0.tiles_n + a1.tiles_m * a1.tiles_n)), PC ? 512 : 256, lds, st>>>(a0, a1);
-  VH_LAUNCH_CHECK();
-  return VH_OK;
-}
 }  // namespace
 
 int dense_bf16_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStream_t st) {
@@ -866,8 +657,7 @@ int dense_bf16_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStre
   };
   if (whole(a0) && whole(a1) && (long)(a0.M / 128) * (a0.N / 256) + (long)(a1.M / 128) * (a1.N / 256) >= 256)
     return launch_d2l_pair(a0, a1, st);
-  const long t256 = (long)((p0.M + 127) / 128) * ((p0.N + 255) / 256) + (long)((p1.M + 127) / 128) * ((p1.N + 255) / 256);
-  return t256 >= 256 ? launch_pair<256, true>(a0, a1, st) : launch_pair<128, false>(a0, a1, st);
+  return VH_ERR_UNSUPPORTED;
 }
 
 }  // namespace vh

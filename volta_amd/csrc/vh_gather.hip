@@ -24,56 +24,16 @@
 // fragments come from transposing LDS reads (ds_read_b64_tr_b16), fp32 ones from
 // 4-byte reads.  Split over positions, fp32 partials added in a fixed order by
 // gather_wgrad_reduce_kernel.
-#include <type_traits>
-
 #include "vh_kernels.hpp"
+#include "vh_tiles.hpp"
 
 namespace vh {
 
 namespace {
 
-typedef unsigned int u32x4g __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2g __attribute__((ext_vector_type(2)));
+using namespace tiles;
 
-constexpr int kOORg = (int)0x80000000u;  // buffer offset past every range: loads 0, stores dropped
 constexpr int kMaxPhases = 16;
-constexpr long kMaxBytesG = (1L << 31) - 4096;  // every tensor is addressed with 32-bit byte offsets
-
-template <typename T>
-struct GT {
-  static constexpr int ES = sizeof(typename Elem<T>::storage);
-  static constexpr int UE = 16 / ES;   // elements per 16-byte unit
-  static constexpr int BK = 128 / ES;  // k per stage: 8 units per K-major row
-  // K-major fragment of one step (2 units): 8 bf16, or 4 fp32 = 4 MFMAs of 2 k
-  using frag = std::conditional_t<ES == 2, bf16x8, f32x4>;
-};
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_g(const void* p, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, bytes, 0x00020000);
-}
-
-// s_waitcnt vmcnt(0) lgkmcnt(0), then the block barrier
-__device__ __forceinline__ void gather_sync() {
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// all MFMAs of one fragment step: independent accumulators back to back
-template <int FM, int FN>
-__device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const bf16x8 (&a)[FM], const bf16x8 (&b)[FN]) {
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], c[i][j], 0, 0, 0);
-}
-template <int FM, int FN>
-__device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const f32x4 (&a)[FM], const f32x4 (&b)[FN]) {
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][t], b[j][t], c[i][j], 0, 0, 0);
-}
 
 // ---------------------------------------------------------------- preparation
 // One tensor copied from [N][C][H][W] to [N][Hp][Wp][Cp] with (padT, padL) zero
@@ -332,21 +292,15 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
   };
 
   const int row_l = lane & 31, half_l = lane >> 5;
-  // fragment of rows row0 .. +31, step kk: the lanes of half h take unit 2 kk + h
-  // (fp32: MFMA t of the step multiplies element t of both units)
-  auto read1 = [&](const char* tile, int row0, int kk) {
-    return __builtin_bit_cast(Frag, *reinterpret_cast<const u32x4g*>(
-                                        tile + (row0 + row_l) * 128 + ((2 * kk + half_l) ^ ((row_l >> 1) & 7)) * 16));
-  };
   struct Frags {
     Frag a[FM], b[FN];
   };
   auto read = [&](const u32x4g* st, int kk, Frags& q) {
     const char* at = reinterpret_cast<const char*>(st) + grp * (BM + BN) * 128;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) q.a[i] = read1(at, wm + 32 * i, kk);
+    for (int i = 0; i < FM; ++i) q.a[i] = read_k<T>(at, wm + 32 * i, kk, lane);
 #pragma unroll
-    for (int j = 0; j < FN; ++j) q.b[j] = read1(at + BM * 128, wn + 32 * j, kk);
+    for (int j = 0; j < FN; ++j) q.b[j] = read_k<T>(at + BM * 128, wn + 32 * j, kk, lane);
   };
   f32x16 acc[FM][FN];
 #pragma unroll
@@ -494,18 +448,6 @@ struct WgradArgs {
   FastDiv fPQ, fQ, fCU, fS;
 };
 
-// Operand tile of BK k rows (positions) x R columns: UR units per k row, copy
-// instruction c brings k rows (64 / UR) c ..; slot t of k row kr holds unit
-// t ^ swz(kr), which spreads a fragment's reads over the banks.
-template <typename T, int R>
-struct MnTile {
-  static constexpr int ES = GT<T>::ES, UR = R * ES / 16, RPI = 64 / UR, INSTR = GT<T>::BK / RPI, CPW = INSTR / 4;
-  __device__ static int swz(int kr) {
-    if (ES == 4) return 8 * (kr & 1);
-    return UR == 8 ? 4 * ((kr >> 1) & 1) : 4 * (kr & 3);
-  }
-};
-
 template <typename T, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   using G = GT<T>;
@@ -513,7 +455,8 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   using TB = MnTile<T, BN>;
   constexpr int ES = G::ES, UE = G::UE, BK = G::BK, FM = WM / 32, FN = WN / 32, NWN = BN / WN;
   constexpr int A_UNITS = BK * TA::UR, B_UNITS = BK * TB::UR;
-  static_assert((BM / WM) * (BN / WN) == 4 && TA::CPW >= 1 && TB::CPW >= 1, "tile");
+  constexpr int AC = BM / 32, BC = BN / 32;  // copy instructions per wave and stage
+  static_assert((BM / WM) * (BN / WN) == 4, "four waves");
   __shared__ __attribute__((aligned(16))) u32x4g S0[A_UNITS + B_UNITS];
   __shared__ __attribute__((aligned(16))) u32x4g S1[A_UNITS + B_UNITS];
 
@@ -529,9 +472,11 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave / NWN) * WM, wn = (wave % NWN) * WN;
 
-  // this lane's k row of copy instruction wave + 4 i, and its column unit
-  const int akr = TA::RPI * wave + lane / TA::UR, bkr = TB::RPI * wave + lane / TB::UR;
-  const int au = m0 / UE + ((lane % TA::UR) ^ TA::swz(akr)), bu = n0 / UE + ((lane % TB::UR) ^ TB::swz(bkr));
+  // this lane's k row of copy instruction wave + 4 i, and its column unit (the same
+  // for every i: 4 instructions are a multiple of the swizzle's period)
+  auto akr = [&](int i) { return TA::krow(TA::RPI * (wave + 4 * i) + lane / TA::UR); };
+  auto bkr = [&](int i) { return TB::krow(TB::RPI * (wave + 4 * i) + lane / TB::UR); };
+  const int au = m0 / UE + ((lane % TA::UR) ^ TA::swz(akr(0))), bu = n0 / UE + ((lane % TB::UR) ^ TB::swz(bkr(0)));
   const int acol = au * 16 < g.dcol ? au * 16 : kOORg;  // dcol = bytes of a dy position
   uint32_t tap, cu, r, c;
   g.fCU.divmod((uint32_t)bu, tap, cu);
@@ -547,90 +492,29 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
       return k < ke ? (int)n * img + (int)p * row + (int)q * col : kOORg;
     };
 #pragma unroll
-    for (int i = 0; i < TA::CPW; ++i)
-      lds_copy16(ar, place(k0 + akr + 4 * TA::RPI * i, g.dimg, g.drow, g.dcol) + acol, 0, la + (wave + 4 * i) * 1024);
+    for (int i = 0; i < AC; ++i)
+      lds_copy16(ar, place(k0 + akr(i), g.dimg, g.drow, g.dcol) + acol, 0, la + (wave + 4 * i) * 1024);
 #pragma unroll
-    for (int i = 0; i < TB::CPW; ++i)
-      lds_copy16(br, place(k0 + bkr + 4 * TB::RPI * i, g.ximg, g.xrow, g.xcol) + bcol, 0,
+    for (int i = 0; i < BC; ++i)
+      lds_copy16(br, place(k0 + bkr(i), g.ximg, g.xrow, g.xcol) + bcol, 0,
                  la + A_UNITS * 16 + (wave + 4 * i) * 1024);
   };
 
   const int row_l = lane & 31, half_l = lane >> 5;
-  typedef short v4i16 __attribute__((ext_vector_type(4)));
-  typedef short v8i16 __attribute__((ext_vector_type(8)));
-  // bf16, step of 16 k: fragment f of a wave's columns col0 .. is columns
-  // 32 f + lane % 32, by transposing reads (k rows 8 half + (lane & 15) / 4 and + 4)
-  auto read_tr = [&](auto TILE, const char* tile, int col, int kk) {
-    using Tl = decltype(TILE);
-    const int kr = 8 * half_l + ((lane & 15) >> 2);
-    const int in = (2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * 16 + 8 * (lane & 1);
-    const __attribute__((address_space(3))) char* q = (const __attribute__((address_space(3))) char*)tile +
-                                                      (16 * kk + kr) * Tl::UR * 16 + in + ((col >> 3) ^ Tl::swz(kr)) * 16;
-    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)q);
-    const v4i16 hi =
-        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(q + 4 * Tl::UR * 16));
-    const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    return __builtin_bit_cast(bf16x8, v);
+  struct Frags {
+    typename G::frag a[FM], b[FN];
   };
-  // fp32, step of 8 k (MFMA t: k rows 2 t and 2 t + 1 of it, one per half): with
-  // two fragments per wave they are the even and the odd columns, one 8-byte read
-  auto read_pair = [&](auto TILE, auto F, const char* tile, int col0, int kk, float (&v)[decltype(F)::value][4]) {
-    using Tl = decltype(TILE);
-    constexpr int N = decltype(F)::value;
-    const int col = col0 + N * row_l, u = (col >> 2) ^ (8 * half_l);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const char* q = tile + ((8 * kk + 2 * t + half_l) * Tl::UR + u) * 16 + (col & 3) * 4;
-      if constexpr (N == 2) {
-        const float2 p = *reinterpret_cast<const float2*>(q);
-        v[0][t] = p.x;
-        v[1][t] = p.y;
-      } else {
-        v[0][t] = *reinterpret_cast<const float*>(q);
-      }
-    }
-  };
-  static_assert(FM <= 2 && FN <= 2, "fragments per wave");
-  struct FragsB {
-    bf16x8 a[FM], b[FN];
-  };
-  struct FragsF {
-    float a[FM][4], b[FN][4];
-  };
-  using Frags = std::conditional_t<ES == 2, FragsB, FragsF>;
   auto read = [&](const u32x4g* st, int kk, Frags& q) {
     const char* at = reinterpret_cast<const char*>(st);
-    const char* bt = at + A_UNITS * 16;
-    if constexpr (ES == 2) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i) q.a[i] = read_tr(TA{}, at, wm + 32 * i, kk);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) q.b[j] = read_tr(TB{}, bt, wn + 32 * j, kk);
-    } else {
-      read_pair(TA{}, std::integral_constant<int, FM>{}, at, wm, kk, q.a);
-      read_pair(TB{}, std::integral_constant<int, FN>{}, bt, wn, kk, q.b);
-    }
+    read_mn<T, BM, FM>(at, wm, kk, lane, q.a);
+    read_mn<T, BN, FN>(at + A_UNITS * 16, wn, kk, lane, q.b);
   };
-  // row / column of the wave's tile that element e of fragment f stands for
-  auto spread = [&](int F, int f, int e) { return ES == 4 && F == 2 ? 2 * e + f : 32 * f + e; };
   f32x16 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
-  auto mma = [&](const Frags& q) {
-    if constexpr (ES == 2) {
-      mma_all<FM, FN>(acc, q.a, q.b);
-    } else {
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(q.a[i][t], q.b[j][t], acc[i][j], 0, 0, 0);
-    }
-  };
+  auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
 
   // bias gradient: the blocks of one m-tile share its BM columns of o; each sums
   // 4 << cs_shift of them from the staged tiles, a thread 4 columns of every
@@ -642,7 +526,7 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   auto colsum = [&](const u32x4g* st) {
     const char* at = reinterpret_cast<const char*>(st);
     for (int kr = cs_k0; kr < BK; kr += 256 >> g.cs_shift) {
-      const char* q = at + (kr * TA::UR + ((cs_c / UE) ^ TA::swz(kr))) * 16 + (cs_c % UE) * ES;
+      const char* q = at + (TA::krow(kr) * TA::UR + ((cs_c / UE) ^ TA::swz(kr))) * 16 + (cs_c % UE) * ES;
       if constexpr (ES == 2) {
         const u32x2g v = *reinterpret_cast<const u32x2g*>(q);
         csum[0] += __builtin_bit_cast(float, v[0] << 16);
@@ -698,12 +582,12 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const int row = m0 + wm + spread(FM, i, (v >> 2) * 8 + half_l * 4 + (v & 3));
+      const int row = m0 + wm + mn_spread<T, FM>(i, (v >> 2) * 8 + half_l * 4 + (v & 3));
       if (row < g.O) {
         float* d = g.part + ((size_t)z * g.O + row) * g.NC;
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          const int col = n0 + wn + spread(FN, j, row_l);
+          const int col = n0 + wn + mn_spread<T, FN>(j, row_l);
           if (col < g.NC) d[col] = acc[i][j][v];
         }
       }

@@ -188,15 +188,13 @@ int gather_run(int dt, const GatherCall& c, void* ws, hipStream_t st);
 // [N][ldb] or, with bt, [K][ldb].
 bool dense_bf16_ok(long M, long N, long K, bool at, long lda, bool bt, long ldb, long ldc, const void* a,
                    const void* b, const void* c);
-// colsum (bf16 [N], optional): also the column sums of B over K, for an
-// MN-major B on 128 x 128 tiles without bias (VH_ERR_UNSUPPORTED otherwise,
-// before anything is queued).
+// Whole 256 x 256 tiles, or 128 x 256 ones of a large K-major A and MN-major B;
+// VH_ERR_UNSUPPORTED for every other product.
 int dense_bf16_gemm(const void* a, int lda, bool at, const void* b, int ldb, bool bt, void* c, int ldc, int M,
-                    int N, int K, const void* bias, hipStream_t st, void* colsum = nullptr);
+                    int N, int K, const void* bias, hipStream_t st);
 // Two bias-free products in one launch (each checked by dense_bf16_ok): a
 // K-major A and B next to an MN-major A and B (with optional column sums of
-// that B), when both run 128 x 128 tiles; VH_ERR_UNSUPPORTED otherwise (the
-// caller then runs them one after the other).
+// that B), whole 128 x 256 tiles of both; VH_ERR_UNSUPPORTED otherwise.
 struct DenseProblem {
   const void* a;
   int lda;
@@ -209,14 +207,21 @@ struct DenseProblem {
   void* colsum;
 };
 int dense_bf16_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStream_t st);
-// The same in fp32 (vh_dense_f32.hip): K % 4 == 0, 16-byte aligned A and B.
+// The same in fp32 (vh_dense_f32.hip): K % 4 == 0, 16-byte aligned A and B; the
+// single product whole 256 x 256 tiles of an MN-major A and B.
 bool dense_f32_ok(long M, long N, long K, bool at, long lda, bool bt, long ldb, long ldc, const void* a,
                   const void* b, const void* c);
 int dense_f32_gemm(const void* a, int lda, bool at, const void* b, int ldb, bool bt, void* c, int ldc, int M,
-                   int N, int K, const void* bias, hipStream_t st);
-// Linear's dX and dW (+ column sums) in one launch, fp32 (each problem checked
-// by dense_f32_ok); VH_ERR_UNSUPPORTED: run them separately.
+                   int N, int K, hipStream_t st);
 int dense_f32_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStream_t st);
+
+// ---- products of any size (vh_mm.hip) ----
+// One product, or a Linear layer's dX (K-major x K-major) and dW (MN-major x
+// MN-major) as a pair; colsum (of an MN-major A and B): the column sums of B over K.
+// bias [N] of a single product.  Workspace bytes (possibly 0); *ok false: an empty
+// or too large (32-bit byte offsets) product.
+size_t mm_ws(int dt, const DenseProblem* p, int np, bool* ok);
+int mm_run(int dt, const DenseProblem* p, int np, const void* bias, void* ws, hipStream_t st);
 
 // ---- strided 1x1 bf16 convolutions, pad 0 (vh_pointwise.hip) ----
 // w is the OIHW weight itself ([O][C]).  Each returns VH_ERR_UNSUPPORTED

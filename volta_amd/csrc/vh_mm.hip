@@ -1,0 +1,581 @@
+// vh_mm.hip -- matrix products of any size (bf16 and fp32) that the large-tile
+// kernels of vh_dense.hip and vh_dense_f32.hip do not fill the chip with, or whose
+// rows they cannot load.
+//
+// C[M][N] = A . B (+ bias[N]); A is [M][K] or, "MN-major", [K][M]; B is [N][K] or
+// [K][N].  What bounds these products is not the matrix cores: 16 blocks of 256
+// CUs (256 x 784 -> 512 fp32: 43 us on 64 x 128 tiles), or operands whose rows are
+// not 16-byte aligned and were gathered element by element (K = 2001: 70 - 95 us a
+// product that takes 17 on whole units).  So
+//  * tiles are 64 x 64 and smaller, two to five blocks a CU; below one block a CU
+//    the four waves of a block split K (KS groups of waves, every KS-th stage each,
+//    added in group order), and what is still short is split over blocks (fp32
+//    partials, added in split order by mm_reduce_kernel);
+//  * operands whose rows are not whole 16-byte units are first copied to padded
+//    rows (mm_pad_kernel: both operands in one launch); the products then copy
+//    whole units straight into LDS (vh_tiles.hpp).
+// A Linear layer's two gradients go in one launch, the bias gradient as column
+// sums of the staged dY tiles.
+#include "vh_kernels.hpp"
+#include "vh_tiles.hpp"
+
+namespace vh {
+
+namespace {
+
+using namespace tiles;
+
+struct MmArgs {
+  const void *a, *b;
+  void* c;           // [M][ldc], or fp32 partials [split][M][N]
+  const void* bias;  // [N] or nullptr
+  void* colsum;      // [N] (element type, one split) or fp32 [split][N], or nullptr: column sums of B
+  int M, N, K, lda, ldb, ldc;
+  int a_bytes, b_bytes, c_bytes;
+  int tiles_m, tiles_n, splits, per;  // stages per split
+  int cs_shift;      // column sums: 4 << cs_shift columns per block
+};
+
+// One BM x BN tile (logical block lb).  S0, S1: two LDS stages.
+template <typename T, int BM, int BN, int WM, int WN, bool AT, bool BT, bool CS>
+__device__ __forceinline__ void mm_tile(const MmArgs& g, const int lb, u32x4g* S0, u32x4g* S1) {
+  using ST = typename Elem<T>::storage;
+  using G = GT<T>;
+  using TA = MnTile<T, BM>;
+  using TB = MnTile<T, BN>;
+  constexpr int ES = G::ES, UE = G::UE, BK = G::BK, FM = WM / 32, FN = WN / 32, NWN = BN / WN;
+  constexpr int WPG = (BM / WM) * (BN / WN), KS = 4 / WPG;  // waves per group, groups
+  constexpr int AC = BM / 8 / WPG, BC = BN / 8 / WPG, GS = (BM + BN) * 8;  // copies per wave; units per group
+  static_assert(WPG * KS == 4 && AC >= 1 && BC >= 1, "four waves");
+
+  const int nt = g.tiles_m * g.tiles_n, z = lb / nt, tl = lb - z * nt;
+  // column-major groups of 8 row tiles: a group shares its B panel in L2
+  const int grp8 = tl / (8 * g.tiles_n), gm = min(g.tiles_m - grp8 * 8, 8), ing = tl - grp8 * 8 * g.tiles_n;
+  const int tm = grp8 * 8 + ing % gm, tn = ing / gm, m0 = tm * BM, n0 = tn * BN;
+  const int kb = z * g.per * BK, ke = min(g.K, kb + g.per * BK);
+  const int nst = (ke - kb + BK - 1) / BK;
+
+  const int tid = threadIdx.x, lane = tid & 63, row_l = lane & 31, half_l = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), grp = wv / WPG, wave = wv % WPG;
+  const int wm = (wave / NWN) * WM, wn = (wave % NWN) * WN;
+
+  // copy instruction c = wave + WPG i of an operand: byte offset of this lane's unit
+  // in stage 0, and the k (K-major: of the unit; MN-major: row) it stands for
+  struct Unit {
+    int off, k;
+  };
+  auto unit = [&](auto MN, auto TILE, int rows, int r0, int ld, int c) {
+    using Tl = decltype(TILE);
+    Unit u;
+    if constexpr (decltype(MN)::value) {
+      const int kr = Tl::krow(Tl::RPI * c + lane / Tl::UR);
+      const int col = r0 + ((lane % Tl::UR) ^ Tl::swz(kr)) * UE;
+      u.k = kr;
+      u.off = col < rows ? (kr * ld + col) * ES : kOORg;
+    } else {
+      const int r = 8 * c + (lane >> 3), ku = (lane & 7) ^ ((r >> 1) & 7);
+      u.k = ku * UE;
+      u.off = r0 + r < rows ? ((r0 + r) * ld + ku * UE) * ES : kOORg;
+    }
+    return u;
+  };
+  Unit ua[AC], ub[BC];
+#pragma unroll
+  for (int i = 0; i < AC; ++i) ua[i] = unit(std::integral_constant<bool, AT>{}, TA{}, g.M, m0, g.lda, wave + WPG * i);
+#pragma unroll
+  for (int i = 0; i < BC; ++i) ub[i] = unit(std::integral_constant<bool, BT>{}, TB{}, g.N, n0, g.ldb, wave + WPG * i);
+  const __amdgpu_buffer_rsrc_t ar = rsrc_g(g.a, g.a_bytes), br = rsrc_g(g.b, g.b_bytes);
+  const int astep = AT ? g.lda * ES : ES, bstep = BT ? g.ldb * ES : ES;  // bytes per k
+  auto issue = [&](u32x4g* st, int sk) {
+    const int k0 = kb + (sk * KS + grp) * BK;  // this group's stage
+    const uint32_t la = lds_byte_addr(st) + grp * GS * 16;
+    // k at or past the end of the split: out of every range (sign bit)
+    const int ask = (int)((uint32_t)k0 * astep), bsk = (int)((uint32_t)k0 * bstep), left = ke - 1 - k0;
+#pragma unroll
+    for (int i = 0; i < AC; ++i)
+      lds_copy16(ar, (ua[i].off + ask) | ((left - ua[i].k) & kOORg), 0, la + (wave + WPG * i) * 1024);
+#pragma unroll
+    for (int i = 0; i < BC; ++i)
+      lds_copy16(br, (ub[i].off + bsk) | ((left - ub[i].k) & kOORg), 0,
+                 la + BM * 128 + (wave + WPG * i) * 1024);
+  };
+
+  struct Frags {
+    typename G::frag a[FM], b[FN];
+  };
+  auto read = [&](const u32x4g* st, int kk, Frags& q) {
+    const char* at = reinterpret_cast<const char*>(st + grp * GS);
+    const char* bt = at + BM * 128;
+    if constexpr (AT) {
+      read_mn<T, BM, FM>(at, wm, kk, lane, q.a);
+    } else {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) q.a[i] = read_k<T>(at, wm + 32 * i, kk, lane);
+    }
+    if constexpr (BT) {
+      read_mn<T, BN, FN>(bt, wn, kk, lane, q.b);
+    } else {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) q.b[j] = read_k<T>(bt, wn + 32 * j, kk, lane);
+    }
+  };
+  f32x16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+  auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
+
+  // column sums (B MN-major): the blocks of one column tile share its columns, each
+  // sums 4 << cs_shift of them from the staged tiles, a thread 4 columns of every
+  // (256 / ng)-th k row of all groups
+  const int cs_w = 4 << g.cs_shift, cs_c0 = tm * cs_w, ng = cs_w >> 2;
+  const bool cs_blk = CS && g.colsum != nullptr && cs_c0 < BN;
+  const int cs_c = cs_c0 + 4 * (tid & (ng - 1)), cs_k0 = tid >> g.cs_shift;
+  float csum[4] = {0.f, 0.f, 0.f, 0.f};
+  auto colsum = [&](const u32x4g* st) {
+    for (int r = cs_k0; r < KS * BK; r += 256 >> g.cs_shift) {
+      const int kr = r % BK;
+      const char* q = reinterpret_cast<const char*>(st + (r / BK) * GS) + BM * 128 +
+                      (TB::krow(kr) * TB::UR + ((cs_c / UE) ^ TB::swz(kr))) * 16 + (cs_c % UE) * ES;
+      if constexpr (ES == 2) {
+        const u32x2g v = *reinterpret_cast<const u32x2g*>(q);
+        csum[0] += __builtin_bit_cast(float, v[0] << 16);
+        csum[1] += __builtin_bit_cast(float, v[0] & 0xffff0000u);
+        csum[2] += __builtin_bit_cast(float, v[1] << 16);
+        csum[3] += __builtin_bit_cast(float, v[1] & 0xffff0000u);
+      } else {
+        const float4 v = *reinterpret_cast<const float4*>(q);
+        csum[0] += v.x;
+        csum[1] += v.y;
+        csum[2] += v.z;
+        csum[3] += v.w;
+      }
+    }
+  };
+
+  // the loop of vh_gather.hip: copies of stage s+1 in flight, reads of the next
+  // step ahead of the MFMAs of this one
+  Frags fa, fb;
+  const int ns = (nst + KS - 1) / KS;
+  issue(S0, 0);
+  gather_sync();
+  read(S0, 0, fa);
+  auto body = [&](auto BUF, int s) {
+    constexpr int B = decltype(BUF)::value;
+    u32x4g* cur = B == 0 ? S0 : S1;
+    u32x4g* nxt = B == 0 ? S1 : S0;
+    if (s + 1 < ns) issue(nxt, s + 1);
+    if constexpr (CS) {
+      if (cs_blk) colsum(cur);
+    }
+#pragma unroll
+    for (int kk = 1; kk < 4; kk += 2) {
+      read(cur, kk, fb);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(fa);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kk + 1 < 4) {
+        read(cur, kk + 1, fa);
+      } else if (s + 1 < ns) {
+        gather_sync();
+        read(nxt, 0, fa);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      mma(fb);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int s = 0;
+  for (; s + 1 < ns; s += 2) {
+    body(std::integral_constant<int, 0>{}, s);
+    body(std::integral_constant<int, 1>{}, s + 1);
+  }
+  if (s < ns) body(std::integral_constant<int, 0>{}, s);
+
+  float* red = reinterpret_cast<float*>(S0);
+  if constexpr (CS) {
+    if (cs_blk) {  // the k-row group sums, added in group order
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[cs_k0 * cs_w + cs_c - cs_c0 + e] = csum[e];
+      __syncthreads();
+      const int n = n0 + cs_c0 + tid;
+      if (tid < cs_w && cs_c0 + tid < BN && n < g.N) {
+        float t = 0.f;
+        for (int j = 0; j < 256 >> g.cs_shift; ++j) t += red[j * cs_w + tid];
+        if (g.splits > 1)
+          reinterpret_cast<float*>(g.colsum)[(size_t)z * g.N + n] = t;
+        else
+          reinterpret_cast<ST*>(g.colsum)[n] = Elem<T>::from_f32(t);
+      }
+    }
+  }
+  if constexpr (KS > 1) {  // the groups' sums, added in group order
+    constexpr int TILE = FM * FN * 1024;
+    static_assert((KS - 1) * WPG * TILE * 4 <= KS * GS * 16, "group sums exceed a stage");
+    __syncthreads();
+    if (grp > 0) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            red[((grp - 1) * WPG + wave) * TILE + ((i * FN + j) * 16 + v) * 64 + lane] = acc[i][j][v];
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int q = 0; q < KS - 1; ++q)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][j][v] += red[(q * WPG + wave) * TILE + ((i * FN + j) * 16 + v) * 64 + lane];
+  }
+
+  // epilogue: lanes walk columns
+  const bool part = g.splits > 1;
+  const ST* bias = reinterpret_cast<const ST*>(g.bias);
+  const __amdgpu_buffer_rsrc_t cr = rsrc_g(g.c, g.c_bytes);
+  const int es = part ? 4 : ES, ld = part ? g.N : g.ldc, zoff = part ? z * g.M * g.N * 4 : 0;
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int col = n0 + wn + (BT ? mn_spread<T, FN>(j, row_l) : 32 * j + row_l);
+    const float bv = bias && col < g.N ? Elem<T>::to_f32(bias[col]) : 0.f;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int e = (v >> 2) * 8 + half_l * 4 + (v & 3);
+        const int row = m0 + wm + (AT ? mn_spread<T, FM>(i, e) : 32 * i + e);
+        const int o = row < g.M && col < g.N ? zoff + (row * ld + col) * es : kOORg;
+        const float r = acc[i][j][v] + bv;
+        if (ES == 2 && !part)
+          __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, (__bf16)r), cr, o, 0, 0);
+        else
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), cr, o, 0, 0);
+      }
+  }
+}
+
+template <int BM, int BN, int WM, int WN>
+constexpr int mm_stage() {  // units
+  return 4 / ((BM / WM) * (BN / WN)) * (BM + BN) * 8;
+}
+
+template <typename T, int BM, int BN, int WM, int WN, bool AT, bool BT>
+__global__ __launch_bounds__(256) void mm_kernel(MmArgs g) {
+  __shared__ __attribute__((aligned(16))) u32x4g S0[mm_stage<BM, BN, WM, WN>()];
+  __shared__ __attribute__((aligned(16))) u32x4g S1[mm_stage<BM, BN, WM, WN>()];
+  mm_tile<T, BM, BN, WM, WN, AT, BT, AT && BT>(g, xcd_block(gridDim.x), S0, S1);
+}
+
+// Linear's dX (K-major x K-major) and dW (MN-major x MN-major, with the bias
+// gradient) in one launch: blocks 0 .. t0-1 take dX's tiles, the rest dW's.
+template <typename T, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256) void mm_pair_kernel(MmArgs g0, MmArgs g1) {
+  __shared__ __attribute__((aligned(16))) u32x4g S0[mm_stage<BM, BN, WM, WN>()];
+  __shared__ __attribute__((aligned(16))) u32x4g S1[mm_stage<BM, BN, WM, WN>()];
+  const int t0 = g0.tiles_m * g0.tiles_n * g0.splits, h = blockIdx.x;
+  if (h < t0)
+    mm_tile<T, BM, BN, WM, WN, false, false, false>(g0, xcd_map(h, t0), S0, S1);
+  else
+    mm_tile<T, BM, BN, WM, WN, true, true, true>(g1, xcd_map(h - t0, g1.tiles_m * g1.tiles_n * g1.splits), S0, S1);
+}
+
+// Split products: C (+ bias) and the column sums from the fp32 partials, in split
+// order; blocks b0 .. take a second product's (the pair's dW), ..
+struct MmReduce {
+  const float *part, *cpart;
+  void *c, *colsum;
+  const void* bias;
+  int M, N, ldc, splits, nb, nbc;  // blocks of C and of the column sums
+  FastDiv fN;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void mm_reduce_kernel(MmReduce r0, MmReduce r1) {
+  using ST = typename Elem<T>::storage;
+  const bool first = (int)blockIdx.x < r0.nb + r0.nbc;
+  const MmReduce& r = first ? r0 : r1;
+  const int b = (int)blockIdx.x - (first ? 0 : r0.nb + r0.nbc);
+  const ST* bias = reinterpret_cast<const ST*>(r.bias);
+  if (b < r.nb)
+    reduce_splits_block(r.part, r.splits, (long)r.M * r.N,
+                        [&](long i, float v) {
+                          uint32_t row, col;
+                          r.fN.divmod((uint32_t)i, row, col);
+                          if (bias) v += Elem<T>::to_f32(bias[col]);
+                          reinterpret_cast<ST*>(r.c)[(size_t)row * r.ldc + col] = Elem<T>::from_f32(v);
+                        },
+                        b, r.nb);
+  else
+    reduce_splits_block(r.cpart, r.splits, r.N,
+                        [&](long i, float v) { reinterpret_cast<ST*>(r.colsum)[i] = Elem<T>::from_f32(v); }, b - r.nb, r.nbc);
+}
+
+// Rows of `cols` elements copied to rows of whole 16-byte units (zeros past the
+// end): one unit per thread, a wave's loads contiguous but for the row ends.
+struct PadSeg {
+  const void* src;
+  void* dst;
+  long total;  // units
+  int cols, ld, upr;
+  FastDiv fupr;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void mm_pad_kernel(PadSeg p0, PadSeg p1, int b0) {
+  using ST = typename Elem<T>::storage;
+  constexpr int UE = GT<T>::UE;
+  const PadSeg& p = (int)blockIdx.x < b0 ? p0 : p1;
+  const long id = (long)((int)blockIdx.x < b0 ? blockIdx.x : blockIdx.x - b0) * 256 + threadIdx.x;
+  if (id >= p.total) return;
+  uint32_t row, u;
+  p.fupr.divmod((uint32_t)id, row, u);
+  const ST* s = reinterpret_cast<const ST*>(p.src) + (size_t)row * p.ld + u * UE;
+  uint4 q;
+  if ((int)(u + 1) * UE <= p.cols) {
+    __builtin_memcpy(&q, s, 16);  // one load at the element's alignment
+  } else {
+    ST v[UE];
+#pragma unroll
+    for (int j = 0; j < UE; ++j) v[j] = (int)u * UE + j < p.cols ? s[j] : (ST)0;
+    __builtin_memcpy(&q, v, 16);
+  }
+  reinterpret_cast<uint4*>(p.dst)[id] = q;
+}
+
+// ---------------------------------------------------------------- host side
+size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
+
+struct Tile {
+  int bm, bn;
+};
+
+// The tile of a product, or of a pair launched together (both grids counted), by
+// its cost: rounds of 256 blocks, each of the tile's own weight.  The weights are
+// the times of one round of blocks at K = 4096 relative to 64 x 64 (bf16 4096^3:
+// 108, 143, 175, 252, 505 us on 128 x 128 .. 32 x 32; fp32 978, 1043, 1231 on the
+// last three, the larger ones gain nothing).  A bf16 block alone on a CU cannot
+// cover its copies: less than 1.7 rounds cost as much (2048^3: 30 us on 256 blocks
+// of 128 x 128, 24 on 512 of 64 x 128; 1024^3: 22, 9.4, 7.7, 7.0, 11.5).
+template <typename T>
+Tile mm_pick(const DenseProblem* p, int np) {
+  struct Cand {
+    Tile t;
+    float w;
+  };
+  static constexpr Cand kBf16[] = {{{128, 128}, 2.46f}, {{64, 128}, 1.5f}, {{64, 64}, 1.f}, {{32, 64}, 0.72f}, {{32, 32}, 0.72f}};
+  static constexpr Cand kF32[] = {{{64, 64}, 1.f}, {{32, 64}, 0.54f}, {{32, 32}, 0.3125f}};
+  const bool b16 = GT<T>::ES == 2;
+  const Cand* c = b16 ? kBf16 + (np > 1 ? 2 : 0) : kF32;  // pairs: 64 x 64 and below
+  const int nc = b16 && np == 1 ? 5 : 3;
+  Tile best{64, 64};
+  float least = 1e30f;
+  for (int k = 0; k < nc; ++k) {
+    long n = 0;
+    for (int i = 0; i < np; ++i) n += (long)((p[i].M + c[k].t.bm - 1) / c[k].t.bm) * ((p[i].N + c[k].t.bn - 1) / c[k].t.bn);
+    const float cost = c[k].w * std::max((float)((n + 255) / 256), b16 ? 1.7f : 1.f);
+    if (cost < least) {
+      least = cost;
+      best = c[k].t;
+    }
+  }
+  return best;
+}
+
+template <typename T>
+void mm_plan(MmArgs& a, const Tile& t, long blocks) {
+  constexpr int BK = GT<T>::BK;
+  const int ks = t.bm == 32 ? (t.bn == 32 ? 4 : 2) : 1;
+  const int stages = (a.K + BK - 1) / BK;
+  a.tiles_m = (a.M + t.bm - 1) / t.bm;
+  a.tiles_n = (a.N + t.bn - 1) / t.bn;
+  // below half the CUs: split K for a block on each, at least 2 stages of every
+  // wave group (fp32 32 x 4096 x 64, 2 blocks: 23 -> 6.8 us at 16 splits; 128 x 8192
+  // x 256: 47 -> 11.6).  A bf16 product of over 32 blocks loses more to the partials
+  // (512 x 4096 x 128: 9.9 us, 15 split by 4).
+  int want = blocks < (GT<T>::ES == 2 ? 33 : 128) ? (int)std::min<long>(256 / blocks, stages / (2 * ks)) : 1;
+  want = std::max(1, want);
+  a.per = (stages + want - 1) / want;
+  a.splits = (stages + a.per - 1) / a.per;
+}
+
+// An operand with its rows as whole 16-byte units: stored rows (K-major: M or N;
+// MN-major: K) of `cols` elements.
+struct Opnd {
+  const void* p;
+  int rows, cols, ld, ldp;  // ldp: the padded copy's pitch, 0 if none is needed
+  size_t bytes;             // of the copy
+};
+template <typename T>
+Opnd opnd(const void* p, int rows, int cols, int ld) {
+  constexpr int UE = GT<T>::UE;
+  Opnd o{p, rows, cols, ld, 0, 0};
+  if (cols % UE || ld % UE || ((uintptr_t)p & 15)) {
+    o.ldp = (cols + UE - 1) / UE * UE;
+    o.bytes = align256((size_t)rows * o.ldp * GT<T>::ES);
+  }
+  return o;
+}
+
+struct MmLayout {
+  Opnd a[2], b[2];
+  MmArgs g[2];
+  Tile t;
+  size_t part[2], cpart[2], copies, bytes;
+  bool shared;
+};
+
+template <typename T>
+bool mm_layout(const DenseProblem* p, int np, const void* bias, MmLayout& l) {
+  constexpr int ES = GT<T>::ES;
+  l.bytes = 0;
+  l.t = mm_pick<T>(p, np);
+  long blocks = 0;
+  for (int i = 0; i < np; ++i) blocks += (long)((p[i].M + l.t.bm - 1) / l.t.bm) * ((p[i].N + l.t.bn - 1) / l.t.bn);
+  if (blocks > (1L << 30)) return false;
+  for (int i = 0; i < np; ++i) {
+    const DenseProblem& q = p[i];
+    if (q.M <= 0 || q.N <= 0 || q.K <= 0 || (q.at && !q.bt)) return false;
+    l.a[i] = opnd<T>(q.a, q.at ? q.K : q.M, q.at ? q.M : q.K, q.lda);
+    l.b[i] = opnd<T>(q.b, q.bt ? q.K : q.N, q.bt ? q.N : q.K, q.ldb);
+    MmArgs& g = l.g[i];
+    g = MmArgs{};
+    g.M = q.M;
+    g.N = q.N;
+    g.K = q.K;
+    g.lda = l.a[i].ldp ? l.a[i].ldp : q.lda;
+    g.ldb = l.b[i].ldp ? l.b[i].ldp : q.ldb;
+    g.ldc = q.ldc;
+    g.c = q.c;
+    g.bias = bias;
+    g.colsum = q.colsum;
+    mm_plan<T>(g, l.t, blocks);
+    g.cs_shift = colsum_shift(g.tiles_m, l.t.bn);
+    // with slack: a stage's addresses run past the last row
+    const long ab = ((long)l.a[i].rows + 64) * g.lda * ES, bb = ((long)l.b[i].rows + 64) * g.ldb * ES;
+    const long cb = (long)q.M * q.ldc * ES, pb = g.splits > 1 ? (long)g.splits * q.M * q.N * 4 : 0;
+    if (std::max({ab, bb, cb, pb, (long)q.M * q.N}) > kMaxBytesG) return false;
+    // bytes of the operand as stored: the last row may end before its pitch
+    g.a_bytes = (int)(((long)l.a[i].rows - 1) * g.lda * ES + (l.a[i].ldp ? l.a[i].ldp : l.a[i].cols) * ES);
+    g.b_bytes = (int)(((long)l.b[i].rows - 1) * g.ldb * ES + (l.b[i].ldp ? l.b[i].ldp : l.b[i].cols) * ES);
+    g.c_bytes = (int)(pb ? pb : ((long)q.M - 1) * q.ldc * ES + (long)q.N * ES);
+    l.part[i] = l.bytes;
+    l.bytes += align256((size_t)pb);
+    l.cpart[i] = l.bytes;
+    if (pb && q.colsum) l.bytes += align256((size_t)g.splits * q.N * 4);
+  }
+  // one copy of dY, the rows of dX's A and the k rows of dW's B
+  l.shared = np == 2 && l.b[1].p == l.a[0].p && l.b[1].rows == l.a[0].rows && l.b[1].cols == l.a[0].cols;
+  l.copies = l.bytes;
+  for (int i = 0; i < np; ++i) l.bytes += l.a[i].bytes + (i == 1 && l.shared ? 0 : l.b[i].bytes);
+  return true;
+}
+
+template <typename T, int BM, int BN, int WM, int WN>
+void mm_launch(const MmArgs* g, int np, bool at, bool bt, hipStream_t st) {
+  const unsigned n = (unsigned)(g[0].tiles_m * g[0].tiles_n * g[0].splits);
+  if (np == 2) {
+    if constexpr (BM * BN <= 4096) {
+      const unsigned n1 = (unsigned)(g[1].tiles_m * g[1].tiles_n * g[1].splits);
+      mm_pair_kernel<T, BM, BN, WM, WN><<<dim3(n + n1), 256, 0, st>>>(g[0], g[1]);
+    }
+    return;
+  }
+  if (at && bt)
+    mm_kernel<T, BM, BN, WM, WN, true, true><<<dim3(n), 256, 0, st>>>(g[0]);
+  else if (bt)
+    mm_kernel<T, BM, BN, WM, WN, false, true><<<dim3(n), 256, 0, st>>>(g[0]);
+  else
+    mm_kernel<T, BM, BN, WM, WN, false, false><<<dim3(n), 256, 0, st>>>(g[0]);
+}
+
+template <typename T>
+int mm_run_t(const DenseProblem* p, int np, const void* bias, char* ws, hipStream_t st) {
+  MmLayout l;
+  if (!mm_layout<T>(p, np, bias, l)) return VH_ERR_UNSUPPORTED;
+  size_t at = l.copies;
+  PadSeg seg[4];
+  int ns = 0;
+  auto place = [&](const Opnd& o) -> const void* {
+    if (!o.ldp) return o.p;
+    PadSeg& s = seg[ns++];
+    s.src = o.p;
+    s.dst = ws + at;
+    s.cols = o.cols;
+    s.ld = o.ld;
+    s.upr = o.ldp / GT<T>::UE;
+    s.total = (long)o.rows * s.upr;
+    s.fupr = FastDiv((uint32_t)s.upr);
+    at += o.bytes;
+    return s.dst;
+  };
+  for (int i = 0; i < np; ++i) {
+    l.g[i].a = place(l.a[i]);
+    l.g[i].b = i == 1 && l.shared ? l.g[0].a : place(l.b[i]);
+  }
+  for (int i = 0; i < ns; i += 2) {
+    PadSeg none{};
+    none.fupr = FastDiv(1);
+    const PadSeg& s1 = i + 1 < ns ? seg[i + 1] : none;
+    const long b0 = (seg[i].total + 255) / 256, b1 = (s1.total + 255) / 256;
+    mm_pad_kernel<T><<<dim3((unsigned)(b0 + b1)), 256, 0, st>>>(seg[i], s1, (int)b0);
+    VH_LAUNCH_CHECK();
+  }
+  MmReduce r[2] = {};
+  int nb = 0;
+  for (int i = 0; i < np; ++i) {
+    MmArgs& g = l.g[i];
+    if (g.splits <= 1) continue;
+    r[i].part = reinterpret_cast<float*>(ws + l.part[i]);
+    r[i].c = g.c;
+    r[i].bias = g.bias;
+    r[i].M = g.M;
+    r[i].N = g.N;
+    r[i].ldc = g.ldc;
+    r[i].splits = g.splits;
+    r[i].nb = reduce_splits_grid((long)g.M * g.N);
+    r[i].fN = FastDiv((uint32_t)g.N);
+    g.c = ws + l.part[i];
+    g.bias = nullptr;
+    if (g.colsum) {
+      r[i].cpart = reinterpret_cast<float*>(ws + l.cpart[i]);
+      r[i].colsum = g.colsum;
+      r[i].nbc = reduce_splits_grid(g.N);
+      g.colsum = ws + l.cpart[i];
+    }
+    nb += r[i].nb + r[i].nbc;
+  }
+  const bool ta = p[0].at, tb = p[0].bt;
+  if constexpr (GT<T>::ES == 2) {
+    if (l.t.bm == 128) mm_launch<T, 128, 128, 64, 64>(l.g, np, ta, tb, st);
+    if (l.t.bm == 64 && l.t.bn == 128) mm_launch<T, 64, 128, 32, 64>(l.g, np, ta, tb, st);
+  }
+  if (l.t.bm == 64 && l.t.bn == 64) mm_launch<T, 64, 64, 32, 32>(l.g, np, ta, tb, st);
+  if (l.t.bm == 32 && l.t.bn == 64) mm_launch<T, 32, 64, 32, 32>(l.g, np, ta, tb, st);
+  if (l.t.bm == 32 && l.t.bn == 32) mm_launch<T, 32, 32, 32, 32>(l.g, np, ta, tb, st);
+  VH_LAUNCH_CHECK();
+  if (nb) {
+    mm_reduce_kernel<T><<<dim3((unsigned)nb), 256, 0, st>>>(r[0], r[1]);
+    VH_LAUNCH_CHECK();
+  }
+  return VH_OK;
+}
+
+}  // namespace
+
+size_t mm_ws(int dt, const DenseProblem* p, int np, bool* ok) {
+  MmLayout l;
+  *ok = dt == VH_BF16 ? mm_layout<bf16>(p, np, nullptr, l) : mm_layout<float>(p, np, nullptr, l);
+  return *ok ? l.bytes : 0;
+}
+
+int mm_run(int dt, const DenseProblem* p, int np, const void* bias, void* ws, hipStream_t st) {
+  return dt == VH_BF16 ? mm_run_t<bf16>(p, np, bias, static_cast<char*>(ws), st)
+                       : mm_run_t<float>(p, np, bias, static_cast<char*>(ws), st);
+}
+
+}  // namespace vh

@@ -1,0 +1,138 @@
+// vh_tiles.hpp -- operand tiles of the direct-to-LDS products (vh_gather.hip,
+// vh_mm.hip) on gfx950 MFMA: their layouts in LDS and the fragment reads.
+//
+// A stage holds 128 bytes of k per row of the product (64 k bf16, 32 fp32) of both
+// operands, copied by buffer_load_dwordx4 ... lds: the 64 16-byte units of a copy
+// instruction land contiguously, so a layout is set by which unit each lane fetches.
+//  * K-major tile (R rows x 8 units): slot t of row r holds k unit t ^ ((r >> 1) & 7).
+//  * MN-major tile (k rows of R columns, UR units each): slot t of k row kr holds
+//    unit t ^ swz(kr).
+// A step is 32 bytes of k.  K-major: the lanes of half h (lane / 32) take unit
+// 2 kk + h of their row in one 16-byte read -- 8 bf16, or 4 fp32 for four MFMAs of
+// 2 k.  MN-major tiles give the same k to the same half.
+#pragma once
+#include <type_traits>
+
+#include "vh_common.hpp"
+
+namespace vh {
+
+namespace tiles {
+
+typedef unsigned int u32x4g __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2g __attribute__((ext_vector_type(2)));
+
+constexpr int kOORg = (int)0x80000000u;  // buffer offset past every range: loads 0, stores dropped
+constexpr long kMaxBytesG = (1L << 31) - 4096;  // tensors are addressed with 32-bit byte offsets
+
+template <typename T>
+struct GT {
+  static constexpr int ES = sizeof(typename Elem<T>::storage);
+  static constexpr int UE = 16 / ES;   // elements per 16-byte unit
+  static constexpr int BK = 128 / ES;  // k per stage: 8 units per K-major row
+  using frag = std::conditional_t<ES == 2, bf16x8, f32x4>;
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_g(const void* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, bytes, 0x00020000);
+}
+
+// s_waitcnt vmcnt(0) lgkmcnt(0), then the block barrier
+__device__ __forceinline__ void gather_sync() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// all MFMAs of one fragment step: independent accumulators back to back
+template <int FM, int FN>
+__device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const bf16x8 (&a)[FM], const bf16x8 (&b)[FN]) {
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], c[i][j], 0, 0, 0);
+}
+template <int FM, int FN>
+__device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const f32x4 (&a)[FM], const f32x4 (&b)[FN]) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][t], b[j][t], c[i][j], 0, 0, 0);
+}
+
+// Fragment of rows row0 .. +31 of a K-major tile, step kk.
+template <typename T>
+__device__ __forceinline__ typename GT<T>::frag read_k(const char* tile, int row0, int kk, int lane) {
+  const int r = lane & 31;
+  return __builtin_bit_cast(typename GT<T>::frag,
+                            *reinterpret_cast<const u32x4g*>(tile + (row0 + r) * 128 +
+                                                             ((2 * kk + (lane >> 5)) ^ ((r >> 1) & 7)) * 16));
+}
+
+// MN-major tile of R columns: copy instruction c brings the k rows (64 / UR) c ..
+template <typename T, int R>
+struct MnTile {
+  static constexpr int ES = GT<T>::ES, UR = R * ES / 16, RPI = 64 / UR;
+  // the swizzle puts what the two halves (fp32: k rows 4 apart) or the four k rows
+  // of a transposing read (bf16) take onto different banks
+  __device__ static int swz(int kr) {
+    if (ES == 4) return UR >= 16 ? 8 * ((kr >> 2) & 1) : 0;
+    return UR >= 16 ? 4 * (kr & 3) : UR == 8 ? 4 * ((kr >> 1) & 1) : 0;
+  }
+  // k row held in row pr of the tile: fp32 rows of 128 bytes change places instead
+  // of slots (an involution)
+  __device__ static int krow(int pr) { return ES == 4 && UR == 8 ? pr ^ ((pr >> 2) & 1) : pr; }
+};
+
+// Fragments of F * 32 columns col0 .. of an MN-major tile, step kk.  bf16: fragment
+// f is columns 32 f .. 32 f + 31, by transposing reads; fp32 with two fragments:
+// the even and the odd columns, one 8-byte read per k (mn_spread).
+template <typename T, int R, int F>
+__device__ __forceinline__ void read_mn(const char* tile, int col0, int kk, int lane, typename GT<T>::frag (&v)[F]) {
+  using Tl = MnTile<T, R>;
+  const int row_l = lane & 31, half_l = lane >> 5;
+  if constexpr (Tl::ES == 2) {
+    typedef short v4i16 __attribute__((ext_vector_type(4)));
+    typedef short v8i16 __attribute__((ext_vector_type(8)));
+    // k rows 16 kk + 8 half + (lane & 15) / 4 and + 4
+    const int kr = 8 * half_l + ((lane & 15) >> 2);
+    const int in = (2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * 16 + 8 * (lane & 1);
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const __attribute__((address_space(3))) char* q = (const __attribute__((address_space(3))) char*)tile +
+                                                        (16 * kk + kr) * Tl::UR * 16 + in +
+                                                        (((col0 + 32 * f) >> 3) ^ Tl::swz(kr)) * 16;
+      const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)q);
+      const v4i16 hi =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(q + 4 * Tl::UR * 16));
+      const v8i16 w = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      v[f] = __builtin_bit_cast(bf16x8, w);
+    }
+  } else {
+    static_assert(F <= 2, "fragments per wave");
+    const int col = col0 + F * row_l;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int kr = 8 * kk + 4 * half_l + t;
+      const char* q = tile + (Tl::krow(kr) * Tl::UR + ((col >> 2) ^ Tl::swz(kr))) * 16 + (col & 3) * 4;
+      if constexpr (F == 2) {
+        const float2 p = *reinterpret_cast<const float2*>(q);
+        v[0][t] = p.x;
+        v[1][t] = p.y;
+      } else {
+        v[0][t] = *reinterpret_cast<const float*>(q);
+      }
+    }
+  }
+}
+
+// Row / column of a wave's F * 32 that element e of fragment f of an MN-major
+// operand stands for.
+template <typename T, int F>
+__device__ __forceinline__ int mn_spread(int f, int e) {
+  return GT<T>::ES == 4 && F == 2 ? 2 * e + f : 32 * f + e;
+}
+
+}  // namespace tiles
+
+}  // namespace vh
