@@ -24,7 +24,10 @@
 //   [split][tile][wave][tap][row group j][lane][4]   (element v = 4j + k of lane)
 // written as one 16-byte store per lane and (tap, j), and a second kernel adds
 // them in a fixed order and writes dW (OIHW).  The optional bias gradient (sum of dY over
-// positions) is accumulated by the c-tile-0 blocks from the same LDS copy of dY.
+// positions) is accumulated by the c-tile-0 blocks' loading threads, from the dY
+// values they hold on their way into LDS: the multiplying waves, whose time the
+// grid waits for, carry none of it (summed by them from LDS it cost 17 - 38 us of
+// 41 - 51: 128 @28 N=128 86 us with bias, 47 without; now 51).
 #include <algorithm>
 #include <type_traits>
 
@@ -51,7 +54,7 @@ struct WgradArgs {
   int XV;              // x columns walked per row and step (segment width): multiple of 8
   int nseg;            // column segments per row (1: whole rows)
   int HL;              // dY columns loaded left of the segment: 0 (whole rows) or 8
-  int BW;              // dY columns per row slot summed for the bias gradient (multiple of 8)
+  int BW;              // segments: dY columns of the step's own, summed for the bias gradient
   int RL, XL;          // dY / x elements loaded per row and step
   int DP;              // LDS pitch of a dY row (elements)
   int XP;              // LDS pitch of an x row (elements): XV
@@ -278,12 +281,38 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
       j += a.xadv + wrap;
     }
   };
+  // bias gradient: a thread's dY items all belong to its owner row o; two sums (even
+  // and odd positions) in item order
+  const bool do_bias = a.dbias_part != nullptr && tile_c == 0;
+  float db0 = 0.f, db1 = 0.f;
+  auto bias_add = [&](const VT& v, bool ok) {
+    uint32_t w[V / 2];
+    __builtin_memcpy(w, &v, sizeof(w));
+#pragma unroll
+    for (int e = 0; e < V / 2; ++e) {
+      const uint32_t u = ok ? w[e] : 0u;
+      db0 += __builtin_bit_cast(float, u << 16);
+      db1 += __builtin_bit_cast(float, u & 0xffff0000u);
+    }
+  };
+  auto bias_out = [&]() {  // the TPO threads of an owner are adjacent lanes
+    float t = db0 + db1;
+    t += __shfl_xor(t, 1, 64);
+    t += __shfl_xor(t, 2, 64);
+    if constexpr (TPO == 8) t += __shfl_xor(t, 4, 64);
+    const int o = o0 + own;
+    if (sub == 0 && o < a.O) a.dbias_part[(long)split * a.O + o] = t;
+  };
   auto sstore = [&](auto SET, int st) {
     constexpr int sI = decltype(SET)::value;
     if constexpr (!SEG) {
       uint16_t* base = smem + st * stage;
 #pragma unroll
       for (int it = 0; it < ND; ++it) *reinterpret_cast<VT*>(base + d_lds[it]) = rdy[sI][it];
+      if (do_bias) {
+#pragma unroll
+        for (int it = 0; it < ND; ++it) bias_add(rdy[sI][it], d_lds[it] != sink_el);
+      }
 #pragma unroll
       for (int it = 0; it < NX; ++it) *reinterpret_cast<VT*>(base + x_lds[it]) = rx[sI][it];
       return;
@@ -298,6 +327,8 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
     for (int it = 0; it < ND; ++it) {
       uint16_t* dst = sub + TPO * it < dy_chunks ? d + g * DP + col : sink;
       *reinterpret_cast<VT*>(dst) = rdy[sI][it];
+      // the step's own columns (the halo columns belong to the neighbouring segments)
+      if (do_bias) bias_add(rdy[sI][it], col >= a.HL && col < a.HL + a.BW);
       col += a.cadv;
       const int wrap = col >= a.RL;
       col -= wrap ? a.RL : 0;
@@ -324,9 +355,6 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
       for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
   };
   if (!PC) zero_acc();
-  float dbias = 0.f;
-  const bool do_bias = a.dbias_part != nullptr && tile_c == 0;
-
   const int XV = a.XV;
   const int nchunk = G * (XV >> 3);  // even by construction
   const int grp = lane >> 5, rl = lane & 31;
@@ -425,15 +453,6 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
     }
     if (kk < nkk) mma(fa);
     }
-    if (do_bias) {
-      // thread t sums quarter (t % 4) of the columns [8, 8 + BW) of every dY row
-      // slot of o = t / 4: the step's own dY columns (past Q they hold zeros;
-      // the halo columns of a segment belong to its neighbours)
-      const uint16_t* drow = DYS(st) + own * OS + 8;
-      const int q4 = a.BW / TPO, beg = sub * q4;
-      for (int gg = 0; gg < G; ++gg)
-        for (int k = beg; k < beg + q4; ++k) dbias += bf16_to_f32(drow[gg * DP + k]);
-    }
   };
 
   __syncthreads();
@@ -464,6 +483,7 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
         if (DEPTH == 1 && ks + 3 < nsteps) gload(I0{}, step_b + ks + 3);
         __syncthreads();
       }
+      if (do_bias) bias_out();
       if constexpr (!KQ) return;  // KQ: the producers take part in the epilogue's barriers
     } else {
       zero_acc();
@@ -573,13 +593,8 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
         *reinterpret_cast<float4*>(pb + (t * 4 + j) * 256) = u;
       }
   }
-  if (do_bias && !producer) {
-    // combine the 4 quarter sums of each o (adjacent lanes)
-    dbias += __shfl_xor(dbias, 1, 64);
-    dbias += __shfl_xor(dbias, 2, 64);
-    if constexpr (TPO == 8) dbias += __shfl_xor(dbias, 4, 64);
-    const int o = o0 + own;
-    if (sub == 0 && o < a.O) a.dbias_part[(long)split * a.O + o] = dbias;
+  if constexpr (!PC) {
+    if (do_bias) bias_out();
   }
 }
 
@@ -1086,7 +1101,7 @@ bool plan_wgrad(WgradPlan& pl, int N, int C, int H, int W, int O, int R, int S, 
       a.HL = hl;
       a.RL = rl;
       a.XL = xl;
-      a.BW = whole ? dp - 8 : xv;
+      a.BW = xv;
       a.nseg = whole ? 1 : (span + xv - 1) / xv;
       pl.lds = lds;
       pl.nd = nd;
