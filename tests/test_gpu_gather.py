@@ -125,3 +125,20 @@ def test_gather_falls_back_without_workspace():
         graph.replay()
         torch.cuda.synchronize()
         assert float((out - want).abs().max()) <= 2 * 144 * 2.0 ** -24 * float(want.abs().max()) * 16
+
+
+@pytest.mark.parametrize("B", [3, 33, 60, 64, 65])
+def test_narrow_fp32_layer_on_either_kernel(B):
+    """32 -> 64 channels at 28 x 28: the channels-last path and the halo kernel
+    (40 <= B <= 64, a nearly full round of its blocks) by batch size."""
+    g = rng(B)
+    conv = vnn.Conv2d(32, 64, 3, 1, 1, device=DEV)
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    x, xt = prep(g.standard_normal((B, 32, 28, 28)), "f32")
+    dy, dyt = prep(g.standard_normal((B, 64, 28, 28)), "f32")
+    w, kw = host(conv.weight), dict(stride=(1, 1), pad=(1, 1))
+    check(conv.forward(xt), oracle.direct_conv, (x, w), "f32", "y", kw, k=288)
+    dx, dw, db = conv.backward(dyt, xt)
+    check(dx, oracle.direct_conv_backward_input, (dy, w, x.shape), "f32", "dx", kw, k=576)
+    check(dw, oracle.direct_conv_backward_weight, (dy, x, w.shape), "f32", "dw", kw, k=B * 784)
+    check(db, oracle.conv_bias_grad, (dy,), "f32", "db", k=B * 784)

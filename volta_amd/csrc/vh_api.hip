@@ -311,6 +311,15 @@ static bool is_3x3_s1_p1(const ConvDims& d) {
   return d.KH == 3 && d.KW == 3 && d.SH == 1 && d.SW == 1 && d.PH == 1 && d.PW == 1;
 }
 
+// The fp32 halo kernels (one block per image and 7 rows, 21 us a round of 256
+// blocks however few of them there are) against the channels-last path, whose time
+// grows with the positions.  Measured at 28 x 28, forward, us: N = 16 21.6 / 15.1, 32
+// 22.2 / 20.4, 64 23.4 / 31, 71 42.0 / 34, 128 44.2 / 52, 200 83.2 / 68.
+static bool halo_f32_pays(const ConvDims& d) {
+  const long rounds = (d.B * ((d.H + 6) / 7) + 255) / 256;
+  return 21.3 * (double)rounds <= 11.0 + 0.285 * (double)(d.B * d.H * d.W) / 784.0;
+}
+
 // act: 1 = ReLU on the output (fused into the epilogue where the kernel has it).
 // defer: a pass that takes the channels-last path is only put down in it (the
 // caller runs it, together with the other passes it put down; the same below).
@@ -326,11 +335,14 @@ static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, voi
     // 4x4 stride 2 from a few channels (the up-sampling layer's input gradient)
     int r = cell_fwd_f32(x, w, bias, y, g, act, st);
     if (r != VH_ERR_UNSUPPORTED) return r;
-    if (is_3x3_s1_p1(d)) {  // narrow images: the fp32 halo kernel
-      r = halo_conv3x3_f32(x, w, 0, bias, nullptr, y, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, act, st);
-      if (r != VH_ERR_UNSUPPORTED) return r;
-    }
   }
+  // narrow images: the fp32 halo kernel, also where the channels-last path cannot run
+  const bool halo_f32 = dt == VH_F32 && g_fast_paths && is_3x3_s1_p1(d) && act <= 1 &&
+                        halo_conv3x3_f32_ok(x, w, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O);
+  auto run_halo_f32 = [&] {
+    return halo_conv3x3_f32(x, w, 0, bias, nullptr, y, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, act, st);
+  };
+  if (halo_f32 && halo_f32_pays(d)) return run_halo_f32();
   // weight staging: the generic layout, or the halo kernel's channel-grouped one (padded to 16 channels)
   const size_t wbytes = std::max((size_t)d.O * d.C * RS * elem_size(dt),
                                  halo_conv_bf16_ws((int)d.C, (int)d.O, (int)d.KH, (int)d.KW));
@@ -352,8 +364,8 @@ static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, voi
   size_t ws_gemm = igemm_prepare(p);
   Carve cv;
   size_t o_w = cv.take(wbytes), o_g = cv.take(ws_gemm);
-  void* ws;
-  VH_TRY(ws_get(st, cv.off, &ws));
+  void* ws = nullptr;
+  if (!halo_f32) VH_TRY(ws_get(st, cv.off, &ws));  // (with the halo kernel to fall back on: no workspace)
   void* wt = at(ws, o_w);
   if (dt == VH_BF16 && d.SH == 1 && d.SW == 1 && g_fast_paths && d.C <= 4 && act <= 1) {
     // few input channels: K packed as (c, r, s) instead of 16-channel groups
@@ -377,6 +389,7 @@ static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, voi
     c.act = act;
     int r = VH_OK;
     if (defer || gather_try(dt, gc, st, &r)) return r;
+    if (halo_f32) return run_halo_f32();
     VH_TRY(ws_get(st, cv.off, &ws));
     wt = at(ws, o_w);
   }
@@ -547,10 +560,12 @@ static int igemm_dgrad(int dt, const void* dy, const void* w, void* dx, const Co
   }
   // at most 4 input channels: one lane per input position, no workspace
   if (g_fast_paths && dgrad_smallc_ok(g)) return VH_DISPATCH(dt, run_dgrad_smallc, dy, w, nullptr, mask, dx, g, st);
-  if (halo_f32)  // dX = conv(dY, W rotated, O and C swapped), the ReLU mask in the epilogue
+  auto run_halo_f32 = [&] {  // dX = conv(dY, W rotated, O and C swapped), the ReLU mask in the epilogue
     return halo_conv3x3_f32(dy, w, 1, nullptr, mask, dx, (int)d.B, (int)d.O, (int)d.H, (int)d.W, (int)d.C, 0, st);
-  void* ws;
-  VH_TRY(ws_get(st, cv.off, &ws));
+  };
+  if (halo_f32 && halo_f32_pays(d)) return run_halo_f32();
+  void* ws = nullptr;
+  if (!halo_f32) VH_TRY(ws_get(st, cv.off, &ws));  // (with the halo kernel to fall back on: no workspace)
   void* wd = at(ws, o_w);
   if (dt == VH_BF16 && d.SH == 1 && d.SW == 1 && d.PH <= d.KH - 1 && d.PW <= d.KW - 1 && g_fast_paths) {
     // stride 1: dX = conv(dY, W rotated 180 degrees with O and C swapped), pad K-1-p
@@ -574,6 +589,7 @@ static int igemm_dgrad(int dt, const void* dy, const void* w, void* dx, const Co
     int r = VH_OK;
     if (defer || gather_try(dt, gc, st, &r)) return r;
   }
+  if (halo_f32) return run_halo_f32();
   if ((d.SH > 1 || d.SW > 1) && g_fast_paths) {
     int r = dgrad_phases(dt, dy, w, nullptr, dx, d, st, mask);  // unsupported only beyond 16 phases
     if (r != VH_ERR_UNSUPPORTED) return r;
@@ -631,23 +647,24 @@ static int igemm_wgrad(int dt, const void* dy, const void* x, void* dw, void* db
       if (r != VH_ERR_UNSUPPORTED) return r;
     }
   }
-  if (dt == VH_F32 && g_fast_paths && is_3x3_s1_p1(d)) {
-    // fp32 3x3 of narrow images: the halo weight gradient (bias gradient included)
-    const size_t nb = halo_wgrad3x3_f32_ws(dy, x, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O);
-    if (nb && need) {
-      *need = nb;
-      return VH_OK;
-    }
-    if (nb) {
-      void* ws;
-      VH_TRY(ws_get(st, nb, &ws));
-      int r = halo_wgrad3x3_f32(dy, x, dw, db, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, (float*)ws, nb, st);
-      if (r != VH_ERR_UNSUPPORTED) {
-        if (r == VH_OK && db_done) *db_done = db != nullptr;
-        return r;
-      }
-    }
+  // fp32 3x3 of narrow images: the halo weight gradient (bias gradient included), also
+  // where the channels-last path cannot run
+  const size_t halo_nb = dt == VH_F32 && g_fast_paths && is_3x3_s1_p1(d)
+                             ? halo_wgrad3x3_f32_ws(dy, x, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O)
+                             : 0;
+  if (halo_nb && need) {
+    *need = halo_nb;
+    return VH_OK;
   }
+  auto run_halo_f32 = [&] {
+    void* ws;
+    VH_TRY(ws_get(st, halo_nb, &ws));
+    const int r =
+        halo_wgrad3x3_f32(dy, x, dw, db, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, (float*)ws, halo_nb, st);
+    if (r == VH_OK && db_done) *db_done = db != nullptr;
+    return r;
+  };
+  if (halo_nb && halo_f32_pays(d)) return run_halo_f32();
   ConvGeom g = geom_of(d);
   if (g_fast_paths && !need) {
     GatherCall gc{};
@@ -663,6 +680,7 @@ static int igemm_wgrad(int dt, const void* dy, const void* x, void* dw, void* db
       return r;
     }
   }
+  if (halo_nb) return run_halo_f32();
   const long RS = d.KH * d.KW;
   IgemmPlan p{};
   p.dtype = dt;

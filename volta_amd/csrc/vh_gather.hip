@@ -721,38 +721,49 @@ int launch_conv_tile(ConvArgs& a, hipStream_t st) {
   return VH_OK;
 }
 
-// Measured over 26 shapes of each type (3x3, 32 .. 512 channels, 1.5k .. 1M
-// positions): what counts is the number of 64 x 64 tiles, g64.
-//  * below one block per CU the waves split K instead (8 x 11 x 11 positions, 217
-//    -> 224 channels: 47 us with 64 x 64 tiles, 32 with 32 x 64 in two groups, 23
-//    with 32 x 32 in four; the two cross at about 80 tiles);
-//  * fp32 keeps 64 x 64 above that: five blocks a CU cover each other's copies and
-//    stores, and larger tiles gain nothing (64 x 128: 0 .. 3 % slower);
-//  * bf16 products are ten times shorter, so a CU's copies count: 64 x 128 tiles
-//    from four blocks a CU (64 -> 192 @28x29 N=64: 33.2 -> 29.8 us), 128 x 128
-//    where one round of two blocks a CU covers the grid (3x3 s2 64 -> 128 @56: 29.7
-//    -> 28.2), K in two groups of waves for deep products of one to two blocks a CU
-//    (256 @14x15 N=32: 30.6 -> 26.3; shallow ones lose to the extra sum).
+// The tile, by its cost as in vh_mm.hip: rounds of 256 blocks, each of the tile's
+// weight (tile_cost, vh_tiles.hpp).  Measured over 31 shapes of each type (3x3, 32 .. 512
+// channels, 1.5k .. 1M positions); it finds the fastest or one within 7 %, e.g. us on
+// 64 x 64, 32 x 64 (K in two groups of waves), 32 x 32 (four):
+//   fp32 217 -> 224 @11 N=8:     47.5  31.6  23.4
+//   fp32 128 -> 128 @28x29 N=16: 50.7  56.1  61.9
+//   bf16 64 -> 64 @28x29 N=16:   12.6  11.4  14.8
+// and on 128 x 128, 64 x 128, 64 x 64:
+//   bf16 3x3 s2 64 -> 128 @56:   28.2  32.4  29.7
+//   bf16 96 -> 144 @35x27 N=32:  26.0  24.6  29.5
+// fp32 gains nothing from tiles above 64 x 64: five blocks a CU cover each other's
+// copies and stores.  Deep bf16 products of one or two blocks a CU split K over two
+// groups of waves on the 64 x 64 tile (256 @14x15 N=32: 30.6 -> 26.3; shallow ones
+// lose to the extra sum, 64 channels 13.8 -> 14.3).
 template <typename T>
 int launch_conv(ConvArgs& a, hipStream_t st) {
+  constexpr bool b16 = GT<T>::ES == 2;
+  static constexpr int tile[][2] = {{64, 64}, {32, 128}, {32, 64}, {32, 32}, {64, 128}, {128, 128}};
   long n = 0;
   int nst = 0;
   for (int f = 0; f < a.nph; ++f) {
     n += a.ph[f].N;
     nst = std::max(nst, a.ph[f].nst);
   }
-  auto grid = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((n + bn - 1) / bn); };
-  const long g64 = grid(64, 64);
-  if (a.M <= 32 && grid(32, 128) >= 256) return launch_conv_tile<T, 32, 128, 32, 32>(a, st);
-  if (g64 < 80) return launch_conv_tile<T, 32, 32, 32, 32>(a, st);
-  if (g64 < 256) return launch_conv_tile<T, 32, 64, 32, 32>(a, st);
-  if constexpr (GT<T>::ES == 2) {
-    const bool fits128 = a.M > 64 && round_up(a.M, 128) * 7 <= round_up(a.M, 64) * 8;
-    if (fits128 && grid(128, 128) >= 256 && grid(128, 128) <= 512)
-      return launch_conv_tile<T, 128, 128, 64, 64>(a, st);
-    if (g64 >= 1024) return launch_conv_tile<T, 64, 128, 32, 64>(a, st);
-    if (g64 < 512 && nst >= 16) return launch_conv_tile<T, 64, 64, 64, 32>(a, st);
+  const long g64 = (long)((a.M + 63) / 64) * ((n + 63) / 64);
+  int best = 0;
+  float least = 1e30f;
+  for (int k = 0; k < (b16 ? 6 : 4); ++k) {
+    const long g = (long)((a.M + tile[k][0] - 1) / tile[k][0]) * ((n + tile[k][1] - 1) / tile[k][1]);
+    const float cost = tile_cost<T>(tile[k][0], tile[k][1], nst, g);
+    if (cost < least) {
+      least = cost;
+      best = k;
+    }
   }
+  if constexpr (b16) {
+    if (best == 5) return launch_conv_tile<T, 128, 128, 64, 64>(a, st);
+    if (best == 4) return launch_conv_tile<T, 64, 128, 32, 64>(a, st);
+    if (best == 0 && g64 <= 512 && nst >= 16) return launch_conv_tile<T, 64, 64, 64, 32>(a, st);
+  }
+  if (best == 1) return launch_conv_tile<T, 32, 128, 32, 32>(a, st);
+  if (best == 2) return launch_conv_tile<T, 32, 64, 32, 32>(a, st);
+  if (best == 3) return launch_conv_tile<T, 32, 32, 32, 32>(a, st);
   return launch_conv_tile<T, 64, 64, 32, 32>(a, st);
 }
 

@@ -354,33 +354,24 @@ struct Tile {
   int bm, bn;
 };
 
-// The tile of a product, or of a pair launched together (both grids counted), by
-// its cost: rounds of 256 blocks, each of the tile's own weight.  The weights are
-// the times of one round of blocks at K = 4096 relative to 64 x 64 (bf16 4096^3:
-// 108, 143, 175, 252, 505 us on 128 x 128 .. 32 x 32; fp32 978, 1043, 1231 on the
-// last three, the larger ones gain nothing).  A bf16 block alone on a CU cannot
-// cover its copies: less than 1.7 rounds cost as much (2048^3: 30 us on 256 blocks
-// of 128 x 128, 24 on 512 of 64 x 128; 1024^3: 22, 9.4, 7.7, 7.0, 11.5).
+// The tile of a product, or of a pair launched together (both grids counted; 64 x
+// 64 and below), by its cost.  fp32 gains nothing above 64 x 64 (4096^3: 978 us, 970
+// on 64 x 128).
 template <typename T>
 Tile mm_pick(const DenseProblem* p, int np) {
-  struct Cand {
-    Tile t;
-    float w;
-  };
-  static constexpr Cand kBf16[] = {{{128, 128}, 2.46f}, {{64, 128}, 1.5f}, {{64, 64}, 1.f}, {{32, 64}, 0.72f}, {{32, 32}, 0.72f}};
-  static constexpr Cand kF32[] = {{{64, 64}, 1.f}, {{32, 64}, 0.54f}, {{32, 32}, 0.3125f}};
-  const bool b16 = GT<T>::ES == 2;
-  const Cand* c = b16 ? kBf16 + (np > 1 ? 2 : 0) : kF32;  // pairs: 64 x 64 and below
-  const int nc = b16 && np == 1 ? 5 : 3;
+  static constexpr Tile tile[] = {{64, 64}, {32, 64}, {32, 32}, {64, 128}, {128, 128}};
+  int nst = 1;
+  for (int i = 0; i < np; ++i) nst = std::max(nst, (p[i].K + GT<T>::BK - 1) / GT<T>::BK);
   Tile best{64, 64};
   float least = 1e30f;
-  for (int k = 0; k < nc; ++k) {
+  for (int k = 0; k < (GT<T>::ES == 2 && np == 1 ? 5 : 3); ++k) {
     long n = 0;
-    for (int i = 0; i < np; ++i) n += (long)((p[i].M + c[k].t.bm - 1) / c[k].t.bm) * ((p[i].N + c[k].t.bn - 1) / c[k].t.bn);
-    const float cost = c[k].w * std::max((float)((n + 255) / 256), b16 ? 1.7f : 1.f);
+    for (int i = 0; i < np; ++i)
+      n += (long)((p[i].M + tile[k].bm - 1) / tile[k].bm) * ((p[i].N + tile[k].bn - 1) / tile[k].bn);
+    const float cost = tile_cost<T>(tile[k].bm, tile[k].bn, nst, n);
     if (cost < least) {
       least = cost;
-      best = c[k].t;
+      best = tile[k];
     }
   }
   return best;

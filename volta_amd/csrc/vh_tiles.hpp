@@ -133,6 +133,28 @@ __device__ __forceinline__ int mn_spread(int f, int e) {
   return GT<T>::ES == 4 && F == 2 ? 2 * e + f : 32 * f + e;
 }
 
+// Cost of a product of `blocks` tiles over nst stages: rounds of 256 blocks, each
+// of the tile's weight.
+//  * fp32 rounds are their MFMAs: a weight is the stages of one block, plus 3 to 4
+//    for its prologue and epilogue (half-size tiles in two K groups: half the
+//    stages, slightly longer ones).
+//  * bf16: the times of one round relative to 64 x 64 (4096^3: 108, 143, 175, 252,
+//    505 us on 128 x 128 .. 32 x 32).  A block alone on a CU cannot cover its
+//    copies: less than 1.7 rounds cost as much (2048^3: 30 us on 256 blocks of 128 x
+//    128, 24 on 512 of 64 x 128; 1024^3: 22, 9.4, 7.7, 7.0, 11.5).
+template <typename T>
+float tile_cost(int bm, int bn, int nst, long blocks) {
+  const float rounds = (float)((blocks + 255) / 256);
+  if (GT<T>::ES == 4) {
+    if (bm == 32 && bn == 64) return rounds * (1.05f * (float)((nst + 1) / 2) + 3.5f);
+    if (bm == 32 && bn == 32) return rounds * (1.1f * (float)((nst + 3) / 4) + 4.f);
+    return rounds * ((float)nst + 3.f);  // 64 x 64, 32 x 128
+  }
+  const float w = bm == 128 ? 2.46f : bm == 64 ? (bn == 128 ? 1.5f : 1.f) : bn == 128 ? 1.1f : 0.72f;
+  // deep products: four K groups shorten the chain (217 -> 224 @11 N=8: 17.4 -> 13.9 us)
+  return w * std::max(rounds, bm == 32 && bn == 32 && nst >= 16 ? 1.4f : 1.7f);
+}
+
 }  // namespace tiles
 
 }  // namespace vh
