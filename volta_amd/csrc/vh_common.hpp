@@ -59,8 +59,7 @@ struct FastDiv {
   uint32_t d, m, s;
   FastDiv() : d(1), m(0), s(0) {}
   explicit FastDiv(uint32_t div) : d(div) {
-    s = 0;
-    while ((1u << s) < div) ++s;
+    s = div > 1 ? 32 - __builtin_clz(div - 1) : 0;  // ceil(log2(div))
     uint64_t one = 1;
     m = (uint32_t)(((one << 32) * ((one << s) - div)) / div + 1);
   }

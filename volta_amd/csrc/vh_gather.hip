@@ -34,6 +34,7 @@ namespace {
 using namespace tiles;
 
 constexpr int kMaxPhases = 16;
+constexpr int kLaunchPhases = 4;  // stride 2 in one launch, its arguments below 600 bytes
 
 // ---------------------------------------------------------------- preparation
 // One tensor copied from [N][C][H][W] to [N][Hp][Wp][Cp] with (padT, padL) zero
@@ -210,7 +211,7 @@ struct ConvArgs {
   int OH, OW, osh, osw;  // output extents and strides
   int nph, tiles;
   FastDiv ftail;         // by the channel units of the last chunk
-  ConvPhase ph[kMaxPhases];
+  ConvPhase ph[kLaunchPhases];
 };
 
 // Tile BM x BN, four waves of WM x WN, two LDS stages of 128 bytes per row: row r
@@ -710,14 +711,28 @@ int launch_prep(PrepArgs& a, int npack, bool weights, hipStream_t st) {
   return VH_OK;
 }
 
+// A pass: its arguments and all its phases.
+struct ConvPlan {
+  ConvArgs a;
+  ConvPhase ph[kMaxPhases];
+  int nph;
+};
+
 template <typename T, int BM, int BN, int WM, int WN>
-int launch_conv_tile(ConvArgs& a, hipStream_t st) {
+int launch_conv_tile(ConvPlan& p, hipStream_t st) {
+  ConvArgs& a = p.a;
   a.tiles_m = (a.M + BM - 1) / BM;
-  a.tiles = 0;
-  for (int f = 0; f < a.nph; ++f) a.tiles = std::max(a.tiles, (a.ph[f].N + BN - 1) / BN);
-  a.tiles *= a.tiles_m * a.nph;
-  gather_conv_kernel<T, BM, BN, WM, WN><<<dim3((unsigned)((a.tiles + 7) / 8 * 8)), 256, 0, st>>>(a);
-  VH_LAUNCH_CHECK();
+  for (int f0 = 0; f0 < p.nph; f0 += kLaunchPhases) {
+    a.nph = std::min(kLaunchPhases, p.nph - f0);
+    a.tiles = 0;
+    for (int f = 0; f < a.nph; ++f) {
+      a.ph[f] = p.ph[f0 + f];
+      a.tiles = std::max(a.tiles, (a.ph[f].N + BN - 1) / BN);
+    }
+    a.tiles *= a.tiles_m * a.nph;
+    gather_conv_kernel<T, BM, BN, WM, WN><<<dim3((unsigned)((a.tiles + 7) / 8 * 8)), 256, 0, st>>>(a);
+    VH_LAUNCH_CHECK();
+  }
   return VH_OK;
 }
 
@@ -736,7 +751,7 @@ int launch_conv_tile(ConvArgs& a, hipStream_t st) {
 // groups of waves on the 64 x 64 tile (256 @14x15 N=32: 30.6 -> 26.3; shallow ones
 // lose to the extra sum, 64 channels 13.8 -> 14.3).
 template <typename T>
-int launch_conv(ConvArgs& a, hipStream_t st) {
+int launch_conv(ConvPlan& a, hipStream_t st) {
   constexpr bool b16 = GT<T>::ES == 2;
   static constexpr int tile[][2] = {{64, 64}, {32, 128}, {32, 64}, {32, 32}, {64, 128}, {128, 128}};
   long n = 0;
@@ -745,11 +760,12 @@ int launch_conv(ConvArgs& a, hipStream_t st) {
     n += a.ph[f].N;
     nst = std::max(nst, a.ph[f].nst);
   }
-  const long g64 = (long)((a.M + 63) / 64) * ((n + 63) / 64);
+  const int M = a.a.M;
+  const long g64 = (long)((M + 63) / 64) * ((n + 63) / 64);
   int best = 0;
   float least = 1e30f;
   for (int k = 0; k < (b16 ? 6 : 4); ++k) {
-    const long g = (long)((a.M + tile[k][0] - 1) / tile[k][0]) * ((n + tile[k][1] - 1) / tile[k][1]);
+    const long g = (long)((M + tile[k][0] - 1) / tile[k][0]) * ((n + tile[k][1] - 1) / tile[k][1]);
     const float cost = tile_cost<T>(tile[k][0], tile[k][1], nst, g);
     if (cost < least) {
       least = cost;
@@ -880,9 +896,10 @@ bool make_layout(const GatherCall& c, const Geo& o, Layout& l) {
 }
 
 template <typename T>
-void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, char* ws, const Layout& l) {
+void conv_args(ConvPlan& plan, WeightSeg& s, const GatherCall& c, const Geo& o, char* ws, const Layout& l) {
   constexpr int ES = GT<T>::ES, UE = GT<T>::UE;
   const ConvGeom& g = c.g;
+  ConvArgs& a = plan.a;
   const int RS = g.R * g.S;
   s.src = c.w;
   s.dst = ws + l.w;
@@ -919,9 +936,9 @@ void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, cha
     a.OH = g.P;
     a.OW = g.Q;
     a.osh = a.osw = 1;
-    a.nph = 1;
+    plan.nph = 1;
     a.ftail = FastDiv((uint32_t)std::max(1, CU & 7));
-    ConvPhase& p = a.ph[0];
+    ConvPhase& p = plan.ph[0];
     p.w_bytes = g.O * nst * 128;
     p.nst = nst;
     p.units = units;
@@ -973,7 +990,7 @@ void conv_args(ConvArgs& a, WeightSeg& s, const GatherCall& c, const Geo& o, cha
     s.cols[f] = std::max(1, q.Sc);
     if (!live) continue;
     tails += g.C * (nst * 8 - units);
-    ConvPhase& p = a.ph[a.nph++];
+    ConvPhase& p = plan.ph[plan.nph++];
     p.w_off = off * 16;
     p.w_bytes = g.C * nst * 128;
     p.nst = nst;
@@ -1059,7 +1076,7 @@ int run_call(const GatherCall& c, char* ws, hipStream_t st) {
   if (!make_geo<T>(c.g, o) || !make_layout<T>(c, o, l)) return VH_ERR_UNSUPPORTED;
   const ConvGeom& g = c.g;
   PrepArgs pa{};
-  ConvArgs a{};
+  ConvPlan a{};
   int np = 0;
   if (c.y || c.dw) pa.p[np++] = pack_seg<T>(c.x, ws + l.x, g.N, g.C, g.H, g.W, o.Cp, o.Hp, o.Wp, g.ph, g.pw);
   if (c.dx)

@@ -71,19 +71,30 @@ class Conv2d:
             raise ValueError("Channel mismatch")
         return (B, C, O, H, W, KH, KW, self.stride[0], self.stride[1], self.padding[0], self.padding[1])
 
-    def output_shape(self, x: torch.Tensor):
-        B, C, O, H, W, KH, KW, SH, SW, PH, PW = self._dims(x)
+    @staticmethod
+    def _out_shape(dims):
+        B, C, O, H, W, KH, KW, SH, SW, PH, PW = dims
         return (B, O, conv_out(H, KH, SH, PH), conv_out(W, KW, SW, PW))
+
+    def output_shape(self, x: torch.Tensor):
+        return self._out_shape(self._dims(x))
+
+    def _new_or_checked(self, out, x, dims):
+        shape = self._out_shape(dims)
+        if out is None:
+            return torch.empty(shape, dtype=x.dtype, device=x.device)
+        expect_numel(out, math.prod(shape), "Conv2d.forward out")
+        return out
 
     def forward(self, x: torch.Tensor, out: Optional[torch.Tensor] = None, relu: bool = False) -> torch.Tensor:
         """relu=True: the layer followed by ReLU, fused (vh_conv2d_forward_relu)."""
         dt = _same_dtype(x, self.weight, self.bias)
-        y = out if out is not None else torch.empty(self.output_shape(x), dtype=x.dtype, device=x.device)
-        expect_numel(y, math.prod(self.output_shape(x)), "Conv2d.forward out")
+        dims = self._dims(x)
+        y = self._new_or_checked(out, x, dims)
         used = ctypes.c_int(-1)
         fn = lib().vh_conv2d_forward_relu if relu else lib().vh_conv2d_forward
-        check(fn(dt, int(self.algo), ptr(x), ptr(self.weight), ptr(self.bias), ptr(y), *self._dims(x),
-                 ctypes.byref(used), stream_ptr(x.device)))
+        check(fn(dt, self.algo, ptr(x), ptr(self.weight), ptr(self.bias), ptr(y), *dims, ctypes.byref(used),
+                 stream_ptr(x.device)))
         self.last_algo = ConvAlgo(used.value)
         return y
 
@@ -95,10 +106,10 @@ class Conv2d:
         """Returns (grad_input, grad_weight, grad_bias); None where not requested.
         relu_input=True: x came out of a ReLU; grad_input gets that ReLU's backward
         (zero where x <= 0), fused (vh_conv2d_backward_relu)."""
+        dims = self._dims(x)
         algo = ConvAlgo(algo if algo is not None else (self.last_algo if self.last_algo is not None else self.algo))
         if algo == ConvAlgo.Auto:
-            B, C, O, H, W, KH, KW, SH, SW, PH, PW = self._dims(x)
-            algo = ConvAlgo(lib().vh_conv_algo_select_mi355x(B, C, O, H, W, KH, KW, SH, SW, PH, PW))
+            algo = ConvAlgo(lib().vh_conv_algo_select_mi355x(*dims))
         dt = _same_dtype(out_grad, x, self.weight)
         if outs is not None:
             dx, dw, db = outs
@@ -106,12 +117,13 @@ class Conv2d:
             dx = torch.empty_like(x) if input_grad else None
             dw = torch.empty_like(self.weight) if weight_grad else None
             db = torch.empty_like(self.bias) if (self.bias is not None and weight_grad) else None
-        expect_numel(out_grad, math.prod(self.output_shape(x)), "Conv2d.backward out_grad")
-        expect_numel(dx, x.numel(), "Conv2d.backward grad_input")
-        expect_numel(dw, self.weight.numel(), "Conv2d.backward grad_weight")
+        expect_numel(out_grad, math.prod(self._out_shape(dims)), "Conv2d.backward out_grad")
+        if outs is not None:
+            expect_numel(dx, x.numel(), "Conv2d.backward grad_input")
+            expect_numel(dw, self.weight.numel(), "Conv2d.backward grad_weight")
         expect_numel(db, self.weight.shape[0], "Conv2d.backward grad_bias")
         fn = lib().vh_conv2d_backward_relu if relu_input else lib().vh_conv2d_backward
-        check(fn(dt, int(algo), ptr(out_grad), ptr(x), ptr(self.weight), ptr(dx), ptr(dw), ptr(db), *self._dims(x),
+        check(fn(dt, algo, ptr(out_grad), ptr(x), ptr(self.weight), ptr(dx), ptr(dw), ptr(db), *dims,
                  stream_ptr(x.device)))
         return dx, dw, db
 
