@@ -142,3 +142,15 @@ def test_narrow_fp32_layer_on_either_kernel(B):
     check(dx, oracle.direct_conv_backward_input, (dy, w, x.shape), "f32", "dx", kw, k=576)
     check(dw, oracle.direct_conv_backward_weight, (dy, x, w.shape), "f32", "dw", kw, k=B * 784)
     check(db, oracle.conv_bias_grad, (dy,), "f32", "db", k=B * 784)
+
+
+@pytest.mark.parametrize("C", [60, 128, 190, 250, 300, 550])  # 1x1: 1, 2, 3, 4, 5 and 9 stages
+@pytest.mark.parametrize("B,O", [(2, 40), (96, 130)])  # K over four wave groups; 64-row tiles
+def test_gather_bf16_stages_in_flight(C, B, O):
+    g = rng(C + B)
+    x, xt = prep(g.standard_normal((B, C, 13, 11)), "bf16")
+    w, wt = prep(g.standard_normal((O, C, 1, 1)) * np.sqrt(2.0 / C), "bf16")
+    conv = vnn.Conv2d(C, O, 1, 2, 0, device=DEV, dtype=DTYPES["bf16"])
+    conv.weight = wt
+    conv.bias.zero_()
+    check(conv.forward(xt), oracle.direct_conv, (x, w), "bf16", "y", dict(stride=(2, 2), pad=(0, 0)), k=C)

@@ -87,3 +87,15 @@ def test_mm_padding_does_not_leak(mkn, dt):
     assert c[: m - 1].all() and not c[m - 1].any()
     db = np.isfinite(host(ops.gpu_matmul_backward_b(a, torch.ones((m, n), device=DEV, dtype=DTYPES[dt]), m, k, n)))
     assert db[: k - 1].all() and not db[k - 1].any()
+
+
+@pytest.mark.parametrize("k", [700, 768, 772, 896, 1030])  # 11 stages (two in LDS) .. 17 (three)
+@pytest.mark.parametrize("m,n", [(40, 1200), (520, 264), (1024, 1024), (1500, 1111), (1536, 2048), (1537, 2048)])
+def test_mm_bf16_stages_in_flight(m, k, n):
+    g = rng(m + k + n)
+    a, at = prep(g.standard_normal((m, k)), "bf16")
+    b, bt = prep(g.standard_normal((k, n)), "bf16")
+    check(ops.gpu_matmul(at, bt, m, k, n), oracle.matmul, (a, b), "bf16", "matmul", k=k)
+    gr, grt = prep(g.standard_normal((m, k)), "bf16")  # dA = G [m][k] . B^T, reduced over k
+    w, wt = prep(g.standard_normal((n, k)), "bf16")
+    check(ops.gpu_matmul_backward_a(grt, wt, m, n, k), oracle.matmul_backward_a, (gr, w), "bf16", "dA", k=k)

@@ -221,7 +221,7 @@ struct ConvArgs {
 // A tile of fewer than four waves' WM x WN is computed by KS groups of waves that
 // take every KS-th stage each (their sums added in group order at the end): for
 // grids of few positions, which larger tiles would leave on a part of the CUs.
-template <typename T, int BM, int BN, int WM, int WN>
+template <typename T, int BM, int BN, int WM, int WN, int NB>
 __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
   using ST = typename Elem<T>::storage;
   using G = GT<T>;
@@ -230,8 +230,8 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
   constexpr int WPG = (BM / WM) * (BN / WN), KS = 4 / WPG;  // waves per group, groups
   constexpr int AC = BM / 8 / WPG, BC = BN / 8 / WPG;       // copy instructions per wave and stage
   static_assert(WPG * KS == 4, "four waves");
-  __shared__ __attribute__((aligned(16))) u32x4g S0[KS * (BM + BN) * 8];
-  __shared__ __attribute__((aligned(16))) u32x4g S1[KS * (BM + BN) * 8];
+  constexpr int STAGE = KS * (BM + BN) * 8;
+  __shared__ __attribute__((aligned(16))) u32x4g S[NB * STAGE];
 
   // consecutive tiles on one XCD (the grid is a multiple of 8): the m-tiles of one
   // position tile share its gathered rows in that L2, and so do its stride phases,
@@ -310,21 +310,23 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
   auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
 
-  // stage s sits in buffer s % 2; fa holds its first step on entry.  The copies
-  // of stage s+1 go into the other buffer, whose stage s-1 every wave finished
-  // reading before the last barrier.  The reads of step k+1 are kept ahead of the
+  // stage s sits in buffer s % NB; fa holds its first step on entry.  The copies
+  // of stage s+NB-1 go into the buffer whose stage s-1 every wave finished reading
+  // before the last barrier.  The reads of step k+1 are kept ahead of the
   // MFMAs of step k (left alone the compiler sinks them to their use, and every
   // step waits for LDS).
   Frags fa, fb;
   const int nst = (p.nst + KS - 1) / KS;
-  issue(S0, 0);
-  gather_sync();
-  read(S0, 0, fa);
-  auto body = [&](auto BUF, int s) {
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i)
+    if (i < nst) issue(S + i * STAGE, i);
+  stage_sync<NB, AC + BC>(nst - 1);
+  read(S, 0, fa);
+  for_stages<NB>(nst, [&](auto BUF, int s) {
     constexpr int B = decltype(BUF)::value;
-    u32x4g* cur = B == 0 ? S0 : S1;
-    u32x4g* nxt = B == 0 ? S1 : S0;
-    if (s + 1 < nst) issue(nxt, s + 1);
+    const u32x4g* cur = S + B * STAGE;
+    const u32x4g* nxt = S + (B + 1) % NB * STAGE;
+    if (s + NB - 1 < nst) issue(S + (B + NB - 1) % NB * STAGE, s + NB - 1);
 #pragma unroll
     for (int kk = 1; kk < 4; kk += 2) {
       read(cur, kk, fb);
@@ -334,25 +336,19 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
       if (kk + 1 < 4) {
         read(cur, kk + 1, fa);
       } else if (s + 1 < nst) {
-        gather_sync();
+        stage_sync<NB, AC + BC>(nst - 2 - s);
         read(nxt, 0, fa);
       }
       __builtin_amdgcn_sched_barrier(0);
       mma(fb);
       __builtin_amdgcn_sched_barrier(0);
     }
-  };
-  int s = 0;
-  for (; s + 1 < nst; s += 2) {
-    body(std::integral_constant<int, 0>{}, s);
-    body(std::integral_constant<int, 1>{}, s + 1);
-  }
-  if (s < nst) body(std::integral_constant<int, 0>{}, s);
+  });
 
   if constexpr (KS > 1) {  // the groups' sums, added in group order
-    float* red = reinterpret_cast<float*>(S0);
+    float* red = reinterpret_cast<float*>(S);
     constexpr int TILE = FM * FN * 1024;
-    static_assert((KS - 1) * WPG * TILE * 4 <= (int)sizeof(S0), "group sums exceed a stage");
+    static_assert((KS - 1) * WPG * TILE * 4 <= STAGE * 16, "group sums exceed a stage");
     __syncthreads();
     if (grp > 0) {
 #pragma unroll
@@ -730,7 +726,11 @@ int launch_conv_tile(ConvPlan& p, hipStream_t st) {
       a.tiles = std::max(a.tiles, (a.ph[f].N + BN - 1) / BN);
     }
     a.tiles *= a.tiles_m * a.nph;
-    gather_conv_kernel<T, BM, BN, WM, WN><<<dim3((unsigned)((a.tiles + 7) / 8 * 8)), 256, 0, st>>>(a);
+    const dim3 grid((unsigned)((a.tiles + 7) / 8 * 8));
+    if (GT<T>::ES == 2 && third_stage(BM, BN, 4 / ((BM / WM) * (BN / WN)), a.tiles))
+      gather_conv_kernel<T, BM, BN, WM, WN, GT<T>::ES == 2 ? 3 : 2><<<grid, 256, 0, st>>>(a);
+    else
+      gather_conv_kernel<T, BM, BN, WM, WN, 2><<<grid, 256, 0, st>>>(a);
     VH_LAUNCH_CHECK();
   }
   return VH_OK;

@@ -36,9 +36,9 @@ struct MmArgs {
   int cs_shift;      // column sums: 4 << cs_shift columns per block
 };
 
-// One BM x BN tile (logical block lb).  S0, S1: two LDS stages.
-template <typename T, int BM, int BN, int WM, int WN, bool AT, bool BT, bool CS>
-__device__ __forceinline__ void mm_tile(const MmArgs& g, const int lb, u32x4g* S0, u32x4g* S1) {
+// One BM x BN tile (logical block lb).  S: NB LDS stages.
+template <typename T, int BM, int BN, int WM, int WN, int NB, bool AT, bool BT, bool CS>
+__device__ __forceinline__ void mm_tile(const MmArgs& g, const int lb, u32x4g* S) {
   using ST = typename Elem<T>::storage;
   using G = GT<T>;
   using TA = MnTile<T, BM>;
@@ -154,18 +154,20 @@ __device__ __forceinline__ void mm_tile(const MmArgs& g, const int lb, u32x4g* S
     }
   };
 
-  // the loop of vh_gather.hip: copies of stage s+1 in flight, reads of the next
-  // step ahead of the MFMAs of this one
+  // the loop of vh_gather.hip: copies of the next NB-1 stages in flight, reads of the
+  // next step ahead of the MFMAs of this one
   Frags fa, fb;
   const int ns = (nst + KS - 1) / KS;
-  issue(S0, 0);
-  gather_sync();
-  read(S0, 0, fa);
-  auto body = [&](auto BUF, int s) {
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i)
+    if (i < ns) issue(S + i * KS * GS, i);
+  stage_sync<NB, AC + BC>(ns - 1);
+  read(S, 0, fa);
+  for_stages<NB>(ns, [&](auto BUF, int s) {
     constexpr int B = decltype(BUF)::value;
-    u32x4g* cur = B == 0 ? S0 : S1;
-    u32x4g* nxt = B == 0 ? S1 : S0;
-    if (s + 1 < ns) issue(nxt, s + 1);
+    const u32x4g* cur = S + B * KS * GS;
+    const u32x4g* nxt = S + (B + 1) % NB * KS * GS;
+    if (s + NB - 1 < ns) issue(S + (B + NB - 1) % NB * KS * GS, s + NB - 1);
     if constexpr (CS) {
       if (cs_blk) colsum(cur);
     }
@@ -178,22 +180,16 @@ __device__ __forceinline__ void mm_tile(const MmArgs& g, const int lb, u32x4g* S
       if (kk + 1 < 4) {
         read(cur, kk + 1, fa);
       } else if (s + 1 < ns) {
-        gather_sync();
+        stage_sync<NB, AC + BC>(ns - 2 - s);
         read(nxt, 0, fa);
       }
       __builtin_amdgcn_sched_barrier(0);
       mma(fb);
       __builtin_amdgcn_sched_barrier(0);
     }
-  };
-  int s = 0;
-  for (; s + 1 < ns; s += 2) {
-    body(std::integral_constant<int, 0>{}, s);
-    body(std::integral_constant<int, 1>{}, s + 1);
-  }
-  if (s < ns) body(std::integral_constant<int, 0>{}, s);
+  });
 
-  float* red = reinterpret_cast<float*>(S0);
+  float* red = reinterpret_cast<float*>(S);
   if constexpr (CS) {
     if (cs_blk) {  // the k-row group sums, added in group order
       __syncthreads();
@@ -266,24 +262,22 @@ constexpr int mm_stage() {  // units
   return 4 / ((BM / WM) * (BN / WN)) * (BM + BN) * 8;
 }
 
-template <typename T, int BM, int BN, int WM, int WN, bool AT, bool BT>
+template <typename T, int BM, int BN, int WM, int WN, int NB, bool AT, bool BT>
 __global__ __launch_bounds__(256) void mm_kernel(MmArgs g) {
-  __shared__ __attribute__((aligned(16))) u32x4g S0[mm_stage<BM, BN, WM, WN>()];
-  __shared__ __attribute__((aligned(16))) u32x4g S1[mm_stage<BM, BN, WM, WN>()];
-  mm_tile<T, BM, BN, WM, WN, AT, BT, AT && BT>(g, xcd_block(gridDim.x), S0, S1);
+  __shared__ __attribute__((aligned(16))) u32x4g S[NB * mm_stage<BM, BN, WM, WN>()];
+  mm_tile<T, BM, BN, WM, WN, NB, AT, BT, AT && BT>(g, xcd_block(gridDim.x), S);
 }
 
 // Linear's dX (K-major x K-major) and dW (MN-major x MN-major, with the bias
 // gradient) in one launch: blocks 0 .. t0-1 take dX's tiles, the rest dW's.
 template <typename T, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(256) void mm_pair_kernel(MmArgs g0, MmArgs g1) {
-  __shared__ __attribute__((aligned(16))) u32x4g S0[mm_stage<BM, BN, WM, WN>()];
-  __shared__ __attribute__((aligned(16))) u32x4g S1[mm_stage<BM, BN, WM, WN>()];
+  __shared__ __attribute__((aligned(16))) u32x4g S[2 * mm_stage<BM, BN, WM, WN>()];
   const int t0 = g0.tiles_m * g0.tiles_n * g0.splits, h = blockIdx.x;
   if (h < t0)
-    mm_tile<T, BM, BN, WM, WN, false, false, false>(g0, xcd_map(h, t0), S0, S1);
+    mm_tile<T, BM, BN, WM, WN, 2, false, false, false>(g0, xcd_map(h, t0), S);
   else
-    mm_tile<T, BM, BN, WM, WN, true, true, true>(g1, xcd_map(h - t0, g1.tiles_m * g1.tiles_n * g1.splits), S0, S1);
+    mm_tile<T, BM, BN, WM, WN, 2, true, true, true>(g1, xcd_map(h - t0, g1.tiles_m * g1.tiles_n * g1.splits), S);
 }
 
 // Split products: C (+ bias) and the column sums from the fp32 partials, in split
@@ -476,12 +470,25 @@ void mm_launch(const MmArgs* g, int np, bool at, bool bt, hipStream_t st) {
     }
     return;
   }
+  // A third stage where the grid leaves room for it, from 12 stages on (bf16 900 x 600
+  // x 2000, 10 stages: 8.0 us on two, 8.3 on three; 700 x 3000 x 500: 23.6 and 17.5).
+  // MN-major x MN-major tiles are bound by their transposing reads and lose as often
+  // as they gain (271 x 2368 x 3200: 24.3 and 26.3; 1400^3: 16.9 and 15.9): two.
+  if constexpr (GT<T>::ES == 2) {
+    if (!at && g[0].per >= 12 && third_stage(BM, BN, 4 / ((BM / WM) * (BN / WN)), n)) {
+      if (bt)
+        mm_kernel<T, BM, BN, WM, WN, 3, false, true><<<dim3(n), 256, 0, st>>>(g[0]);
+      else
+        mm_kernel<T, BM, BN, WM, WN, 3, false, false><<<dim3(n), 256, 0, st>>>(g[0]);
+      return;
+    }
+  }
   if (at && bt)
-    mm_kernel<T, BM, BN, WM, WN, true, true><<<dim3(n), 256, 0, st>>>(g[0]);
+    mm_kernel<T, BM, BN, WM, WN, 2, true, true><<<dim3(n), 256, 0, st>>>(g[0]);
   else if (bt)
-    mm_kernel<T, BM, BN, WM, WN, false, true><<<dim3(n), 256, 0, st>>>(g[0]);
+    mm_kernel<T, BM, BN, WM, WN, 2, false, true><<<dim3(n), 256, 0, st>>>(g[0]);
   else
-    mm_kernel<T, BM, BN, WM, WN, false, false><<<dim3(n), 256, 0, st>>>(g[0]);
+    mm_kernel<T, BM, BN, WM, WN, 2, false, false><<<dim3(n), 256, 0, st>>>(g[0]);
 }
 
 template <typename T>

@@ -42,6 +42,32 @@ __device__ __forceinline__ void gather_sync() {
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// The same once the oldest stage in flight has landed: NB buffers, COPIES copy
+// instructions per wave and stage, `later` stages of the product after that one (the
+// last ones are waited for together).
+template <int NB, int COPIES>
+__device__ __forceinline__ void stage_sync(int later) {
+  if (NB > 2 && later >= NB - 2)
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NB - 2) * COPIES) : "memory");
+  else
+    gather_sync();
+}
+
+// body(buffer, stage) for stages 0 .. ns-1, the buffers in turn and known to the compiler
+template <int NB, typename F>
+__device__ __forceinline__ void for_stages(int ns, F body) {
+  static_assert(NB == 2 || NB == 3, "buffers");
+  int s = 0;
+  for (; s + NB - 1 < ns; s += NB) {
+    body(std::integral_constant<int, 0>{}, s);
+    body(std::integral_constant<int, 1>{}, s + 1);
+    if constexpr (NB > 2) body(std::integral_constant<int, 2>{}, s + 2);
+  }
+  if (s < ns) body(std::integral_constant<int, 0>{}, s);
+  if constexpr (NB > 2)
+    if (s + 1 < ns) body(std::integral_constant<int, 1>{}, s + 1);
+}
+
 // all MFMAs of one fragment step: independent accumulators back to back
 template <int FM, int FN>
 __device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const bf16x8 (&a)[FM], const bf16x8 (&b)[FN]) {
@@ -153,6 +179,16 @@ float tile_cost(int bm, int bn, int nst, long blocks) {
   const float w = bm == 128 ? 2.46f : bm == 64 ? (bn == 128 ? 1.5f : 1.f) : bn == 128 ? 1.1f : 0.72f;
   // deep products: four K groups shorten the chain (217 -> 224 @11 N=8: 17.4 -> 13.9 us)
   return w * std::max(rounds, bm == 32 && bn == 32 && nst >= 16 ? 1.4f : 1.7f);
+}
+
+// Whether a grid of bf16 tiles (ks wave groups) keeps a third stage: the whole grid
+// still fits on the 256 CUs at once, 160 KB of LDS each.  Its few blocks cannot cover
+// a copy's latency with two (3x3 217 -> 224 @11 N=8: 14.0 -> 12.5 us; 512 -> 512 @7
+// N=32: 36.1 -> 30.5); where it takes blocks off a CU it costs more than it gives
+// (256 -> 256 @14x15 N=32, 420 blocks in two K groups: 26.4 us on two, 31.2 on three).
+// fp32 stages take four times as long to compute: within 2 % on either.
+inline bool third_stage(int bm, int bn, int ks, long blocks) {
+  return blocks <= 256L * (160 * 1024 / (3 * ks * (bm + bn) * 128));
 }
 
 }  // namespace tiles
