@@ -282,7 +282,8 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
     }
   };
   // bias gradient: a thread's dY items all belong to its owner row o; two sums (even
-  // and odd positions) in item order
+  // and odd positions) in item order, items that no thread uses left out (one of 8 is
+  // used at 32 -> 112 @13x56)
   const bool do_bias = a.dbias_part != nullptr && tile_c == 0;
   float db0 = 0.f, db1 = 0.f;
   auto bias_add = [&](const VT& v, bool ok) {
@@ -311,7 +312,8 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
       for (int it = 0; it < ND; ++it) *reinterpret_cast<VT*>(base + d_lds[it]) = rdy[sI][it];
       if (do_bias) {
 #pragma unroll
-        for (int it = 0; it < ND; ++it) bias_add(rdy[sI][it], d_lds[it] != sink_el);
+        for (int it = 0; it < ND; ++it)
+          if (TPO * it < dy_chunks) bias_add(rdy[sI][it], d_lds[it] != sink_el);
       }
 #pragma unroll
       for (int it = 0; it < NX; ++it) *reinterpret_cast<VT*>(base + x_lds[it]) = rx[sI][it];
@@ -328,7 +330,7 @@ __global__ __launch_bounds__(PC ? 512 : 256) void wgrad_rows_bf16_kernel(WgradAr
       uint16_t* dst = sub + TPO * it < dy_chunks ? d + g * DP + col : sink;
       *reinterpret_cast<VT*>(dst) = rdy[sI][it];
       // the step's own columns (the halo columns belong to the neighbouring segments)
-      if (do_bias) bias_add(rdy[sI][it], col >= a.HL && col < a.HL + a.BW);
+      if (do_bias && TPO * it < dy_chunks) bias_add(rdy[sI][it], col >= a.HL && col < a.HL + a.BW);
       col += a.cadv;
       const int wrap = col >= a.RL;
       col -= wrap ? a.RL : 0;
