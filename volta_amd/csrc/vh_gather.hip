@@ -308,6 +308,8 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+  Totals<T, FM, FN> tot;
+  tot.init();
   auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
 
   // stage s sits in buffer s % NB; fa holds its first step on entry.  The copies
@@ -343,7 +345,9 @@ __global__ __launch_bounds__(256) void gather_conv_kernel(ConvArgs g) {
       mma(fb);
       __builtin_amdgcn_sched_barrier(0);
     }
+    tot.template stage<B>(acc);
   });
+  tot.finish(acc);
 
   if constexpr (KS > 1) {  // the groups' sums, added in group order
     float* red = reinterpret_cast<float*>(S);
@@ -441,7 +445,7 @@ struct WgradArgs {
   int dimg, drow, dcol;       // bytes between images, rows and columns of dy
   int ximg, xrow, xcol;       // the same of x, per output row / column (strides applied)
   int trow, tcol;             // bytes between tap rows and columns
-  int cs_shift;               // bias gradient: 4 << cs_shift columns of o per block
+  int cs_shift;               // bias gradient: 4 << cs_shift columns of o per block (ColSum)
   FastDiv fPQ, fQ, fCU, fS;
 };
 
@@ -450,7 +454,7 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   using G = GT<T>;
   using TA = MnTile<T, BM>;
   using TB = MnTile<T, BN>;
-  constexpr int ES = G::ES, UE = G::UE, BK = G::BK, FM = WM / 32, FN = WN / 32, NWN = BN / WN;
+  constexpr int UE = G::UE, BK = G::BK, FM = WM / 32, FN = WN / 32, NWN = BN / WN;
   constexpr int A_UNITS = BK * TA::UR, B_UNITS = BK * TB::UR;
   constexpr int AC = BM / 32, BC = BN / 32;  // copy instructions per wave and stage
   static_assert((BM / WM) * (BN / WN) == 4, "four waves");
@@ -511,34 +515,13 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+  Totals<T, FM, FN> tot;
+  tot.init();
   auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
 
-  // bias gradient: the blocks of one m-tile share its BM columns of o; each sums
-  // 4 << cs_shift of them from the staged tiles, a thread 4 columns of every
-  // (256 / ng)-th k row
-  const int cs_w = 4 << g.cs_shift, cs_c0 = tn * cs_w, ng = cs_w >> 2;
-  const bool cs_blk = g.dbpart != nullptr && cs_c0 < BM;
-  const int cs_c = cs_c0 + 4 * (tid & (ng - 1)), cs_k0 = tid >> g.cs_shift;
-  float csum[4] = {0.f, 0.f, 0.f, 0.f};
-  auto colsum = [&](const u32x4g* st) {
-    const char* at = reinterpret_cast<const char*>(st);
-    for (int kr = cs_k0; kr < BK; kr += 256 >> g.cs_shift) {
-      const char* q = at + (TA::krow(kr) * TA::UR + ((cs_c / UE) ^ TA::swz(kr))) * 16 + (cs_c % UE) * ES;
-      if constexpr (ES == 2) {
-        const u32x2g v = *reinterpret_cast<const u32x2g*>(q);
-        csum[0] += __builtin_bit_cast(float, v[0] << 16);
-        csum[1] += __builtin_bit_cast(float, v[0] & 0xffff0000u);
-        csum[2] += __builtin_bit_cast(float, v[1] << 16);
-        csum[3] += __builtin_bit_cast(float, v[1] & 0xffff0000u);
-      } else {
-        const float4 v = *reinterpret_cast<const float4*>(q);
-        csum[0] += v.x;
-        csum[1] += v.y;
-        csum[2] += v.z;
-        csum[3] += v.w;
-      }
-    }
-  };
+  // bias gradient: the blocks of one m-tile share its BM columns of o
+  ColSum<T, BM, 1> cs;
+  cs.init(g.dbpart != nullptr, tn, g.cs_shift);
 
   Frags fa, fb;
   const int nst = (ke - kb + BK - 1) / BK;
@@ -550,7 +533,7 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
     u32x4g* cur = B == 0 ? S0 : S1;
     u32x4g* nxt = B == 0 ? S1 : S0;
     if (s + 1 < nst) issue(nxt, kb + (s + 1) * BK);
-    if (cs_blk) colsum(cur);
+    if (cs.on) cs.stage(reinterpret_cast<const char*>(cur), 0, s);
 #pragma unroll
     for (int kk = 1; kk < 4; kk += 2) {
       read(cur, kk, fb);
@@ -567,6 +550,7 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
       mma(fb);
       __builtin_amdgcn_sched_barrier(0);
     }
+    tot.template stage<B>(acc);
   };
   int s = 0;
   for (; s + 1 < nst; s += 2) {
@@ -574,6 +558,7 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
     body(std::integral_constant<int, 1>{}, s + 1);
   }
   if (s < nst) body(std::integral_constant<int, 0>{}, s);
+  tot.finish(acc);
 
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -589,19 +574,10 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
         }
       }
     }
-  if (cs_blk) {  // the k-row group sums, added in group order
-    __syncthreads();
-    float* red = reinterpret_cast<float*>(S0);  // [256 / ng][cs_w]
-#pragma unroll
-    for (int e = 0; e < 4; ++e) red[cs_k0 * cs_w + cs_c - cs_c0 + e] = csum[e];
-    __syncthreads();
-    const int o = m0 + cs_c0 + tid;
-    if (tid < cs_w && cs_c0 + tid < BM && o < g.O) {
-      float t = 0.f;
-      for (int j = 0; j < 256 >> g.cs_shift; ++j) t += red[j * cs_w + tid];
-      g.dbpart[(size_t)z * g.O + o] = t;
-    }
-  }
+  if (cs.on)
+    cs.finish(reinterpret_cast<float*>(S0), [&](int col, float t) {
+      if (m0 + col < g.O) g.dbpart[(size_t)z * g.O + m0 + col] = t;
+    });
 }
 
 // dW[o][c][tap] and db[o] from the splits' partials [split][o][tap][Cp], added in
@@ -646,9 +622,12 @@ __global__ __launch_bounds__(256) void gather_wgrad_reduce_vec4_kernel(const flo
                                                                        void* db, int O, int C, FastDiv fCp, FastDiv fRS,
                                                                        int splits, int lg_g, int nb) {
   using ST = typename Elem<T>::storage;
-  if ((int)blockIdx.x >= nb) {
-    reduce_splits_block(dbpart, splits, O, [&](long i, float v) { reinterpret_cast<ST*>(db)[i] = Elem<T>::from_f32(v); },
-                        (int)blockIdx.x - nb, (int)gridDim.x - nb);
+  if ((int)blockIdx.x >= nb) {  // a wave per output, its lanes' sums added in pairs
+    const int o = ((int)blockIdx.x - nb) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    float t = 0.f;
+    for (int z = lane; z < splits && o < O; z += 64) t += dbpart[(size_t)z * O + o];
+    for (int d = 1; d < 64; d <<= 1) t += __shfl_xor(t, d, 64);
+    if (lane == 0 && o < O) reinterpret_cast<ST*>(db)[o] = Elem<T>::from_f32(t);
     return;
   }
   const int RS = (int)fRS.d;
@@ -1049,7 +1028,7 @@ int run_wgrad(const GatherCall& c, const Geo& o, char* ws, const Layout& l, hipS
   const int RS = g.R * g.S;
   if (p.splits > 8) {
     const int lg = reduce_vec4_lg_groups(p.splits), nb = reduce_vec4_grid((long)g.O * a.NC, lg);
-    const int ndb = c.db ? reduce_splits_grid(g.O) : 0;
+    const int ndb = c.db ? (g.O + 3) / 4 : 0;
     gather_wgrad_reduce_vec4_kernel<T><<<dim3((unsigned)(nb + ndb)), 256, 0, st>>>(
         a.part, a.dbpart, c.dw, c.db, g.O, g.C, FastDiv((uint32_t)o.Cp), FastDiv((uint32_t)RS), p.splits, lg, nb);
   } else {

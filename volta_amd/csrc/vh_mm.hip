@@ -33,7 +33,7 @@ struct MmArgs {
   int M, N, K, lda, ldb, ldc;
   int a_bytes, b_bytes, c_bytes;
   int tiles_m, tiles_n, splits, per;  // stages per split
-  int cs_shift;      // column sums: 4 << cs_shift columns per block
+  int cs_shift;      // column sums: 4 << cs_shift columns per block (ColSum)
 };
 
 // One BM x BN tile (logical block lb).  S: NB LDS stages.
@@ -124,35 +124,13 @@ __device__ __forceinline__ void mm_tile(const MmArgs& g, const int lb, u32x4g* S
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+  Totals<T, FM, FN> tot;
+  tot.init();
   auto mma = [&](const Frags& q) { mma_all<FM, FN>(acc, q.a, q.b); };
 
-  // column sums (B MN-major): the blocks of one column tile share its columns, each
-  // sums 4 << cs_shift of them from the staged tiles, a thread 4 columns of every
-  // (256 / ng)-th k row of all groups
-  const int cs_w = 4 << g.cs_shift, cs_c0 = tm * cs_w, ng = cs_w >> 2;
-  const bool cs_blk = CS && g.colsum != nullptr && cs_c0 < BN;
-  const int cs_c = cs_c0 + 4 * (tid & (ng - 1)), cs_k0 = tid >> g.cs_shift;
-  float csum[4] = {0.f, 0.f, 0.f, 0.f};
-  auto colsum = [&](const u32x4g* st) {
-    for (int r = cs_k0; r < KS * BK; r += 256 >> g.cs_shift) {
-      const int kr = r % BK;
-      const char* q = reinterpret_cast<const char*>(st + (r / BK) * GS) + BM * 128 +
-                      (TB::krow(kr) * TB::UR + ((cs_c / UE) ^ TB::swz(kr))) * 16 + (cs_c % UE) * ES;
-      if constexpr (ES == 2) {
-        const u32x2g v = *reinterpret_cast<const u32x2g*>(q);
-        csum[0] += __builtin_bit_cast(float, v[0] << 16);
-        csum[1] += __builtin_bit_cast(float, v[0] & 0xffff0000u);
-        csum[2] += __builtin_bit_cast(float, v[1] << 16);
-        csum[3] += __builtin_bit_cast(float, v[1] & 0xffff0000u);
-      } else {
-        const float4 v = *reinterpret_cast<const float4*>(q);
-        csum[0] += v.x;
-        csum[1] += v.y;
-        csum[2] += v.z;
-        csum[3] += v.w;
-      }
-    }
-  };
+  // column sums (B MN-major): the blocks of one column tile share its columns
+  ColSum<T, BN, KS> cs;
+  if constexpr (CS) cs.init(g.colsum != nullptr, tm, g.cs_shift);
 
   // the loop of vh_gather.hip: copies of the next NB-1 stages in flight, reads of the
   // next step ahead of the MFMAs of this one
@@ -169,7 +147,7 @@ __device__ __forceinline__ void mm_tile(const MmArgs& g, const int lb, u32x4g* S
     const u32x4g* nxt = S + (B + 1) % NB * KS * GS;
     if (s + NB - 1 < ns) issue(S + (B + NB - 1) % NB * KS * GS, s + NB - 1);
     if constexpr (CS) {
-      if (cs_blk) colsum(cur);
+      if (cs.on) cs.stage(reinterpret_cast<const char*>(cur) + BM * 128, GS * 16, s);
     }
 #pragma unroll
     for (int kk = 1; kk < 4; kk += 2) {
@@ -187,25 +165,21 @@ __device__ __forceinline__ void mm_tile(const MmArgs& g, const int lb, u32x4g* S
       mma(fb);
       __builtin_amdgcn_sched_barrier(0);
     }
+    tot.template stage<B>(acc);
   });
+  tot.finish(acc);
 
   float* red = reinterpret_cast<float*>(S);
   if constexpr (CS) {
-    if (cs_blk) {  // the k-row group sums, added in group order
-      __syncthreads();
-#pragma unroll
-      for (int e = 0; e < 4; ++e) red[cs_k0 * cs_w + cs_c - cs_c0 + e] = csum[e];
-      __syncthreads();
-      const int n = n0 + cs_c0 + tid;
-      if (tid < cs_w && cs_c0 + tid < BN && n < g.N) {
-        float t = 0.f;
-        for (int j = 0; j < 256 >> g.cs_shift; ++j) t += red[j * cs_w + tid];
+    if (cs.on)
+      cs.finish(red, [&](int col, float t) {
+        const int n = n0 + col;
+        if (n >= g.N) return;
         if (g.splits > 1)
           reinterpret_cast<float*>(g.colsum)[(size_t)z * g.N + n] = t;
         else
           reinterpret_cast<ST*>(g.colsum)[n] = Elem<T>::from_f32(t);
-      }
-    }
+      });
   }
   if constexpr (KS > 1) {  // the groups' sums, added in group order
     constexpr int TILE = FM * FN * 1024;

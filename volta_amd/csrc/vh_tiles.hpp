@@ -86,6 +86,46 @@ __device__ __forceinline__ void mma_all(f32x16 (&c)[FM][FN], const f32x4 (&a)[FM
       for (int j = 0; j < FN; ++j) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][t], b[j][t], c[i][j], 0, 0, 0);
 }
 
+// fp32 sums in two levels: an accumulator takes the products of 64 k (two stages),
+// then goes into the total and starts again.  The error of a sum grows with the root
+// of the additions in a row: one accumulator over all of K was up to 3 times further
+// off 64 bits (512 channels 3x3 @7: 5.7e-7; 32768 positions: 1.1e-6) than sums of a
+// few hundred; so it is 1.7e-7.  Always after the second buffer, so that the zeros are
+// the compiler's and no registers (at the fourth stage, by a test of s: 2.1e-7, 8 - 15 %
+// slower): 2048^3 forward and gradients 386 -> 399 us.  bf16 results are rounded at
+// 2^-9: one level.
+template <typename T, int FM, int FN>
+struct Totals {
+  static constexpr bool two = GT<T>::ES == 4;
+  f32x16 t[two ? FM : 1][two ? FN : 1];
+  __device__ __forceinline__ void init() {
+    if constexpr (two)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) t[i][j] = f32x16{};
+  }
+  // after the stage in buffer B of two
+  template <int B>
+  __device__ __forceinline__ void stage(f32x16 (&acc)[FM][FN]) {
+    if constexpr (two && B == 1)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          t[i][j] += acc[i][j];
+          acc[i][j] = f32x16{};
+        }
+  }
+  __device__ __forceinline__ void finish(f32x16 (&acc)[FM][FN]) const {
+    if constexpr (two)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] += t[i][j];
+  }
+};
+
 // Fragment of rows row0 .. +31 of a K-major tile, step kk.
 template <typename T>
 __device__ __forceinline__ typename GT<T>::frag read_k(const char* tile, int row0, int kk, int lane) {
@@ -158,6 +198,75 @@ template <typename T, int F>
 __device__ __forceinline__ int mn_spread(int f, int e) {
   return GT<T>::ES == 4 && F == 2 ? 2 * e + f : 32 * f + e;
 }
+
+// Column sums (a bias gradient) of an MN-major operand of R columns from its staged
+// tiles, KG of them `group_bytes` apart: of the blocks that share the columns, block
+// idx sums 4 << shift of them, a thread 4 columns of every (256 >> shift)-th k row.
+// Added in pairs of lanes, then of waves: the rounding stays that of the threads' own
+// sums, which start again every 8 stages.
+template <typename T, int R, int KG>
+struct ColSum {
+  using Tl = MnTile<T, R>;
+  static constexpr int ES = GT<T>::ES, UE = GT<T>::UE, BK = GT<T>::BK;
+  int shift, c0, c, k0;
+  bool on;
+  float part[4], tot[4];
+  __device__ __forceinline__ void init(bool want, int idx, int sh) {
+    shift = sh;
+    c0 = idx * (4 << sh);
+    on = want && c0 < R;
+    c = c0 + 4 * ((int)threadIdx.x & ((1 << sh) - 1));
+    k0 = (int)threadIdx.x >> sh;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) part[e] = tot[e] = 0.f;
+  }
+  __device__ __forceinline__ void stage(const char* tile, int group_bytes, int s) {
+    for (int r = k0; r < KG * BK; r += 256 >> shift) {
+      const int kr = r % BK;
+      const char* q =
+          tile + (r / BK) * group_bytes + (Tl::krow(kr) * Tl::UR + ((c / UE) ^ Tl::swz(kr))) * 16 + (c % UE) * ES;
+      if constexpr (ES == 2) {
+        const u32x2g v = *reinterpret_cast<const u32x2g*>(q);
+        part[0] += __builtin_bit_cast(float, v[0] << 16);
+        part[1] += __builtin_bit_cast(float, v[0] & 0xffff0000u);
+        part[2] += __builtin_bit_cast(float, v[1] << 16);
+        part[3] += __builtin_bit_cast(float, v[1] & 0xffff0000u);
+      } else {
+        const float4 v = *reinterpret_cast<const float4*>(q);
+        part[0] += v.x;
+        part[1] += v.y;
+        part[2] += v.z;
+        part[3] += v.w;
+      }
+    }
+    if ((s & 7) == 7) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        tot[e] += part[e];
+        part[e] = 0.f;
+      }
+    }
+  }
+  // all threads of the block, `on` the same for all; red: 4 * R floats.  out(column
+  // of the tile, sum)
+  template <typename F>
+  __device__ __forceinline__ void finish(float* red, F out) {
+    const int tid = threadIdx.x, w = 4 << shift;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tot[e] += part[e];
+    for (int d = 1 << shift; d < 64; d <<= 1) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tot[e] += __shfl_xor(tot[e], d, 64);
+    }
+    __syncthreads();
+    if ((tid & 63) < (1 << shift)) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[(tid >> 6) * w + c - c0 + e] = tot[e];
+    }
+    __syncthreads();
+    if (tid < w && c0 + tid < R) out(c0 + tid, (red[tid] + red[w + tid]) + (red[2 * w + tid] + red[3 * w + tid]));
+  }
+};
 
 // Cost of a product of `blocks` tiles over nst stages: rounds of 256 blocks, each
 // of the tile's weight.
