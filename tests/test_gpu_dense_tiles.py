@@ -103,3 +103,14 @@ def test_linear_backward_pair_tiles(dt):
     assert_parity(host(dx), ref[0], sc[0], dt, "dX", k=o)
     assert_parity(host(dw), ref[1], sc[1], dt, "dW", k=m)
     assert_parity(host(db), ref[2], sc[2], dt, "db", k=m)
+
+
+@pytest.mark.parametrize("m", [8, 64, 72, 200])
+def test_matmul_backward_b_128x256_tiles(m):
+    # dB on the producer / consumer tiles (bf16, rounds of 256 tiles nearly full), with
+    # remainders in M, N and the contraction: one k row group .. three stages and a bit
+    k, n = 2040, 4088
+    g = np.random.default_rng(m)
+    a, at = prep(g.standard_normal((m, k)), "bf16")
+    gr, grt = prep(g.standard_normal((m, n)), "bf16")
+    check(ops.gpu_matmul_backward_b(at, grt, m, k, n), oracle.matmul_backward_b, (a, gr), "dB", m, "bf16")

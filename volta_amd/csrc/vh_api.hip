@@ -882,7 +882,7 @@ static int dense_large(int dt, const DenseProblem* p, int np, const void* bias, 
   if (np == 2) return b16 ? dense_bf16_gemm_pair(p[0], p[1], st) : dense_f32_gemm_pair(p[0], p[1], st);
   const DenseProblem& q = *p;
   if (b16) return dense_bf16_gemm(q.a, q.lda, q.at, q.b, q.ldb, q.bt, q.c, q.ldc, q.M, q.N, q.K, bias, st);
-  return bias ? VH_ERR_UNSUPPORTED : dense_f32_gemm(q.a, q.lda, q.at, q.b, q.ldb, q.bt, q.c, q.ldc, q.M, q.N, q.K, st);
+  return dense_f32_gemm(q.a, q.lda, q.at, q.b, q.ldb, q.bt, q.c, q.ldc, q.M, q.N, q.K, bias, st);
 }
 
 // The large kernels, or those for any size (vh_mm.hip) where their workspace can be

@@ -13,7 +13,7 @@
 // consecutive k of column j.  No operand is transposed in memory.
 //
 // Two kernels: whole 256 x 256 (a Linear pair: 128 x 256) tiles copied straight into
-// LDS, and 128 x 256 producer / consumer tiles for large K-major x MN-major products
+// LDS, and 128 x 256 producer / consumer tiles for large products with an MN-major B
 // that are not whole (4104 x 4096 x 4104: 162 us, 180 on the tiles of vh_mm.hip,
 // which take every other product).  XCD-aware block order: the blocks resident on
 // one XCD cover groups of 8 m-tiles x a few n-tiles, sharing A and B slices in L2.
@@ -47,6 +47,7 @@ struct DenseArgs {
   int tiles_m, tiles_n;
 };
 
+template <bool AT>
 struct DenseCfg {
   static constexpr int BM = 128, BN = 256;
   static constexpr int BK = 64;            // contraction elements per stage
@@ -56,8 +57,8 @@ struct DenseCfg {
   static constexpr int AIT = BM * KU / 256, BIT = BN * KU / 256;  // load units per thread
   // MN-major tile: BK rows of R elements, pitch R + 32 elements (row starts 64
   // bytes apart mod 256: the four rows of a transposing read hit disjoint banks)
-  static constexpr int BPU = BN / 8 + 4;
-  static constexpr int A_UNITS = BM * PU, B_UNITS = BK * BPU;
+  static constexpr int APU = BM / 8 + 4, BPU = BN / 8 + 4;
+  static constexpr int A_UNITS = AT ? BK * APU : BM * PU, B_UNITS = BK * BPU;
   static constexpr int STAGE = A_UNITS + B_UNITS;  // units per LDS stage
 };
 
@@ -65,15 +66,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, int bytes)
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, bytes, 0x00020000);
 }
 
-// 128 x 256 tiles of a K-major A and an MN-major B, any M and N.  512 threads;
+// 128 x 256 tiles of a K-major (or, AT, MN-major) A and an MN-major B, any M and N.  512 threads;
 // waves 0-3 only multiply (consumers, the accumulators), waves 4-7 only load the
 // next stages into registers and store them into the other LDS buffer (producers,
 // threads 256-511).  Neither role holds the other's registers, so two waves run per
 // SIMD and the loads leave the multiplying waves' instruction stream.
-template <bool BIAS>
+template <bool BIAS, bool AT>
 __global__ __launch_bounds__(512) void gemm_bf16_kernel(DenseArgs g) {
-  using Cfg = DenseCfg;
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, FM = Cfg::FM, FN = Cfg::FN, PU = Cfg::PU, BPU = Cfg::BPU, STAGE = Cfg::STAGE;
+  using Cfg = DenseCfg<AT>;
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, FM = Cfg::FM, FN = Cfg::FN, PU = Cfg::PU, APU = Cfg::APU, BPU = Cfg::BPU,
+                STAGE = Cfg::STAGE;
   extern __shared__ __attribute__((aligned(16))) u32x4d lds[];
   const int lb = xcd_block(g.tiles_m * g.tiles_n);
   const bool producer = threadIdx.x >= 256;
@@ -89,18 +91,27 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(DenseArgs g) {
   const int in_grp = lb - grp * kGroupM * g.tiles_n;
   const int m0 = (first_m + in_grp % gm) * BM, n0 = (in_grp / gm) * BN;
 
-  // Load items.  A: unit u = tid + 256*it -> row u / KU, k unit u % KU (= tid %
-  // KU); global offset of k0 = 0 (the stage's k0 is a scalar offset).  B: unit u ->
-  // k row u / (BN/8), row unit u % (BN/8); the k row's bound is checked per unit (a
+  // Load items.  K-major A: unit u = tid + 256*it -> row u / KU, k unit u % KU (= tid %
+  // KU); global offset of k0 = 0 (the stage's k0 is a scalar offset).  MN-major: unit u
+  // -> k row u / (R/8), row unit u % (R/8); the k row's bound is checked per unit (a
   // scalar offset is not range-checked, so an unused unit carries an out-of-range
   // per-lane offset).
   const int cu = tid % Cfg::KU;
-  int a_off[Cfg::AIT], b_off[Cfg::BIT], b_kr[Cfg::BIT], a_l[Cfg::AIT], b_l[Cfg::BIT];
+  int a_off[Cfg::AIT], b_off[Cfg::BIT], a_kr[Cfg::AIT], b_kr[Cfg::BIT], a_l[Cfg::AIT], b_l[Cfg::BIT];
 #pragma unroll
   for (int it = 0; it < Cfg::AIT; ++it) {
-    const int r = (tid + it * 256) / Cfg::KU;
-    a_off[it] = m0 + r < g.M ? ((m0 + r) * g.lda + cu * 8) * 2 : kOOR;
-    a_l[it] = r * PU + cu;
+    const int u = tid + it * 256;
+    if constexpr (AT) {
+      const int kr = u / (BM / 8), ru = u % (BM / 8);
+      a_kr[it] = kr;
+      a_off[it] = m0 + ru * 8 < g.M ? (kr * g.lda + m0 + ru * 8) * 2 : kOOR;
+      a_l[it] = kr * APU + ru;
+    } else {
+      const int r = u / Cfg::KU;
+      a_kr[it] = cu * 8;
+      a_off[it] = m0 + r < g.M ? ((m0 + r) * g.lda + cu * 8) * 2 : kOOR;
+      a_l[it] = r * PU + cu;
+    }
   }
 #pragma unroll
   for (int it = 0; it < Cfg::BIT; ++it) {
@@ -114,11 +125,11 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(DenseArgs g) {
   u32x4d areg[2][Cfg::AIT], breg[2][Cfg::BIT];
   auto gload = [&](auto SET, int k0) {
     constexpr int s = decltype(SET)::value;
-    const int ask = k0 * 2, bsk = k0 * g.ldb * 2;
+    const int ask = AT ? k0 * g.lda * 2 : k0 * 2, bsk = k0 * g.ldb * 2;
 #pragma unroll
     for (int it = 0; it < Cfg::AIT; ++it)  // K % 8 == 0: a K-major unit is all in or all out
       areg[s][it] = __builtin_bit_cast(
-          u32x4d, __builtin_amdgcn_raw_buffer_load_b128(ar, k0 + cu * 8 < g.K ? a_off[it] : kOOR, ask, 0));
+          u32x4d, __builtin_amdgcn_raw_buffer_load_b128(ar, k0 + a_kr[it] < g.K ? a_off[it] : kOOR, ask, 0));
 #pragma unroll
     for (int it = 0; it < Cfg::BIT; ++it)
       breg[s][it] = __builtin_bit_cast(
@@ -134,16 +145,16 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(DenseArgs g) {
   };
 
   const int row_l = lane & 31, half_l = lane >> 5;
-  // transposing reads of the MN-major tile: lane l reads k row 8*(l/32) + (l%16)/4
+  // transposing reads of an MN-major tile: lane l reads k row 8*(l/32) + (l%16)/4
   // (+4 for the second half of the fragment), elements 16*((l/16)%2) + 4*(l%4) .. +3
   const int tr_row = 8 * half_l + ((lane & 15) >> 2), tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  auto frag_mn = [&](const u32x4d* tile, int ks, int col0) {
+  auto frag_mn = [&](const u32x4d* tile, int pitch, int ks, int col0) {
     typedef short v4i16 __attribute__((ext_vector_type(4)));
     const __attribute__((address_space(3))) char* p =
-        (const __attribute__((address_space(3))) char*)(tile) + (((ks * 8 + tr_row) * BPU) * 16 + (col0 + tr_col) * 2);
+        (const __attribute__((address_space(3))) char*)(tile) + (((ks * 8 + tr_row) * pitch) * 16 + (col0 + tr_col) * 2);
     const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)p);
     const v4i16 hi =
-        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(p + 4 * BPU * 16));
+        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16*)(p + 4 * pitch * 16));
     typedef short v8i16 __attribute__((ext_vector_type(8)));
     const v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     return __builtin_bit_cast(bf16x8, v);
@@ -180,15 +191,17 @@ __global__ __launch_bounds__(512) void gemm_bf16_kernel(DenseArgs g) {
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
-    const u32x4d* ap = lds + (kt & 1) * STAGE + (wm + row_l) * PU + half_l;
-    const u32x4d* bt = lds + (kt & 1) * STAGE + Cfg::A_UNITS;
+    const u32x4d* at = lds + (kt & 1) * STAGE;
+    const u32x4d* ap = at + (wm + row_l) * PU + half_l;
+    const u32x4d* bt = at + Cfg::A_UNITS;
 #pragma unroll
     for (int ks = 0; ks < Cfg::KU; ks += 2) {
       bf16x8 af[FM], bf[FN];
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = __builtin_bit_cast(bf16x8, ap[i * 32 * PU + ks]);
+      for (int i = 0; i < FM; ++i)
+        af[i] = AT ? frag_mn(at, APU, ks, wm + i * 32) : __builtin_bit_cast(bf16x8, ap[i * 32 * PU + ks]);
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bf[j] = frag_mn(bt, ks, wn + j * 32);
+      for (int j = 0; j < FN; ++j) bf[j] = frag_mn(bt, BPU, ks, wn + j * 32);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -547,14 +560,15 @@ void gemm_bf16_d2l_pair_kernel(DenseArgs g0, DenseArgs g1) {
 
 bool fits(long bytes) { return bytes >= 0 && bytes < (1L << 31) - 64; }
 
-template <bool BIAS>
+template <bool BIAS, bool AT>
 int launch_gemm(const DenseArgs& a0, hipStream_t st) {
-  auto kern = gemm_bf16_kernel<BIAS>;
+  using Cfg = DenseCfg<AT>;
+  auto kern = gemm_bf16_kernel<BIAS, AT>;
   VH_LDS_LIMIT_ONCE(kern);
   DenseArgs a = a0;
-  a.tiles_m = (a.M + DenseCfg::BM - 1) / DenseCfg::BM;
-  a.tiles_n = (a.N + DenseCfg::BN - 1) / DenseCfg::BN;
-  kern<<<dim3((unsigned)(a.tiles_m * a.tiles_n)), 512, (size_t)2 * DenseCfg::STAGE * 16, st>>>(a);
+  a.tiles_m = (a.M + Cfg::BM - 1) / Cfg::BM;
+  a.tiles_n = (a.N + Cfg::BN - 1) / Cfg::BN;
+  kern<<<dim3((unsigned)(a.tiles_m * a.tiles_n)), 512, (size_t)2 * Cfg::STAGE * 16, st>>>(a);
   VH_LAUNCH_CHECK();
   return VH_OK;
 }
@@ -591,8 +605,14 @@ DenseArgs dense_args(const void* a, int lda, bool at, const void* b, int ldb, bo
   return g;
 }
 
-// 128 x 256 tiles when they still give at least one block per CU
-bool dense_big(int M, int N) { return (long)((M + 127) / 128) * ((N + 255) / 256) >= 256; }
+// 128 x 256 tiles when they still give at least one block per CU; of an MN-major A
+// where their rounds of 256 are at least four fifths full (us here and on the tiles of
+// vh_mm.hip: 2688 x 8064 x 2816, 672 tiles: 131 and 153; 8064 x 2816 x 2688, 693: 127 and 130;
+// 5632 x 1408 x 1920, 264: 59 and 34)
+bool dense_big(long M, long N, bool at) {
+  const long t = ((M + 127) / 128) * ((N + 255) / 256);
+  return t >= 256 && (!at || t * 5 >= (t + 255) / 256 * 256 * 4);
+}
 
 // The 256 x 256 direct-to-LDS kernel: whole tiles only (no bounds checks in
 // its loads or stores), K in whole stages, 16-byte aligned rows of every
@@ -623,8 +643,9 @@ int dense_bf16_gemm(const void* a, int lda, bool at, const void* b, int ldb, boo
     return bt ? launch_d2l<false, true>(g, st) : launch_d2l<false, false>(g, st);
   }
   // not whole tiles, at least one block per CU
-  if (at || !bt || !dense_big(M, N)) return VH_ERR_UNSUPPORTED;
-  return bias ? launch_gemm<true>(g, st) : launch_gemm<false>(g, st);
+  if (!bt || (at && bias) || !dense_big(M, N, at)) return VH_ERR_UNSUPPORTED;
+  if (at) return launch_gemm<false, true>(g, st);
+  return bias ? launch_gemm<true, false>(g, st) : launch_gemm<false, false>(g, st);
 }
 
 namespace {

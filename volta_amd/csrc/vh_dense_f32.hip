@@ -23,6 +23,7 @@ struct DenseF32Args {
   const float* a;     // [M][lda] (K-major) or [K][lda] (MN-major)
   const float* b;     // [N][ldb] (K-major) or [K][ldb] (MN-major)
   float* c;           // [M][ldc]
+  const float* bias;  // [N] or nullptr
   float* colsum;      // [N] or nullptr: column sums of an MN-major B over K (pair kernel)
   int M, N, K, lda, ldb, ldc;
   int a_bytes, b_bytes, c_bytes;
@@ -71,7 +72,7 @@ struct F32D2lCfg {
 // own 4 << cs_shift of its columns, so every column is summed by exactly one
 // block over all K; a thread adds 4 consecutive owned columns of one k row per
 // stage, in stage order, and the k-row group sums are added in group order.
-template <int BM, bool AT, bool BT, bool CS>
+template <int BM, bool AT, bool BT, bool CS, bool BIAS = false>
 __device__ __forceinline__ void f32_d2l_tile(const DenseF32Args& g, const int lb, u32x4f* S0, u32x4f* S1) {
   using Cfg = F32D2lCfg<BM>;
   constexpr int FM = Cfg::FM, FN = Cfg::FN, UNITS_A = Cfg::A_UNITS;
@@ -234,28 +235,30 @@ __device__ __forceinline__ void f32_d2l_tile(const DenseF32Args& g, const int lb
     }
   }
 
-  // epilogue: fp32 stores, lanes walk columns (32 columns x 2 rows per store)
+  // epilogue: (+ bias) fp32 stores, lanes walk columns (32 columns x 2 rows per store)
   const __amdgpu_buffer_rsrc_t cr = rsrc_f(g.c, g.c_bytes);
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     const int col = n0 + wn + j * 32 + row_l;
     const int voff = (col + half_l * 4 * g.ldc) * 4;
+    const float bv = BIAS ? g.bias[col] : 0.f;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int row = m0 + wm + i * 32 + (v >> 2) * 8 + (v & 3);  // + 4 * half_l
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, (float)acc[i][j][v]), cr, voff,
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, acc[i][j][v] + bv), cr, voff,
                                               row * g.ldc * 4, 0);
       }
   }
 }
 
+template <bool AT, bool BT, bool BIAS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_f32_d2l_kernel(DenseF32Args g) {
   __shared__ __attribute__((aligned(16))) u32x4f S0[F32D2lCfg<256>::STAGE];
   __shared__ __attribute__((aligned(16))) u32x4f S1[F32D2lCfg<256>::STAGE];
-  f32_d2l_tile<256, true, true, false>(g, xcd_block(g.tiles_m * g.tiles_n), S0, S1);
+  f32_d2l_tile<256, AT, BT, false, BIAS>(g, xcd_block(g.tiles_m * g.tiles_n), S0, S1);
 }
 
 // Two products in one launch on 128 x 256 tiles (Linear's dX, K-major x
@@ -327,16 +330,26 @@ int dense_f32_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStrea
 }
 
 int dense_f32_gemm(const void* a, int lda, bool at, const void* b, int ldb, bool bt, void* c, int ldc, int M,
-                   int N, int K, hipStream_t st) {
+                   int N, int K, const void* bias, hipStream_t st) {
   // whole 256 x 256 tiles that fill the chip (16-byte aligned operand rows; the
-  // stores are 4-byte)
-  if (!at || !bt || M % 256 || N % 256 || K % (2 * kF32D2lBK) || lda % 4 || ldb % 4 ||
+  // stores are 4-byte): 4096 x 4096 x 1024 254 us, 272 on the tiles of vh_mm.hip; 4096^3 979
+  // and 1044, of MN-major A and B 931 and 985
+  if ((at && !bt) || (at && bias) || M % 256 || N % 256 || K % (2 * kF32D2lBK) || lda % 4 || ldb % 4 ||
       (long)(M / 256) * (N / 256) < 256)
     return VH_ERR_UNSUPPORTED;
   DenseF32Args g = f32_args(a, lda, at, b, ldb, bt, c, ldc, M, N, K);
+  g.bias = (const float*)bias;
   g.tiles_m = M / 256;
   g.tiles_n = N / 256;
-  gemm_f32_d2l_kernel<<<dim3((unsigned)(g.tiles_m * g.tiles_n)), 512, 0, st>>>(g);
+  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n));
+  if (at)
+    gemm_f32_d2l_kernel<true, true, false><<<grid, 512, 0, st>>>(g);
+  else if (bt)
+    bias ? gemm_f32_d2l_kernel<false, true, true><<<grid, 512, 0, st>>>(g)
+         : gemm_f32_d2l_kernel<false, true, false><<<grid, 512, 0, st>>>(g);
+  else
+    bias ? gemm_f32_d2l_kernel<false, false, true><<<grid, 512, 0, st>>>(g)
+         : gemm_f32_d2l_kernel<false, false, false><<<grid, 512, 0, st>>>(g);
   VH_LAUNCH_CHECK();
   return VH_OK;
 }

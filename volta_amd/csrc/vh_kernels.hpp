@@ -188,7 +188,7 @@ int gather_run(int dt, const GatherCall& c, void* ws, hipStream_t st);
 // [N][ldb] or, with bt, [K][ldb].
 bool dense_bf16_ok(long M, long N, long K, bool at, long lda, bool bt, long ldb, long ldc, const void* a,
                    const void* b, const void* c);
-// Whole 256 x 256 tiles, or 128 x 256 ones of a large K-major A and MN-major B;
+// Whole 256 x 256 tiles, or 128 x 256 ones of a large product with an MN-major B;
 // VH_ERR_UNSUPPORTED for every other product.
 int dense_bf16_gemm(const void* a, int lda, bool at, const void* b, int ldb, bool bt, void* c, int ldc, int M,
                     int N, int K, const void* bias, hipStream_t st);
@@ -208,11 +208,11 @@ struct DenseProblem {
 };
 int dense_bf16_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStream_t st);
 // The same in fp32 (vh_dense_f32.hip): K % 4 == 0, 16-byte aligned A and B; the
-// single product whole 256 x 256 tiles of an MN-major A and B.
+// single product whole 256 x 256 tiles only.
 bool dense_f32_ok(long M, long N, long K, bool at, long lda, bool bt, long ldb, long ldc, const void* a,
                   const void* b, const void* c);
 int dense_f32_gemm(const void* a, int lda, bool at, const void* b, int ldb, bool bt, void* c, int ldc, int M,
-                   int N, int K, hipStream_t st);
+                   int N, int K, const void* bias, hipStream_t st);
 int dense_f32_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStream_t st);
 
 // ---- products of any size (vh_mm.hip) ----
