@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import oracle
+from tests.parity import assert_parity
 from tests.test_gpu_parity import DEV, DTYPES, check, host, prep, rng
 from volta_amd import nn as vnn
 from volta_amd import ops
@@ -99,3 +100,28 @@ def test_mm_bf16_stages_in_flight(m, k, n):
     gr, grt = prep(g.standard_normal((m, k)), "bf16")  # dA = G [m][k] . B^T, reduced over k
     w, wt = prep(g.standard_normal((n, k)), "bf16")
     check(ops.gpu_matmul_backward_a(grt, wt, m, n, k), oracle.matmul_backward_a, (gr, w), "bf16", "dA", k=k)
+
+
+# a long batch over few features (dW: few tiles of a deep K, split beside dX's many), then
+# the pair on 64 x 128 and 128 x 128 tiles (bf16) with remainders, aligned rows and padded ones
+@pytest.mark.parametrize("shape", [(5000, 12, 30), (4100, 70, 64), (1030, 1032, 2056), (1700, 1544, 1800), (2056, 1290, 2312)])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_mm_linear_gradients_in_one_launch(shape, dt):
+    m, i, o = shape
+    g = rng(m + i + o)
+    x, xt = prep(g.standard_normal((m, i)), dt)
+    w, wt = prep(g.uniform(-0.5, 0.5, (i, o)), dt)
+    dy, dyt = prep(g.standard_normal((m, o)), dt)
+    lin = vnn.Linear(i, o, device=DEV, dtype=DTYPES[dt])
+    lin.weight = wt
+    ref = oracle.linear_backward(dy, x, w)
+    scale = oracle.linear_backward(np.abs(dy), np.abs(x), np.abs(w))
+    for got, r, s, what, k in zip(lin.backward(dyt, xt), ref, scale, ("dx", "dw", "db"), (o, m, m)):
+        assert_parity(host(got), r, s, dt, what, k=k)
+
+
+# K short or an operand long: the implicit GEMM's side of the rule, and just past it
+@pytest.mark.parametrize("mkn", [(30, 38, 139), (60, 161, 120), (4000, 9, 37), (4000, 25, 150), (3, 2050, 1003), (17, 1030, 3001)])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_mm_or_implicit_gemm(mkn, dt):
+    test_mm_family(mkn, dt)

@@ -5,15 +5,68 @@
 // Every backward composition is run in its sizing mode (the same dispatch as
 // a real call: algorithm choice, stride phases, weight-gradient plans,
 // split-K plans, im2col sizes; it stops before any launch) over a grid of
-// shapes, dtypes and algorithms, together with the algorithm selectors and the
-// shape checks of the entry points.  A sanitizer report or a bad size fails.
+// shapes, dtypes and algorithms, together with the plans of products and Linear
+// layers up to the largest sizes, the algorithm selectors and the shape checks of the
+// entry points.  A sanitizer report, a bad size or a bad plan fails.
 #include "vh_api.hip"
 
 #include <cstdio>
 
+namespace {
+using namespace vh;
+long n = 0, fails = 0;
+
+// The plan of a product or a Linear layer's pair: the splits cover K, the workspace
+// holds them, and no block is left with a long K of its own beside an idle chip.
+void check_mm(int dt, const DenseProblem* p, int np) {
+  MmInfo o;
+  ++n;
+  if (!mm_info(dt, p, np, &o)) return;
+  const long bk = dt == VH_BF16 ? 64 : 32;
+  double work = 0;
+  size_t part = 0;
+  for (int i = 0; i < np; ++i) {
+    const long st = (p[i].K + bk - 1) / bk;
+    work += (double)((p[i].M + o.bm - 1L) / o.bm) * ((p[i].N + o.bn - 1L) / o.bn) * st;
+    if (o.splits[i] > 1) part += (size_t)o.splits[i] * p[i].M * p[i].N * 4;
+    if (o.splits[i] < 1 || (long)o.splits[i] * o.per[i] < st || (long)(o.splits[i] - 1) * o.per[i] >= st) {
+      printf("bad splits %d x %d of %ld stages: %d %d %d\n", o.splits[i], o.per[i], st, p[i].M, p[i].N, p[i].K);
+      ++fails;
+    }
+  }
+  for (int i = 0; i < np; ++i)
+    if (o.per[i] > 64 + 3 * work / 256) {
+      printf("a block of %d stages, %.0f a CU: dt%d np%d %d %d %d\n", o.per[i], work / 256, dt, np, p[i].M, p[i].N, p[i].K);
+      ++fails;
+    }
+  if (o.bytes < part) {
+    printf("workspace %zu below the partials %zu: %d %d %d\n", o.bytes, part, p[0].M, p[0].N, p[0].K);
+    ++fails;
+  }
+}
+
+void check_products() {
+  char* q = reinterpret_cast<char*>(4096);
+  const int dims[] = {1, 2, 7, 10, 31, 64, 65, 130, 500, 513, 1000, 2048, 4097, 16384, 100003, 1 << 24, (1 << 30) + 1, INT32_MAX};
+  for (int dt : {(int)VH_F32, (int)VH_BF16})
+    for (int M : dims)
+      for (int N : dims)
+        for (int K : dims) {
+          if (std::max({(long)M * K, (long)K * N, (long)M * N}) > kMaxElems) continue;
+          const DenseProblem nn{q, K, false, q, N, true, q, N, M, N, K, nullptr}, nt{q, K, false, q, K, false, q, N, M, N, K, nullptr},
+              tn{q, M, true, q, N, true, q, N, M, N, K, nullptr};
+          check_mm(dt, &nn, 1);
+          check_mm(dt, &nt, 1);
+          check_mm(dt, &tn, 1);
+          // a Linear layer of M rows, K -> N features
+          const DenseProblem pair[2] = {{q, N, false, q, N, false, q, K, M, K, N, nullptr}, {q, K, true, q, N, true, q, N, K, N, M, q}};
+          check_mm(dt, pair, 2);
+          (void)linear_pair(dt, pair);
+        }
+}
+}  // namespace
+
 int main() {
-  using namespace vh;
-  long n = 0, fails = 0;
   const long Bs[] = {1, 2, 3, 16, 128};
   const long Cs[] = {1, 3, 16, 27, 64, 256};
   const long Hs[] = {1, 5, 14, 28, 56, 256};
@@ -69,6 +122,7 @@ int main() {
       ++fails;
     }
   }
+  check_products();
   printf("host_check: %ld plans, %ld failures\n", n, fails);
   return fails ? 1 : 0;
 }

@@ -894,12 +894,8 @@ static bool product_try(int dt, const DenseProblem* p, int np, const void* bias,
     plain = plain && (np == 2 || !p[i].colsum);
   }
   if (plain && (*r = dense_large(dt, p, np, bias, st)) != VH_ERR_UNSUPPORTED) return true;
-  bool ok;
-  const size_t bytes = mm_ws(dt, p, np, &ok);
-  void* ws = nullptr;
-  if (!ok || (bytes && !ws_try(st, bytes, &ws))) return false;
-  *r = mm_run(dt, p, np, bias, ws, st);
-  return true;
+  *r = mm_run(dt, p, np, bias, ws_get, st);
+  return *r != VH_ERR_UNSUPPORTED && *r != VH_ERR_OOM && *r != VH_ERR_CAPTURE;
 }
 
 static int gemm(int dt, int ak, int bk, const void* a, int lda, const void* b, int ldb, void* c, int ldc,
@@ -1579,16 +1575,22 @@ int vh_linear_forward(int dtype, const void* x, const void* weight, const void* 
               m, out_features, in_features, bias, 2, S(stream));
 }
 
-// Whether a Linear layer's dX and dW go in one launch: on the whole-tile pair
-// kernels, or where the two grids of 64 x 64 tiles leave room in four blocks a CU.
+// Whether a Linear layer's dX and dW go in one launch: on the whole-tile pair kernels,
+// or where the pair's plan is the faster one.  A product of whole 256 x 256 tiles that
+// fill the chip keeps its own kernel, ahead of any pair of smaller ones.
 static bool linear_pair(int dt, const DenseProblem* p) {
-  long g64 = 0;
-  bool whole = true;
+  bool whole = true, large = false;
+  long tiles = 0;
   for (int i = 0; i < 2; ++i) {
-    g64 += ((p[i].M + 63L) / 64) * ((p[i].N + 63L) / 64);
     whole = whole && p[i].M % 128 == 0 && p[i].N % 256 == 0 && p[i].K % 128 == 0;
+    tiles += (p[i].M / 128L) * (p[i].N / 256L);
+    large = large || (p[i].M % 256 == 0 && p[i].N % 256 == 0 && p[i].K % 128 == 0 &&
+                      (p[i].M / 256L) * (p[i].N / 256L) >= 256);
   }
-  return dt == VH_F32 || whole || g64 <= 1024;
+  if (whole && tiles >= 256) return true;
+  MmInfo pair, dx, dw;
+  if (large || !mm_info(dt, p, 2, &pair)) return false;
+  return !mm_info(dt, p, 1, &dx) || !mm_info(dt, p + 1, 1, &dw) || pair.us <= dx.us + dw.us + 2.f;
 }
 
 int vh_linear_backward(int dtype, const void* out_grad, const void* x, const void* weight, void* grad_x,

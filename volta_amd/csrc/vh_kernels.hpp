@@ -218,10 +218,20 @@ int dense_f32_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStrea
 // ---- products of any size (vh_mm.hip) ----
 // One product, or a Linear layer's dX (K-major x K-major) and dW (MN-major x
 // MN-major) as a pair; colsum (of an MN-major A and B): the column sums of B over K.
-// bias [N] of a single product.  Workspace bytes (possibly 0); *ok false: an empty
-// or too large (32-bit byte offsets) product.
-size_t mm_ws(int dt, const DenseProblem* p, int np, bool* ok);
-int mm_run(int dt, const DenseProblem* p, int np, const void* bias, void* ws, hipStream_t st);
+// bias [N] of a single product.  VH_ERR_UNSUPPORTED: an empty or too large (32-bit
+// byte offsets) product, or one that the implicit GEMM computes sooner; the status of
+// `get`, asked for the call's workspace if it needs any, where that is not VH_OK.
+// Nothing is queued then.
+using WsGet = int (*)(hipStream_t st, size_t bytes, void** out);
+int mm_run(int dt, const DenseProblem* p, int np, const void* bias, WsGet get, hipStream_t st);
+// The plan of a call: tile, K splits and stages of each, workspace, the time it was
+// chosen by (us); false: unsupported.
+struct MmInfo {
+  int bm, bn, splits[2], per[2];
+  size_t bytes;
+  float us;
+};
+bool mm_info(int dt, const DenseProblem* p, int np, MmInfo* o);
 
 // ---- strided 1x1 bf16 convolutions, pad 0 (vh_pointwise.hip) ----
 // w is the OIHW weight itself ([O][C]).  Each returns VH_ERR_UNSUPPORTED

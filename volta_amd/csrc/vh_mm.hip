@@ -7,10 +7,11 @@
 // CUs (256 x 784 -> 512 fp32: 43 us on 64 x 128 tiles), or operands whose rows are
 // not 16-byte aligned and were gathered element by element (K = 2001: 70 - 95 us a
 // product that takes 17 on whole units).  So
-//  * tiles are 64 x 64 and smaller, two to five blocks a CU; below one block a CU
-//    the four waves of a block split K (KS groups of waves, every KS-th stage each,
-//    added in group order), and what is still short is split over blocks (fp32
-//    partials, added in split order by mm_reduce_kernel);
+//  * tiles are 32 x 32 to 64 x 64 (bf16: to 128 x 128), two to five blocks a CU; the
+//    four waves of a block of the smaller ones split K (KS groups of waves, every KS-th
+//    stage each, added in group order), and what is still short is split over blocks
+//    (fp32 partials, added in split order by mm_reduce_kernel); a cost model of the
+//    tiles picks both (mm_plan);
 //  * operands whose rows are not whole 16-byte units are first copied to padded
 //    rows (mm_pad_kernel: both operands in one launch); the products then copy
 //    whole units straight into LDS (vh_tiles.hpp).
@@ -318,48 +319,114 @@ __global__ __launch_bounds__(256) void mm_pad_kernel(PadSeg p0, PadSeg p1, int b
 // ---------------------------------------------------------------- host side
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
-struct Tile {
-  int bm, bn;
+// What a tile costs, us: `alone`, a pass of the wave groups over their stages by a
+// block that has its CU to itself; `busy`, the same as a share of a CU full of blocks;
+// both larger by a fraction where operand rows do not start on 128-byte lines (every
+// copy of a row then reads two); `ends`, prologue and epilogue, in passes; `fit`, the
+// blocks that fit a CU.  Fitted to 2600 timings of all tiles and splits over 130
+// products of 1 .. 8192 rows (K to 65536); the plan it picks takes 1.01 - 1.06 times
+// the best one's time in the mean.
+struct TileCost {
+  int bm, bn, ks, fit;
+  float alone, busy, busy_off, ends, alone_off;
 };
-
-// The tile of a product, or of a pair launched together (both grids counted; 64 x
-// 64 and below), by its cost.  fp32 gains nothing above 64 x 64 (4096^3: 978 us, 970
-// on 64 x 128).
 template <typename T>
-Tile mm_pick(const DenseProblem* p, int np) {
-  static constexpr Tile tile[] = {{64, 64}, {32, 64}, {32, 32}, {64, 128}, {128, 128}};
-  int nst = 1;
-  for (int i = 0; i < np; ++i) nst = std::max(nst, (p[i].K + GT<T>::BK - 1) / GT<T>::BK);
-  Tile best{64, 64};
-  float least = 1e30f;
-  for (int k = 0; k < (GT<T>::ES == 2 && np == 1 ? 5 : 3); ++k) {
-    long n = 0;
-    for (int i = 0; i < np; ++i)
-      n += (long)((p[i].M + tile[k].bm - 1) / tile[k].bm) * ((p[i].N + tile[k].bn - 1) / tile[k].bn);
-    const float cost = tile_cost<T>(tile[k].bm, tile[k].bn, nst, n);
-    if (cost < least) {
-      least = cost;
-      best = tile[k];
-    }
-  }
-  return best;
+constexpr int mm_tiles() {  // fp32 gains nothing above 64 x 64 (4096^3: 978 us, 970 on 64 x 128)
+  return GT<T>::ES == 2 ? 5 : 3;
+}
+template <typename T>
+const TileCost* mm_costs(bool at) {
+  static constexpr TileCost b16[] = {{64, 64, 1, 5, .25f, .196f, .20f, 2.0f, .25f},
+                                     {32, 64, 2, 3, .25f, .232f, .20f, 2.2f, .26f},
+                                     {32, 32, 4, 2, .40f, .325f, .11f, 2.0f, .26f},
+                                     {64, 128, 1, 3, .27f, .307f, .21f, 2.5f, .29f},
+                                     {128, 128, 1, 2, .42f, .471f, 0.f, 5.6f, .24f}};
+  // MN-major A and B: bound by their transposing reads
+  static constexpr TileCost b16t[] = {{64, 64, 1, 5, .48f, .200f, .30f, 2.0f, .35f},
+                                      {32, 64, 2, 3, .40f, .300f, .25f, 2.0f, .30f},
+                                      {32, 32, 4, 2, .60f, .480f, .10f, 2.0f, .30f},
+                                      {64, 128, 1, 3, .55f, .305f, .25f, 2.7f, .15f},
+                                      {128, 128, 1, 2, .74f, .520f, 0.f, 3.3f, .07f}};
+  static constexpr TileCost f32[] = {{64, 64, 1, 5, .58f, .512f, .02f, 2.0f, 0.f},
+                                     {32, 64, 2, 3, .58f, .585f, .02f, 2.0f, .02f},
+                                     {32, 32, 4, 2, .75f, .630f, .05f, 2.5f, .15f}};
+  return GT<T>::ES == 4 ? f32 : at ? b16t : b16;
 }
 
+constexpr float kSplitUs = 4.f;  // of the reduction's launch
+
+// Tile and K splits of a product, or of a Linear layer's pair in one launch.
+struct MmPlan {
+  TileCost t;
+  int per[2], splits[2];  // stages per split
+  float us;
+};
 template <typename T>
-void mm_plan(MmArgs& a, const Tile& t, long blocks) {
-  constexpr int BK = GT<T>::BK;
-  const int ks = t.bm == 32 ? (t.bn == 32 ? 4 : 2) : 1;
-  const int stages = (a.K + BK - 1) / BK;
-  a.tiles_m = (a.M + t.bm - 1) / t.bm;
-  a.tiles_n = (a.N + t.bn - 1) / t.bn;
-  // below half the CUs: split K for a block on each, at least 2 stages of every
-  // wave group (fp32 32 x 4096 x 64, 2 blocks: 23 -> 6.8 us at 16 splits; 128 x 8192
-  // x 256: 47 -> 11.6).  A bf16 product of over 32 blocks loses more to the partials
-  // (512 x 4096 x 128: 9.9 us, 15 split by 4).
-  int want = blocks < (GT<T>::ES == 2 ? 33 : 128) ? (int)std::min<long>(256 / blocks, stages / (2 * ks)) : 1;
-  want = std::max(1, want);
-  a.per = (stages + want - 1) / want;
-  a.splits = (stages + a.per - 1) / a.per;
+MmPlan mm_plan(const DenseProblem* p, int np) {
+  constexpr int BK = GT<T>::BK, ES = GT<T>::ES;
+  MmPlan best{};
+  best.us = 1e30f;
+  long stages[2] = {0, 0}, deepest = 0;
+  bool off = false;
+  for (int i = 0; i < np; ++i) {
+    stages[i] = ((long)p[i].K + BK - 1) / BK;
+    deepest = std::max(deepest, stages[i]);
+    off = off || (long)p[i].lda * ES % 128 || (long)p[i].ldb * ES % 128;
+  }
+  const TileCost* costs = mm_costs<T>(p[np - 1].at);
+  // (sizes of tiles and groups are powers of two: no divisions without splits, the plan of
+  // a small call takes 0.1 us)
+  auto consider = [&](const TileCost& t, int s) -> long {
+    const long cap = s > 1 ? (deepest + s - 1) / s : deepest;
+    // every split computes at least two passes of each wave group: its copies cover
+    // nothing otherwise
+    if (s > 1 && cap < 2 * t.ks) return 1L << 30;
+    const int lm = __builtin_ctz(t.bm), ln = __builtin_ctz(t.bn), lk = __builtin_ctz(t.ks);
+    MmPlan m{t, {0, 0}, {1, 1}, 0.f};
+    long blocks = 0, longest = 0;
+    float work = 0.f;
+    for (int i = 0; i < np; ++i) {
+      long tiles = (((long)p[i].M + t.bm - 1) >> lm) * (((long)p[i].N + t.bn - 1) >> ln), per = stages[i];
+      if (per > cap) {
+        const long n = std::min(256L, (per + cap - 1) / cap);
+        per = (per + n - 1) / n;
+        m.splits[i] = (int)((stages[i] + per - 1) / per);
+        if (tiles > 256) return 1L << 30;
+        tiles *= m.splits[i];
+        // partials: written and read at 6 TB/s
+        m.us += (float)m.splits[i] * (float)p[i].M * (float)p[i].N * 1.33e-6f;
+      }
+      m.per[i] = (int)per;
+      const long passes = (per + t.ks - 1) >> lk;
+      blocks += tiles;
+      longest = std::max(longest, passes);
+      work += (float)tiles * ((float)passes + t.ends);
+    }
+    if (m.splits[0] > 1 || m.splits[1] > 1) m.us += kSplitUs;
+    const float alone = t.alone * (off ? 1.f + t.alone_off : 1.f), busy = t.busy * (off ? 1.f + t.busy_off : 1.f);
+    const long rounds = (blocks + 255) >> 8;   // blocks on the fullest CU
+    const float mean = work / (float)blocks;   // passes of a block
+    float deep;                                // a block's share of the CU's time
+    if (rounds <= t.fit)
+      deep = busy * (float)rounds;
+    else if (rounds <= 2 * t.fit)  // what does not fit starts when the first blocks end, all about together
+      deep = busy * (float)t.fit + std::max(alone, busy * (float)(rounds - t.fit));
+    else
+      deep = busy * (float)blocks / 256.f + .5f * alone;
+    m.us += std::max(alone * ((float)longest + t.ends), deep * mean);
+    if (m.us < best.us) best = m;
+    return blocks;
+  };
+  constexpr int nt = mm_tiles<T>();
+  long blocks[nt];
+  for (int k = 0; k < nt; ++k) blocks[k] = consider(costs[k], 1);
+  // A split pays for its reduction where the grid leaves room (fp32 512 x 512 x 8192: 52
+  // -> 43 us at 16 splits, 64 x 2048 x 2048: 14.8 -> 12.5) or one product of a pair has
+  // few deep blocks (Linear 16384 x 64 -> 64 backward, one tile of dW: 112 -> 20).
+  for (int k = 0; k < 3 && best.us > 2 * kSplitUs; ++k)
+    for (int s = 2; s <= 256; s += std::max(1, s / 4))
+      if (consider(costs[k], s) > blocks[k] + 2048) break;
+  return best;
 }
 
 // An operand with its rows as whole 16-byte units: stored rows (K-major: M or N;
@@ -380,11 +447,41 @@ Opnd opnd(const void* p, int rows, int cols, int ld) {
   return o;
 }
 
+// Products that the implicit GEMM (element-wise gathers, no copies) computes sooner:
+// an operand's rows need a copy, and
+//  * the product is over in less than the copy's launch (us here and there: bf16 30 x 139
+//    x 38 8.5 and 10.0; fp32 10 x 55 x 9 8.3 and 9.1; but 298 x 9 x 254 21.7 and 9.1), or
+//    K is so short that the copy doubles the traffic (fp32 4766 x 89 x 9: 7.7 and 9.3; 7028 x
+//    657 x 4 11.9 and 9.3);
+//  * it reads a long operand once, by many blocks or with K split: of few rows (fp32 3 x
+//    1274 x 11586 24.7 and 37, 42 x 1817 x 4365 24.3 and 29.1; 62 x 1002 x 945, 16 tiles of a K
+//    not split there, 44 and 13), or few columns of an MN-major A (fp32 15665 x 31 x 14088
+//    347 and 505).  bf16 gathers of K-major rows are slow (35 x 2764 x 4314 39 and 20), those
+//    of an MN-major B ahead at 3 x 1490 x 5800 (15.8 and 24) and 48 x 3511 x 9048 (32 and 38),
+//    not at 56 x 10447 x 1455 (31 and 23); of both operands MN-major at 35 x 2764 x 4314 (19.7
+//    and 21.6), not at 18 x 220 x 71840 (74 and 32).
+template <typename T>
+bool mm_generic(const DenseProblem& q, const Opnd& a, const Opnd& b, bool alone) {
+  if (!a.ldp && !b.ldp) return false;
+  const double mnk = (double)q.M * q.N * q.K;
+  constexpr bool b16 = GT<T>::ES == 2;
+  if (alone && ((q.K <= (b16 ? 160 : 96) && mnk <= 5e5) || (q.K <= 24 && mnk <= 1.5e7 && !q.at))) return true;
+  const bool wide = q.M <= (b16 ? 64 : 96);
+  const int len = wide ? q.N : q.M;  // it is read by len / 64 tiles at once, or split
+  if ((q.K < 1024 && (b16 || len < 8192)) || (!wide && (q.N > 64 || !q.at))) return false;
+  const Opnd& o = wide ? b : a;
+  if (!o.ldp || (q.at && (b16 || !wide) && len < (b16 ? 1500 : 1000))) return false;
+  const double bytes = (double)o.rows * o.cols * GT<T>::ES;
+  if (q.at || !b16) return bytes > (wide && !b16 ? 2e6 : 8e6);
+  return q.bt && bytes > (q.M <= 16 ? 14e6 : 40e6);
+}
+
 struct MmLayout {
   Opnd a[2], b[2];
   MmArgs g[2];
-  Tile t;
+  TileCost t;
   size_t part[2], cpart[2], copies, bytes;
+  float us;
   bool shared;
 };
 
@@ -392,15 +489,19 @@ template <typename T>
 bool mm_layout(const DenseProblem* p, int np, const void* bias, MmLayout& l) {
   constexpr int ES = GT<T>::ES;
   l.bytes = 0;
-  l.t = mm_pick<T>(p, np);
+  for (int i = 0; i < np; ++i)
+    if (std::min({p[i].M, p[i].N, p[i].K}) <= 0 || std::max({p[i].M, p[i].N, p[i].K}) > (1 << 30) ||
+        (p[i].at && !p[i].bt))
+      return false;
+  const MmPlan m = mm_plan<T>(p, np);
+  l.t = m.t;
+  l.us = m.us;
   long blocks = 0;
-  for (int i = 0; i < np; ++i) blocks += (long)((p[i].M + l.t.bm - 1) / l.t.bm) * ((p[i].N + l.t.bn - 1) / l.t.bn);
-  if (blocks > (1L << 30)) return false;
   for (int i = 0; i < np; ++i) {
     const DenseProblem& q = p[i];
-    if (q.M <= 0 || q.N <= 0 || q.K <= 0 || (q.at && !q.bt)) return false;
     l.a[i] = opnd<T>(q.a, q.at ? q.K : q.M, q.at ? q.M : q.K, q.lda);
     l.b[i] = opnd<T>(q.b, q.bt ? q.K : q.N, q.bt ? q.N : q.K, q.ldb);
+    if (mm_generic<T>(q, l.a[i], l.b[i], np == 1)) return false;
     MmArgs& g = l.g[i];
     g = MmArgs{};
     g.M = q.M;
@@ -412,7 +513,13 @@ bool mm_layout(const DenseProblem* p, int np, const void* bias, MmLayout& l) {
     g.c = q.c;
     g.bias = bias;
     g.colsum = q.colsum;
-    mm_plan<T>(g, l.t, blocks);
+    const long tm = ((long)q.M + m.t.bm - 1) / m.t.bm, tn = ((long)q.N + m.t.bn - 1) / m.t.bn;
+    blocks += tm * tn * m.splits[i];
+    if (blocks > (1L << 30)) return false;
+    g.tiles_m = (int)tm;
+    g.tiles_n = (int)tn;
+    g.per = m.per[i];
+    g.splits = m.splits[i];
     g.cs_shift = colsum_shift(g.tiles_m, l.t.bn);
     // with slack: a stage's addresses run past the last row
     const long ab = ((long)l.a[i].rows + 64) * g.lda * ES, bb = ((long)l.b[i].rows + 64) * g.ldb * ES;
@@ -438,10 +545,8 @@ template <typename T, int BM, int BN, int WM, int WN>
 void mm_launch(const MmArgs* g, int np, bool at, bool bt, hipStream_t st) {
   const unsigned n = (unsigned)(g[0].tiles_m * g[0].tiles_n * g[0].splits);
   if (np == 2) {
-    if constexpr (BM * BN <= 4096) {
-      const unsigned n1 = (unsigned)(g[1].tiles_m * g[1].tiles_n * g[1].splits);
-      mm_pair_kernel<T, BM, BN, WM, WN><<<dim3(n + n1), 256, 0, st>>>(g[0], g[1]);
-    }
+    const unsigned n1 = (unsigned)(g[1].tiles_m * g[1].tiles_n * g[1].splits);
+    mm_pair_kernel<T, BM, BN, WM, WN><<<dim3(n + n1), 256, 0, st>>>(g[0], g[1]);
     return;
   }
   // A third stage where the grid leaves room for it, from 12 stages on (bf16 900 x 600
@@ -466,9 +571,15 @@ void mm_launch(const MmArgs* g, int np, bool at, bool bt, hipStream_t st) {
 }
 
 template <typename T>
-int mm_run_t(const DenseProblem* p, int np, const void* bias, char* ws, hipStream_t st) {
+int mm_run_t(const DenseProblem* p, int np, const void* bias, WsGet get, hipStream_t st) {
   MmLayout l;
   if (!mm_layout<T>(p, np, bias, l)) return VH_ERR_UNSUPPORTED;
+  void* wsp = nullptr;
+  if (l.bytes) {
+    const int r = get(st, l.bytes, &wsp);
+    if (r != VH_OK) return r;
+  }
+  char* ws = static_cast<char*>(wsp);
   size_t at = l.copies;
   PadSeg seg[4];
   int ns = 0;
@@ -539,15 +650,15 @@ int mm_run_t(const DenseProblem* p, int np, const void* bias, char* ws, hipStrea
 
 }  // namespace
 
-size_t mm_ws(int dt, const DenseProblem* p, int np, bool* ok) {
+bool mm_info(int dt, const DenseProblem* p, int np, MmInfo* o) {
   MmLayout l;
-  *ok = dt == VH_BF16 ? mm_layout<bf16>(p, np, nullptr, l) : mm_layout<float>(p, np, nullptr, l);
-  return *ok ? l.bytes : 0;
+  if (!(dt == VH_BF16 ? mm_layout<bf16>(p, np, nullptr, l) : mm_layout<float>(p, np, nullptr, l))) return false;
+  *o = MmInfo{l.t.bm, l.t.bn, {l.g[0].splits, np > 1 ? l.g[1].splits : 0}, {l.g[0].per, np > 1 ? l.g[1].per : 0}, l.bytes, l.us};
+  return true;
 }
 
-int mm_run(int dt, const DenseProblem* p, int np, const void* bias, void* ws, hipStream_t st) {
-  return dt == VH_BF16 ? mm_run_t<bf16>(p, np, bias, static_cast<char*>(ws), st)
-                       : mm_run_t<float>(p, np, bias, static_cast<char*>(ws), st);
+int mm_run(int dt, const DenseProblem* p, int np, const void* bias, WsGet get, hipStream_t st) {
+  return dt == VH_BF16 ? mm_run_t<bf16>(p, np, bias, get, st) : mm_run_t<float>(p, np, bias, get, st);
 }
 
 }  // namespace vh
