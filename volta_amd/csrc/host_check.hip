@@ -6,15 +6,110 @@
 // a real call: algorithm choice, stride phases, weight-gradient plans,
 // split-K plans, im2col sizes; it stops before any launch) over a grid of
 // shapes, dtypes and algorithms, together with the plans of products and Linear
-// layers up to the largest sizes, the algorithm selectors and the shape checks of the
+// layers up to the largest sizes, the growth of a stream's workspace over a played
+// device, the algorithm selectors and the shape checks of the
 // entry points.  A sanitizer report, a bad size or a bad plan fails.
-#include "vh_api.hip"
+#include <hip/hip_runtime.h>
 
 #include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <vector>
+
+// The allocator and the stream queries behind the workspaces, played by the host: a
+// device of `room` bytes whose calls are written down in order (m, s, f).
+namespace fake {
+size_t room = SIZE_MAX;
+bool capturing = false;
+hipError_t sync = hipSuccess;
+std::vector<char> calls;
+hipError_t alloc(void** p, size_t bytes) {
+  calls.push_back('m');
+  if (bytes > room) return hipErrorOutOfMemory;
+  *p = malloc(bytes);
+  return hipSuccess;
+}
+hipError_t release(void* p) {
+  calls.push_back('f');
+  free(p);
+  return hipSuccess;
+}
+hipError_t synchronize(hipStream_t) {
+  calls.push_back('s');
+  return sync;
+}
+hipError_t is_capturing(hipStream_t, hipStreamCaptureStatus* s) {
+  *s = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+}  // namespace fake
+#define hipMalloc fake::alloc
+#define hipFree fake::release
+#define hipStreamSynchronize fake::synchronize
+#define hipStreamIsCapturing fake::is_capturing
+#include "vh_api.hip"
 
 namespace {
 using namespace vh;
 long n = 0, fails = 0;
+
+void expect(bool ok, const char* what) {
+  ++n;
+  if (!ok) {
+    printf("workspace: %s\n", what);
+    ++fails;
+  }
+}
+bool called(const char* seq) {
+  const bool same = std::string(fake::calls.begin(), fake::calls.end()) == seq;
+  fake::calls.clear();
+  return same;
+}
+
+// Growth of a stream's workspace: an optional request that cannot be had changes nothing.
+void check_workspace() {
+  const hipStream_t st = reinterpret_cast<hipStream_t>(64), st2 = reinterpret_cast<hipStream_t>(128);
+  void *a, *b;
+  expect(ws_get(st, 1000, &a) == VH_OK && a && called("m"), "first request");
+  fake::room = 1 << 20;
+  set_error(VH_OK, "before");
+  expect(ws_optional(st, 2 << 20, &b) == VH_ERR_OOM && !b && called("m"), "optional request without memory");
+  expect(falls_back(VH_ERR_OOM) && !strcmp(g_err, "before"), "an error was left by a call that falls back");
+  expect(ws_get(st, 1000, &b) == VH_OK && b == a && called(""), "the old buffer is gone");
+  expect(ws_optional(st, 2 << 20, &b) == VH_ERR_OOM && called(""), "a second try right away");
+  expect(ws_optional(st, 3000, &b) == VH_OK && b != a && called("msf"), "a smaller optional request; new buffer before the old goes");
+  fake::room = 2 << 20;
+  for (int i = 0; i < kRefusals; ++i) {
+    fake::room = SIZE_MAX;
+    if (ws_optional(st, 2 << 20, &b) == VH_OK) break;
+  }
+  expect(ws_optional(st, 2 << 20, &b) == VH_OK && b, "tried again once there is memory");
+  fake::calls.clear();
+  // capture: never grows; what is there serves, and is retired when outgrown
+  fake::capturing = true;
+  set_error(VH_OK, "before");
+  expect(ws_optional(st, 8 << 20, &a) == VH_ERR_CAPTURE && !a && !strcmp(g_err, "before") && called(""), "optional growth in a capture");
+  expect(ws_get(st, 1000, &a) == VH_OK && a == b && called(""), "use in a capture");
+  expect(ws_get(st, 8 << 20, &a) == VH_ERR_CAPTURE && called(""), "growth in a capture");
+  fake::capturing = false;
+  const size_t retired = g_ws_retired.size();
+  expect(ws_optional(st, 8 << 20, &a) == VH_OK && called("m") && g_ws_retired.size() == retired + 1, "a captured buffer is retired");
+  // a required request frees first; a failed synchronisation is the call's own error
+  expect(ws_get(st, 16 << 20, &a) == VH_OK && called("sfm"), "required growth");
+  fake::sync = hipErrorLaunchFailure;
+  expect(ws_optional(st, 32 << 20, &a) == VH_ERR_LAUNCH && !falls_back(VH_ERR_LAUNCH), "a failed synchronisation");
+  fake::sync = hipSuccess;
+  fake::calls.clear();
+  // the fixed scratch
+  char scr[64];
+  {
+    FixedWs guard(scr, sizeof(scr));
+    set_error(VH_OK, "before");
+    expect(ws_optional(st2, 65, &a) == VH_ERR_UNSUPPORTED && !strcmp(g_err, "before"), "optional beyond the scratch");
+    expect(ws_optional(st2, 64, &a) == VH_OK && a == scr && called(""), "the scratch");
+  }
+}
 
 // The plan of a product or a Linear layer's pair: the splits cover K, the workspace
 // holds them, and no block is left with a long K of its own beside an idle chip.
@@ -122,6 +217,7 @@ int main() {
       ++fails;
     }
   }
+  check_workspace();
   check_products();
   printf("host_check: %ld plans, %ld failures\n", n, fails);
   return fails ? 1 : 0;

@@ -27,6 +27,12 @@ int set_error(int status, const char* fmt, ...) {
   return status;
 }
 
+#define VH_TRY(expr)          \
+  do {                        \
+    int _s = (expr);          \
+    if (_s != VH_OK) return _s; \
+  } while (0)
+
 // Specialised kernels (halo conv, ...) are used where their envelope allows
 // unless the policy says otherwise (vh_set_kernel_policy; the environment
 // variable VOLTA_HIP_GENERIC=1 sets the initial policy to generic).
@@ -92,7 +98,10 @@ struct Ws {
   void* ptr = nullptr;
   size_t bytes = 0;
   bool captured = false;  // a call captured into a graph used this buffer
+  size_t refused = 0;     // an optional request that the device had no memory for ..
+  int skip = 0;           // .. and how many more of its size are refused without a try
 };
+static constexpr int kRefusals = 64;
 static std::mutex g_ws_mu;
 static std::unordered_map<hipStream_t, Ws> g_ws;
 static std::vector<void*> g_ws_retired;
@@ -108,14 +117,38 @@ static size_t ws_grow_to(size_t have, size_t need) {
   return round_bytes(std::max(need, have * 5 / 4));
 }
 
+// Frees a buffer that the stream's workspace has outgrown, or retires it.
+static int ws_drop(hipStream_t st, void* old, bool captured) {
+  if (!old) return VH_OK;
+  if (captured) {
+    g_ws_retired.push_back(old);  // a graph holds its address: freed by vh_release_cache only
+    return VH_OK;
+  }
+  // only this stream's queued calls can still use it
+  const hipError_t e = hipStreamSynchronize(st);
+  if (e != hipSuccess) {
+    g_ws_retired.push_back(old);
+    return set_error(VH_ERR_LAUNCH, "hipStreamSynchronize before a workspace grows failed: %s", hipGetErrorString(e));
+  }
+  VH_HIP_CHECK(hipFree(old));
+  return VH_OK;
+}
+
 // Returns a device buffer of >= bytes private to `st`.
-static int ws_get(hipStream_t st, size_t bytes, void** out) {
+//
+// optional: the caller has another path to fall back on where the fixed scratch is too
+// small (VH_ERR_UNSUPPORTED), the stream is being captured and its workspace would have
+// to grow (VH_ERR_CAPTURE), or the device is out of memory (VH_ERR_OOM).  Such a
+// request leaves vh_last_error alone, and the old buffer -- which may be all that the
+// fallback needs -- in place until the larger one is there.
+static int ws_request(hipStream_t st, size_t bytes, void** out, bool optional) {
   *out = nullptr;
   if (bytes == 0) return VH_OK;
   if (t_ws_fixed) {
     if (bytes > t_ws_fixed_bytes)
-      return set_error(VH_ERR_UNSUPPORTED, "call needs %zu bytes of scratch; the static scratch holds %zu", bytes,
-                       t_ws_fixed_bytes);
+      return optional ? VH_ERR_UNSUPPORTED
+                      : set_error(VH_ERR_UNSUPPORTED, "call needs %zu bytes of scratch; the static scratch holds %zu",
+                                  bytes, t_ws_fixed_bytes);
     *out = t_ws_fixed;
     return VH_OK;
   }
@@ -127,47 +160,49 @@ static int ws_get(hipStream_t st, size_t bytes, void** out) {
   const size_t nb = ws_grow_to(w.bytes, bytes);
   if (nb) {
     if (capturing)
-      return set_error(VH_ERR_CAPTURE,
-                       "workspace of this stream (%zu bytes) must grow to %zu while the stream is captured: "
-                       "run the call once eagerly on the stream before capturing",
-                       w.bytes, bytes);
-    if (w.ptr) {
+      return optional ? VH_ERR_CAPTURE
+                      : set_error(VH_ERR_CAPTURE,
+                                  "workspace of this stream (%zu bytes) must grow to %zu while the stream is captured: "
+                                  "run the call once eagerly on the stream before capturing",
+                                  w.bytes, bytes);
+    if (optional && w.skip > 0 && bytes >= w.refused) {
+      --w.skip;
+      return VH_ERR_OOM;
+    }
+    if (!optional) {  // no room for both is no reason to fail: the old buffer goes first
       void* old = w.ptr;
-      const bool keep = w.captured;
+      const bool captured = w.captured;
       w.ptr = nullptr;
       w.bytes = 0;
       w.captured = false;
-      if (keep) {
-        g_ws_retired.push_back(old);  // a graph holds its address: freed by vh_release_cache only
-      } else {
-        // only this stream's queued calls can still use it
-        const hipError_t e = hipStreamSynchronize(st);
-        if (e != hipSuccess) {
-          g_ws_retired.push_back(old);
-          return set_error(VH_ERR_LAUNCH, "hipStreamSynchronize before a workspace grows failed: %s",
-                           hipGetErrorString(e));
-        }
-        VH_HIP_CHECK(hipFree(old));
-      }
+      VH_TRY(ws_drop(st, old, captured));
     }
     void* p = nullptr;
     if (hipMalloc(&p, nb) != hipSuccess) {
       (void)hipGetLastError();
-      return set_error(VH_ERR_OOM, "workspace allocation of %zu bytes failed", nb);
+      if (!optional) return set_error(VH_ERR_OOM, "workspace allocation of %zu bytes failed", nb);
+      w.refused = bytes;
+      w.skip = kRefusals;
+      return VH_ERR_OOM;
     }
+    void* old = w.ptr;
+    const bool captured = w.captured;
     w.ptr = p;
     w.bytes = nb;
     w.captured = false;
+    w.skip = 0;
+    VH_TRY(ws_drop(st, old, captured));
   }
   if (capturing) w.captured = true;
   *out = w.ptr;
   return VH_OK;
 }
+static int ws_get(hipStream_t st, size_t bytes, void** out) { return ws_request(st, bytes, out, false); }
+static int ws_optional(hipStream_t st, size_t bytes, void** out) { return ws_request(st, bytes, out, true); }
 
-// A request of a path that has another to fall back on: no workspace where the
-// fixed scratch is too small, the stream is being captured and its workspace
-// would have to grow, or the device is out of memory.
-static bool ws_try(hipStream_t st, size_t bytes, void** out) { return bytes > 0 && ws_get(st, bytes, out) == VH_OK; }
+// Whether a path whose optional request (or own envelope) ended with r leaves the call
+// to its fallback; any other failure is the call's.
+static bool falls_back(int r) { return r == VH_ERR_UNSUPPORTED || r == VH_ERR_OOM || r == VH_ERR_CAPTURE; }
 
 // Carves aligned sub-buffers out of one workspace request.
 struct Carve {
@@ -273,21 +308,17 @@ static ConvGeom geom_of(const ConvDims& d) {
                    (int)d.SH, (int)d.SW, (int)d.PH, (int)d.PW);
 }
 
-#define VH_TRY(expr)          \
-  do {                        \
-    int _s = (expr);          \
-    if (_s != VH_OK) return _s; \
-  } while (0)
-
 #define VH_DISPATCH(dtype, FN, ...) \
   ((dtype) == VH_BF16 ? FN<bf16>(__VA_ARGS__) : FN<float>(__VA_ARGS__))
 
 // The channels-last path, where its workspace can be had: true with its status in *r.
 static bool gather_try(int dt, const GatherCall& c, hipStream_t st, int* r) {
+  const size_t bytes = gather_ws(dt, c);
+  if (!bytes) return false;
   void* ws;
-  if (!ws_try(st, gather_ws(dt, c), &ws)) return false;
-  *r = gather_run(dt, c, ws, st);
-  return true;
+  *r = ws_optional(st, bytes, &ws);
+  if (*r == VH_OK) *r = gather_run(dt, c, ws, st);
+  return !falls_back(*r);
 }
 
 // ------------------------------------------------------------------ conv passes
@@ -894,8 +925,8 @@ static bool product_try(int dt, const DenseProblem* p, int np, const void* bias,
     plain = plain && (np == 2 || !p[i].colsum);
   }
   if (plain && (*r = dense_large(dt, p, np, bias, st)) != VH_ERR_UNSUPPORTED) return true;
-  *r = mm_run(dt, p, np, bias, ws_get, st);
-  return *r != VH_ERR_UNSUPPORTED && *r != VH_ERR_OOM && *r != VH_ERR_CAPTURE;
+  *r = mm_run(dt, p, np, bias, ws_optional, st);
+  return !falls_back(*r);
 }
 
 static int gemm(int dt, int ak, int bk, const void* a, int lda, const void* b, int ldb, void* c, int ldc,
