@@ -42,6 +42,13 @@
  *    captured the library never allocates, frees or synchronises for it: a
  *    call whose workspace would have to grow returns VH_ERR_CAPTURE (run the
  *    call once eagerly on that stream before capturing).
+ *  - Convolutions over channels-last copies (up to 256 MiB of workspace) and products
+ *    over padded copies (up to 1 GiB) can do without: where the workspace would
+ *    have to grow inside a capture, or the device is out of memory, and a form
+ *    without the copies fits in what is there, the call succeeds on that form: 2 to
+ *    4 times slower, its sums in another order (results may differ in the last
+ *    bits), and recorded so in a graph.  A call that has run once eagerly on the
+ *    stream is captured as it ran.
  */
 #ifndef VOLTA_HIP_H
 #define VOLTA_HIP_H
@@ -327,11 +334,13 @@ int vh_conv2d_backward_relu(int dtype, int algo, const void* out_grad, const voi
 /* Allocation-free variant of vh_conv2d_backward (no counterpart in the reference):
  * for callers that cannot allocate device memory -- code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc.  Same arguments, algorithms,
- * kernels and results as vh_conv2d_backward; its workspace (re-laid-out weights,
- * split-K partial sums, im2col matrices) is a static device array of
- * VH_NOALLOC_SCRATCH_BYTES per GPU, held from the library's first use on that GPU
- * until the process ends.  The call never allocates or frees: a call that would
- * need more workspace returns VH_ERR_UNSUPPORTED before anything is queued.  Every
+ * kernels and results as vh_conv2d_backward; its workspace is a static device array
+ * per GPU, held from the library's first use on that GPU until the process ends:
+ * VH_NOALLOC_SCRATCH_BYTES of it for re-laid-out weights, split-K partial sums and
+ * im2col matrices, 256 MiB in all with the channels-last copies (which neither
+ * entry lets grow beyond that).  The call never allocates or frees: a call that
+ * would need more than VH_NOALLOC_SCRATCH_BYTES (channels-last copies and their
+ * partial sums aside) returns VH_ERR_UNSUPPORTED before anything is queued.  Every
  * call on one GPU shares that GPU's array, so calls that overlap on one GPU (two
  * streams, two threads, without ordering between them) race; order them. */
 #define VH_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)

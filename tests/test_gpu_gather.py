@@ -154,3 +154,37 @@ def test_gather_bf16_stages_in_flight(C, B, O):
     conv.weight = wt
     conv.bias.zero_()
     check(conv.forward(xt), oracle.direct_conv, (x, w), "bf16", "y", dict(stride=(2, 2), pad=(0, 0)), k=C)
+
+
+# copies of all images above the workspace's bound: chunks of images, the last smaller
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_gather_gradients_in_chunks(dt):
+    B, C, O, H, W, K, S = (41, 96, 24, 131, 130, 1, 1) if dt == "f32" else (67, 72, 24, 171, 165, 2, 2)
+    g = rng(B)
+    x, xt = prep(g.standard_normal((B, C, H, W)), dt)
+    w, wt = prep(g.standard_normal((O, C, K, K)) * np.sqrt(2.0 / (C * K * K)), dt)
+    conv = vnn.Conv2d(C, O, K, S, 0, device=DEV, dtype=DTYPES[dt])
+    conv.weight = wt
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    kw = dict(stride=(S, S), pad=(0, 0))
+    HO, WO = (H - K) // S + 1, (W - K) // S + 1
+    dy, dyt = prep(g.standard_normal((B, O, HO, WO)), dt)
+    dx, dw, db = conv.backward(dyt, xt)
+    check(dx, oracle.direct_conv_backward_input, (dy, w, x.shape), dt, "dx", kw, k=k_conv_dgrad(O, K, K))
+    check(dw, oracle.direct_conv_backward_weight, (dy, x, w.shape), dt, "dw", kw, k=k_conv_wgrad(B, HO, WO))
+    check(db, oracle.conv_bias_grad, (dy,), dt, "db", k=B * HO * WO)
+    masked = host(conv.backward(dyt, xt, weight_grad=False, relu_input=True)[0])
+    assert np.array_equal(masked, np.where(x > 0, host(dx), 0))
+
+
+def test_gather_forward_in_chunks():
+    B, C, O, H, W = 37, 32, 8, 270, 247
+    g = rng(B)
+    x, xt = prep(g.standard_normal((B, C, H, W)), "f32")
+    w, wt = prep(g.standard_normal((O, C, 1, 1)), "f32")
+    b, bt = prep(g.uniform(-1, 1, (O,)), "f32")
+    conv = vnn.Conv2d(C, O, 1, 1, 0, device=DEV)
+    conv.weight, conv.bias = wt, bt
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    bb = b[None, :, None, None]
+    check(conv.forward(xt), oracle.direct_conv, (x, w), "f32", "y", extra_ref=bb, extra_scale=np.abs(bb), k=C + 1)

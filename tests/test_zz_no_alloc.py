@@ -55,6 +55,11 @@ CASES = [
     # the weight gradient only the few-channel kernel's partials (what the sizing must report)
     ("bf16", _lib.ALGO_IGEMM, (256, 3, 64, 64, 64, 5, 1, 2), (4, 3, 64, 16, 16, 5, 1, 2)),
     ("f32", _lib.ALGO_IGEMM, (512, 4, 32, 28, 28, 3, 1, 1), (2, 4, 32, 9, 9, 3, 1, 1)),
+    # channels-last copies of 70 MiB; of 300 MiB, in chunks; of one image above the scratch
+    ("f32", _lib.ALGO_IGEMM, (64, 64, 128, 32, 32, 3, 1, 1), (65, 64, 128, 32, 32, 3, 1, 1)),
+    ("f32", _lib.ALGO_IGEMM, (96, 128, 256, 45, 44, 1, 1, 0), (7, 48, 40, 130, 120, 1, 1, 0)),
+    ("bf16", _lib.ALGO_IGEMM, (96, 64, 128, 113, 113, 3, 2, 1), (40, 96, 144, 60, 57, 3, 1, 1)),
+    ("f32", _lib.ALGO_IGEMM, (1, 24, 16, 1500, 1400, 3, 1, 1), (2, 24, 16, 30, 30, 3, 1, 1)),
 ]
 
 

@@ -222,7 +222,9 @@ static inline char* at(void* base, size_t off) { return static_cast<char*>(base)
 // In host code `scratch` names a host-side stand-in, not device memory: its
 // device address comes from hipGetSymbolAddress, once per device with that
 // device current, and only that address is ever passed to kernels.
-static constexpr size_t kScratchBytes = VH_NOALLOC_SCRATCH_BYTES;
+// (what a call may ask for, VH_NOALLOC_SCRATCH_BYTES, and room for channels-last copies)
+static constexpr size_t kScratchBytes = kGatherMostWs;
+static_assert(kScratchBytes >= VH_NOALLOC_SCRATCH_BYTES, "static scratch");
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 static constexpr int kMaxDevices = 64;
 static std::once_flag g_scratch_once[kMaxDevices];
@@ -1441,11 +1443,11 @@ int vh_conv2d_backward_noalloc(int dtype, int algo, const void* out_grad, const 
   VH_TRY(conv2d_backward_impl(dtype, algo, out_grad, input, weight, grad_input, grad_weight, grad_bias, batch,
                               in_channels, out_channels, height, width, kernel_h, kernel_w, stride_h, stride_w,
                               pad_h, pad_w, stream, false, &need));
-  if (need > kScratchBytes)
+  if (need > VH_NOALLOC_SCRATCH_BYTES)
     return set_error(VH_ERR_UNSUPPORTED,
                      "vh_conv2d_backward_noalloc: this call needs %zu bytes of scratch, above the static "
                      "maximum of %zu bytes; use vh_conv2d_backward",
-                     need, kScratchBytes);
+                     need, VH_NOALLOC_SCRATCH_BYTES);
   FixedWs guard(sp, kScratchBytes);
   return conv2d_backward_impl(dtype, algo, out_grad, input, weight, grad_input, grad_weight, grad_bias, batch,
                               in_channels, out_channels, height, width, kernel_h, kernel_w, stride_h, stride_w,

@@ -441,6 +441,7 @@ struct WgradArgs {
   float* dbpart;   // [split][O] or nullptr
   int O, NC, K;    // rows, columns (RS * Cp), positions
   int tiles_m, tiles_n, per;  // stages per split
+  int add;         // onto the partials of the images before these
   int dy_bytes, x_bytes;
   int dimg, drow, dcol;       // bytes between images, rows and columns of dy
   int ximg, xrow, xcol;       // the same of x, per output row / column (strides applied)
@@ -570,13 +571,14 @@ __global__ __launch_bounds__(256) void gather_wgrad_kernel(WgradArgs g) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
           const int col = n0 + wn + mn_spread<T, FN>(j, row_l);
-          if (col < g.NC) d[col] = acc[i][j][v];
+          if (col < g.NC) d[col] = g.add ? d[col] + acc[i][j][v] : acc[i][j][v];
         }
       }
     }
   if (cs.on)
     cs.finish(reinterpret_cast<float*>(S0), [&](int col, float t) {
-      if (m0 + col < g.O) g.dbpart[(size_t)z * g.O + m0 + col] = t;
+      float* d = g.dbpart + (size_t)z * g.O + m0 + col;
+      if (m0 + col < g.O) *d = g.add ? *d + t : t;
     });
 }
 
@@ -847,10 +849,10 @@ WgradPlan wgrad_plan(const ConvGeom& g, const Geo& o) {
 // Workspace of a call: the copies of x and dy, the weights, the partials.
 struct Layout {
   size_t x = 0, dy = 0, w = 0, part = 0, bytes = 0;
-};
+};  // for the images of one chunk
 
 template <typename T>
-bool make_layout(const GatherCall& c, const Geo& o, Layout& l) {
+bool make_layout(const GatherCall& c, const Geo& o, const WgradPlan& wg, Layout& l) {
   const ConvGeom& g = c.g;
   constexpr int UE = GT<T>::UE;
   auto take = [&](size_t b) {
@@ -870,7 +872,7 @@ bool make_layout(const GatherCall& c, const Geo& o, Layout& l) {
     for (int f = 0; f < n; ++f) wu += (size_t)g.C * ((ph[f].Rc * ph[f].Sc * (o.Op / UE) + 7) / 8) * 8;
     l.w = take(wu * 16);
   }
-  if (c.dw) l.part = take((size_t)wgrad_plan<T>(g, o).splits * g.O * (g.R * g.S * o.Cp + 1) * sizeof(float));
+  if (c.dw) l.part = take((size_t)wg.splits * g.O * (g.R * g.S * o.Cp + 1) * sizeof(float));
   return true;
 }
 
@@ -988,11 +990,13 @@ void conv_args(ConvPlan& plan, WeightSeg& s, const GatherCall& c, const Geo& o, 
   s.total = s.units + tails;
 }
 
+// The partials of one chunk's images (the first: add false), and after the last chunk
+// their sums.
 template <typename T>
-int run_wgrad(const GatherCall& c, const Geo& o, char* ws, const Layout& l, hipStream_t st) {
+int run_wgrad(const GatherCall& c, const Geo& o, const WgradPlan& p, char* ws, const Layout& l, bool add, bool last,
+              hipStream_t st) {
   constexpr int ES = GT<T>::ES, UE = GT<T>::UE;
   const ConvGeom& g = c.g;
-  const WgradPlan p = wgrad_plan<T>(g, o);
   // the copy of dy has the input gradient's border when both are computed
   const int Pd = c.dx ? o.Pp : g.P, Qd = c.dx ? o.Qp : g.Q, dT = c.dx ? o.dT : 0, dL = c.dx ? o.dL : 0;
   WgradArgs a{};
@@ -1012,6 +1016,7 @@ int run_wgrad(const GatherCall& c, const Geo& o, char* ws, const Layout& l, hipS
   a.tiles_m = (g.O + 63) / 64;
   a.tiles_n = (a.NC + 63) / 64;
   a.per = p.per;
+  a.add = add;
   a.tcol = o.Cp * ES;
   a.trow = o.Wp * a.tcol;
   a.xcol = g.sw * a.tcol;
@@ -1025,6 +1030,7 @@ int run_wgrad(const GatherCall& c, const Geo& o, char* ws, const Layout& l, hipS
   const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * p.splits));
   gather_wgrad_kernel<T, 64, 64, 32, 32><<<grid, 256, 0, st>>>(a);
   VH_LAUNCH_CHECK();
+  if (!last) return VH_OK;
   const int RS = g.R * g.S;
   if (p.splits > 8) {
     const int lg = reduce_vec4_lg_groups(p.splits), nb = reduce_vec4_grid((long)g.O * a.NC, lg);
@@ -1039,34 +1045,79 @@ int run_wgrad(const GatherCall& c, const Geo& o, char* ws, const Layout& l, hipS
   return VH_OK;
 }
 
-template <typename T>
-size_t call_ws(const GatherCall& c) {
+// A call's workspace is bounded, so that no stream holds copies of whole large tensors,
+// by what the allocation-free entry point has (it then runs the same kernels).  More
+// images are taken in equal chunks, each with its own copies; the partials of the
+// weight gradient add up over them.  Eight chunks of 64 MiB had cost a 1x1 128 -> 256 @64
+// N=64 fp32 backward 730 us where two take 500.
+struct CallPlan {
   Geo o;
   Layout l;
+  WgradPlan wg;
+  int images;  // per chunk
+};
+
+template <typename T>
+bool plan_call(const GatherCall& c, CallPlan& p) {
   // more than 64 taps: beyond the reduction's LDS tile
-  if (c.g.N <= 0 || c.g.R * c.g.S > 64 || !make_geo<T>(c.g, o) || !make_layout<T>(c, o, l)) return 0;
-  return l.bytes;
+  if (c.g.N <= 0 || c.g.R * c.g.S > 64 || !make_geo<T>(c.g, p.o)) return false;
+  GatherCall part = c;
+  auto fits = [&](int images) {
+    part.g.N = p.images = images;
+    p.l = Layout{};
+    p.wg = wgrad_plan<T>(part.g, p.o);
+    return make_layout<T>(part, p.o, p.wg, p.l) && p.l.bytes <= kGatherMostWs;
+  };
+  if (fits(c.g.N)) return true;
+  if (!fits(1)) return false;
+  int lo = 1, hi = c.g.N;  // lo fits, hi does not
+  while (hi - lo > 1) {
+    const int mid = lo + (hi - lo) / 2;
+    (fits(mid) ? lo : hi) = mid;
+  }
+  const int chunks = (c.g.N + lo - 1) / lo;
+  return fits((c.g.N + chunks - 1) / chunks);
+}
+
+template <typename T>
+size_t call_ws(const GatherCall& c) {
+  CallPlan p;
+  return plan_call<T>(c, p) ? p.l.bytes : 0;
 }
 
 template <typename T>
 int run_call(const GatherCall& c, char* ws, hipStream_t st) {
-  Geo o;
-  Layout l;
-  if (!make_geo<T>(c.g, o) || !make_layout<T>(c, o, l)) return VH_ERR_UNSUPPORTED;
-  const ConvGeom& g = c.g;
-  PrepArgs pa{};
-  ConvPlan a{};
-  int np = 0;
-  if (c.y || c.dw) pa.p[np++] = pack_seg<T>(c.x, ws + l.x, g.N, g.C, g.H, g.W, o.Cp, o.Hp, o.Wp, g.ph, g.pw);
-  if (c.dx)
-    pa.p[np++] = pack_seg<T>(c.dy, ws + l.dy, g.N, g.O, g.P, g.Q, o.Op, o.Pp, o.Qp, o.dT, o.dL);
-  else if (c.dw)
-    pa.p[np++] = pack_seg<T>(c.dy, ws + l.dy, g.N, g.O, g.P, g.Q, o.Op, g.P, g.Q, 0, 0);
-  if (c.y || c.dx) conv_args<T>(a, pa.w, c, o, ws, l);
-  int r = launch_prep<T>(pa, np, c.y || c.dx, st);
-  if (r == VH_OK && (c.y || c.dx)) r = launch_conv<T>(a, st);
-  if (r == VH_OK && c.dw) r = run_wgrad<T>(c, o, ws, l, st);
-  return r;
+  CallPlan cp;
+  if (!plan_call<T>(c, cp)) return VH_ERR_UNSUPPORTED;
+  const Geo& o = cp.o;
+  const Layout& l = cp.l;
+  const size_t in = (size_t)c.g.C * c.g.H * c.g.W * GT<T>::ES, out = (size_t)c.g.O * c.g.P * c.g.Q * GT<T>::ES;
+  auto image = [](const void* p, size_t off) { return p ? static_cast<const char*>(p) + off : nullptr; };
+  for (int n0 = 0; n0 < c.g.N; n0 += cp.images) {
+    GatherCall d = c;
+    d.g.N = std::min(cp.images, c.g.N - n0);
+    d.x = image(c.x, n0 * in);
+    d.mask = image(c.mask, n0 * in);
+    d.dx = const_cast<char*>(image(c.dx, n0 * in));
+    d.dy = image(c.dy, n0 * out);
+    d.y = const_cast<char*>(image(c.y, n0 * out));
+    const ConvGeom& g = d.g;
+    PrepArgs pa{};
+    ConvPlan a{};
+    int np = 0;
+    if (d.y || d.dw) pa.p[np++] = pack_seg<T>(d.x, ws + l.x, g.N, g.C, g.H, g.W, o.Cp, o.Hp, o.Wp, g.ph, g.pw);
+    if (d.dx)
+      pa.p[np++] = pack_seg<T>(d.dy, ws + l.dy, g.N, g.O, g.P, g.Q, o.Op, o.Pp, o.Qp, o.dT, o.dL);
+    else if (d.dw)
+      pa.p[np++] = pack_seg<T>(d.dy, ws + l.dy, g.N, g.O, g.P, g.Q, o.Op, g.P, g.Q, 0, 0);
+    const bool conv = d.y || d.dx;
+    if (conv) conv_args<T>(a, pa.w, d, o, ws, l);
+    int r = launch_prep<T>(pa, np, conv && n0 == 0, st);
+    if (r == VH_OK && conv) r = launch_conv<T>(a, st);
+    if (r == VH_OK && d.dw) r = run_wgrad<T>(d, o, cp.wg, ws, l, n0 > 0, n0 + cp.images >= c.g.N, st);
+    if (r != VH_OK) return r;
+  }
+  return VH_OK;
 }
 
 }  // namespace

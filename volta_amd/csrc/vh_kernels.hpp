@@ -177,8 +177,10 @@ struct GatherCall {
   void *y, *dx, *dw, *db;
   int act;
 };
-// Workspace bytes; 0: unsupported (a tensor beyond 32-bit byte offsets, more than
-// 64 taps, more than 16 stride phases).
+// Workspace bytes (at most kGatherMostWs; more images than fit are taken in chunks); 0:
+// unsupported (a tensor beyond 32-bit byte offsets, more than 64 taps, more than 16
+// stride phases, one image beyond the bound).
+constexpr size_t kGatherMostWs = (size_t)256 << 20;
 size_t gather_ws(int dt, const GatherCall& c);
 int gather_run(int dt, const GatherCall& c, void* ws, hipStream_t st);
 

@@ -353,6 +353,7 @@ const TileCost* mm_costs(bool at) {
   return GT<T>::ES == 4 ? f32 : at ? b16t : b16;
 }
 
+constexpr size_t kMostWs = (size_t)1 << 30;  // workspace of a call
 constexpr float kSplitUs = 4.f;  // of the reduction's launch
 
 // Tile and K splits of a product, or of a Linear layer's pair in one launch.
@@ -538,7 +539,7 @@ bool mm_layout(const DenseProblem* p, int np, const void* bias, MmLayout& l) {
   l.shared = np == 2 && l.b[1].p == l.a[0].p && l.b[1].rows == l.a[0].rows && l.b[1].cols == l.a[0].cols;
   l.copies = l.bytes;
   for (int i = 0; i < np; ++i) l.bytes += l.a[i].bytes + (i == 1 && l.shared ? 0 : l.b[i].bytes);
-  return true;
+  return l.bytes <= kMostWs;
 }
 
 template <typename T, int BM, int BN, int WM, int WN>
