@@ -129,8 +129,8 @@ def test_gather_falls_back_without_workspace():
 
 @pytest.mark.parametrize("B", [3, 33, 60, 64, 65])
 def test_narrow_fp32_layer_on_either_kernel(B):
-    """32 -> 64 channels at 28 x 28: the channels-last path and the halo kernel
-    (40 <= B <= 64, a nearly full round of its blocks) by batch size."""
+    """32 -> 64 channels at 28 x 28: all passes on the channels-last path (3), on the
+    halo kernels (60, 64), the weight and the input gradient on them (33), none (65)."""
     g = rng(B)
     conv = vnn.Conv2d(32, 64, 3, 1, 1, device=DEV)
     conv.set_algo(vnn.ConvAlgo.IGEMM)
@@ -188,3 +188,19 @@ def test_gather_forward_in_chunks():
     conv.set_algo(vnn.ConvAlgo.IGEMM)
     bb = b[None, :, None, None]
     check(conv.forward(xt), oracle.direct_conv, (x, w), "f32", "y", extra_ref=bb, extra_scale=np.abs(bb), k=C + 1)
+
+
+def test_narrow_fp32_layer_with_passes_on_both_paths():
+    """64 -> 32 channels at 20 x 20, 128 images: the weight gradient on the halo kernel,
+    the input gradient and the forward pass over channels-last copies."""
+    g = rng(20)
+    conv = vnn.Conv2d(64, 32, 3, 1, 1, device=DEV)
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    x, xt = prep(g.standard_normal((128, 64, 20, 20)), "f32")
+    dy, dyt = prep(g.standard_normal((128, 32, 20, 20)), "f32")
+    w, kw = host(conv.weight), dict(stride=(1, 1), pad=(1, 1))
+    check(conv.forward(xt), oracle.direct_conv, (x, w), "f32", "y", kw, k=576)
+    dx, dw, db = conv.backward(dyt, xt)
+    check(dx, oracle.direct_conv_backward_input, (dy, w, x.shape), "f32", "dx", kw, k=288)
+    check(dw, oracle.direct_conv_backward_weight, (dy, x, w.shape), "f32", "dw", kw, k=128 * 400)
+    check(db, oracle.conv_bias_grad, (dy,), "f32", "db", k=128 * 400)

@@ -344,13 +344,39 @@ static bool is_3x3_s1_p1(const ConvDims& d) {
   return d.KH == 3 && d.KW == 3 && d.SH == 1 && d.SW == 1 && d.PH == 1 && d.PW == 1;
 }
 
-// The fp32 halo kernels (one block per image and 7 rows, 21 us a round of 256
-// blocks however few of them there are) against the channels-last path, whose time
-// grows with the positions.  Measured at 28 x 28, forward, us: N = 16 21.6 / 15.1, 32
-// 22.2 / 20.4, 64 23.4 / 31, 71 42.0 / 34, 128 44.2 / 52, 200 83.2 / 68.
-static bool halo_f32_pays(const ConvDims& d) {
-  const long rounds = (d.B * ((d.H + 6) / 7) + 255) / 256;
-  return 21.3 * (double)rounds <= 11.0 + 0.285 * (double)(d.B * d.H * d.W) / 784.0;
+// The fp32 halo kernels (one block per image and 7 rows, about 20 us a round of 256
+// blocks however few or narrow they are) against the channels-last path, whose time
+// grows with the positions (u: in images of 28 x 28).  Fitted to each pass at 8 extents of 4 .. 28
+// columns, 1 .. 512 images; us at 28 x 28, halo / channels-last:
+//   images               16          32          64          71          128         256
+//   32 -> 64 (and the input gradient of 64 -> 32)
+//                    21.4 15.8   22.3 21.7   23.4 33.0   41.8 33.8   43.3 54.1   84.0 87.1
+//   64 -> 32 (... 32 -> 64)
+//                    21.7 16.7   22.3 24.4   22.9 38.0   42.1 38.4   44.6 57.8   87.3 96.8
+//   weight gradient 32 -> 64
+//                    23.6 22.9   26.2 28.0   28.8 40.7   45.8 43.4   52.3 64.9   99.5 113
+//   weight gradient 64 -> 32
+//                    24.3 26.8   27.1 36.4   29.2 52.1   47.4 56.7   53.2 90.6   101 168
+// Both gradients over the copies share that of the output gradient (saved, below).
+enum HaloPass { HALO_TO_64, HALO_TO_32, HALO_WGRAD };
+struct HaloUs {
+  double halo, copies, saved;
+};
+static HaloUs halo_f32_us(const ConvDims& d, HaloPass pass) {
+  const double rounds = (double)((d.B * ((d.H + 6) / 7) + 255) / 256), u = (double)(d.B * d.H * d.W) / 784.0;
+  const double saved = 3.5 + (d.O == 64 ? 0.07 : 0.023) * u;
+  if (pass == HALO_TO_64) return {1.0 + 20.5 * rounds, 11.0 + 0.31 * u, saved};
+  if (pass == HALO_TO_32) return {21.1 * rounds, 13.5 + 0.31 * u, saved};
+  return {3.0 + 19.0 * rounds + 0.085 * u, 16.0 + (d.C == 32 ? 0.39 : 0.615) * u, saved};
+}
+// pass is TO_64 or TO_32: with_wgrad, the weight gradient of the same call is still to
+// be placed.  HALO_WGRAD: with_copies, the other gradient went over the copies.
+static bool halo_f32_pays(const ConvDims& d, HaloPass pass, bool with_wgrad, bool with_copies) {
+  const HaloUs t = halo_f32_us(d, pass);
+  if (pass == HALO_WGRAD) return t.halo <= t.copies - (with_copies ? t.saved : 0.0);
+  if (!with_wgrad) return t.halo <= t.copies;
+  const HaloUs w = halo_f32_us(d, HALO_WGRAD);
+  return t.halo + std::min(w.halo, w.copies) <= t.copies + std::min(w.halo, w.copies - w.saved);
 }
 
 // act: 1 = ReLU on the output (fused into the epilogue where the kernel has it).
@@ -375,7 +401,7 @@ static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, voi
   auto run_halo_f32 = [&] {
     return halo_conv3x3_f32(x, w, 0, bias, nullptr, y, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, act, st);
   };
-  if (halo_f32 && halo_f32_pays(d)) return run_halo_f32();
+  if (halo_f32 && halo_f32_pays(d, d.O == 64 ? HALO_TO_64 : HALO_TO_32, defer, false)) return run_halo_f32();
   // weight staging: the generic layout, or the halo kernel's channel-grouped one (padded to 16 channels)
   const size_t wbytes = std::max((size_t)d.O * d.C * RS * elem_size(dt),
                                  halo_conv_bf16_ws((int)d.C, (int)d.O, (int)d.KH, (int)d.KW));
@@ -596,7 +622,7 @@ static int igemm_dgrad(int dt, const void* dy, const void* w, void* dx, const Co
   auto run_halo_f32 = [&] {  // dX = conv(dY, W rotated, O and C swapped), the ReLU mask in the epilogue
     return halo_conv3x3_f32(dy, w, 1, nullptr, mask, dx, (int)d.B, (int)d.O, (int)d.H, (int)d.W, (int)d.C, 0, st);
   };
-  if (halo_f32 && halo_f32_pays(d)) return run_halo_f32();
+  if (halo_f32 && halo_f32_pays(d, d.C == 64 ? HALO_TO_64 : HALO_TO_32, defer, false)) return run_halo_f32();
   void* ws = nullptr;
   if (!halo_f32) VH_TRY(ws_get(st, cv.off, &ws));  // (with the halo kernel to fall back on: no workspace)
   void* wd = at(ws, o_w);
@@ -697,7 +723,7 @@ static int igemm_wgrad(int dt, const void* dy, const void* x, void* dw, void* db
     if (r == VH_OK && db_done) *db_done = db != nullptr;
     return r;
   };
-  if (halo_nb && halo_f32_pays(d)) return run_halo_f32();
+  if (halo_nb && halo_f32_pays(d, HALO_WGRAD, false, defer && (defer->dx || defer->y))) return run_halo_f32();
   ConvGeom g = geom_of(d);
   if (g_fast_paths && !need) {
     GatherCall gc{};
