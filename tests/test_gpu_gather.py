@@ -204,3 +204,11 @@ def test_narrow_fp32_layer_with_passes_on_both_paths():
     check(dx, oracle.direct_conv_backward_input, (dy, w, x.shape), "f32", "dx", kw, k=288)
     check(dw, oracle.direct_conv_backward_weight, (dy, x, w.shape), "f32", "dw", kw, k=128 * 400)
     check(db, oracle.conv_bias_grad, (dy,), "f32", "db", k=128 * 400)
+
+
+# fp32: forward / input gradient with K too long for their positions (the implicit GEMM
+# with K split), next to a weight gradient over the copies
+@pytest.mark.parametrize("case", [(1, 130, 33, 5, 7, 5, 1, 2), (2, 9, 310, 4, 6, 3, 1, 1), (1, 300, 20, 7, 9, 3, 1, 1)], ids=_ids)
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_few_positions(case, dt):
+    test_gather_conv_all_passes(case, dt)

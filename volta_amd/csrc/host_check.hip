@@ -191,6 +191,22 @@ void check_halo_rule() {
     ++fails;
   }
 }
+// fp32 layers of few positions: M, positions, channels, taps; us generic, channels-last.
+void check_few_positions() {
+  const struct {
+    long M, pos, C, RS;
+    float generic, copies;
+  } rows[] = {{60, 32, 778, 25, 26.3f, 136.f}, {33, 162, 459, 9, 18.7f, 35.4f},   {512, 49, 512, 9, 33.7f, 47.f},   {72, 225, 468, 16, 24.5f, 59.5f},
+              {577, 98, 453, 16, 43.5f, 65.2f}, {108, 1053, 940, 9, 47.6f, 68.7f}, {60, 1734, 625, 25, 103.f, 112.f}, {333, 343, 721, 9, 63.1f, 56.8f}, {228, 768, 618, 25, 157.f, 112.f},
+              {512, 392, 512, 9, 53.1f, 48.2f}, {164, 256, 192, 9, 22.8f, 21.f},   {199, 125, 240, 9, 28.7f, 25.3f},  {68, 936, 170, 9, 21.8f, 19.8f}};
+  for (const auto& r : rows) {
+    ++n;
+    if (copies_pay(VH_F32, r.M, r.pos, r.C, r.RS) != (r.copies < r.generic)) {
+      printf("fp32 %ld x %ld, %ld channels, %ld taps: the slower path\n", r.M, r.pos, r.C, r.RS);
+      ++fails;
+    }
+  }
+}
 }  // namespace
 
 int main() {
@@ -252,6 +268,7 @@ int main() {
   check_workspace();
   check_products();
   check_halo_rule();
+  check_few_positions();
   printf("host_check: %ld plans, %ld failures\n", n, fails);
   return fails ? 1 : 0;
 }

@@ -379,6 +379,17 @@ static bool halo_f32_pays(const ConvDims& d, HaloPass pass, bool with_wgrad, boo
   return t.halo + std::min(w.halo, w.copies) <= t.copies + std::min(w.halo, w.copies - w.saved);
 }
 
+// fp32 passes with a long K over few positions: the channels-last kernel, whose waves
+// alone split K, leaves CUs idle where the generic one splits it over blocks too.
+// Fitted to 173 layers of 9 .. 6400 positions (M rows, RS taps of C channels), us generic /
+// channels-last: 33 x 162, K 4131 18.7 / 35.4; 512 x 49, K 4608 33.7 / 47; 60 x 1734, K 15700
+// 103 / 112; 333 x 343, K 6489 63 / 57; 228 x 768, K 15450 157 / 112.  bf16: at most 12 % apart.
+static bool copies_pay(int dt, long M, long positions, long C, long RS) {
+  const long stages = (RS * ((C + 3) / 4 * 4) + 31) / 32, blocks = ((M + 31) / 32) * ((positions + 31) / 32);
+  return dt == VH_BF16 || blocks > 160 ||
+         (double)stages < 64 + 0.75 * (double)blocks + 2.4 * (double)std::max(0L, blocks - 100);
+}
+
 // act: 1 = ReLU on the output (fused into the epilogue where the kernel has it).
 // defer: a pass that takes the channels-last path is only put down in it (the
 // caller runs it, together with the other passes it put down; the same below).
@@ -437,7 +448,7 @@ static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, voi
                            (int)d.KW, (int)d.PH, (int)d.PW, st, act);
     if (r != VH_ERR_UNSUPPORTED) return r;
   }
-  if (g_fast_paths) {
+  if (g_fast_paths && copies_pay(dt, d.O, d.B * d.HO * d.WO, d.C, RS)) {
     GatherCall gc{};
     GatherCall& c = defer ? *defer : gc;
     c.g = g;
@@ -448,10 +459,10 @@ static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, voi
     c.act = act;
     int r = VH_OK;
     if (defer || gather_try(dt, gc, st, &r)) return r;
-    if (halo_f32) return run_halo_f32();
-    VH_TRY(ws_get(st, cv.off, &ws));
-    wt = at(ws, o_w);
   }
+  if (halo_f32) return run_halo_f32();
+  VH_TRY(ws_get(st, cv.off, &ws));
+  wt = at(ws, o_w);
   VH_TRY(VH_DISPATCH(dt, run_relayout, w, wt, (int)d.O, (int)d.C, (int)RS, 0, st));
   const int vec = dt == VH_BF16 ? 8 : 4;
   p.args.a = Operand{wt, (int)(RS * d.C), (int)d.O, ((RS * d.C) % vec) == 0};
@@ -637,7 +648,7 @@ static int igemm_dgrad(int dt, const void* dy, const void* w, void* dx, const Co
     int r = pw_conv_bf16_dgrad(dy, w, dx, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, (int)d.SH, st);
     if (r != VH_ERR_UNSUPPORTED) return r == VH_OK && mask ? mask_after(dt, mask, dx, d.B * d.C * d.H * d.W, st) : r;
   }
-  if (g_fast_paths) {
+  if (g_fast_paths && (d.SH > 1 || d.SW > 1 || copies_pay(dt, d.C, d.B * d.H * d.W, d.O, RS))) {
     GatherCall gc{};
     GatherCall& c = defer ? *defer : gc;
     c.g = g;
@@ -1523,7 +1534,7 @@ int vh_conv_transpose2d_forward(int dtype, const void* input, const void* weight
   const ConvGeom gs = geom_of(d);
   if (g_fast_paths && dgrad_smallc_ok(gs))  // at most 4 output channels
     return VH_DISPATCH(dtype, run_dgrad_smallc, input, weight, bias, nullptr, output, gs, st);
-  if (g_fast_paths) {
+  if (g_fast_paths && (d.SH > 1 || d.SW > 1 || copies_pay(dtype, d.C, d.B * d.H * d.W, d.O, d.KH * d.KW))) {
     GatherCall gc{};
     gc.g = gs;
     gc.dy = input;
