@@ -6,7 +6,8 @@
 // a real call: algorithm choice, stride phases, weight-gradient plans,
 // split-K plans, im2col sizes; it stops before any launch) over a grid of
 // shapes, dtypes and algorithms, together with the plans of products and Linear
-// layers up to the largest sizes, the growth of a stream's workspace over a played
+// layers up to the largest sizes, of convolutions over channels-last copies (and that
+// their addresses stay within the copies), the growth of a stream's workspace over a played
 // device, the algorithm selectors and the shape checks of the
 // entry points.  A sanitizer report, a bad size or a bad plan fails.
 #include <hip/hip_runtime.h>
@@ -159,6 +160,70 @@ void check_products() {
           (void)linear_pair(dt, pair);
         }
 }
+// A convolution's plans over channels-last copies: forward, both gradients apart and together.
+void check_gather(int dt, const ConvDims& d) {
+  char* q = reinterpret_cast<char*>(4096);
+  GatherCall y{}, dx{}, dw{}, both{};
+  y.g = dx.g = dw.g = both.g = geom_of(d);
+  y.x = y.w = dx.dy = dx.w = dw.x = dw.dy = both.x = both.dy = both.w = q;
+  y.y = dx.dx = dw.dw = dw.db = both.dx = both.dw = q;
+  for (const GatherCall* c : {&y, &dx, &dw, &both}) {
+    GatherInfo o;
+    ++n;
+    if (!gather_info(dt, *c, &o)) continue;
+    if (!o.ok || o.bytes != gather_ws(dt, *c) || o.bytes > kGatherMostWs || o.images < 1 || o.images > d.B) {
+      printf("channels-last plan: dt%d B%ld C%ld O%ld %ldx%ld K%ldx%ld S%ldx%ld P%ldx%ld: %d images, %zu bytes, ok %d\n", dt, d.B,
+             d.C, d.O, d.H, d.W, d.KH, d.KW, d.SH, d.SW, d.PH, d.PW, o.images, o.bytes, (int)o.ok);
+      ++fails;
+    }
+  }
+}
+
+void check_gathers() {
+  const long Bs[] = {1, 3, 64, 1000}, Cs[] = {1, 7, 64, 513}, Hs[] = {1, 2, 9, 57, 300}, Ks[] = {1, 2, 3, 8};
+  for (int dt : {(int)VH_F32, (int)VH_BF16})
+    for (long B : Bs)
+      for (long C : Cs)
+        for (long O : Cs)
+          for (long H : Hs)
+            for (long W : Hs)
+              for (long K : Ks)
+                for (long S : {1L, 2L, 3L, 5L})
+                  for (long P : {0L, 1L, K, 40L}) {
+                    ConvDims d{B, C, O, H, W, K, std::min(K, 3L), S, S > 3 ? 1 : S, P, P / 2, 0, 0};
+                    if (H + 2 * d.PH < d.KH || W + 2 * d.PW < d.KW) continue;
+                    d.HO = (H + 2 * d.PH - d.KH) / d.SH + 1;
+                    d.WO = (W + 2 * d.PW - d.KW) / d.SW + 1;
+                    if (check_conv(d, true) == VH_OK) check_gather(dt, d);
+                  }
+  // padding beyond what 32 bits hold when doubled
+  const ConvDims wide{1, 1, 1, INT32_MAX, 1, 1, 1, 1, 1, 0, 0, INT32_MAX, 1}, pad{1, 1, 1, 1, 1, 3, 3, 1 << 29, 1 << 29, 1 << 30, 1 << 30, 4, 4};
+  for (int dt : {(int)VH_F32, (int)VH_BF16}) {
+    check_gather(dt, wide);
+    check_gather(dt, pad);
+  }
+  // tiles that tests/test_gpu_gather.py is after (bf16)
+  const struct {
+    long B, C, O, H, W, K, S;
+    int bm, bn, ks;
+  } tiles[] = {{16, 120, 130, 21, 23, 3, 1, 64, 64, 2},  {5, 120, 250, 33, 31, 3, 1, 64, 64, 2},  {64, 60, 64, 39, 41, 1, 2, 64, 64, 1},
+               {64, 300, 64, 39, 41, 1, 2, 64, 64, 1},   {128, 60, 64, 39, 41, 1, 2, 64, 128, 1}, {128, 250, 64, 39, 41, 1, 2, 64, 128, 1},
+               {96, 100, 120, 29, 31, 3, 1, 128, 128, 1}, {2, 250, 40, 13, 11, 3, 1, 32, 32, 4},  {4, 40, 100, 27, 29, 3, 1, 32, 64, 2}};
+  for (const auto& t : tiles) {
+    const long HO = (t.H + (t.K / 2) * 2 - t.K) / t.S + 1, WO = (t.W + (t.K / 2) * 2 - t.K) / t.S + 1;
+    const ConvDims d{t.B, t.C, t.O, t.H, t.W, t.K, t.K, t.S, t.S, t.K / 2, t.K / 2, HO, WO};
+    GatherCall c{};
+    c.g = geom_of(d);
+    c.x = c.w = c.y = const_cast<char*>("");
+    GatherInfo o;
+    ++n;
+    if (!gather_info(VH_BF16, c, &o) || o.bm != t.bm || o.bn != t.bn || o.ks != t.ks) {
+      printf("tile of B%ld C%ld O%ld %ldx%ld: %d x %d, %d groups\n", t.B, t.C, t.O, t.H, t.W, o.bm, o.bn, o.ks);
+      ++fails;
+    }
+  }
+}
+
 // The narrow fp32 layers take the faster of their two paths, pass by pass, where one
 // was measured 8 % ahead (us: halo, channels-last).
 void check_halo_rule() {
@@ -266,6 +331,7 @@ int main() {
     }
   }
   check_workspace();
+  check_gathers();
   check_products();
   check_halo_rule();
   check_few_positions();

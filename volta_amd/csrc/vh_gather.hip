@@ -13,8 +13,8 @@
 //    memory straight into LDS (buffer_load_dwordx4 ... lds), no registers;
 //  * a unit's address is base(position) + offset(tap, channel unit): no bounds
 //    checks, whatever the stride and padding.
-// The copy costs one read and one write of the tensor, 2 of the R*S + 1 times
-// that the product reads it.
+// The copy costs one read and one write of the tensor; the product reads it once
+// per tap (mostly from L2) and row of tiles.
 //
 // gather_conv_kernel: D[o][position], forward and (one stride phase at a time,
 // every phase a stride-1 convolution over its own taps) input gradient; weights
@@ -214,7 +214,7 @@ struct ConvArgs {
   ConvPhase ph[kLaunchPhases];
 };
 
-// Tile BM x BN, four waves of WM x WN, two LDS stages of 128 bytes per row: row r
+// Tile BM x BN, four waves of WM x WN, NB LDS stages of 128 bytes per row: row r
 // of 8 units, slot t holds k unit t ^ ((r >> 1) & 7), so that a fragment read (16
 // lanes = 16 rows of one unit) is spread over all banks.  Copy instruction c
 // brings rows 8c .. 8c+7, a lane's k unit depends on c's parity.
@@ -697,6 +697,7 @@ struct ConvPlan {
 
 template <typename T, int BM, int BN, int WM, int WN>
 int launch_conv_tile(ConvPlan& p, hipStream_t st) {
+  constexpr bool b16 = GT<T>::ES == 2, three = b16 && BM * BN < 128 * 128;  // (256 tiles of 128 x 128: never picked)
   ConvArgs& a = p.a;
   a.tiles_m = (a.M + BM - 1) / BM;
   for (int f0 = 0; f0 < p.nph; f0 += kLaunchPhases) {
@@ -708,8 +709,8 @@ int launch_conv_tile(ConvPlan& p, hipStream_t st) {
     }
     a.tiles *= a.tiles_m * a.nph;
     const dim3 grid((unsigned)((a.tiles + 7) / 8 * 8));
-    if (GT<T>::ES == 2 && third_stage(BM, BN, 4 / ((BM / WM) * (BN / WN)), a.tiles))
-      gather_conv_kernel<T, BM, BN, WM, WN, GT<T>::ES == 2 ? 3 : 2><<<grid, 256, 0, st>>>(a);
+    if (three && third_stage(BM, BN, 4 / ((BM / WM) * (BN / WN)), a.tiles))
+      gather_conv_kernel<T, BM, BN, WM, WN, three ? 3 : 2><<<grid, 256, 0, st>>>(a);
     else
       gather_conv_kernel<T, BM, BN, WM, WN, 2><<<grid, 256, 0, st>>>(a);
     VH_LAUNCH_CHECK();
@@ -717,8 +718,8 @@ int launch_conv_tile(ConvPlan& p, hipStream_t st) {
   return VH_OK;
 }
 
-// The tile, by its cost as in vh_mm.hip: rounds of 256 blocks, each of the tile's
-// weight (tile_cost, vh_tiles.hpp).  Measured over 31 shapes of each type (3x3, 32 .. 512
+// The tile, by its cost: rounds of 256 blocks, each of the tile's weight (tile_cost,
+// vh_tiles.hpp).  Measured over 31 shapes of each type (3x3, 32 .. 512
 // channels, 1.5k .. 1M positions); it finds the fastest or one within 7 %, e.g. us on
 // 64 x 64, 32 x 64 (K in two groups of waves), 32 x 32 (four):
 //   fp32 217 -> 224 @11 N=8:     47.5  31.6  23.4
@@ -731,8 +732,11 @@ int launch_conv_tile(ConvPlan& p, hipStream_t st) {
 // copies and stores.  Deep bf16 products of one or two blocks a CU split K over two
 // groups of waves on the 64 x 64 tile (256 @14x15 N=32: 30.6 -> 26.3; shallow ones
 // lose to the extra sum, 64 channels 13.8 -> 14.3).
+struct ConvTile {
+  int bm, bn, ks;
+};
 template <typename T>
-int launch_conv(ConvPlan& a, hipStream_t st) {
+ConvTile pick_conv(const ConvPlan& a) {
   constexpr bool b16 = GT<T>::ES == 2;
   static constexpr int tile[][2] = {{64, 64}, {32, 128}, {32, 64}, {32, 32}, {64, 128}, {128, 128}};
   long n = 0;
@@ -753,14 +757,21 @@ int launch_conv(ConvPlan& a, hipStream_t st) {
       best = k;
     }
   }
-  if constexpr (b16) {
-    if (best == 5) return launch_conv_tile<T, 128, 128, 64, 64>(a, st);
-    if (best == 4) return launch_conv_tile<T, 64, 128, 32, 64>(a, st);
-    if (best == 0 && g64 <= 512 && nst >= 16) return launch_conv_tile<T, 64, 64, 64, 32>(a, st);
+  const int ks = b16 && best == 0 && g64 <= 512 && nst >= 16 ? 2 : best == 2 ? 2 : best == 3 ? 4 : 1;
+  return {tile[best][0], tile[best][1], ks};
+}
+
+template <typename T>
+int launch_conv(ConvPlan& a, hipStream_t st) {
+  const ConvTile t = pick_conv<T>(a);
+  if constexpr (GT<T>::ES == 2) {
+    if (t.bm == 128) return launch_conv_tile<T, 128, 128, 64, 64>(a, st);
+    if (t.bm == 64 && t.bn == 128) return launch_conv_tile<T, 64, 128, 32, 64>(a, st);
+    if (t.bm == 64 && t.ks == 2) return launch_conv_tile<T, 64, 64, 64, 32>(a, st);
   }
-  if (best == 1) return launch_conv_tile<T, 32, 128, 32, 32>(a, st);
-  if (best == 2) return launch_conv_tile<T, 32, 64, 32, 32>(a, st);
-  if (best == 3) return launch_conv_tile<T, 32, 32, 32, 32>(a, st);
+  if (t.bm == 32 && t.bn == 128) return launch_conv_tile<T, 32, 128, 32, 32>(a, st);
+  if (t.bm == 32 && t.bn == 64) return launch_conv_tile<T, 32, 64, 32, 32>(a, st);
+  if (t.bm == 32) return launch_conv_tile<T, 32, 32, 32, 32>(a, st);
   return launch_conv_tile<T, 64, 64, 32, 32>(a, st);
 }
 
@@ -774,8 +785,10 @@ bool make_geo(const ConvGeom& g, Geo& o) {
   constexpr int UE = GT<T>::UE;
   o.Cp = round_up(g.C, UE);
   o.Op = round_up(g.O, UE);
-  o.Hp = (g.P - 1) * g.sh + g.R;
-  o.Wp = (g.Q - 1) * g.sw + g.S;
+  const long Hp = (long)(g.P - 1) * g.sh + g.R, Wp = (long)(g.Q - 1) * g.sw + g.S;
+  if (std::max(Hp, Wp) > (1 << 30) || std::max(g.ph, g.pw) > (1 << 30)) return false;
+  o.Hp = (int)Hp;
+  o.Wp = (int)Wp;
   // dy rows that the input-gradient phases reach: i + (a + ph) / sh - t
   int lo_h = 0, hi_h = g.P - 1, lo_w = 0, hi_w = g.Q - 1;
   auto reach = [](int in, int s, int p, int k, int& lo, int& hi) {
@@ -1120,9 +1133,52 @@ int run_call(const GatherCall& c, char* ws, hipStream_t st) {
   return VH_OK;
 }
 
+// The plan of a call and, of its first chunk, the farthest bytes that the kernels
+// address: every one within its buffer.
+template <typename T>
+bool call_info(const GatherCall& c, GatherInfo& o) {
+  constexpr int UE = GT<T>::UE;
+  CallPlan cp;
+  if (!plan_call<T>(c, cp)) return false;
+  GatherCall d = c;
+  d.g.N = cp.images;
+  PrepArgs pa{};
+  ConvPlan a{};
+  o = GatherInfo{cp.images, 0, 0, 0, cp.wg.splits, cp.wg.per, cp.l.bytes, true};
+  if (c.dw) {
+    const long stages = ((long)cp.images * c.g.P * c.g.Q + GT<T>::BK - 1) / GT<T>::BK;
+    o.ok = (long)cp.wg.splits * cp.wg.per >= stages && (long)(cp.wg.splits - 1) * cp.wg.per < stages;
+  }
+  if (!c.y && !c.dx) return true;
+  conv_args<T>(a, pa.w, d, cp.o, reinterpret_cast<char*>(256), cp.l);  // (nothing is read)
+  const ConvTile t = pick_conv<T>(a);
+  o.bm = t.bm;
+  o.bn = t.bn;
+  o.ks = t.ks;
+  const long planes = (long)a.a.OH * a.a.OW * GT<T>::ES;
+  for (int f = 0; f < a.nph; ++f) {
+    const ConvPhase& p = a.ph[f];
+    const long hw = p.fHW.d, wc = p.fW.d, hc = hw / wc, images = p.N / hw, taps = p.fT.d, tc = p.fS.d, tr = taps / tc;
+    const long in = (images - 1) * a.a.img + (hc - 1) * a.a.sh * a.a.rowb + (wc - 1) * a.a.sw * a.a.colb + p.off0;
+    const long units = (c.y ? cp.o.Cp : cp.o.Op) / UE;
+    const long tap = (tr - 1) * a.a.rowb + (tc - 1) * a.a.colb + units * 16;
+    const long out = ((images - 1) * a.a.M + a.a.M - 1) * planes +
+                     (((hc - 1) * a.a.osh + p.sub_a) * a.a.OW + (wc - 1) * a.a.osw + p.sub_b + 1) * GT<T>::ES;
+    const bool live = p.nst > 0;
+    o.ok = o.ok && (!live || (p.off0 >= 0 && in + tap <= a.a.x_bytes)) && out <= a.a.y_bytes &&
+           (long)a.a.M * p.nst * 128 == p.w_bytes && (long)p.w_off + p.w_bytes <= (long)(cp.l.bytes - cp.l.w) &&
+           p.units <= p.nst * 8;
+  }
+  return true;
+}
+
 }  // namespace
 
 size_t gather_ws(int dt, const GatherCall& c) { return dt == VH_BF16 ? call_ws<bf16>(c) : call_ws<float>(c); }
+
+bool gather_info(int dt, const GatherCall& c, GatherInfo* o) {
+  return dt == VH_BF16 ? call_info<bf16>(c, *o) : call_info<float>(c, *o);
+}
 
 int gather_run(int dt, const GatherCall& c, void* ws, hipStream_t st) {
   return dt == VH_BF16 ? run_call<bf16>(c, static_cast<char*>(ws), st) : run_call<float>(c, static_cast<char*>(ws), st);

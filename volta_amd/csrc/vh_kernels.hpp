@@ -183,6 +183,15 @@ struct GatherCall {
 constexpr size_t kGatherMostWs = (size_t)256 << 20;
 size_t gather_ws(int dt, const GatherCall& c);
 int gather_run(int dt, const GatherCall& c, void* ws, hipStream_t st);
+// The plan of a call: images per chunk, tile and wave groups of y or dx, position
+// splits and stages of dw, workspace; ok: its addresses lie within its buffers.  False:
+// unsupported.
+struct GatherInfo {
+  int images, bm, bn, ks, splits, per;
+  size_t bytes;
+  bool ok;
+};
+bool gather_info(int dt, const GatherCall& c, GatherInfo* o);
 
 // ---- dense bf16 products (vh_dense.hip) ----
 // C[M][N] = A . B (+ bias[N] per column), bf16 in and out.  A is stored
