@@ -1,5 +1,7 @@
 """GPU: convolutions over channels-last copies (vh_gather.hip) at the edges of
 their tiles, stages and stride phases, against the oracle under the parity gate."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -7,7 +9,7 @@ import torch
 import oracle
 from tests.parity import k_conv_dgrad, k_conv_fwd, k_conv_wgrad
 from tests.test_gpu_parity import DEV, DTYPES, check, host, prep, rng
-from volta_amd import nn as vnn
+from volta_amd import lib, nn as vnn
 
 pytestmark = pytest.mark.gpu
 
@@ -22,7 +24,7 @@ CASES = [
     (2, 7, 9, 10, 3, 2, 4, 0),       # stride 4 past the width, taps missing in most phases
     (2, 12, 20, 11, 13, 3, 1, 3),    # padding wider than the kernel reaches
     (64, 9, 80, 33, 31, 3, 1, 1),    # 128-row tiles, channels 9 -> 16 padded
-    (80, 24, 64, 33, 31, 3, 1, 1),   # 64 x 256 tiles
+    (80, 24, 64, 33, 31, 3, 1, 1),   # 64-row tiles of many positions
     (16, 16, 16, 45, 45, 3, 1, 1),   # weight gradient split many ways
     (2, 72, 136, 5, 7, 3, 1, 1),     # weight gradient split a few ways, channels past 64
 ]
@@ -104,22 +106,33 @@ def test_gather_conv_transpose(dt):
     assert np.array_equal(host(ct.backward(dyt, xt, weight_grad=False)[0]), host(got[0]))
 
 
+def _workspace(stream):
+    n = ctypes.c_size_t()
+    assert lib().vh_workspace_info(ctypes.c_void_p(stream.cuda_stream), None, ctypes.byref(n), None) == 0
+    return n.value
+
+
 def test_gather_falls_back_without_workspace():
     """A capture on a stream whose workspace holds what the generic path needs
-    but not the copies is still accepted, and right."""
+    but not the copies is still accepted, and right; the workspace does not move."""
     conv = vnn.Conv2d(16, 16, 3, 1, 1, use_bias=False, device=DEV)
     conv.set_algo(vnn.ConvAlgo.IGEMM)
     small, big = torch.randn(1, 16, 31, 31, device=DEV), torch.randn(64, 16, 31, 31, device=DEV)
     want = conv.forward(big)
     out = torch.empty_like(want)
-    cap = torch.cuda.Stream()
+    cap = torch.cuda.Stream()  # (its handle may be one that earlier work has grown a workspace on)
+    torch.cuda.synchronize()
+    assert lib().vh_release_cache() == 0
     cap.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(cap):
         conv.forward(small)
     torch.cuda.synchronize()
+    have = _workspace(cap)
+    assert 0 < have < big.shape[0] * 33 * 33 * 16 * 4, "the copy of the input fits: nothing falls back"
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=cap):
         conv.forward(big, out=out)
+    assert _workspace(cap) == have
     for _ in range(3):
         out.fill_(float("nan"))
         graph.replay()
@@ -144,8 +157,8 @@ def test_narrow_fp32_layer_on_either_kernel(B):
     check(db, oracle.conv_bias_grad, (dy,), "f32", "db", k=B * 784)
 
 
-@pytest.mark.parametrize("C", [60, 128, 190, 250, 300, 550])  # 1x1: 1, 2, 3, 4, 5 and 9 stages
-@pytest.mark.parametrize("B,O", [(2, 40), (96, 130)])  # K over four wave groups; 64-row tiles
+@pytest.mark.parametrize("C", [60, 120, 190, 250, 300, 550])  # 1x1: 1, 2, 3, 4, 5 and 9 stages
+@pytest.mark.parametrize("B,O", [(2, 40), (96, 130)])  # 32 x 64 tiles, K over two wave groups
 def test_gather_bf16_stages_in_flight(C, B, O):
     g = rng(C + B)
     x, xt = prep(g.standard_normal((B, C, 13, 11)), "bf16")
@@ -212,3 +225,26 @@ def test_narrow_fp32_layer_with_passes_on_both_paths():
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 def test_few_positions(case, dt):
     test_gather_conv_all_passes(case, dt)
+
+
+# bf16 on the tiles that the cases above do not pick (host_check pins the choice): 64 x 64 and
+# 64 x 128 with three LDS stages of 1 .. 5, 64 x 64 with two wave groups of 9 and 8 stages
+@pytest.mark.parametrize("case", [(64, 60, 64, 39, 41, 1, 2), (64, 120, 64, 39, 41, 1, 2), (64, 190, 64, 39, 41, 1, 2),
+                                  (64, 250, 64, 39, 41, 1, 2), (64, 300, 64, 39, 41, 1, 2), (128, 60, 64, 39, 41, 1, 2),
+                                  (128, 190, 64, 39, 41, 1, 2), (128, 250, 64, 39, 41, 1, 2), (16, 120, 130, 21, 23, 3, 1),
+                                  (5, 120, 250, 33, 31, 3, 1)])
+def test_gather_bf16_tiles(case):
+    B, C, O, H, W, K, S = case
+    g = rng(C + B)
+    x, xt = prep(g.standard_normal((B, C, H, W)), "bf16")
+    w, wt = prep(g.standard_normal((O, C, K, K)) * np.sqrt(2.0 / (C * K * K)), "bf16")
+    conv = vnn.Conv2d(C, O, K, S, K // 2, use_bias=False, device=DEV, dtype=DTYPES["bf16"])
+    conv.weight = wt
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    kw = dict(stride=(S, S), pad=(K // 2, K // 2))
+    y = conv.forward(xt)
+    check(y, oracle.direct_conv, (x, w), "bf16", "y", kw, k=C * K * K)
+    if S == 1:  # the same tiles in the input gradient, O and C changing places
+        dy, dyt = prep(g.standard_normal(tuple(y.shape)), "bf16")
+        dx = conv.backward(dyt, xt, weight_grad=False)[0]
+        check(dx, oracle.direct_conv_backward_input, (dy, w, x.shape), "bf16", "dx", kw, k=O * K * K)

@@ -19,11 +19,11 @@ CASES = [
     (40, 3000, 24),              # few tiles: K split over blocks
     (129, 4097, 70),             # the same with padded rows, a split's last stage partial
     (300, 96, 1000), (257, 130, 255),
-    (520, 250, 520),             # 64 x 64 tiles (bf16: 32 x 64)
-    (1030, 72, 1100),            # 64 x 64 / 64 x 128 tiles with remainders
-    (2060, 40, 2072),            # 128 x 128 tiles (bf16) with remainders, aligned rows
+    (520, 250, 520),             # 32 x 64 tiles in two K groups, dA and dB of 9 stages
+    (1030, 72, 1100),            # bf16 64 x 128 tiles with remainders; dA 32 x 64, dB 32 x 32 of 17 stages
+    (2060, 40, 2072),            # many 64 x 64 tiles of one stage, aligned rows; dB split
     (2050, 33, 2310),            # the same, padded rows
-    (4100, 16, 2056),            # 128 x 256 producer / consumer tiles (bf16 forward)
+    (4100, 16, 2056),            # 2145 tiles of a quarter stage; dA and dB of few deep tiles
 ]
 
 
@@ -90,7 +90,7 @@ def test_mm_padding_does_not_leak(mkn, dt):
     assert db[: k - 1].all() and not db[k - 1].any()
 
 
-@pytest.mark.parametrize("k", [700, 768, 772, 896, 1030])  # 11 stages (two in LDS) .. 17 (three)
+@pytest.mark.parametrize("k", [700, 768, 772, 896, 1030])  # 11 stages (two in LDS) .. 17 (three), on every tile
 @pytest.mark.parametrize("m,n", [(40, 1200), (520, 264), (1024, 1024), (1500, 1111), (1536, 2048), (1537, 2048)])
 def test_mm_bf16_stages_in_flight(m, k, n):
     g = rng(m + k + n)
@@ -125,3 +125,13 @@ def test_mm_linear_gradients_in_one_launch(shape, dt):
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 def test_mm_or_implicit_gemm(mkn, dt):
     test_mm_family(mkn, dt)
+
+
+# dB alone on 128 x 128 tiles (bf16) with remainders, aligned rows and padded ones
+@pytest.mark.parametrize("mkn", [(300, 2056, 2064), (289, 2299, 2308)])
+def test_mm_bf16_backward_b_128x128_tiles(mkn):
+    m, k, n = mkn
+    g = rng(m + k + n)
+    a, at = prep(g.standard_normal((m, k)), "bf16")
+    gr, grt = prep(g.standard_normal((m, n)), "bf16")
+    check(ops.gpu_matmul_backward_b(at, grt, m, k, n), oracle.matmul_backward_b, (a, gr), "bf16", "dB", k=m)

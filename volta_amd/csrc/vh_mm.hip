@@ -423,7 +423,7 @@ MmPlan mm_plan(const DenseProblem* p, int np) {
   for (int k = 0; k < nt; ++k) blocks[k] = consider(costs[k], 1);
   // A split pays for its reduction where the grid leaves room (fp32 512 x 512 x 8192: 52
   // -> 43 us at 16 splits, 64 x 2048 x 2048: 14.8 -> 12.5) or one product of a pair has
-  // few deep blocks (Linear 16384 x 64 -> 64 backward, one tile of dW: 112 -> 20).
+  // few deep blocks (Linear 16384 x 64 -> 64 backward, one tile of dW: 112 -> 14).
   for (int k = 0; k < 3 && best.us > 2 * kSplitUs; ++k)
     for (int s = 2; s <= 256; s += std::max(1, s / 4))
       if (consider(costs[k], s) > blocks[k] + 2048) break;

@@ -268,12 +268,12 @@ struct ColSum {
   }
 };
 
-// Cost of a product of `blocks` tiles over nst stages: rounds of 256 blocks, each
-// of the tile's weight.
+// Cost of a convolution of `blocks` tiles over nst stages (matrix products have their
+// own, mm_plan): rounds of 256 blocks, each of the tile's weight.
 //  * fp32 rounds are their MFMAs: a weight is the stages of one block, plus 3 to 4
 //    for its prologue and epilogue (half-size tiles in two K groups: half the
 //    stages, slightly longer ones).
-//  * bf16: the times of one round relative to 64 x 64 (4096^3: 108, 143, 175, 252,
+//  * bf16: the times of one round relative to 64 x 64 (products, 4096^3: 108, 143, 175, 252,
 //    505 us on 128 x 128 .. 32 x 32).  A block alone on a CU cannot cover its
 //    copies: less than 1.7 rounds cost as much (2048^3: 30 us on 256 blocks of 128 x
 //    128, 24 on 512 of 64 x 128; 1024^3: 22, 9.4, 7.7, 7.0, 11.5).
