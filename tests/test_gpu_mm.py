@@ -135,3 +135,24 @@ def test_mm_bf16_backward_b_128x128_tiles(mkn):
     a, at = prep(g.standard_normal((m, k)), "bf16")
     gr, grt = prep(g.standard_normal((m, n)), "bf16")
     check(ops.gpu_matmul_backward_b(at, grt, m, k, n), oracle.matmul_backward_b, (a, gr), "bf16", "dB", k=m)
+
+
+def test_stream_of_a_device():
+    """The current stream by a tensor's device, an index, a name or nothing; no other device has one."""
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for d in (torch.zeros(1, device=DEV).device, 0, "cuda", "cuda:0", torch.device("cuda"), None):
+            assert ops.stream_ptr(d) == side.cuda_stream
+    for d in ("cpu", torch.device("cpu")):
+        with pytest.raises(ValueError):
+            ops.stream_ptr(d)
+
+
+def test_algorithm_given_as_a_plain_number():
+    conv = vnn.Conv2d(3, 4, 3, 1, 1, device=DEV)
+    x = torch.randn(2, 3, 6, 6, device=DEV)
+    conv.algo = np.int64(int(vnn.ConvAlgo.IGEMM))
+    y = conv.forward(x)
+    assert conv.last_algo == vnn.ConvAlgo.IGEMM
+    conv.algo = vnn.ConvAlgo.IGEMM
+    assert torch.equal(conv.forward(x), y)

@@ -93,7 +93,7 @@ class Conv2d:
         y = self._new_or_checked(out, x, dims)
         used = ctypes.c_int(-1)
         fn = lib().vh_conv2d_forward_relu if relu else lib().vh_conv2d_forward
-        check(fn(dt, self.algo, ptr(x), ptr(self.weight), ptr(self.bias), ptr(y), *dims, ctypes.byref(used),
+        check(fn(dt, int(self.algo), ptr(x), ptr(self.weight), ptr(self.bias), ptr(y), *dims, ctypes.byref(used),
                  stream_ptr(x.device)))
         self.last_algo = ConvAlgo(used.value)
         return y

@@ -28,10 +28,11 @@ def dtype_code(t: torch.Tensor) -> int:
 
 
 def stream_ptr(device=None) -> int:
-    """The current stream's handle (without building a torch Stream object: 0.1
-    instead of 1.8 us, on a call that launches in 4 to 10)."""
-    index = torch.device(device).index if isinstance(device, (str, torch.device)) else device
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    """The current stream's handle.  For a tensor's device without building a torch
+    Stream object: 0.4 instead of 1.9 us, on a call that launches in 4 to 10."""
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None and torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
