@@ -156,3 +156,28 @@ def test_algorithm_given_as_a_plain_number():
     assert conv.last_algo == vnn.ConvAlgo.IGEMM
     conv.algo = vnn.ConvAlgo.IGEMM
     assert torch.equal(conv.forward(x), y)
+
+
+# fp32 dX + dW in one launch: whole tiles with sums in two levels (no product fills the chip with
+# 256 x 256 tiles), dX or a dW without db in one level (it does: 16384 x 1024, 4096 x 4096),
+# smaller tiles; where a product alone has the same groups and splits of K, its bits (dW of
+# 16384 x 1024 x 256 is split alone)
+@pytest.mark.parametrize("shape", [(4096, 2048, 2048), (16384, 1024, 128), (4096, 4096, 4096), (300, 200, 260), (16384, 1024, 256),
+                                   (1024, 4096, 4096)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_linear_gradients_together_and_alone(shape, bias):
+    m, i, o = shape
+    torch.manual_seed(m + i + o)
+    lin = vnn.Linear(i, o, use_bias=bias, device=DEV)
+    x, dy = torch.randn(m, i, device=DEV), torch.randn(m, o, device=DEV)
+    dx, dw, db = lin.backward(dy, x)
+    assert torch.equal(lin.backward(dy, x, weight_grad=False)[0], dx)
+    _, dw1, db1 = lin.backward(dy, x, input_grad=False)
+    if shape != (16384, 1024, 256):
+        assert torch.equal(dw1, dw)
+    if not bias:
+        return
+    # (db: column sums of the staged tiles, or of dY: the bound of m additions in any order)
+    bound = 2.0 ** -24 * m * dy.double().abs().sum(0)
+    assert bool(((db.double() - dy.double().sum(0)).abs() <= bound).all())
+    assert bool(((db1.double() - dy.double().sum(0)).abs() <= bound).all())

@@ -1,14 +1,14 @@
 // vh_dense_f32.hip -- dense fp32 matrix products (matmul, its gradients,
 // Linear) on gfx950 MFMA (v_mfma_f32_32x32x2_f32), fp32 accumulation.
 //
-// Products of whole tiles: dW = A^T . G on 256 x 256 tiles (4096^3: 925 us, 983 on
-// the 64 x 64 tiles of vh_mm.hip, which take every other product: whole 256 x 256
-// tiles of the other layouts measured equal or slower, 978 / 971 and 1003 / 970 us),
-// and a Linear layer's dX and dW as one launch.  "K-major": [rows][K], the contraction
-// index contiguous; "MN-major": [K][rows].
+// Products of whole 256 x 256 tiles that fill the chip (4096^3: 979 us, 1044 on the 64 x
+// 64 tiles of vh_mm.hip, which take every other product), and a Linear layer's dX and dW
+// as one launch.  "K-major": [rows][K], the contraction index contiguous; "MN-major":
+// [K][rows].
 #include <type_traits>
 
 #include "vh_kernels.hpp"
+#include "vh_tiles.hpp"
 
 namespace vh {
 
@@ -72,7 +72,7 @@ struct F32D2lCfg {
 // own 4 << cs_shift of its columns, so every column is summed by exactly one
 // block over all K; a thread adds 4 consecutive owned columns of one k row per
 // stage, in stage order, and the k-row group sums are added in group order.
-template <int BM, bool AT, bool BT, bool CS, bool BIAS = false>
+template <int BM, bool AT, bool BT, bool CS, bool BIAS, bool TWO>
 __device__ __forceinline__ void f32_d2l_tile(const DenseF32Args& g, const int lb, u32x4f* S0, u32x4f* S1) {
   using Cfg = F32D2lCfg<BM>;
   constexpr int FM = Cfg::FM, FN = Cfg::FN, UNITS_A = Cfg::A_UNITS;
@@ -116,8 +116,10 @@ __device__ __forceinline__ void f32_d2l_tile(const DenseF32Args& g, const int lb
 
   // fragments of step kk (8 k) of a stage: MFMA t multiplies k 8 kk + 4 half_l + t of
   // the lane's half -- K-major one 16-byte read of unit 2 kk + half_l, MN-major 4-byte
-  // reads of four k rows.  The same k pairs in the same order as in vh_mm.hip, so a
-  // product is bit-identical on either.
+  // reads of four k rows.  The same k pairs in the same order as in vh_mm.hip, and with TWO
+  // the same two levels of sums, for which 256 x 256 tiles have no registers: a product of
+  // the pair takes them unless it would go on such tiles alone, so that dX and dW are bit
+  // for bit those of separate calls.
   const int row_l = lane & 31, half_l = lane >> 5;
   struct Frags {
     f32x4 a[FM], b[FN];
@@ -149,6 +151,8 @@ __device__ __forceinline__ void f32_d2l_tile(const DenseF32Args& g, const int lb
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
+  tiles::Totals<float, TWO ? FM : 1, TWO ? FN : 1> tot;
+  if constexpr (TWO) tot.init();
   auto mma = [&](const Frags& f) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -211,6 +215,7 @@ __device__ __forceinline__ void f32_d2l_tile(const DenseF32Args& g, const int lb
       mma(fb);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (TWO) tot.template stage<B>(acc);
   };
   using C0 = std::integral_constant<int, 0>;
   using C1 = std::integral_constant<int, 1>;
@@ -218,6 +223,7 @@ __device__ __forceinline__ void f32_d2l_tile(const DenseF32Args& g, const int lb
     body(C0{}, s);
     body(C1{}, s + 1);
   }
+  if constexpr (TWO) tot.finish(acc);
 
   if constexpr (CS) {
     if (cs_blk) {  // per owned column: the k-row group sums, added in group order
@@ -258,21 +264,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_f32_d2l_kernel(DenseF32Args g) {
   __shared__ __attribute__((aligned(16))) u32x4f S0[F32D2lCfg<256>::STAGE];
   __shared__ __attribute__((aligned(16))) u32x4f S1[F32D2lCfg<256>::STAGE];
-  f32_d2l_tile<256, AT, BT, false, BIAS>(g, xcd_block(g.tiles_m * g.tiles_n), S0, S1);
+  f32_d2l_tile<256, AT, BT, false, BIAS, false>(g, xcd_block(g.tiles_m * g.tiles_n), S0, S1);
 }
 
 // Two products in one launch on 128 x 256 tiles (Linear's dX, K-major x
 // K-major, and dW, MN-major x MN-major with the bias gradient's column sums):
 // blocks 0 .. T0-1 take the first product's tiles, the rest the second's.
+// (4096 x 1024 -> 4096, both in two levels: 478 -> 496 us.)
+template <bool TWO0, bool TWO1>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_f32_d2l_pair_kernel(DenseF32Args g0, DenseF32Args g1) {
   __shared__ __attribute__((aligned(16))) u32x4f S0[F32D2lCfg<128>::STAGE];
   __shared__ __attribute__((aligned(16))) u32x4f S1[F32D2lCfg<128>::STAGE];
   const int t0 = g0.tiles_m * g0.tiles_n, h = blockIdx.x;
   if (h < t0)
-    f32_d2l_tile<128, false, false, false>(g0, xcd_map(h, t0), S0, S1);
+    f32_d2l_tile<128, false, false, false, false, TWO0>(g0, xcd_map(h, t0), S0, S1);
   else
-    f32_d2l_tile<128, true, true, true>(g1, xcd_map(h - t0, g1.tiles_m * g1.tiles_n), S0, S1);
+    f32_d2l_tile<128, true, true, true, false, TWO1>(g1, xcd_map(h - t0, g1.tiles_m * g1.tiles_n), S0, S1);
 }
 
 bool fits_f(long bytes) { return bytes >= 0 && bytes < (1L << 31) - 64; }
@@ -305,6 +313,8 @@ DenseF32Args f32_args(const void* a, int lda, bool at, const void* b, int ldb, b
   g.c_bytes = (int)((long)M * ldc * 4);
   return g;
 }
+// whole 256 x 256 tiles that fill the chip
+bool f32_large(int M, int N) { return M % 256 == 0 && N % 256 == 0 && (long)(M / 256) * (N / 256) >= 256; }
 }  // namespace
 
 int dense_f32_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStream_t st) {
@@ -323,19 +333,24 @@ int dense_f32_gemm_pair(const DenseProblem& p0, const DenseProblem& p1, hipStrea
     a->tiles_n = a->N / 256;
     a->cs_shift = colsum_shift(a->tiles_m, 256);
   }
-  gemm_f32_d2l_pair_kernel<<<dim3((unsigned)(a0.tiles_m * a0.tiles_n + a1.tiles_m * a1.tiles_n)), 512, 0, st>>>(a0,
-                                                                                                                a1);
+  const dim3 grid((unsigned)(a0.tiles_m * a0.tiles_n + a1.tiles_m * a1.tiles_n));
+  // (with column sums a product alone is one of vh_mm.hip)
+  const bool two0 = !f32_large(p0.M, p0.N), two1 = p1.colsum || !f32_large(p1.M, p1.N);
+  if (two0)
+    two1 ? gemm_f32_d2l_pair_kernel<true, true><<<grid, 512, 0, st>>>(a0, a1)
+         : gemm_f32_d2l_pair_kernel<true, false><<<grid, 512, 0, st>>>(a0, a1);
+  else
+    two1 ? gemm_f32_d2l_pair_kernel<false, true><<<grid, 512, 0, st>>>(a0, a1)
+         : gemm_f32_d2l_pair_kernel<false, false><<<grid, 512, 0, st>>>(a0, a1);
   VH_LAUNCH_CHECK();
   return VH_OK;
 }
 
 int dense_f32_gemm(const void* a, int lda, bool at, const void* b, int ldb, bool bt, void* c, int ldc, int M,
                    int N, int K, const void* bias, hipStream_t st) {
-  // whole 256 x 256 tiles that fill the chip (16-byte aligned operand rows; the
-  // stores are 4-byte): 4096 x 4096 x 1024 254 us, 272 on the tiles of vh_mm.hip; 4096^3 979
+  // large whole tiles (16-byte aligned operand rows; the stores are 4-byte): 4096 x 4096 x 1024 254 us, 272 on the tiles of vh_mm.hip; 4096^3 979
   // and 1044, of MN-major A and B 931 and 985
-  if ((at && !bt) || (at && bias) || M % 256 || N % 256 || K % (2 * kF32D2lBK) || lda % 4 || ldb % 4 ||
-      (long)(M / 256) * (N / 256) < 256)
+  if ((at && !bt) || (at && bias) || !f32_large(M, N) || K % (2 * kF32D2lBK) || lda % 4 || ldb % 4)
     return VH_ERR_UNSUPPORTED;
   DenseF32Args g = f32_args(a, lda, at, b, ldb, bt, c, ldc, M, N, K);
   g.bias = (const float*)bias;
