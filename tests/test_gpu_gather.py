@@ -227,6 +227,33 @@ def test_few_positions(case, dt):
     test_gather_conv_all_passes(case, dt)
 
 
+# fp32 1x1 layers on either side of the rule for a forward or a lone input gradient: one row of tiles
+# over the implicit GEMM (48, 64 and 24 rows), two rows or few positions over the copies
+@pytest.mark.parametrize("case", [(100, 64, 48, 13, 13), (65, 65, 64, 16, 16), (64, 64, 64, 16, 16), (3, 24, 66, 77, 73),
+                                  (2, 24, 8, 257, 256)])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_pointwise_layer_on_either_kernel(case, dt):
+    B, C, O, H, W = case
+    g = rng(B + C)
+    conv = vnn.Conv2d(C, O, 1, 1, 0, device=DEV, dtype=DTYPES[dt])
+    conv.set_algo(vnn.ConvAlgo.IGEMM)
+    x, xt = prep(g.standard_normal((B, C, H, W)), dt)
+    w, wt = prep(g.standard_normal((O, C, 1, 1)) / np.sqrt(C), dt)
+    b, bt = prep(g.standard_normal(O), dt)
+    dy, dyt = prep(g.standard_normal((B, O, H, W)), dt)
+    conv.weight, conv.bias = wt, bt
+    kw = dict(stride=(1, 1), pad=(0, 0))
+    y = conv.forward(xt)
+    bb = b[None, :, None, None]
+    check(y, oracle.direct_conv, (x, w), dt, "y", kw, extra_ref=bb, extra_scale=np.abs(bb), k=C + 1)
+    assert np.array_equal(host(conv.forward(xt, relu=True)), np.maximum(host(y), 0))
+    check(conv.backward(dyt, xt, weight_grad=False)[0], oracle.direct_conv_backward_input, (dy, w, x.shape), dt, "dx", kw, k=O)
+    dx, dw, db = conv.backward(dyt, xt)
+    check(dx, oracle.direct_conv_backward_input, (dy, w, x.shape), dt, "dx together", kw, k=O)
+    check(dw, oracle.direct_conv_backward_weight, (dy, x, w.shape), dt, "dw", kw, k=B * H * W)
+    check(db, oracle.conv_bias_grad, (dy,), dt, "db", k=B * H * W)
+
+
 # bf16 on the tiles that the cases above do not pick (host_check pins the choice): 64 x 64 and
 # 64 x 128 with three LDS stages of 1 .. 5, 64 x 64 with two wave groups of 9 and 8 stages
 @pytest.mark.parametrize("case", [(64, 60, 64, 39, 41, 1, 2), (64, 120, 64, 39, 41, 1, 2), (64, 190, 64, 39, 41, 1, 2),

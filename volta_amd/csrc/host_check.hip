@@ -261,13 +261,30 @@ void check_few_positions() {
   const struct {
     long M, pos, C, RS;
     float generic, copies;
-  } rows[] = {{60, 32, 778, 25, 26.3f, 136.f}, {33, 162, 459, 9, 18.7f, 35.4f},   {512, 49, 512, 9, 33.7f, 47.f},   {72, 225, 468, 16, 24.5f, 59.5f},
+  } rows[] = {{60, 32, 778, 25, 26.3f, 136.f}, {33, 162, 459, 9, 18.7f, 35.4f},   {512, 49, 512, 9, 33.7f, 47.f},  {256, 49, 256, 9, 21.9f, 25.7f},  {72, 225, 468, 16, 24.5f, 59.5f},
               {577, 98, 453, 16, 43.5f, 65.2f}, {108, 1053, 940, 9, 47.6f, 68.7f}, {60, 1734, 625, 25, 103.f, 112.f}, {333, 343, 721, 9, 63.1f, 56.8f}, {228, 768, 618, 25, 157.f, 112.f},
               {512, 392, 512, 9, 53.1f, 48.2f}, {164, 256, 192, 9, 22.8f, 21.f},   {199, 125, 240, 9, 28.7f, 25.3f},  {68, 936, 170, 9, 21.8f, 19.8f}};
   for (const auto& r : rows) {
     ++n;
     if (copies_pay(VH_F32, r.M, r.pos, r.C, r.RS) != (r.copies < r.generic)) {
       printf("fp32 %ld x %ld, %ld channels, %ld taps: the slower path\n", r.M, r.pos, r.C, r.RS);
+      ++fails;
+    }
+  }
+}
+
+// fp32 1x1 layers: the path measured as the faster for a forward (or lone input gradient) of M rows
+void check_pointwise() {
+  const struct {
+    long M, K, B, H;
+    float generic, copies;
+  } rows[] = {{64, 256, 64, 56, 97.8f, 156.7f}, {64, 64, 32, 56, 25.3f, 29.6f}, {16, 64, 32, 56, 20.9f, 23.3f}, {16, 64, 64, 56, 39.4f, 36.9f},
+              {48, 64, 100, 13, 12.0f, 13.3f},  {128, 64, 64, 56, 87.1f, 71.1f}, {64, 128, 16, 14, 13.7f, 10.1f}, {48, 160, 12, 56, 22.0f, 27.0f}};
+  for (const auto& r : rows) {
+    const ConvDims d{r.B, r.K, r.M, r.H, r.H, 1, 1, 1, 1, 0, 0, r.H, r.H};
+    ++n;
+    if (pointwise_once(VH_F32, d, r.M) != (r.generic < r.copies)) {
+      printf("fp32 1x1 %ld -> %ld, %ld images of %ld: the slower path\n", r.K, r.M, r.B, r.H);
       ++fails;
     }
   }
@@ -335,6 +352,7 @@ int main() {
   check_products();
   check_halo_rule();
   check_few_positions();
+  check_pointwise();
   printf("host_check: %ld plans, %ld failures\n", n, fails);
   return fails ? 1 : 0;
 }
