@@ -228,21 +228,22 @@ def test_few_positions(case, dt):
 
 
 # fp32 1x1 layers on either side of the rule for a forward or a lone input gradient: one row of tiles
-# over the implicit GEMM (48, 64 and 24 rows), two rows or few positions over the copies
-@pytest.mark.parametrize("case", [(100, 64, 48, 13, 13), (65, 65, 64, 16, 16), (64, 64, 64, 16, 16), (3, 24, 66, 77, 73),
-                                  (2, 24, 8, 257, 256)])
+# over the implicit GEMM (48, 64 and 24 rows), two rows or few positions over the copies; stride 2
+# forward over the implicit GEMM and (257 rows, few positions) the copies
+@pytest.mark.parametrize("case", [(100, 64, 48, 13, 13, 1), (65, 65, 64, 16, 16, 1), (64, 64, 64, 16, 16, 1), (3, 24, 66, 77, 73, 1),
+                                  (2, 24, 8, 257, 256, 1), (8, 20, 70, 65, 67, 2), (8, 12, 257, 65, 67, 2), (8, 20, 70, 64, 64, 2)])
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 def test_pointwise_layer_on_either_kernel(case, dt):
-    B, C, O, H, W = case
+    B, C, O, H, W, S = case
     g = rng(B + C)
-    conv = vnn.Conv2d(C, O, 1, 1, 0, device=DEV, dtype=DTYPES[dt])
+    conv = vnn.Conv2d(C, O, 1, S, 0, device=DEV, dtype=DTYPES[dt])
     conv.set_algo(vnn.ConvAlgo.IGEMM)
     x, xt = prep(g.standard_normal((B, C, H, W)), dt)
     w, wt = prep(g.standard_normal((O, C, 1, 1)) / np.sqrt(C), dt)
     b, bt = prep(g.standard_normal(O), dt)
-    dy, dyt = prep(g.standard_normal((B, O, H, W)), dt)
+    dy, dyt = prep(g.standard_normal((B, O, (H - 1) // S + 1, (W - 1) // S + 1)), dt)
     conv.weight, conv.bias = wt, bt
-    kw = dict(stride=(1, 1), pad=(0, 0))
+    kw = dict(stride=(S, S), pad=(0, 0))
     y = conv.forward(xt)
     bb = b[None, :, None, None]
     check(y, oracle.direct_conv, (x, w), dt, "y", kw, extra_ref=bb, extra_scale=np.abs(bb), k=C + 1)

@@ -261,7 +261,7 @@ void check_few_positions() {
   const struct {
     long M, pos, C, RS;
     float generic, copies;
-  } rows[] = {{60, 32, 778, 25, 26.3f, 136.f}, {33, 162, 459, 9, 18.7f, 35.4f},   {512, 49, 512, 9, 33.7f, 47.f},  {256, 49, 256, 9, 21.9f, 25.7f},  {72, 225, 468, 16, 24.5f, 59.5f},
+  } rows[] = {{60, 32, 778, 25, 26.3f, 136.f}, {33, 162, 459, 9, 18.7f, 35.4f},   {512, 49, 512, 9, 33.7f, 47.f},  {256, 49, 256, 9, 21.9f, 25.7f}, {16, 784, 256, 9, 13.9f, 25.f}, {48, 432, 192, 9, 16.5f, 20.7f}, {192, 224, 64, 25, 22.6f, 21.3f}, {2, 1250, 128, 16, 14.1f, 20.7f},  {72, 225, 468, 16, 24.5f, 59.5f},
               {577, 98, 453, 16, 43.5f, 65.2f}, {108, 1053, 940, 9, 47.6f, 68.7f}, {60, 1734, 625, 25, 103.f, 112.f}, {333, 343, 721, 9, 63.1f, 56.8f}, {228, 768, 618, 25, 157.f, 112.f},
               {512, 392, 512, 9, 53.1f, 48.2f}, {164, 256, 192, 9, 22.8f, 21.f},   {199, 125, 240, 9, 28.7f, 25.3f},  {68, 936, 170, 9, 21.8f, 19.8f}};
   for (const auto& r : rows) {
@@ -273,18 +273,21 @@ void check_few_positions() {
   }
 }
 
-// fp32 1x1 layers: the path measured as the faster for a forward (or lone input gradient) of M rows
+// fp32 1x1 layers: the path measured as the faster for a forward of M rows
 void check_pointwise() {
   const struct {
-    long M, K, B, H;
+    long M, K, B, H, S;
     float generic, copies;
-  } rows[] = {{64, 256, 64, 56, 97.8f, 156.7f}, {64, 64, 32, 56, 25.3f, 29.6f}, {16, 64, 32, 56, 20.9f, 23.3f}, {16, 64, 64, 56, 39.4f, 36.9f},
-              {48, 64, 100, 13, 12.0f, 13.3f},  {128, 64, 64, 56, 87.1f, 71.1f}, {64, 128, 16, 14, 13.7f, 10.1f}, {48, 160, 12, 56, 22.0f, 27.0f}};
+  } rows[] = {{64, 256, 64, 56, 1, 97.8f, 156.7f}, {64, 64, 32, 56, 1, 25.3f, 29.6f},    {16, 64, 32, 56, 1, 20.9f, 23.3f},
+              {16, 64, 64, 56, 1, 39.4f, 36.9f},   {48, 64, 100, 13, 1, 12.0f, 13.3f},   {128, 64, 64, 56, 1, 87.1f, 71.1f},
+              {64, 128, 16, 14, 1, 13.7f, 10.1f},  {48, 160, 12, 56, 1, 22.0f, 27.0f},   {64, 256, 16, 112, 2, 36.5f, 111.5f},
+              {256, 64, 32, 56, 2, 26.6f, 29.9f},  {512, 128, 16, 112, 2, 131.6f, 124.5f}, {64, 64, 32, 28, 2, 11.0f, 10.6f}};
   for (const auto& r : rows) {
-    const ConvDims d{r.B, r.K, r.M, r.H, r.H, 1, 1, 1, 1, 0, 0, r.H, r.H};
+    const long HO = (r.H - 1) / r.S + 1;
+    const ConvDims d{r.B, r.K, r.M, r.H, r.H, 1, 1, r.S, r.S, 0, 0, HO, HO};
     ++n;
-    if (pointwise_once(VH_F32, d, r.M) != (r.generic < r.copies)) {
-      printf("fp32 1x1 %ld -> %ld, %ld images of %ld: the slower path\n", r.K, r.M, r.B, r.H);
+    if (pointwise_once(VH_F32, d, r.M, true) != (r.generic < r.copies)) {
+      printf("fp32 1x1 %ld -> %ld, %ld images of %ld, stride %ld: the slower path\n", r.K, r.M, r.B, r.H, r.S);
       ++fails;
     }
   }

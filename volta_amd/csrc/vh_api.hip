@@ -381,26 +381,32 @@ static bool halo_f32_pays(const ConvDims& d, HaloPass pass, bool with_wgrad, boo
 
 // fp32 passes with a long K over few positions: the channels-last kernel, whose waves
 // alone split K, leaves CUs idle where the generic one splits it over blocks too.
-// Fitted to 175 layers of 9 .. 6400 positions (M rows, RS taps of C channels), us generic /
-// channels-last: 33 x 162, K 4131 18.7 / 35.4; 512 x 49, K 4608 33.7 / 47; 256 x 49, K 2304 21.9 /
-// 25.7; 60 x 1734, K 15700 103 / 112; 333 x 343, K 6489 63 / 57; 228 x 768, K 15450 157 / 112.
-// bf16: at most 12 % apart.
+// Fitted to 430 layers (M rows, RS taps of C channels), us generic / channels-last: 33 x
+// 162, K 4131 18.7 / 35.4; 512 x 49, K 4608 33.7 / 47; 256 x 49, K 2304 21.9 / 25.7; 60 x 1734,
+// K 15700 103 / 112; 333 x 343, K 6489 63 / 57; 228 x 768, K 15450 157 / 112.  Of few rows the
+// generic one also has a small weight matrix to lay out again: 16 x 784, K 2304 13.9 / 25;
+// 48 x 432, K 1728 16.5 / 20.7; 224 x 192, K 1600 22.6 / 21.3.  bf16: at most 12 % apart.
 static bool copies_pay(int dt, long M, long positions, long C, long RS) {
   const long stages = (RS * ((C + 3) / 4 * 4) + 31) / 32, blocks = ((M + 31) / 32) * ((positions + 31) / 32);
   return dt == VH_BF16 || blocks > 160 ||
-         (double)stages < 62 + 0.6 * (double)blocks + 3.6 * (double)std::max(0L, blocks - 100);
+         (double)stages < (M <= 32 ? 28 : M <= 64 ? 34 : 62) + 0.6 * (double)blocks + 3.6 * (double)std::max(0L, blocks - 100);
 }
 
-// fp32 1x1 layers of stride 1 read every value of the input once per row of tiles: with
-// one such row (M output rows) and more blocks than CUs a copy costs more than the gather.
-// 64 images of 56 x 56, us generic / channels-last: 256 -> 64 98 / 157, 64 -> 64 40 / 49, 64 ->
-// 16 39.4 / 36.9 (32 images 20.9 / 23.3); with two rows 64 -> 128 87 / 71; 12544 positions
-// 64 -> 64 11.2 / 11.4.  (The gradients of one call share the copy of the output gradient
-// and keep it: 64 -> 64 97 / 100 together, 64 -> 128 134 / 144, 128 -> 64 168 / 158.)
-static bool pointwise_once(int dt, const ConvDims& d, long M) {
-  const long positions = d.B * d.H * d.W;
-  return dt == VH_F32 && d.KH == 1 && d.KW == 1 && d.SH == 1 && d.SW == 1 && d.PH == 0 && d.PW == 0 && M <= 64 &&
-         positions > 16384 && (M > 32 || positions <= 131072);
+// fp32 1x1 layers read every value of the input at most once per row of tiles, where a copy
+// costs more than the gather that it replaces (us generic / channels-last):
+//  * stride 1, one such row (M output rows), more blocks than CUs.  64 images of 56 x 56:
+//    256 -> 64 98 / 157, 64 -> 64 40 / 49, 64 -> 16 39.4 / 36.9 (32 images 20.9 / 23.3); two rows
+//    64 -> 128 87 / 71; 12544 positions 64 -> 64 11.2 / 11.4.  (The gradients of one call
+//    share the copy of the output gradient and keep it: 64 -> 64 97 / 100 together, 64 -> 128
+//    134 / 144, 128 -> 64 168 / 158.)
+//  * strided forward: the copy holds the skipped values too.  16 images of 112 x 112, stride
+//    2: 256 -> 64 36.5 / 111, 512 -> 128 105 / 247, 256 -> 256 121 / 162, 128 -> 512 132 / 125; 6272
+//    outputs 256 -> 64 20.3 / 19.8.
+static bool pointwise_once(int dt, const ConvDims& d, long M, bool forward) {
+  if (dt != VH_F32 || d.KH != 1 || d.KW != 1 || d.PH != 0 || d.PW != 0) return false;
+  const long positions = d.B * d.HO * d.WO;
+  if (d.SH > 1 || d.SW > 1) return forward && M <= 256 && positions > 8192;
+  return M <= 64 && positions > 16384 && (M > 32 || positions <= 131072);
 }
 
 // act: 1 = ReLU on the output (fused into the epilogue where the kernel has it).
@@ -461,7 +467,7 @@ static int igemm_fwd(int dt, const void* x, const void* w, const void* bias, voi
                            (int)d.KW, (int)d.PH, (int)d.PW, st, act);
     if (r != VH_ERR_UNSUPPORTED) return r;
   }
-  if (g_fast_paths && (defer || !pointwise_once(dt, d, d.O)) && copies_pay(dt, d.O, d.B * d.HO * d.WO, d.C, RS)) {
+  if (g_fast_paths && (defer || !pointwise_once(dt, d, d.O, true)) && copies_pay(dt, d.O, d.B * d.HO * d.WO, d.C, RS)) {
     GatherCall gc{};
     GatherCall& c = defer ? *defer : gc;
     c.g = g;
@@ -661,7 +667,7 @@ static int igemm_dgrad(int dt, const void* dy, const void* w, void* dx, const Co
     int r = pw_conv_bf16_dgrad(dy, w, dx, (int)d.B, (int)d.C, (int)d.H, (int)d.W, (int)d.O, (int)d.SH, st);
     if (r != VH_ERR_UNSUPPORTED) return r == VH_OK && mask ? mask_after(dt, mask, dx, d.B * d.C * d.H * d.W, st) : r;
   }
-  if (g_fast_paths && (defer || !pointwise_once(dt, d, d.C)) &&
+  if (g_fast_paths && (defer || !pointwise_once(dt, d, d.C, false)) &&
       (d.SH > 1 || d.SW > 1 || copies_pay(dt, d.C, d.B * d.H * d.W, d.O, RS))) {
     GatherCall gc{};
     GatherCall& c = defer ? *defer : gc;
