@@ -181,3 +181,21 @@ def test_linear_gradients_together_and_alone(shape, bias):
     bound = 2.0 ** -24 * m * dy.double().abs().sum(0)
     assert bool(((db.double() - dy.double().sum(0)).abs() <= bound).all())
     assert bool(((db1.double() - dy.double().sum(0)).abs() <= bound).all())
+
+
+# dW deep beside a dX that fills the chip: two launches (fp32; whole tiles of either type), whose
+# outputs are those of separate calls
+@pytest.mark.parametrize("shape", [(20600, 260, 50), (16384, 512, 256)])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_linear_gradients_of_a_long_batch(shape, dt):
+    m, i, o = shape
+    torch.manual_seed(m + i + o)
+    lin = vnn.Linear(i, o, device=DEV, dtype=DTYPES[dt])
+    x, dy = (torch.randn(m, n, device=DEV).to(DTYPES[dt]) for n in (i, o))
+    dx, dw, db = (t.double().cpu() for t in lin.backward(dy, x))
+    x, dy, w = (t.double().cpu() for t in (x, dy, lin.weight))
+    u = 2.0 ** (-24 if dt == "f32" else -8)
+    for got, a, b in ((dx, dy, w.t()), (dw, x.t(), dy)):  # random signs: the error is far below k u S
+        ref, s, k = a @ b, a.abs() @ b.abs(), a.shape[1]
+        assert bool(((got - ref).abs() <= 2.0 ** -24 * k * s + u * ref.abs()).all())
+    assert bool(((db - dy.sum(0)).abs() <= 2.0 ** -24 * m * dy.abs().sum(0) + u * dy.sum(0).abs()).all())

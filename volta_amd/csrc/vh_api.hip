@@ -1667,19 +1667,31 @@ int vh_linear_forward(int dtype, const void* x, const void* weight, const void* 
 
 // Whether a Linear layer's dX and dW go in one launch: on the whole-tile pair kernels,
 // or where the pair's plan is the faster one.  A product of whole 256 x 256 tiles that
-// fill the chip keeps its own kernel, ahead of any pair of smaller ones.
+// fill the chip keeps its own kernel, ahead of any pair of smaller ones.  dW's blocks, few and
+// deep for a long batch, start behind dX's: where those fill the chip by themselves,
+// they would be a tail of one block's depth (fp32 50000 x 1000 -> 100 541 us in one
+// launch, 260 in two, 20000 x 300 -> 1024 246 and 257; whole tiles 16384 x 1024 -> 4096 2893
+// and 2009, 65536 x 256 -> 256 7950 and 176; bf16 small tiles 50000 x 1000 -> 100 93 either
+// way, 32768 x 256 -> 100 28 and 39).
 static bool linear_pair(int dt, const DenseProblem* p) {
   bool whole = true, large = false;
-  long tiles = 0;
+  long tiles[2];
+  double depth = 0;  // of a CU, evenly shared
   for (int i = 0; i < 2; ++i) {
     whole = whole && p[i].M % 128 == 0 && p[i].N % 256 == 0 && p[i].K % 128 == 0;
-    tiles += (p[i].M / 128L) * (p[i].N / 256L);
+    tiles[i] = (p[i].M / 128L) * (p[i].N / 256L);
+    depth += (double)tiles[i] * p[i].K / 256;
     large = large || (p[i].M % 256 == 0 && p[i].N % 256 == 0 && p[i].K % 128 == 0 &&
                       (p[i].M / 256L) * (p[i].N / 256L) >= 256);
   }
-  if (whole && tiles >= 256) return true;
+  if (whole && tiles[0] + tiles[1] >= 256) {
+    const double longest = tiles[0] + tiles[1] == 256 ? (double)std::max(p[0].K, p[1].K)
+                                                      : (double)tiles[0] / 256 * p[0].K + (double)((tiles[1] + 255) / 256) * p[1].K;
+    if (longest <= 1.25 * depth) return true;
+  }
   MmInfo pair, dx, dw;
   if (large || !mm_info(dt, p, 2, &pair)) return false;
+  if (dt == VH_F32 && (p[0].M + pair.bm - 1L) / pair.bm * ((p[0].N + pair.bn - 1L) / pair.bn) > pair.fit * 256L) return false;
   return !mm_info(dt, p, 1, &dx) || !mm_info(dt, p + 1, 1, &dw) || pair.us <= dx.us + dw.us + 2.f;
 }
 

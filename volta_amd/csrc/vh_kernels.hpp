@@ -238,7 +238,7 @@ int mm_run(int dt, const DenseProblem* p, int np, const void* bias, WsGet get, h
 // The plan of a call: tile, K splits and stages of each, workspace, the time it was
 // chosen by (us); false: unsupported.
 struct MmInfo {
-  int bm, bn, splits[2], per[2];
+  int bm, bn, fit, splits[2], per[2];  // fit: blocks a CU
   size_t bytes;
   float us;
 };

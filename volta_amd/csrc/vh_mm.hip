@@ -654,7 +654,7 @@ int mm_run_t(const DenseProblem* p, int np, const void* bias, WsGet get, hipStre
 bool mm_info(int dt, const DenseProblem* p, int np, MmInfo* o) {
   MmLayout l;
   if (!(dt == VH_BF16 ? mm_layout<bf16>(p, np, nullptr, l) : mm_layout<float>(p, np, nullptr, l))) return false;
-  *o = MmInfo{l.t.bm, l.t.bn, {l.g[0].splits, np > 1 ? l.g[1].splits : 0}, {l.g[0].per, np > 1 ? l.g[1].per : 0}, l.bytes, l.us};
+  *o = MmInfo{l.t.bm, l.t.bn, l.t.fit, {l.g[0].splits, np > 1 ? l.g[1].splits : 0}, {l.g[0].per, np > 1 ? l.g[1].per : 0}, l.bytes, l.us};
   return true;
 }
 
